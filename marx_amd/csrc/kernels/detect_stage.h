@@ -17,18 +17,11 @@
 
 namespace mxg {
 
-__device__ __forceinline__ vec3 rot (const double *m, vec3 v)
-{
-   return v3 (m[0] * v.x + m[1] * v.y + m[2] * v.z,
-              m[3] * v.x + m[4] * v.y + m[5] * v.z,
-              m[6] * v.x + m[7] * v.y + m[8] * v.z);
-}
-
 __device__ __forceinline__ vec3 rot_inv (const double *m, vec3 v)
 {
-   return v3 (m[0] * v.x + m[3] * v.y + m[6] * v.z,
-              m[1] * v.x + m[4] * v.y + m[7] * v.z,
-              m[2] * v.x + m[5] * v.y + m[8] * v.z);
+   return v3 (fma (m[6], v.z, fma (m[3], v.y, m[0] * v.x)),
+              fma (m[7], v.z, fma (m[4], v.y, m[1] * v.x)),
+              fma (m[8], v.z, fma (m[5], v.y, m[2] * v.x)));
 }
 
 // 1 inside, 0 outside (must_hit), -1 parallel; writes x/dx/dy unless 0
@@ -36,19 +29,19 @@ __device__ __forceinline__ int plane_hit (const mxg_chip &g, vec3 x0, vec3 p, ve
                                           double &dx, double &dy, bool must_hit)
 {
    vec3 normal = ld3 (g.normal);
-   double pdotn = dot (p, normal);
+   double pdotn = dot_f (p, normal);
    if (pdotn == 0) return -1;
    vec3 xll = ld3 (g.x_ll);
    vec3 r = sub (x0, xll);
-   r = ax1_bx2 (1.0, r, -1.0 * dot (r, normal) / pdotn, p);
+   r = along_f (r, -div_n (dot_f (r, normal), pdotn), p);
    int hit = 1;
-   double rx = dot (r, ld3 (g.xhat));
+   double rx = dot_f (r, ld3 (g.xhat));
    if ((rx < 0.0) || (rx >= g.xlen))
      {
         if (must_hit) return 0;
         hit = 0;
      }
-   double ry = dot (r, ld3 (g.yhat));
+   double ry = dot_f (r, ld3 (g.yhat));
    if ((ry < 0.0) || (ry >= g.ylen))
      {
         if (must_hit) return 0;
@@ -130,15 +123,15 @@ __device__ __forceinline__ int drake_hit (const mxg_detector_cfg &d, vec3 &x, ve
      {
         const mxg_rect &r = d.drake[k];
         vec3 nrm = ld3 (r.normal);
-        p_dot_n = dot (p, nrm);
+        p_dot_n = dot_f (p, nrm);
         if (p_dot_n == 0.0) continue;
         vec3 a = ld3 (r.a);
-        double t = dot (sub (a, old_x), nrm) / p_dot_n;
-        vec3 new_x = ax1_bx2 (1.0, old_x, t, p);
+        const double t = div_n (dot_f (sub (a, old_x), nrm), p_dot_n);
+        vec3 new_x = along_f (old_x, t, p);
         vec3 xp = sub (new_x, a);
-        double xx = dot (xp, ld3 (r.e1));
+        double xx = dot_f (xp, ld3 (r.e1));
         if ((xx < 0.0) || (xx >= r.len1)) continue;
-        double yy = dot (xp, ld3 (r.e2));
+        double yy = dot_f (xp, ld3 (r.e2));
         if ((yy < 0.0) || (yy >= r.len2)) continue;
         use_cr = (xx < d.drake_cr_width);
         x = new_x;
@@ -411,8 +404,8 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
              x.x -= d.offset[0];
              x.y -= d.offset[1];
              x.z -= d.offset[2];
-             x = rot (d.matrix, x);
-             p = rot (d.matrix, p);
+             x = mul_m3_f (d.matrix, x);
+             p = mul_m3_f (d.matrix, p);
              double dx = 0.0, dy = 0.0;
              int k = find_chip (d, x, p, dx, dy);
              if (k < 0)
@@ -424,8 +417,8 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
                {
                   const mxg_chip &g = d.chip[k];
                   s.ccd[id] = (int8_t) g.id;
-                  float ypix = (float) (dx / g.x_pixel_size);
-                  float zpix = (float) (dy / g.y_pixel_size);
+                  float ypix = (float) div_n (dx, g.x_pixel_size);
+                  float zpix = (float) div_n (dy, g.y_pixel_size);
                   bool detected = true;
                   if (d.ideal == 0)
                     {
@@ -496,7 +489,7 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
                        const mxg_qe_table *fq;
                        if (is_hrc_s)
                          {
-                            double t = (d.shield_x - x.x) / p.x;
+                            double t = div_n (d.shield_x - x.x, p.x);
                             region = filter_region (d, x.y + t * p.y, x.z + t * p.z);
                             if (region < 0) ok = false;
                             fq = d.filter_qe + (region < 0 ? 0 : region);
@@ -525,14 +518,14 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
                               {
                                  double c;
                                  do c = uniform (st); while (c == 0.0);
-                                 rr = d.g1_sigma * sqrt (-2 * log (c));
+                                 rr = d.g1_sigma * sqrt_n (-2.0 * log_n (c));
                                  x_0 = d.g1_xctr; y_0 = d.g1_yctr;
                               }
                             else if (r < d.g1_wgt + d.g2_wgt)
                               {
                                  double c;
                                  do c = uniform (st); while (c == 0.0);
-                                 rr = d.g2_sigma * sqrt (-2 * log (c));
+                                 rr = d.g2_sigma * sqrt_n (-2.0 * log_n (c));
                                  x_0 = d.g2_xctr; y_0 = d.g2_yctr;
                               }
                             else
@@ -542,9 +535,8 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
                                  rr = d.l1_hwhm * sqrt (expm1 (c * log1p (rmax * rmax)));
                                  x_0 = d.l1_xctr; y_0 = d.l1_yctr;
                               }
-                            double theta = (2.0 * MXG_PI) * uniform (st);
                             double sn, cs;
-                            sincos (theta, &sn, &cs);
+                            sincos_turn (uniform (st), sn, cs);
                             dx += x_0 + rr * cs;
                             dy += y_0 + rr * sn;
                             if (d.extend == 0)
@@ -558,8 +550,8 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
                          {
                             const int cid = g.id;
                             double u = d.pix_u[cid], v = d.pix_v[cid];
-                            u += dx / d.u_pixel_size;
-                            v += dy / d.v_pixel_size;
+                            u += div_n (dx, d.u_pixel_size);
+                            v += div_n (dy, d.v_pixel_size);
                             s.upix[id] = (float) u;
                             s.vpix[id] = (float) v;
                             s.ypix[id] = (float) (d.pix_x0[cid] + (u - d.pix_u0[cid]));
@@ -567,8 +559,8 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
                          }
                        else
                          {
-                            s.ypix[id] = (float) (d.pix_x0[0] + dx / d.u_pixel_size);
-                            s.zpix[id] = (float) (d.pix_y0[0] + dy / d.v_pixel_size);
+                            s.ypix[id] = (float) (d.pix_x0[0] + div_n (dx, d.u_pixel_size));
+                            s.zpix[id] = (float) (d.pix_y0[0] + div_n (dy, d.v_pixel_size));
                          }
                     }
                }

@@ -1,11 +1,12 @@
 // dev_common.h -- per-photon device primitives for gfx950.
 //
-// Everything here runs in one lane per photon.  Arithmetic that feeds
-// positions, directions and threshold tests is written in the operation
-// order of the reference's jdmath routines (jdmath/src/vector.c,
-// finterpo.c, dinterpo.c, qroot.c, complex.c) and the file is compiled with
-// -ffp-contract=off, so a lane rounds exactly like the reference's CPU code
-// apart from the last-bit differences of the transcendental functions.
+// Everything here runs in one lane per photon.  The file is compiled with
+// -ffp-contract=off; the stages' vectors, roots and rotations use the
+// explicit fused multiply-adds and the primitives of dev_math.h, so a
+// function rounds alike in every kernel it is part of, and apart from the
+// reference's arithmetic (jdmath/src/vector.c, qroot.c, complex.c) in the
+// last bits only.  Energies, table interpolations (finterpo.c, dinterpo.c)
+// and arrival times keep the reference's operation order and values.
 //
 // Random numbers: one Philox4x32-10 counter stream per (photon tag, stage):
 // key = seed, counter = (tag, stage, block, source id); 4 uniforms per
@@ -16,13 +17,12 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "marx_gpu_cfg.h"
+#include "dev_math.h"
 
 #define MXG_PI 3.14159265358979323846264338327950288
 #define MXG_HBAR_C 1.973269631e-4
 
 namespace mxg {
-
-struct vec3 { double x, y, z; };
 
 __device__ __forceinline__ vec3 v3 (double x, double y, double z) { vec3 a; a.x = x; a.y = y; a.z = z; return a; }
 
@@ -44,7 +44,8 @@ struct Stream
 
 // Philox4x32-10 (Salmon et al., SC'11).  Each round's two 32x32->64-bit
 // products are formed as one 64-bit multiply (v_mad_u64_u32), half the
-// multiply issue of separate low and high products.
+// multiply issue of separate low and high products, and its three-way
+// exclusive ors are one instruction (v_bitop3_b32).
 __device__ __forceinline__ void philox (uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                         uint32_t k0, uint32_t k1,
                                         uint32_t &o0, uint32_t &o1, uint32_t &o2, uint32_t &o3)
@@ -55,8 +56,8 @@ __device__ __forceinline__ void philox (uint32_t c0, uint32_t c1, uint32_t c2, u
         if (r > 0) { k0 += 0x9E3779B9u; k1 += 0xBB67AE85u; }
         uint64_t p0 = (uint64_t) 0xD2511F53u * c0;
         uint64_t p1 = (uint64_t) 0xCD9E8D57u * c2;
-        uint32_t n0 = (uint32_t) (p1 >> 32) ^ c1 ^ k0;
-        uint32_t n2 = (uint32_t) (p0 >> 32) ^ c3 ^ k1;
+        uint32_t n0 = xor3 ((uint32_t) (p1 >> 32), c1, k0);
+        uint32_t n2 = xor3 ((uint32_t) (p0 >> 32), c3, k1);
         c0 = n0; c1 = (uint32_t) p1; c2 = n2; c3 = (uint32_t) p0;
      }
    o0 = c0; o1 = c1; o2 = c2; o3 = c3;
@@ -105,7 +106,9 @@ __device__ __forceinline__ double gaussian (Stream &s)
         g = g1 * g1 + g2 * g2;
      }
    while ((g >= 1.0) || (g == 0.0));
-   double f = sqrt (-2.0 * log (g) / g);
+   // sqrt (l / g) as l / sqrt (l g): 0 < g < 1, so l > 0
+   const double l = -2.0 * log_n (g);
+   const double f = l * rsqrt_n (l * g);
    s.g2 = g2 * f;
    return g1 * f;
 }
@@ -152,26 +155,6 @@ __device__ __forceinline__ float interp_f (float x, const float *__restrict__ xp
    float y0 = yp[n0];
    float dy = yp[n1] - y0;
    return (float) ((double) y0 + (double) dy / (x1 - x0) * ((double) x - x0));
-}
-
-// interp_f of two tables on one abscissa with one search (the same values)
-__device__ __forceinline__ void interp_f2 (float x, const float *__restrict__ xp, const float *__restrict__ ya,
-                                           const float *__restrict__ yb, unsigned int n, float &a, float &b)
-{
-   if (n == 1) { a = ya[0]; b = yb[0]; return; }
-   unsigned int n1 = search_f (x, xp, n);
-   unsigned int n0 = n1 - 1;
-   if ((n1 < n) && (x == xp[n1])) { a = ya[n1]; b = yb[n1]; return; }
-   if (n1 == n) { n1--; n0--; }
-   if (n1 == 0) n0 = 1;
-   double x0 = xp[n0], x1 = xp[n1];
-   if (x1 == x0) { a = ya[n1]; b = yb[n1]; return; }
-   float y0 = ya[n0];
-   float dy = ya[n1] - y0;
-   a = (float) ((double) y0 + (double) dy / (x1 - x0) * ((double) x - x0));
-   y0 = yb[n0];
-   dy = yb[n1] - y0;
-   b = (float) ((double) y0 + (double) dy / (x1 - x0) * ((double) x - x0));
 }
 
 __device__ __forceinline__ unsigned int search_d (double x, const double *__restrict__ xp, unsigned int n)
@@ -286,7 +269,7 @@ __device__ __forceinline__ float interp_fb (float x, const float *__restrict__ x
    if (x1 == x0) return yp[n1];
    float y0 = yp[n0];
    float dy = yp[n1] - y0;
-   return (float) ((double) y0 + (double) dy / (x1 - x0) * ((double) x - x0));
+   return (float) ((double) y0 + div_n ((double) dy, x1 - x0) * ((double) x - x0));
 }
 
 __device__ __forceinline__ void interp_f2b (float x, const float *__restrict__ xp, const float *__restrict__ ya,
@@ -301,12 +284,13 @@ __device__ __forceinline__ void interp_f2b (float x, const float *__restrict__ x
    if (n1 == 0) n0 = 1;
    double x0 = xp[n0], x1 = xp[n1];
    if (x1 == x0) { a = ya[n1]; b = yb[n1]; return; }
+   const double dx = x1 - x0, r = rcp_n (dx);
    float y0 = ya[n0];
    float dy = ya[n1] - y0;
-   a = (float) ((double) y0 + (double) dy / (x1 - x0) * ((double) x - x0));
+   a = (float) ((double) y0 + div_r ((double) dy, dx, r) * ((double) x - x0));
    y0 = yb[n0];
    dy = yb[n1] - y0;
-   b = (float) ((double) y0 + (double) dy / (x1 - x0) * ((double) x - x0));
+   b = (float) ((double) y0 + div_r ((double) dy, dx, r) * ((double) x - x0));
 }
 
 // search_d over a strictly increasing table with the linear bucket index b
@@ -339,7 +323,7 @@ __device__ __forceinline__ double interp_d_at (double x, const double *__restric
    if (n1 == 0) n0 = 1;
    double x0 = xp[n0], x1 = xp[n1];
    if (x1 == x0) return yp[n1];
-   return yp[n0] + (yp[n1] - yp[n0]) / (x1 - x0) * (x - x0);
+   return yp[n0] + div_n (yp[n1] - yp[n0], x1 - x0) * (x - x0);
 }
 
 __device__ __forceinline__ double interp_d (double x, const double *__restrict__ xp,
@@ -347,30 +331,6 @@ __device__ __forceinline__ double interp_d (double x, const double *__restrict__
 {
    if (n == 1) return yp[0];
    return interp_d_at (x, xp, yp, n, search_d (x, xp, n));
-}
-
-// numerically stable roots; returns 1 real, 0 complex, -1 if a == 0
-__device__ __forceinline__ int quadratic_root (double a, double b, double c, double &rplus, double &rminus)
-{
-   if (a == 0.0) return -1;
-   double bsqr = b * b;
-   double ac4 = a * c * 4;
-   double neg_b_over_2a = -b / (2.0 * a);
-   if (bsqr > ac4)
-     {
-        double factor = 1.0 + sqrt (1.0 - ac4 / bsqr);
-        rplus = -2.0 * c / (b * factor);
-        rminus = neg_b_over_2a * factor;
-        return 1;
-     }
-   if (bsqr == ac4)
-     {
-        rplus = rminus = neg_b_over_2a;
-        return 1;
-     }
-   rplus = neg_b_over_2a;
-   rminus = sqrt (c / a) * sqrt (1.0 - bsqr / ac4);
-   return 0;
 }
 
 // ---- vectors -------------------------------------------------------------------
@@ -438,41 +398,22 @@ __device__ __forceinline__ vec3 rotate_vector1 (vec3 p, vec3 n, double c, double
    return ax1_bx2_cx3 (c, p, pn * (1.0 - c), n, s, cross (n, p));
 }
 
-__device__ __forceinline__ vec3 rotate_unit_vector1 (vec3 p, vec3 n, double c, double s)
-{
-   vec3 u = rotate_vector1 (p, n, c, s);
-   normalize (u);
-   return u;
-}
-
 // sin and cos of t; below 2^-6 rad (the arcsecond-to-arcminute angles of
 // the mirror blur, WFold scatter and dither offsets) from their Taylor
 // polynomials through t^7 and t^8 (truncation below 1e-20 relative: the
-// result differs from sincos's by rounding only), else sincos.
+// result differs from sincos's by rounding only), else sincos_r.
 __device__ __forceinline__ void sincos_small (double t, double *sn, double *cs)
 {
    if (fabs (t) < 0.015625)
      {
         const double t2 = t * t;
-        *sn = t * (1.0 - t2 * (1.0 / 6.0 - t2 * (1.0 / 120.0 - t2 * (1.0 / 5040.0))));
-        *cs = 1.0 - t2 * (0.5 - t2 * (1.0 / 24.0 - t2 * (1.0 / 720.0 - t2 * (1.0 / 40320.0))));
+        const double a = fma (t2, fma (t2, 1.0 / 5040.0, -1.0 / 120.0), 1.0 / 6.0);
+        *sn = fma (-t2 * a, t, t);
+        const double b = fma (t2, fma (t2, fma (t2, 1.0 / 40320.0, -1.0 / 720.0), 1.0 / 24.0), -0.5);
+        *cs = fma (t2, b, 1.0);
      }
    else
-     sincos (t, sn, cs);
-}
-
-__device__ __forceinline__ vec3 rotate_unit_vector (vec3 p, vec3 n, double theta)
-{
-   double s, c;
-   sincos (theta, &s, &c);
-   return rotate_unit_vector1 (p, n, c, s);
-}
-
-__device__ __forceinline__ vec3 m3_vmul (const double *__restrict__ a, vec3 v)
-{
-   return v3 (a[0] * v.x + a[1] * v.y + a[2] * v.z,
-              a[3] * v.x + a[4] * v.y + a[5] * v.z,
-              a[6] * v.x + a[7] * v.y + a[8] * v.z);
+     sincos_r (t, *sn, *cs);
 }
 
 __device__ __forceinline__ vec3 ld3 (const double *a) { return v3 (a[0], a[1], a[2]); }
@@ -548,7 +489,7 @@ __device__ __forceinline__ double fold_theta (const double *__restrict__ fa, con
    if (p > p_max) return pow (fa[4] * (1.0 - p), fa[5]);
    unsigned int num = (unsigned int) fa[6];
    const float *t = farena + (unsigned int) fa[7];
-   double delta_i = (p - p_min) / fa[2];
+   double delta_i = div_n (p - p_min, fa[2]);
    unsigned int i = (unsigned int) delta_i;
    if (i + 1 >= num) return (double) t[num - 1];
    delta_i -= (double) i;
@@ -582,35 +523,37 @@ __device__ __forceinline__ double wfold_interp (const mxg_wfold &w, const float 
    double theta_0 = fold_theta (arrays + (i - 1) * MXG_FOLD_STRIDE, fa, r);
    double theta_1 = fold_theta (arrays + i * MXG_FOLD_STRIDE, fa, r);
    double e0 = (double) e_alphas[i - 1], e1 = (double) e_alphas[i];
-   return theta_0 + (theta_1 - theta_0) * (e_alpha - e0) / (e1 - e0);
+   return theta_0 + div_n ((theta_1 - theta_0) * (e_alpha - e0), e1 - e0);
 }
 
 // ---- shared by the mirror and source kernels --------------------------------------
 
-// precollimator / cap / post-collimator strut shadows (hrma.c:900-981)
-__device__ __forceinline__ bool in_strut_shadow (const mxg_hrma_cfg &h, vec3 x, vec3 p,
+// precollimator / cap / post-collimator strut shadows (hrma.c:900-981);
+// ipx: rcp_n (p.x)
+__device__ __forceinline__ bool in_strut_shadow (const mxg_hrma_cfg &h, vec3 x, vec3 p, double ipx,
                                                  const mxg_strut *s)
 {
    const double cos_theta = h.strut_cos, sin_theta = h.strut_sin;
+   bool hit = false;
    for (int k = 0; k < 2; k++)
      {
-        double half_width = s[k].half_width;
-        double t = (s[k].xpos + h.cap_position - x.x) / p.x;
-        double y = x.y + p.y * t;
-        double z = x.z + p.z * t;
+        const double half_width = s[k].half_width;
+        const double t = div_r (s[k].xpos + h.cap_position - x.x, p.x, ipx);
+        double y = fma (p.y, t, x.y);
+        double z = fma (p.z, t, x.z);
         for (int i = 0; i < 3; i++)
           {
              if (i != 0)
                {
-                  double tmp = cos_theta * y - sin_theta * z;
-                  z = sin_theta * y + cos_theta * z;
+                  const double tmp = fma (cos_theta, y, -(sin_theta * z));
+                  z = fma (sin_theta, y, cos_theta * z);
                   y = tmp;
                }
-             if (((-half_width < y) && (y < half_width)) || ((-half_width < z) && (z < half_width)))
-               return true;
+             // no early return: lanes of a wave leave at different bands
+             hit |= (fabs (y) < half_width) | (fabs (z) < half_width);
           }
      }
-   return false;
+   return hit;
 }
 
 // energy of the FLAT or FILE spectrum (spectrum.c:138-147, 184-189); one

@@ -557,7 +557,7 @@ __device__ __forceinline__ bool diff_enter (const mxg_hrma_cfg &h, const mxg_sou
         p = dax1_bx2 (dc<N> (1.0), x, dc<N> (src.distance), p);
         dnormalize (p);
      }
-   if (h.use_struts && in_strut_shadow (h, val (x), val (p), h.pre_struts))
+   if (h.use_struts && in_strut_shadow (h, val (x), val (p), rcp_n (p.x.v), h.pre_struts))
      return false;
    x = dadd (x, ph.t0);
    x = dm3_vmul (D.fwd[0], D.dfwd[0], x);
@@ -672,7 +672,7 @@ void k_diff_forward (const mxg_config *__restrict__ cfg, const float *__restrict
              p = dm3_vmul (D.bwd[k], D.dbwd[k], p);
              x = dm3_vmul (D.bwd[k], D.dbwd[k], x);
              x = dsub (x, (k == 0) ? ph.t0 : ph.t1);
-             if (h.use_struts && in_strut_shadow (h, val (x), val (p), (k == 0) ? h.cap_struts : h.post_struts))
+             if (h.use_struts && in_strut_shadow (h, val (x), val (p), rcp_n (p.x.v), (k == 0) ? h.cap_struts : h.post_struts))
                alive = false;
           }
 

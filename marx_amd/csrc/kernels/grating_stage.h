@@ -18,54 +18,48 @@
 
 namespace mxg {
 
-// rotation about x by the angle of cosine c and sine s
-__device__ __forceinline__ vec3 rotate_x (vec3 a, double c, double s)
+// The root of the quartic t^4 + a t^3 + b t^2 + c t + d by Newton's method
+// from t0, as the reference takes it (at most ten steps, to 1e-4 between
+// the last two: the root is then good to the square of that over its size).
+__device__ __forceinline__ bool newtons_quartic (double a, double b, double c, double d, double t0, double &tp)
 {
-   double ay = a.y, az = a.z;
-   a.y = c * ay - s * az;
-   a.z = s * ay + c * az;
-   return a;
-}
-
-__device__ __forceinline__ int newtons_quartic (double a, double b, double c, double d, double t0,
-                                                double &tp)
-{
-   unsigned int max_it = 10;
-   double a2 = 2.0 * a, a3 = 3.0 * a, b2 = 2.0 * b, t;
-   while (true)
+   const double a2 = 2.0 * a, a3 = 3.0 * a, b2 = 2.0 * b;
+   for (int it = 0; it < 10; it++)
      {
-        double t2 = t0 * t0;
-        double num = t2 * (3.0 * t2 + a2 * t0 + b) - d;
-        double den = t2 * (4.0 * t0 + a3) + b2 * t0 + c;
-        t = num / den;
-        if (fabs (t - t0) < 1.0e-4) break;
-        max_it--;
-        if (max_it == 0) return -1;
+        const double t2 = t0 * t0;
+        const double num = fma (t2, fma (3.0, t2, fma (a2, t0, b)), -d);
+        const double den = fma (t2, fma (4.0, t0, a3), fma (b2, t0, c));
+        const double t = div_n (num, den);
+        if (fabs (t - t0) < 1.0e-4)
+          {
+             tp = t;
+             return true;
+          }
         t0 = t;
      }
-   tp = t;
-   return 0;
+   return false;
 }
 
-__device__ __forceinline__ int torus_intersect (vec3 &x0, vec3 p, double rowland)
+// the hit of a ray on the Rowland torus (diffract.c:622-687)
+__device__ __forceinline__ bool torus_intersect (vec3 &x0, vec3 p, double rowland)
 {
-   double t = -x0.x / p.x;
+   const double t = -div_n (x0.x, p.x);
    x0.x = 0.0;
-   x0.y = x0.y + p.y * t;
-   x0.z = x0.z + p.z * t;
-   double pxpz_len = p.x * p.x + p.z * p.z;
-   double x2 = x0.z * x0.z + x0.y * x0.y;
-   double r2 = rowland * rowland;
-   double pdotx = dot (p, x0);
-   double a = 4.0 * pdotx;
-   double b = 2.0 * x2 + a * pdotx - r2 * pxpz_len;
-   double c = a * x2 - 2.0 * r2 * p.z * x0.z;
-   double d = x2 * x2 - r2 * x0.z * x0.z;
-   double t0 = -rowland * sqrt (pxpz_len);
-   if (-1 == newtons_quartic (a, b, c, d, t0, t))
-     return -1;
-   x0 = ax1_bx2 (1.0, x0, t, p);
-   return 0;
+   x0.y = fma (p.y, t, x0.y);
+   x0.z = fma (p.z, t, x0.z);
+   const double pxpz = fma (p.x, p.x, p.z * p.z);
+   const double x2 = fma (x0.z, x0.z, x0.y * x0.y);
+   const double r2 = rowland * rowland;
+   const double a = 4.0 * fma (p.z, x0.z, p.y * x0.y);
+   const double pdotx = 0.25 * a;
+   const double b = fma (2.0, x2, fma (a, pdotx, -(r2 * pxpz)));
+   const double c = fma (a, x2, -2.0 * r2 * p.z * x0.z);
+   const double d = fma (x2, x2, -(r2 * x0.z * x0.z));
+   double root;
+   if (!newtons_quartic (a, b, c, d, -rowland * sqrt_n (pxpz), root))
+     return false;
+   x0 = along_f (x0, root, p);
+   return true;
 }
 
 // Order draw: first k with r <= cumulative efficiency(E); -1 when none.
@@ -140,7 +134,7 @@ __device__ __forceinline__ int draw_order (const mxg_grating &g, const float *__
         else
           {
              double a = ya, b = yb;
-             v = (float) (a + (b - a) * (e - x_0) / dx_10);
+             v = (float) (a + div_n ((b - a) * (e - x_0), dx_10));
           }
         if (r <= (double) v)
           return (int) k;
@@ -154,12 +148,14 @@ __device__ __forceinline__ int diffract_photon (const mxg_grating &g, unsigned i
                                                 double theta, double energy, vec3 x, vec3 &p, int order,
                                                 Stream &st)
 {
-   double n_lambda_over_d = (double) order * (2.0 * MXG_PI * MXG_HBAR_C) / g.period / energy;
-   vec3 n = unit (x);
+   const double n_lambda_over_d = div_n ((double) order * (2.0 * MXG_PI * MXG_HBAR_C), g.period * energy);
+   // the facet's normal -x / |x|, and the directions along (l, in the x-z
+   // plane) and across (d) its grooves: n . l = 0, so d has length 1
+   vec3 n = unit_f (x);
    n.x = -n.x; n.y = -n.y; n.z = -n.z;
-   vec3 l = v3 (n.z, 0.0, -n.x);
-   l = unit (l);
-   vec3 d = cross (n, l);
+   const double il = rsqrt_n (fma (n.x, n.x, n.z * n.z));
+   vec3 l = v3 (n.z * il, 0.0, -n.x * il);
+   vec3 d = cross_f (n, l);
    double dtheta, dp_over_p;
 
    if (nsec > 0)
@@ -185,26 +181,23 @@ __device__ __forceinline__ int diffract_photon (const mxg_grating &g, unsigned i
    if (theta != 0.0)
      {
         double s, c;
-        sincos (theta, &s, &c);
-        vec3 l_tmp = l, d_tmp = d;
-        l = ax1_bx2 (c, l_tmp, s, d_tmp);
-        d = ax1_bx2 (-s, l_tmp, c, d_tmp);
+        sincos_small (theta, &s, &c);
+        const vec3 l_tmp = l, d_tmp = d;
+        l = lin2_f (c, l_tmp, s, d_tmp);
+        d = lin2_f (-s, l_tmp, c, d_tmp);
      }
 
-   double p_d = n_lambda_over_d + dot (p, d);
-   double p_l = dot (p, l);
-   double p_n = 1.0 - p_l * p_l - p_d * p_d;
-   if (p_n < 0.0) return -1;
-   p_n = sqrt (p_n);
-   vec3 q = ax1_bx2 (p_d, d, p_n, n);
-   p = ax1_bx2 (1.0, q, p_l, l);
+   const double p_d = n_lambda_over_d + dot_f (p, d);
+   const double p_l = dot_f (p, l);
+   const double pn2 = fma (-p_d, p_d, fma (-p_l, p_l, 1.0));
+   if (pn2 < 0.0) return -1;
+   double ipn;
+   const double p_n = sqrt_rsqrt_n (fmax (pn2, 1e-300), ipn);
+   p = along_f (lin2_f (p_d, d, p_n, n), p_l, l);
    if (dp_over_p == 0) return 0;
-   double factor = n_lambda_over_d * dp_over_p;
-   vec3 dp = ax1_bx2 (-factor, d, factor * (p_d / p_n), n);
-   p.x += dp.x;
-   p.y += dp.y;
-   p.z += dp.z;
-   p = unit (p);
+   // dp = -f d + f (p_d / p_n) n
+   const double f = n_lambda_over_d * dp_over_p;
+   p = unit_f (along_f (along_f (p, -f, d), f * (p_d * ipn), n));
    return 0;
 }
 
@@ -379,9 +372,9 @@ __device__ __forceinline__ bool grating_one (const mxg_grating_cfg &gc, const fl
              const double ef = (double) (float) energy;
              int8_t order = s.order[id];
 
-             x = rotate_x (x, g.disp_cos, -g.disp_sin);
-             p = rotate_x (p, g.disp_cos, -g.disp_sin);
-             if (-1 == torus_intersect (x, p, gc.rowland[shell]))
+             x = turn_x_f (x, g.disp_cos, -g.disp_sin);
+             p = turn_x_f (p, g.disp_cos, -g.disp_sin);
+             if (!torus_intersect (x, p, gc.rowland[shell]))
                flags |= PHOTON_UNDIFFRACTED;
              if (-1 == diffract_from (g, grating_tabs<STAGED> (gc, shell, fa, da, L, ltab), fa, 0.0, energy,
                                       ef, x, p, order, st))
@@ -408,8 +401,8 @@ __device__ __forceinline__ bool grating_one (const mxg_grating_cfg &gc, const fl
                     }
                }
 
-             x = rotate_x (x, g.disp_cos, g.disp_sin);
-             p = rotate_x (p, g.disp_cos, g.disp_sin);
+             x = turn_x_f (x, g.disp_cos, g.disp_sin);
+             p = turn_x_f (p, g.disp_cos, g.disp_sin);
              keep = (flags & BAD_PHOTON_MASK) == 0;
              if (!(HANDOFF && keep))
                {

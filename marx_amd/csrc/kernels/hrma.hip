@@ -28,7 +28,7 @@ __global__ __launch_bounds__ (kBlock, MXG_ENTER_WAVES)
 __global__ __launch_bounds__ (kBlock)
 #endif
 void k_hrma_enter (const mxg_config *__restrict__ cfg, Soa s, ListIO io,
-                   uint32_t *__restrict__ rng_pos, double source_distance,
+                   uint32_t *__restrict__ rng_pos, uint32_t tilted, double source_distance,
                    unsigned long long seed, uint32_t source_id)
 {
    __shared__ __align__ (16) unsigned char lds[sizeof (mxg_hrma_cfg)];
@@ -47,7 +47,7 @@ void k_hrma_enter (const mxg_config *__restrict__ cfg, Soa s, ListIO io,
         if (i < range.hi)
           {
              id = io.idx_in[i];
-             keep = hrma_enter_one<FRESH> (h, s, id, rng_pos, source_distance, seed, source_id);
+             keep = hrma_enter_one<FRESH> (h, tilted, s, id, rng_pos, source_distance, seed, source_id);
           }
         survivors.add (keep, id);
      }
@@ -140,10 +140,10 @@ hipError_t launch_hrma (const mxg_config *cfg, const mxg_config *hcfg, const flo
    if (e != hipSuccess) return e;
    if (fresh)
      hipLaunchKernelGGL (k_hrma_enter<true>, dim3 (a.grid), dim3 (kBlock), 0, st, cfg, s, a, hs.rng_pos,
-                         source_distance, seed, source_id);
+                         lay.tilted, source_distance, seed, source_id);
    else
      hipLaunchKernelGGL (k_hrma_enter<false>, dim3 (a.grid), dim3 (kBlock), 0, st, cfg, s, a, hs.rng_pos,
-                         source_distance, seed, source_id);
+                         lay.tilted, source_distance, seed, source_id);
    e = hipGetLastError ();
    if ((e == hipSuccess) && ev) e = hipEventRecord (ev[1], st);
    if (e == hipSuccess) e = launch_compact (a, st);

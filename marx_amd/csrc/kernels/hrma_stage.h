@@ -26,83 +26,116 @@
 namespace mxg {
 
 // The hit of a ray on the quadric x^2+y^2+z^2 = a x^2 + b x + c between
-// xmin <= x < xmax (the larger valid root in x).  On success x0 becomes the
-// hit; on a miss x0 is unchanged and -1 is returned.
-__device__ __forceinline__ int conic_intersection (double a, double b, double c, vec3 &x0, vec3 p,
-                                                   double xmin, double xmax)
+// xmin <= x < xmax (the larger valid root in x); ipx = rcp_n (p.x).  On
+// success x0 becomes the hit; on a miss x0 is unchanged and false is
+// returned.  The second root, -q / (2 alpha) of alpha t^2 + beta t + gamma,
+// is formed only where it can lie between the limits: alpha is of the order
+// of the squared angle to the axis, so it hardly ever does.
+__device__ __forceinline__ bool conic_hit (double a, double b, double c, vec3 &x0, vec3 p, double ipx,
+                                           double xmin, double xmax)
 {
-   double t_plus = -x0.x / p.x;
-   double x_y = x0.y + t_plus * p.y;
-   double x_z = x0.z + t_plus * p.z;
-   double alpha = a * p.x * p.x - 1.0;
-   double beta = b * p.x - 2.0 * (p.y * x_y + p.z * x_z);
-   double gamma = c - x_z * x_z - x_y * x_y;
-   double t_minus;
+   const double t0 = div_r (-x0.x, p.x, ipx);
+   const double x_y = fma (t0, p.y, x0.y);
+   const double x_z = fma (t0, p.z, x0.z);
+   const double alpha = fma (a * p.x, p.x, -1.0);
+   const double beta = fma (b, p.x, -2.0 * fma (p.y, x_y, p.z * x_z));
+   const double gamma = fma (-x_y, x_y, fma (-x_z, x_z, c));
+   double t_plus, t_minus;
+   bool minus_ok = false;
 
    if (alpha == 0.0)
      {
-        if (beta == 0.0) return -1;
-        t_plus = t_minus = -gamma / beta;
+        if (beta == 0.0) return false;
+        t_plus = t_minus = -div_n (gamma, beta);
      }
-   else if (0 >= quadratic_root (alpha, beta, gamma, t_plus, t_minus))
-     return -1;
-
-   double x_plus = p.x * t_plus;
-   double x_minus = p.x * t_minus;
-   bool plus_ok = (x_plus >= xmin) && (x_plus < xmax);
-   bool minus_ok = (x_minus >= xmin) && (x_minus < xmax);
-   double t;
-   if (plus_ok)
-     t = (minus_ok && (x_minus > x_plus)) ? t_minus : t_plus;
-   else if (minus_ok)
-     t = t_minus;
    else
-     return -1;
+     {
+        const double disc = fma (beta, beta, -4.0 * alpha * gamma);
+        if (!(disc >= 0.0)) return false;
+        const double q = beta + copysign (sqrt_n (disc), beta);
+        t_plus = -2.0 * div_n (gamma, q);
+        t_minus = t_plus;
+        if (fabs (p.x * q) <= 2.0001 * fmax (fabs (xmin), fabs (xmax)) * fabs (alpha))
+          {
+             t_minus = -0.5 * div_n (q, alpha);
+             const double x_minus = p.x * t_minus;
+             minus_ok = (x_minus >= xmin) && (x_minus < xmax);
+          }
+     }
 
+   const double x_plus = p.x * t_plus;
+   const bool plus_ok = (x_plus >= xmin) && (x_plus < xmax);
+   if (!(plus_ok || minus_ok)) return false;
+   const double t = (minus_ok && !(plus_ok && (x_plus >= p.x * t_minus))) ? t_minus : t_plus;
    x0.x = p.x * t;
-   x0.y = x_y + p.y * t;
-   x0.z = x_z + p.z * t;
-   return 0;
+   x0.y = fma (p.y, t, x_y);
+   x0.z = fma (p.z, t, x_z);
+   return true;
 }
 
 // inward unit normal of the quadric at a point on it (hrma.c:470-476)
 __device__ __forceinline__ vec3 conic_normal (double a, double b, vec3 x)
 {
-   vec3 n;
-   n.x = (a - 1) * x.x + 0.5 * b;
-   n.y = -x.y;
-   n.z = -x.z;
-   normalize (n);
-   return n;
+   return unit_f (v3 (fma (a - 1.0, x.x, 0.5 * b), -x.y, -x.z));
 }
 
-// The rotation of rotate_unit_vector, for the small angles of the normal
-// blur and the WFold scatter (see sincos_small).
-__device__ __forceinline__ vec3 rotate_small (vec3 p, vec3 n, double t)
-{
-   double sn, cs;
-   sincos_small (t, &sn, &cs);
-   return rotate_unit_vector1 (p, n, cs, sn);
-}
-
+// The normal n turned by a Gaussian angle about a random direction u in the
+// surface (hrma.c:1054-1093).  u is (0, n_z, -n_y) / |(n_y, n_z)| turned
+// about n by a uniform azimuth; the two are at right angles, and u and n are,
+// so the rotations have no component along their axes, and they keep the
+// length 1 to rounding.
 __device__ __forceinline__ void blur_normal (vec3 &n, double blur, Stream &st)
 {
-   double n_y = n.y, n_z = n.z;
-   double len = sqrt (n_y * n_y + n_z * n_z);
-   vec3 perp = v3 (0.0, n_z / len, -n_y / len);
-   double phi = (2.0 * MXG_PI) * uniform (st);
-   perp = rotate_unit_vector (perp, n, phi);
-   phi = blur * (1.0 / 3600.0 * MXG_PI / 180.0);
+   const double n2 = fma (n.y, n.y, n.z * n.z);
+   const double il = rsqrt_n (n2);
+   double s, c;
+   sincos_turn (uniform (st), s, c);
+   const double cl = c * il, sl = s * il, sx = sl * n.x;
+   const vec3 u = v3 (-(sl * n2), fma (sx, n.y, cl * n.z), fma (sx, n.z, -(cl * n.y)));
+   double phi = blur * (1.0 / 3600.0 * MXG_PI / 180.0);
    phi = phi * gaussian (st);
-   n = rotate_small (n, perp, phi);
+   sincos_small (phi, &s, &c);
+   n = reunit_f (lin2_f (c, n, s, cross_f (u, n)));
+}
+
+// The photon's index of refraction at the mirror, n = 1 - delta + i beta,
+// as the Fresnel draw uses it: the real and imaginary part of n^2, and the
+// real part less one (from delta and beta: no cancellation); corr: the
+// square root of its shell's area correction.
+struct MirrorIndex
+{
+   double n2r, n2i, n2r1, corr;
+};
+
+// The Fresnel draw u against reflectivity times corr (reflect.c:39-77):
+// true when absorbed.  The reflectivity is the mean of A / B = |c - w|^2 /
+// |c + w|^2 and C / D = |n^2 c - w|^2 / |n^2 c + w|^2 with c the cosine of
+// the angle to the normal and w = sqrt (n^2 - 1 + c^2); the draw is compared
+// without the divisions.
+__device__ __forceinline__ bool fresnel_absorbs (double u, double c, const MirrorIndex &m)
+{
+   const double wr = fma (c, c, m.n2r1), wi = m.n2i;
+   // the principal square root by the half-angle formulas
+   double inv;
+   const double mod = sqrt_n (fma (wr, wr, wi * wi));
+   const double big = sqrt_rsqrt_n (fmax (0.5 * (mod + fabs (wr)), 1e-300), inv);
+   const double small = 0.5 * wi * inv;
+   const double re = (wr >= 0.0) ? big : fabs (small);
+   const double im = (wr >= 0.0) ? small : copysign (big, small);
+   const double i2 = im * im;
+   const double d1 = c - re, s1 = c + re;
+   const double A = fma (d1, d1, i2), B = fma (s1, s1, i2);
+   const double xr = m.n2r * c, xi = m.n2i * c;
+   const double dr = xr - re, di = xi - im, sr = xr + re, si = xi + im;
+   const double C = fma (dr, dr, di * di), D = fma (sr, sr, si * si);
+   return 2.0 * u * (B * D) >= fma (A, D, C * B) * m.corr;
 }
 
 // Reflection at a surface point x already on conic k of shell S: normal
 // blur, Fresnel draw, specular reflection, WFold scatter (hrma.c:488-545).
 // 0 reflected, -1 absorbed or scattered out.
 __device__ __forceinline__ int reflect_at (const mxg_hrma_cfg &h, const mxg_shell_cfg &S, int k,
-                                           vec3 x, vec3 &p, double energy, double beta,
-                                           double delta, double corr,
+                                           vec3 x, vec3 &p, double energy, const MirrorIndex &m,
                                            const float *__restrict__ fa,
                                            const double *__restrict__ da,
                                            const float *__restrict__ e_alphas,
@@ -111,15 +144,10 @@ __device__ __forceinline__ int reflect_at (const mxg_hrma_cfg &h, const mxg_shel
    vec3 normal = conic_normal (S.conic_a[k], S.conic_b[k], x);
    if (h.use_blur)
      blur_normal (normal, S.blur[k], st);
-   double p_dot_n = dot (p, normal);
-   if (h.ideal == 0)
-     {
-        double r = uniform (st);
-        double rfl = reflectivity (fabs (p_dot_n), beta, delta);
-        if (r >= rfl * corr)
-          return -1;
-     }
-   p = ax1_bx2 (1.0, p, -2.0 * p_dot_n, normal);
+   const double p_dot_n = dot_f (p, normal);
+   if ((h.ideal == 0) && fresnel_absorbs (uniform (st), fabs (p_dot_n), m))
+     return -1;
+   p = along_f (p, -2.0 * p_dot_n, normal);
    if (h.use_wfold == 0)
      return 0;
    double r = uniform (st);
@@ -127,7 +155,12 @@ __device__ __forceinline__ int reflect_at (const mxg_hrma_cfg &h, const mxg_shel
    dg *= S.scat_factor[k];
    if (dg > MXG_PI / 4) return -1;
    if (uniform (st) < 0.5) dg = -dg;
-   p = rotate_small (p, cross (p, normal), dg);
+   // p turned by dg about p x n, which is at right angles to p and not of
+   // length 1: cos p + sin (p x n) x p, with (p x n) x p = n - p (p . n)
+   // and p . n = -p_dot_n after the reflection
+   double sn, cs;
+   sincos_small (dg, &sn, &cs);
+   p = unit_f (lin2_f (fma (sn, p_dot_n, cs), p, sn, normal));
    return 0;
 }
 
@@ -149,7 +182,25 @@ struct HrmaLds
    // the bucket counts of the searched tables (mxg_bucket)
    uint32_t bk_opt, bk_corr[MXG_NUM_SHELLS], bk_ea[MXG_NUM_SHELLS][2];
    uint32_t floats;               // staged floats after the configuration copy
+   // bit k: some shell's tilt matrix of surface k is not the identity (with
+   // the standard geometry file the paraboloids' all are, and the products
+   // with them are left out)
+   uint32_t tilted;
 };
+
+// HrmaLds::tilted of configuration h (host side)
+inline uint32_t hrma_tilted (const mxg_hrma_cfg &h)
+{
+   uint32_t t = 0;
+   for (int sh = 0; sh < MXG_NUM_SHELLS; sh++)
+     for (int k = 0; k < 2; k++)
+       for (int q = 0; q < 9; q++)
+         {
+            const double one = (q % 4 == 0) ? 1.0 : 0.0;
+            if ((h.shell[sh].fwd[k][q] != one) || (h.shell[sh].bwd[k][q] != one)) t |= 1u << k;
+         }
+   return t;
+}
 
 // Dynamic LDS of the reflection: the configuration copy, a copy of the
 // layout at kHrmaLayOff (the reflection reads a table's offset by the
@@ -180,6 +231,7 @@ inline HrmaLds hrma_lds_layout (const mxg_hrma_cfg &h)
           }
      }
    lay.floats = f;
+   lay.tilted = hrma_tilted (h);
    return lay;
 }
 
@@ -229,12 +281,13 @@ __device__ __forceinline__ void stage_hrma_tables (const mxg_config *__restrict_
 }
 
 // The source-to-paraboloid part of the mirror for an unabsorbed photon with
-// tag `tag` and direction p: vignetting, aperture, precollimator struts,
+// tag `tag` and direction p (tilted: HrmaLds): vignetting, aperture, precollimator struts,
 // frame change and the paraboloid intersection.  False when vignetting
 // blocks the photon (nothing else is drawn); else true, with its position
 // x, direction p, shell si and the mirror's marks added to flags; *hit: it
 // hit the paraboloid, its random-stream position in *rng.
-__device__ __forceinline__ bool hrma_enter_core (const mxg_hrma_cfg &h, uint32_t tag, double source_distance,
+__device__ __forceinline__ bool hrma_enter_core (const mxg_hrma_cfg &h, uint32_t tilted, uint32_t tag,
+                                                 double source_distance,
                                                  unsigned long long seed, uint32_t source_id, vec3 &x,
                                                  vec3 &p, int &si, uint32_t &flags, bool &hit, uint32_t &rng)
 {
@@ -263,9 +316,8 @@ __device__ __forceinline__ bool hrma_enter_core (const mxg_hrma_cfg &h, uint32_t
         quad = (unsigned int) (4.0 * theta);
      }
    while (0 == (S.shutter_bitmap & (1u << quad)));
-   theta = (2.0 * MXG_PI) * (theta - 1.0 / 8.0);
    double sn, cs;
-   sincos (theta, &sn, &cs);
+   sincos_turn (theta - 1.0 / 8.0, sn, cs);
    x.z = radius * cs;
    x.y = radius * sn;
    x.x = S.front_position;
@@ -276,15 +328,19 @@ __device__ __forceinline__ bool hrma_enter_core (const mxg_hrma_cfg &h, uint32_t
         p = ax1_bx2 (1.0, x, source_distance, p);
         normalize (p);
      }
-   if (h.use_struts && in_strut_shadow (h, x, p, h.pre_struts))
+   double ipx = rcp_n (p.x);
+   if (h.use_struts && in_strut_shadow (h, x, p, ipx, h.pre_struts))
      flags |= PHOTON_MIRROR_VBLOCKED;
 
    x = add (x, ld3 (S.to_osac[0]));
-   x = m3_vmul (S.fwd[0], x);
-   p = m3_vmul (S.fwd[0], p);
+   if (tilted & 1u)
+     {
+        x = mul_m3_f (S.fwd[0], x);
+        p = mul_m3_f (S.fwd[0], p);
+        ipx = rcp_n (p.x);
+     }
 
-   if (-1 == conic_intersection (S.conic_a[0], S.conic_b[0], S.conic_c[0], x, p,
-                                 S.conic_xmin[0], S.conic_xmax[0]))
+   if (!conic_hit (S.conic_a[0], S.conic_b[0], S.conic_c[0], x, p, ipx, S.conic_xmin[0], S.conic_xmax[0]))
      flags |= PHOTON_UNREFLECTED;
    else
      {
@@ -301,7 +357,7 @@ __device__ __forceinline__ bool hrma_enter_core (const mxg_hrma_cfg &h, uint32_t
 // they are written here, the position and shell zero when vignetting
 // blocks it.
 template <bool FRESH = false>
-__device__ __forceinline__ bool hrma_enter_one (const mxg_hrma_cfg &h, Soa s, uint32_t id,
+__device__ __forceinline__ bool hrma_enter_one (const mxg_hrma_cfg &h, uint32_t tilted, Soa s, uint32_t id,
                                                 uint32_t *__restrict__ rng_pos, double source_distance,
                                                 unsigned long long seed, uint32_t source_id)
 {
@@ -312,7 +368,7 @@ __device__ __forceinline__ bool hrma_enter_one (const mxg_hrma_cfg &h, Soa s, ui
         vec3 x, p = v3 (s.p0[id], s.p1[id], s.p2[id]);
         int si;
         uint32_t rng = 0;
-        if (!hrma_enter_core (h, s.tag[id], source_distance, seed, source_id, x, p, si, flags, keep, rng))
+        if (!hrma_enter_core (h, tilted, s.tag[id], source_distance, seed, source_id, x, p, si, flags, keep, rng))
           {
              s.flags[id] = flags | PHOTON_MIRROR_VBLOCKED;
              if (FRESH)
@@ -352,16 +408,15 @@ __device__ __forceinline__ void resume_stream (Stream &st, const uint32_t *__res
      }
 }
 
-// The photon's optical constants (beta, delta) and the square root of its
-// shell's area correction factor, interpolated at its energy from the
-// tables in LDS (the same values at both surfaces).
-__device__ __forceinline__ void mirror_constants (const mxg_hrma_cfg &h, const mxg_shell_cfg &S, int si,
-                                                  const float *ltab, const HrmaLds &lay, double energy,
-                                                  double &beta, double &delta, double &corr)
+// The photon's optical constants and the square root of its shell's area
+// correction factor, interpolated at its energy from the tables in LDS (the
+// same values at both surfaces).
+__device__ __forceinline__ MirrorIndex mirror_index (const mxg_hrma_cfg &h, const mxg_shell_cfg &S, int si,
+                                                     const float *ltab, const HrmaLds &lay, double energy)
 {
-   beta = 0.0;
-   delta = 1.0;
-   corr = 1.0;
+   double beta = 0.0, delta = 1.0;
+   MirrorIndex m;
+   m.corr = 1.0;
    if (h.opt_n != 0)
      {
         const float *opt_e = ltab + lay.opt;
@@ -371,12 +426,13 @@ __device__ __forceinline__ void mirror_constants (const mxg_hrma_cfg &h, const m
         beta = fb;
         delta = fd;
         if (h.use_scale)
-          {
-             corr = interp_fb (ef, ltab + lay.corr_e[si], ltab + lay.corr_f[si], S.corr_n, S.corr_bucket,
-                               ltab + lay.bk_corr[si]);
-             corr = sqrt (corr);
-          }
+          m.corr = sqrt_n (interp_fb (ef, ltab + lay.corr_e[si], ltab + lay.corr_f[si], S.corr_n, S.corr_bucket,
+                                      ltab + lay.bk_corr[si]));
      }
+   m.n2r1 = fma (delta, delta - 2.0, -(beta * beta));
+   m.n2r = 1.0 + m.n2r1;
+   m.n2i = 2.0 * (1.0 - delta) * beta;
+   return m;
 }
 
 // k_hrma_reflect's work for photon id of the middle list: paraboloid
@@ -401,35 +457,44 @@ __device__ __forceinline__ bool hrma_reflect_one (const mxg_hrma_cfg &h, const f
    vec3 x = v3 (s.x0[id], s.x1[id], s.x2[id]);
    vec3 p = v3 (s.p0[id], s.p1[id], s.p2[id]);
    const double energy = s.energy[id];
-   double beta, delta, corr;
-   mirror_constants (h, S, si, ltab, lay, energy, beta, delta, corr);
+   const MirrorIndex m = mirror_index (h, S, si, ltab, lay, energy);
+   const uint32_t tilted = __builtin_amdgcn_readfirstlane (lay.tilted);
 
-   if (0 != reflect_at (h, S, 0, x, p, energy, beta, delta, corr, fa, da,
-                        ltab + lay.ea[si][0], ltab + lay.bk_ea[si][0], st))
+   if (0 != reflect_at (h, S, 0, x, p, energy, m, fa, da, ltab + lay.ea[si][0], ltab + lay.bk_ea[si][0], st))
      flags |= PHOTON_UNREFLECTED;
    else
      {
-        p = m3_vmul (S.bwd[0], p);
-        x = m3_vmul (S.bwd[0], x);
+        if (tilted & 1u)
+          {
+             p = mul_m3_f (S.bwd[0], p);
+             x = mul_m3_f (S.bwd[0], x);
+          }
         x = sub (x, ld3 (S.to_osac[0]));
-        if (h.use_struts && in_strut_shadow (h, x, p, h.cap_struts))
+        double ipx = rcp_n (p.x);
+        if (h.use_struts && in_strut_shadow (h, x, p, ipx, h.cap_struts))
           flags |= PHOTON_MIRROR_VBLOCKED;
         else
           {
              x = add (x, ld3 (S.to_osac[1]));
-             p = m3_vmul (S.fwd[1], p);
-             x = m3_vmul (S.fwd[1], x);
-             if ((-1 == conic_intersection (S.conic_a[1], S.conic_b[1], S.conic_c[1], x, p,
-                                            S.conic_xmin[1], S.conic_xmax[1]))
-                 || (0 != reflect_at (h, S, 1, x, p, energy, beta, delta, corr, fa, da,
+             if (tilted & 2u)
+               {
+                  p = mul_m3_f (S.fwd[1], p);
+                  x = mul_m3_f (S.fwd[1], x);
+                  ipx = rcp_n (p.x);
+               }
+             if (!conic_hit (S.conic_a[1], S.conic_b[1], S.conic_c[1], x, p, ipx, S.conic_xmin[1], S.conic_xmax[1])
+                 || (0 != reflect_at (h, S, 1, x, p, energy, m, fa, da,
                                       ltab + lay.ea[si][1], ltab + lay.bk_ea[si][1], st)))
                flags |= PHOTON_UNREFLECTED;
              else
                {
-                  p = m3_vmul (S.bwd[1], p);
-                  x = m3_vmul (S.bwd[1], x);
+                  if (tilted & 2u)
+                    {
+                       p = mul_m3_f (S.bwd[1], p);
+                       x = mul_m3_f (S.bwd[1], x);
+                    }
                   x = sub (x, ld3 (S.to_osac[1]));
-                  if (h.use_struts && in_strut_shadow (h, x, p, h.post_struts))
+                  if (h.use_struts && in_strut_shadow (h, x, p, rcp_n (p.x), h.post_struts))
                     flags |= PHOTON_MIRROR_VBLOCKED;
                }
           }

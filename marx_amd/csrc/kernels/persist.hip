@@ -136,7 +136,7 @@ void k_batch_persistent (PersistArgs a)
                {
                   batch_source_one<true, true> (src, a.da, a.s, i, a.off, a.nsrc, a.dir, t0, a.exposure,
                                                 a.start_time, a.seed);
-                  keep = hrma_enter_one<true> (h, a.s, i, a.rng_pos, distance, a.seed, 0u);
+                  keep = hrma_enter_one<true> (h, a.lay.tilted, a.s, i, a.rng_pos, distance, a.seed, 0u);
                }
              c.add (keep, i, list);
           }

@@ -59,26 +59,31 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
                                                     vec3 p, vec3 p_normal, vec3 line_normal, double line_alpha,
                                                     Stream &st)
 {
+   double sn, cs;
    if (src.type == MXG_SOURCE_DISK)
      {
-        vec3 normal = rotate_unit_vector (p_normal, p, 2.0 * MXG_PI * uniform (st));
+        sincos_turn (uniform (st), sn, cs);
+        const vec3 normal = reunit_f (turn_f (p_normal, p, cs, sn));
         double x0 = src.disk_theta_min / src.disk_theta;
         x0 = x0 * x0;
         double x1 = 1.0 - x0;
-        double rnd = src.disk_theta * sqrt (x0 + x1 * uniform (st));
-        return rotate_unit_vector (p, normal, rnd);
+        double rnd = src.disk_theta * sqrt_n (x0 + x1 * uniform (st));
+        sincos_small (rnd, &sn, &cs);
+        return reunit_f (turn_f (p, normal, cs, sn));
      }
    if ((src.type == MXG_SOURCE_GAUSS) || (src.type == MXG_SOURCE_BETA))
      {
-        vec3 normal = rotate_unit_vector (p_normal, p, 2.0 * MXG_PI * uniform (st));
+        sincos_turn (uniform (st), sn, cs);
+        const vec3 normal = reunit_f (turn_f (p_normal, p, cs, sn));
         double rnd;
         do rnd = uniform (st);
         while (rnd == 0.0);
         if (src.type == MXG_SOURCE_GAUSS)
-          rnd = src.gauss_sigma * sqrt (-log (rnd));
+          rnd = src.gauss_sigma * sqrt_n (-log_n (rnd));
         else
           rnd = src.beta_core * sqrt (pow (rnd, src.beta_xpon) - 1.0);
-        return rotate_unit_vector (p, normal, rnd);
+        sincos_small (rnd, &sn, &cs);
+        return reunit_f (turn_f (p, normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_IMAGE)
      {
@@ -90,18 +95,19 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         y = y * src.image_yscale;
         x = x * src.image_xscale;
         double sx, cx, sy, cy;
-        sincos (x, &sx, &cx);
-        sincos (y, &sy, &cy);
-        return rotate_unit_vector (v3 (-cy * cx, cy * sx, -sy), line_normal, line_alpha);
+        sincos_small (x, &sx, &cx);
+        sincos_small (y, &sy, &cy);
+        sincos_r (line_alpha, sn, cs);
+        return reunit_f (turn_f (v3 (-cy * cx, cy * sx, -sy), line_normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_LINE)
      {
         double theta = src.line_theta * (-1.0 + 2.0 * uniform (st));
-        double sn, cs;
-        sincos (theta, &sn, &cs);
+        sincos_small (theta, &sn, &cs);
         const double sin_theta = -sn;
         vec3 q = v3 (-cs, sin_theta * src.line_cos_phi, sin_theta * src.line_sin_phi);
-        return rotate_unit_vector (q, line_normal, line_alpha);
+        sincos_r (line_alpha, sn, cs);
+        return reunit_f (turn_f (q, line_normal, cs, sn));
      }
    return p;
 }
@@ -136,32 +142,32 @@ __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3
 {
    Stream st;
    stream_init (st, seed, tag, MXG_STAGE_DITHER, source_id);
-   double tt = (2.0 * MXG_PI) * (start_time + t);
-   float fra = (float) (src.ra_amp * sin (tt / src.ra_period + src.ra_phase));
-   float fdec = (float) (src.dec_amp * sin (tt / src.dec_period + src.dec_phase));
-   float froll = (float) (src.nominal_roll + src.roll_amp * sin (tt / src.roll_period + src.roll_phase));
+   // the angles as the reference rounds them: the state is kept as float
+   const double tt = (2.0 * MXG_PI) * (start_time + t);
+   float fra = (float) (src.ra_amp * sin_r (div_n (tt, src.ra_period) + src.ra_phase));
+   float fdec = (float) (src.dec_amp * sin_r (div_n (tt, src.dec_period) + src.dec_phase));
+   float froll = (float) src.nominal_roll;
+   if (src.roll_amp != 0.0)
+     froll = (float) (src.nominal_roll + src.roll_amp * sin_r (div_n (tt, src.roll_period) + src.roll_phase));
    d[0] = fra; d[1] = fdec; d[2] = froll;
    double delta_ra = src.aspect_blur * gaussian (st);
    double delta_dec = src.aspect_blur * gaussian (st);
    double ra = (double) fra + delta_ra, dec = (double) fdec + delta_dec, roll = froll;
 
-   {
-      double sr, cr;
-      sincos_small (-roll, &sr, &cr);
-      p = rotate_unit_vector1 (p, v3 (1, 0, 0), cr, sr);
-   }
+   double sr, cr;
+   sincos_small (-roll, &sr, &cr);
+   p = reunit_f (turn_x_f (p, cr, sr));
    double sin_ra, cos_ra, sin_dec, cos_dec;
    sincos_small (ra, &sin_ra, &cos_ra);
    sincos_small (dec, &sin_dec, &cos_dec);
-   double cos_theta = cos_dec * cos_ra;
-   vec3 nv = v3 (0, sin_dec, -cos_dec * sin_ra);
-   double sin_theta = length (nv);
-   if (sin_theta > 1e-20)
+   // the pointing's axis (0, a, b) / sin(theta)
+   const double a = sin_dec, b = -cos_dec * sin_ra;
+   const double s2 = fma (a, a, b * b);
+   if (s2 > 1e-40)
      {
-        nv.x /= sin_theta;
-        nv.y /= sin_theta;
-        nv.z /= sin_theta;
-        p = rotate_unit_vector1 (p, nv, cos_theta, sin_theta);
+        double inv;
+        const double sin_theta = sqrt_rsqrt_n (s2, inv);
+        p = reunit_f (turn_f (p, v3 (0.0, a * inv, b * inv), cos_dec * cos_ra, sin_theta));
      }
    return p;
 }
