@@ -299,11 +299,12 @@ void mxg_set_uniform_times (double tmax);
  * Marx_Photon_Type.  *num_collected receives the number of photons created
  * (fewer than num when exposure_time truncates the chunk), *num_detected
  * the number that survive every stage.  stage_ms, when non-NULL, receives
- * 6 per-stage GPU times in ms measured with HIP events recorded on the
- * library's stream around each stage's kernels (read after the call's
- * final synchronisation, so timing adds no host round trip): source
- * (including dither), 0 (dither is fused into the source stage), mirror,
- * grating, detector, and their sum. */
+ * 6 per-stage GPU times in ms: source (including dither and the arrival-time
+ * scan), 0 (dither is part of the source stage), mirror, grating, detector,
+ * and their sum.  A kernel that runs two stages is timed by the device's
+ * clock, and the stages share its time by the cycles that a sample of its
+ * blocks spent in each; with a FEF file the stages run as kernels of their
+ * own, timed by HIP events around each. */
 int mxg_trace_device (unsigned int num, unsigned int tag_start,
                       double start_time, double exposure_time,
                       unsigned int *num_collected, unsigned int *num_detected,
@@ -414,16 +415,18 @@ int mxg_trace_batch (unsigned int num_sources, const double *dirs, const unsigne
                      unsigned int tag_start, double start_time, double exposure, int use_graph,
                      unsigned int *num_detected, float *ms);
 
-/* Launch schedule of the batched pass.  Staged (persistent_tile = 0): one
- * kernel per stage, with blocks per CU of the source, paraboloid,
- * reflection, grating and detector kernels (1..32; for the grating also 0,
+/* Launch schedule: blocks per CU of the stages' kernels, in the order source,
+ * paraboloid, reflection, grating, detector (1..32; for the grating also 0,
  * the default: one round of the blocks a CU holds at once, which its LDS
- * tables and register budget set) and the minimum waves per
- * SIMD the reflection kernel is compiled for (2, 3, 4).  Persistent
- * (persistent_tile = a multiple of 256 up to 4096): the whole pass as one
- * launch of persistent_blocks_per_cu (1..8) blocks per CU that take tiles of
- * persistent_tile photons from a work counter and run every stage on them
- * (a FEF run takes the staged pass).  Both give the same photons. */
+ * tables and register budget set).  Where one kernel runs several stages it
+ * takes the paraboloid's (source and paraboloid), the reflection's
+ * (reflection, torus and order draw, or detector), and the detector's
+ * (diffraction and detector).  reflect_waves (2, 3, 4): the minimum waves per
+ * SIMD the reflection's own kernel is compiled for, where it runs by itself
+ * (the host photon lists, a FEF file).  persistent_tile (0, or a multiple of
+ * 256 up to 4096) and persistent_blocks_per_cu (1..8) are kept for programs
+ * that set them: the batched pass is the same kernels with and without.  The
+ * photons do not depend on the schedule. */
 typedef struct
 {
    unsigned int blocks_per_cu[5];
@@ -436,24 +439,20 @@ int mxg_set_schedule (const mxg_schedule *s);
 int mxg_get_schedule (mxg_schedule *s);
 
 /* Autotuner: times the batch of mxg_trace_batch (same arguments) under
- * candidate schedules -- for the staged pass, blocks per CU in {2, 4, 8, 16}
- * for every stage kernel and one round (0) for the grating, then 2, 3 and 4
- * waves for the reflection kernel,
- * keeping for each kernel the fastest (HIP-event time, best of `repeats`
- * runs); then the persistent pass with tiles of {512, 1024, 2048, 4096}
- * photons at {2, 3, 4} blocks per CU -- and installs the schedule whose
- * graph-launched pass is fastest, returning it in *best and that pass time
- * in *best_ms. */
+ * candidate schedules -- blocks per CU in {2, 4, 8, 16} for every stage and
+ * one round (0) for the grating, then 2, 3 and 4 waves for the reflection --
+ * keeping for each the fastest (best of `repeats` runs), installs the
+ * schedule found, and returns it in *best and the time of its graph-launched
+ * pass in *best_ms. */
 int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsigned int *counts,
                         unsigned int tag_start, double start_time, double exposure,
                         unsigned int repeats, mxg_schedule *best, float *best_ms);
 
-/* The two mirror kernels of the last mxg_trace_device call, each timed
- * alone with HIP events on the library's stream: [0] aperture + paraboloid
- * intersection, [1] the two reflections.  ms receives their device times in
- * milliseconds, photons_in the photons each one processed (the photons
- * entering the mirror, and those that hit the paraboloid).  Either pointer
- * may be NULL. */
+/* The two parts of the mirror in the last mxg_trace_device call: [0] aperture
+ * + paraboloid intersection, [1] the two reflections.  ms receives their
+ * device times in milliseconds (as mxg_trace_device's stage times),
+ * photons_in the photons each one processed (the photons entering the mirror,
+ * and those that hit the paraboloid).  Either pointer may be NULL. */
 int mxg_last_kernel_stats (float ms[2], unsigned int photons_in[2]);
 
 /* Copies the device-resident photons of the last mxg_trace_device call into

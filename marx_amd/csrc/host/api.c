@@ -618,10 +618,9 @@ int mxg_trace_device (unsigned int num, unsigned int tag_start, double start_tim
    unsigned int n = 0, ndet;
    unsigned long hist = MARX_ENERGY_OK | MARX_TIME_OK | MARX_X_VECTOR_OK | MARX_P_VECTOR_OK | MARX_TAG_OK;
    int with_grating = (Grating_Type == MARX_GRATING_HETG) || (Grating_Type == MARX_GRATING_LETG);
-   /* stages hand their survivors densely to the next one: the grating to
-    * the detector; the mirror to the LETG grating (HETG + ACIS-S measured
-    * the reflection's extra writes costing what its lighter grating pass
-    * saves, LETG + HRC-S 4 percent faster per step) */
+   /* with a FEF file, kernels a stage: they hand their survivors densely to
+    * the next one, the grating to the detector and the mirror to the LETG
+    * grating */
    int relay = (Grating_Type == MARX_GRATING_LETG);
 
    if (-1 == sync_config ())
@@ -640,7 +639,16 @@ int mxg_trace_device (unsigned int num, unsigned int tag_start, double start_tim
    /* timing slots: 0 source+dither (its count: the photons created, read
     * back with the timings, so no stage waits on the host), 1 mirror, 2
     * grating, 3 detector, 4 and 5 the two mirror kernels alone */
-   if ((-1 == mxgd_launch_source (num, tag_start, start_time, exposure_time, Seed, 0, 0, 1))
+   if ((num > 0) && mxgd_passes_fit ())
+     {
+        if ((-1 == mxgd_run_passes (num, tag_start, start_time, exposure_time, Seed, ms, counts))
+            || (-1 == mxgd_set_created (counts[0])))
+          {
+             mxg_error ("%s", mxgd_last_error ());
+             return -1;
+          }
+     }
+   else if ((-1 == mxgd_launch_source (num, tag_start, start_time, exposure_time, Seed, 0, 0, 1))
        || (-1 == mxgd_run_mirror (Mxg_Cfg.src.distance, Seed, 1, NULL, relay, 1))
        || (with_grating && (-1 == mxgd_run_grating (Seed, 2, NULL, relay, Detector_Type > 0)))
        || ((Detector_Type > 0) && (-1 == mxgd_run_detect (start_time, Seed, 3, NULL, with_grating)))
@@ -732,21 +740,17 @@ static Batch_Key Batch_Graph_Key;
 
 
 /* one pass over the uploaded batch (n photons): source, mirror, grating,
- * detector, in timing slots 0-3, or the persistent pass in slot 0 (during
- * graph capture the stages record no events but still copy their survivor
- * counts) */
+ * detector, as chunk kernels or, with a FEF file, as kernels a stage in
+ * timing slots 0-3 (during graph capture those record no events but still
+ * copy their survivor counts) */
 static int batch_pass (unsigned int n, double start_time, double exposure, int with_grating)
 {
-   /* stages hand their survivors densely to the next one: the grating to
-    * the detector; the mirror to the LETG grating (HETG + ACIS-S measured
-    * the reflection's extra writes costing what its lighter grating pass
-    * saves, LETG + HRC-S 4 percent faster per step) */
+   /* with a FEF file, kernels a stage: they hand their survivors densely to
+    * the next one, the grating to the detector and the mirror to the LETG
+    * grating */
    int relay = (Grating_Type == MARX_GRATING_LETG);
-   mxgd_schedule sched;
-   mxgd_get_schedule (&sched);
-   /* the persistent pass traces point sources without the FEF step */
-   if (sched.persist_tile && !Mxg_Cfg.det.fef_on && (Mxg_Cfg.src.type == MXG_SOURCE_POINT))
-     return mxgd_run_batch_persistent (n, exposure, start_time, Seed, 0);
+   if ((n > 0) && mxgd_passes_fit ())
+     return mxgd_run_batch_passes (n, exposure, start_time, Seed);
    if ((-1 == mxgd_run_batch_source (n, exposure, start_time, Seed, 0, 1))
        || (-1 == mxgd_run_mirror (Mxg_Cfg.src.distance, Seed, 1, NULL, relay, 1))
        || (with_grating && (-1 == mxgd_run_grating (Seed, 2, NULL, relay, Detector_Type > 0)))
@@ -755,14 +759,21 @@ static int batch_pass (unsigned int n, double start_time, double exposure, int w
    return 0;
 }
 
-static int batch_finish (unsigned int n, unsigned int tag_start, int with_grating,
+static int batch_finish (unsigned int n, unsigned int tag_start, int with_grating, int timed,
                          unsigned int *num_detected)
 {
    float ms[8];
    unsigned int counts[8];
    unsigned long hist = MARX_ENERGY_OK | MARX_TIME_OK | MARX_X_VECTOR_OK | MARX_P_VECTOR_OK
      | MARX_TAG_OK | MARX_MIRROR_SHELL_OK;
-   if (-1 == mxgd_read_timings (ms, counts, 8))
+   if ((n > 0) && mxgd_passes_fit ())
+     {
+        if (-1 == mxgd_read_passes (n, ms, counts))
+          return -1;
+        /* no stage times when a graph launched the pass */
+        if (!timed) memset (ms, 0, sizeof (ms));
+     }
+   else if (-1 == mxgd_read_timings (ms, counts, 8))
      return -1;
    Stage_Counts[0] = n;
    Stage_Counts[1] = counts[1];
@@ -872,12 +883,12 @@ int mxg_trace_batch (unsigned int num_sources, const double *dirs, const unsigne
      {
         if ((-1 == mxgd_batch_set_tag_start (tag_start))
             || (-1 == batch_pass (n, start_time, exposure, with_grating))
-            || (-1 == batch_finish (n, tag_start, with_grating, num_detected)))
+            || (-1 == batch_finish (n, tag_start, with_grating, 1, num_detected)))
           goto device_error;
         if (ms) *ms = Last_Slot_Ms[0] + Last_Slot_Ms[1] + Last_Slot_Ms[2] + Last_Slot_Ms[3];
         return 0;
      }
-   if (-1 == batch_finish (n, tag_start, with_grating, num_detected))
+   if (-1 == batch_finish (n, tag_start, with_grating, 0, num_detected))
      goto device_error;
    return 0;
 
@@ -961,10 +972,8 @@ int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsi
                         unsigned int repeats, mxg_schedule *best, float *best_ms)
 {
    static const unsigned int bpc[4] = {2, 4, 8, 16};
-   static const unsigned int tiles[4] = {512, 1024, 2048, 4096};
-   static const unsigned int tile_bpc[3] = {2, 3, 4};
    mxg_schedule cur, sel;
-   float best_t[5], t[5], pass_ms, ms;
+   float best_t[5], t[5], pass_ms;
    int k, c;
 
    if (repeats == 0) repeats = 1;
@@ -973,8 +982,7 @@ int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsi
    sel = cur;
    sel.persistent_tile = 0;
    for (k = 0; k < 5; k++) best_t[k] = 1e30f;
-   /* the staged pass: blocks per CU, every kernel at once (their times are
-    * independent) */
+   /* blocks per CU, every stage at once (their times are independent) */
    for (c = 0; c < 4; c++)
      {
         mxg_schedule s = sel;
@@ -1021,33 +1029,8 @@ int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsi
              sel.reflect_waves = (unsigned int) c;
           }
      }
-   /* the staged pass against the persistent one, whole graph-launched
-    * passes (the persistent pass traces point sources without the FEF
-    * step) */
    if ((-1 == mxg_set_schedule (&sel))
        || (-1 == graph_pass_ms (num_sources, dirs, counts, tag_start, start_time, exposure, repeats, &pass_ms)))
-     goto fail;
-   if (!Mxg_Cfg.det.fef_on && (Mxg_Cfg.src.type == MXG_SOURCE_POINT))
-     {
-        mxg_schedule staged = sel;
-        for (c = 0; c < 4; c++)
-          for (k = 0; k < 3; k++)
-            {
-               mxg_schedule s = staged;
-               s.persistent_tile = tiles[c];
-               s.persistent_blocks_per_cu = tile_bpc[k];
-               if ((-1 == mxg_set_schedule (&s))
-                   || (-1 == graph_pass_ms (num_sources, dirs, counts, tag_start, start_time, exposure, repeats,
-                                            &ms)))
-                 goto fail;
-               if (ms < pass_ms)
-                 {
-                    pass_ms = ms;
-                    sel = s;
-                 }
-            }
-     }
-   if (-1 == mxg_set_schedule (&sel))
      goto fail;
    if (best) *best = sel;
    if (best_ms) *best_ms = pass_ms;

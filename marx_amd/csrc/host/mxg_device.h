@@ -94,12 +94,19 @@ int mxgd_batch_set_tag_start (unsigned int tag_start);
  * for mxgd_launch_source (mxgd_run_mirror with fresh set runs next). */
 int mxgd_run_batch_source (unsigned int n, double exposure, double start_time,
                            unsigned long long seed, int slot, int entry_follows);
-/* The whole batched pass (source, mirror, grating, detector) as one
- * persistent launch under the schedule's tile (not with a FEF file): the
- * same photons and final list as the staged pass; timing slot `slot` holds
- * the pass, the survivor counts land in the stage slots. */
-int mxgd_run_batch_persistent (unsigned int n, double exposure, double start_time,
-                               unsigned long long seed, int slot);
+/* The batched pass over n > 0 photons as kernels over the whole batch
+ * (without a wait); mxgd_read_passes then gives its counts and times. */
+int mxgd_run_batch_passes (unsigned int n, double exposure, double start_time, unsigned long long seed);
+/* The trace as kernels over the chunk (after the arrival-time scan of Poisson
+ * arrivals): source, mirror, grating and detector of n > 0 photons, then a
+ * wait.  counts and ms (8 each) by timing slot as mxgd_read_timings gives
+ * them.  mxgd_passes_fit: whether the device's configuration can take it
+ * (no FEF step, tables that fit LDS). */
+int mxgd_passes_fit (void);
+int mxgd_run_passes (unsigned int n, unsigned int tag_start, double start_time, double exposure_time,
+                     unsigned long long seed, float *ms, unsigned int *counts);
+/* Waits for the stream; ms and counts of the batch pass that ran last. */
+int mxgd_read_passes (unsigned int n, float *ms, unsigned int *counts);
 
 /* Launch schedule: blocks per CU of the stage kernels (the grating's 0: one
  * round of the blocks a CU holds at once) and the minimum waves

@@ -344,238 +344,243 @@ static __device__ __noinline__ double contam_transmission (const mxg_contam &c, 
    return exp (-v);
 }
 
-// k_detect's work for photon id (KIND: MXG_DET_ACIS, MXG_DET_HRC_S,
-// MXG_DET_HRC_I; FEF: with the ACIS FEF step).  True when the photon is
-// detected.  RELAY: the photon's incoming x, p, energy, tag and flags are
-// read from row `slot` of *relay instead of the store.
+// The detection of photon id, unabsorbed so far, with tag `tag`, position x,
+// direction p and flags (KIND: MXG_DET_ACIS, MXG_DET_HRC_S, MXG_DET_HRC_I;
+// FEF: with the ACIS FEF step): every column it changes is stored.  True when
+// the photon is detected.
+template <bool FEF, int KIND>
+__device__ __forceinline__ bool detect_core (const mxg_detector_cfg &d, const float *__restrict__ fa,
+                                             const double *__restrict__ da, const Soa &s, uint32_t id, uint32_t tag,
+                                             double energy, vec3 x, vec3 p, uint32_t flags, double tstart,
+                                             unsigned long long seed, uint32_t source_id)
+{
+   constexpr bool is_acis = (KIND == MXG_DET_ACIS);
+   constexpr bool is_hrc_s = (KIND == MXG_DET_HRC_S);
+   Stream st;
+   stream_init (st, seed, tag, MXG_STAGE_DETECT, source_id);
+   bool detect = true;
+
+   if (is_hrc_s && d.use_drake)
+     {
+        double p_dot_n = 0.0;
+        bool use_cr = false;
+        int k = drake_hit (d, x, p, p_dot_n, use_cr);
+        if (k >= 0)
+          {
+             unsigned int nt = use_cr ? d.drake_cr_n : d.drake_c_n;
+             double rfl = 1.0;
+             if (nt != 0)
+               {
+                  unsigned int eo = use_cr ? d.drake_cr_e_off : d.drake_c_e_off;
+                  unsigned int bo = use_cr ? d.drake_cr_beta_off : d.drake_c_beta_off;
+                  unsigned int dof = use_cr ? d.drake_cr_delta_off : d.drake_c_delta_off;
+                  float ef = (float) energy;
+                  float beta = interp_f (ef, fa + eo, fa + bo, nt);
+                  float delta = interp_f (ef, fa + eo, fa + dof, nt);
+                  rfl = reflectivity (fabs (p_dot_n), (double) beta, (double) delta);
+               }
+             if (rfl < uniform (st))
+               {
+                  flags |= PHOTON_DRAKE_BLOCKED;
+                  detect = false;
+               }
+             else
+               {
+                  p = ax1_bx2 (1.0, p, -2.0 * p_dot_n, ld3 (d.drake[k].normal));
+                  flags |= PHOTON_DRAKE_REFLECTED;
+               }
+          }
+     }
+
+   if (detect)
+     {
+        x.x -= d.offset[0];
+        x.y -= d.offset[1];
+        x.z -= d.offset[2];
+        x = mul_m3_f (d.matrix, x);
+        p = mul_m3_f (d.matrix, p);
+        double dx = 0.0, dy = 0.0;
+        int k = find_chip (d, x, p, dx, dy);
+        if (k < 0)
+          {
+             flags |= PHOTON_MISSED_DETECTOR;
+             at (s.ccd, id) = -1;
+          }
+        else if constexpr (is_acis)
+          {
+             const mxg_chip &g = d.chip[k];
+             at (s.ccd, id) = (int8_t) g.id;
+             float ypix = (float) div_n (dx, g.x_pixel_size);
+             float zpix = (float) div_n (dy, g.y_pixel_size);
+             bool detected = true;
+             if (d.ideal == 0)
+               {
+                  double r = uniform (st);
+                  double qe = 1.0, qe_contam = 1.0;
+                  if (g.qe_n != 0)
+                    qe = interp_fb ((float) energy, fa + g.qe_e_off, fa + g.qe_off, g.qe_n, g.qe_bucket,
+                                    fa + g.qe_bucket.off);
+                  if (d.contam_on && d.contam[k].num_layers)
+                    qe_contam = contam_transmission (d.contam[k], fa, energy, ypix, zpix);
+                  // the filter table is empty on the CALDB QE path
+                  // (acis-s.c:303-304): filter transmission 1
+                  if (r >= qe * 1.0 * qe_contam)
+                    {
+                       flags |= PHOTON_UNDETECTED;
+                       detected = false;
+                    }
+               }
+             if (FEF && detected && d.fef_on)
+               {
+                  short pha = -1;
+                  float pi = 0.0f;
+                  if (apply_fef (d, fa, da, g.id, ypix, zpix, energy, st, pha, pi))
+                    {
+                       at (s.pha, id) = pha;
+                       at (s.pi, id) = pi;
+                    }
+                  else
+                    {
+                       at (s.pha, id) = -1;
+                       at (s.pi, id) = 0.0f;
+                       flags |= PHOTON_UNDETECTED;
+                       detected = false;
+                    }
+               }
+             if (detected && (d.frame_transfer_time > 0.0))
+               {
+                  double t = fmod (tstart + at (s.t, id), d.frame_time);
+                  if (t > d.exposure_time)
+                    {
+                       zpix = (float) (1.0 + 1022.0 * uniform (st));
+                       double xpixel = ((double) ypix - g.xpixel_offset) * g.x_pixel_size;
+                       double ypixel = ((double) zpix - g.ypixel_offset) * g.y_pixel_size;
+                       vec3 dxv = ax1_bx2 (xpixel, ld3 (g.xhat), ypixel, ld3 (g.yhat));
+                       x = add (ld3 (g.x_ll), dxv);
+                       p = sub (x, v3 (d.focal_length, 0, 0));
+                       normalize (p);
+                       flags |= PHOTON_ACIS_STREAKED;
+                    }
+               }
+             at (s.ypix, id) = ypix;
+             at (s.zpix, id) = zpix;
+          }
+        else
+          {
+             const mxg_chip &g = d.chip[k];
+             // MCP QE, shield region, filter QE, pulse height
+             bool ok = true;
+             int region = 0;
+             const mxg_qe_table &mq = d.mcp_qe[d.mcp_map[g.id]];
+             if (mq.n != 0)
+               {
+                  double qe = qe_at (mq, fa, energy);
+                  if (uniform (st) >= qe) ok = false;
+               }
+             if (ok)
+               {
+                  const mxg_qe_table *fq;
+                  if (is_hrc_s)
+                    {
+                       double t = div_n (d.shield_x - x.x, p.x);
+                       region = filter_region (d, x.y + t * p.y, x.z + t * p.z);
+                       if (region < 0) ok = false;
+                       fq = d.filter_qe + (region < 0 ? 0 : region);
+                    }
+                  else
+                    fq = d.filter_qe + g.id;
+                  if (ok && (fq->n != 0))
+                    {
+                       double qe = qe_at (*fq, fa, energy);
+                       if (uniform (st) >= qe) ok = false;
+                    }
+               }
+             if (!ok)
+               {
+                  flags |= PHOTON_UNDETECTED;
+                  at (s.ccd, id) = -1;
+               }
+             else
+               {
+                  if (is_hrc_s) at (s.region, id) = (int8_t) region;
+                  at (s.pha, id) = hrc_pha (energy, st);
+                  if (d.ideal == 0)
+                    {
+                       double r = uniform (st), rr, x_0, y_0;
+                       if (r < d.g1_wgt)
+                         {
+                            double c;
+                            do c = uniform (st); while (c == 0.0);
+                            rr = d.g1_sigma * sqrt_n (-2.0 * log_n (c));
+                            x_0 = d.g1_xctr; y_0 = d.g1_yctr;
+                         }
+                       else if (r < d.g1_wgt + d.g2_wgt)
+                         {
+                            double c;
+                            do c = uniform (st); while (c == 0.0);
+                            rr = d.g2_sigma * sqrt_n (-2.0 * log_n (c));
+                            x_0 = d.g2_xctr; y_0 = d.g2_yctr;
+                         }
+                       else
+                         {
+                            double c = uniform (st);
+                            double rmax = d.l1_rmax / d.l1_hwhm;
+                            rr = d.l1_hwhm * sqrt (expm1 (c * log1p (rmax * rmax)));
+                            x_0 = d.l1_xctr; y_0 = d.l1_yctr;
+                         }
+                       double sn, cs;
+                       sincos_turn (uniform (st), sn, cs);
+                       dx += x_0 + rr * cs;
+                       dy += y_0 + rr * sn;
+                       if (d.extend == 0)
+                         {
+                            if (dx < 0.0) dx = 0.0;
+                            if (dy < 0.0) dy = 0.0;
+                         }
+                    }
+                  at (s.ccd, id) = (int8_t) g.id;
+                  if (is_hrc_s)
+                    {
+                       const int cid = g.id;
+                       double u = d.pix_u[cid], v = d.pix_v[cid];
+                       u += div_n (dx, d.u_pixel_size);
+                       v += div_n (dy, d.v_pixel_size);
+                       at (s.upix, id) = (float) u;
+                       at (s.vpix, id) = (float) v;
+                       at (s.ypix, id) = (float) (d.pix_x0[cid] + (u - d.pix_u0[cid]));
+                       at (s.zpix, id) = (float) (d.pix_y0[cid] + (v - d.pix_v0[cid]));
+                    }
+                  else
+                    {
+                       at (s.ypix, id) = (float) (d.pix_x0[0] + div_n (dx, d.u_pixel_size));
+                       at (s.zpix, id) = (float) (d.pix_y0[0] + div_n (dy, d.v_pixel_size));
+                    }
+               }
+          }
+        p = rot_inv (d.matrix, p);
+        x = rot_inv (d.matrix, x);
+        x.x += d.offset[0];
+        x.y += d.offset[1];
+        x.z += d.offset[2];
+     }
+store_path (s, id, x, p, flags);
+   return (flags & BAD_PHOTON_MASK) == 0;
+}
+
+// k_detect's work for photon id: detect_core on the store's columns or,
+// RELAY, with its x, p, energy, tag and flags from row `slot` of *relay.
 template <bool FEF, int KIND, bool RELAY = false>
 __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const float *__restrict__ fa,
                                             const double *__restrict__ da, Soa s, uint32_t id, double tstart,
                                             unsigned long long seed, uint32_t source_id,
                                             const Relay *relay = nullptr, uint32_t slot = 0)
 {
-   constexpr bool is_acis = (KIND == MXG_DET_ACIS);
-   constexpr bool is_hrc_s = (KIND == MXG_DET_HRC_S);
-   bool keep = false;
-   uint32_t flags = RELAY ? relay->flags[slot] : s.flags[id];
-   if ((flags & BAD_PHOTON_MASK) == 0)
-     {
-        Stream st;
-        stream_init (st, seed, RELAY ? relay->tag[slot] : s.tag[id], MXG_STAGE_DETECT, source_id);
-        vec3 x = RELAY ? v3 (relay->x0[slot], relay->x1[slot], relay->x2[slot]) : v3 (s.x0[id], s.x1[id], s.x2[id]);
-        vec3 p = RELAY ? v3 (relay->p0[slot], relay->p1[slot], relay->p2[slot]) : v3 (s.p0[id], s.p1[id], s.p2[id]);
-        const double energy = RELAY ? relay->energy[slot] : s.energy[id];
-        bool detect = true;
-
-        if (is_hrc_s && d.use_drake)
-          {
-             double p_dot_n = 0.0;
-             bool use_cr = false;
-             int k = drake_hit (d, x, p, p_dot_n, use_cr);
-             if (k >= 0)
-               {
-                  unsigned int nt = use_cr ? d.drake_cr_n : d.drake_c_n;
-                  double rfl = 1.0;
-                  if (nt != 0)
-                    {
-                       unsigned int eo = use_cr ? d.drake_cr_e_off : d.drake_c_e_off;
-                       unsigned int bo = use_cr ? d.drake_cr_beta_off : d.drake_c_beta_off;
-                       unsigned int dof = use_cr ? d.drake_cr_delta_off : d.drake_c_delta_off;
-                       float ef = (float) energy;
-                       float beta = interp_f (ef, fa + eo, fa + bo, nt);
-                       float delta = interp_f (ef, fa + eo, fa + dof, nt);
-                       rfl = reflectivity (fabs (p_dot_n), (double) beta, (double) delta);
-                    }
-                  if (rfl < uniform (st))
-                    {
-                       flags |= PHOTON_DRAKE_BLOCKED;
-                       detect = false;
-                    }
-                  else
-                    {
-                       p = ax1_bx2 (1.0, p, -2.0 * p_dot_n, ld3 (d.drake[k].normal));
-                       flags |= PHOTON_DRAKE_REFLECTED;
-                    }
-               }
-          }
-
-        if (detect)
-          {
-             x.x -= d.offset[0];
-             x.y -= d.offset[1];
-             x.z -= d.offset[2];
-             x = mul_m3_f (d.matrix, x);
-             p = mul_m3_f (d.matrix, p);
-             double dx = 0.0, dy = 0.0;
-             int k = find_chip (d, x, p, dx, dy);
-             if (k < 0)
-               {
-                  flags |= PHOTON_MISSED_DETECTOR;
-                  s.ccd[id] = -1;
-               }
-             else if constexpr (is_acis)
-               {
-                  const mxg_chip &g = d.chip[k];
-                  s.ccd[id] = (int8_t) g.id;
-                  float ypix = (float) div_n (dx, g.x_pixel_size);
-                  float zpix = (float) div_n (dy, g.y_pixel_size);
-                  bool detected = true;
-                  if (d.ideal == 0)
-                    {
-                       double r = uniform (st);
-                       double qe = 1.0, qe_contam = 1.0;
-                       if (g.qe_n != 0)
-                         qe = interp_fb ((float) energy, fa + g.qe_e_off, fa + g.qe_off, g.qe_n, g.qe_bucket,
-                                         fa + g.qe_bucket.off);
-                       if (d.contam_on && d.contam[k].num_layers)
-                         qe_contam = contam_transmission (d.contam[k], fa, energy, ypix, zpix);
-                       // the filter table is empty on the CALDB QE path
-                       // (acis-s.c:303-304): filter transmission 1
-                       if (r >= qe * 1.0 * qe_contam)
-                         {
-                            flags |= PHOTON_UNDETECTED;
-                            detected = false;
-                         }
-                    }
-                  if (FEF && detected && d.fef_on)
-                    {
-                       short pha = -1;
-                       float pi = 0.0f;
-                       if (apply_fef (d, fa, da, g.id, ypix, zpix, energy, st, pha, pi))
-                         {
-                            s.pha[id] = pha;
-                            s.pi[id] = pi;
-                         }
-                       else
-                         {
-                            s.pha[id] = -1;
-                            s.pi[id] = 0.0f;
-                            flags |= PHOTON_UNDETECTED;
-                            detected = false;
-                         }
-                    }
-                  if (detected && (d.frame_transfer_time > 0.0))
-                    {
-                       double t = fmod (tstart + s.t[id], d.frame_time);
-                       if (t > d.exposure_time)
-                         {
-                            zpix = (float) (1.0 + 1022.0 * uniform (st));
-                            double xpixel = ((double) ypix - g.xpixel_offset) * g.x_pixel_size;
-                            double ypixel = ((double) zpix - g.ypixel_offset) * g.y_pixel_size;
-                            vec3 dxv = ax1_bx2 (xpixel, ld3 (g.xhat), ypixel, ld3 (g.yhat));
-                            x = add (ld3 (g.x_ll), dxv);
-                            p = sub (x, v3 (d.focal_length, 0, 0));
-                            normalize (p);
-                            flags |= PHOTON_ACIS_STREAKED;
-                         }
-                    }
-                  s.ypix[id] = ypix;
-                  s.zpix[id] = zpix;
-               }
-             else
-               {
-                  const mxg_chip &g = d.chip[k];
-                  // MCP QE, shield region, filter QE, pulse height
-                  bool ok = true;
-                  int region = 0;
-                  const mxg_qe_table &mq = d.mcp_qe[d.mcp_map[g.id]];
-                  if (mq.n != 0)
-                    {
-                       double qe = qe_at (mq, fa, energy);
-                       if (uniform (st) >= qe) ok = false;
-                    }
-                  if (ok)
-                    {
-                       const mxg_qe_table *fq;
-                       if (is_hrc_s)
-                         {
-                            double t = div_n (d.shield_x - x.x, p.x);
-                            region = filter_region (d, x.y + t * p.y, x.z + t * p.z);
-                            if (region < 0) ok = false;
-                            fq = d.filter_qe + (region < 0 ? 0 : region);
-                         }
-                       else
-                         fq = d.filter_qe + g.id;
-                       if (ok && (fq->n != 0))
-                         {
-                            double qe = qe_at (*fq, fa, energy);
-                            if (uniform (st) >= qe) ok = false;
-                         }
-                    }
-                  if (!ok)
-                    {
-                       flags |= PHOTON_UNDETECTED;
-                       s.ccd[id] = -1;
-                    }
-                  else
-                    {
-                       if (is_hrc_s) s.region[id] = (int8_t) region;
-                       s.pha[id] = hrc_pha (energy, st);
-                       if (d.ideal == 0)
-                         {
-                            double r = uniform (st), rr, x_0, y_0;
-                            if (r < d.g1_wgt)
-                              {
-                                 double c;
-                                 do c = uniform (st); while (c == 0.0);
-                                 rr = d.g1_sigma * sqrt_n (-2.0 * log_n (c));
-                                 x_0 = d.g1_xctr; y_0 = d.g1_yctr;
-                              }
-                            else if (r < d.g1_wgt + d.g2_wgt)
-                              {
-                                 double c;
-                                 do c = uniform (st); while (c == 0.0);
-                                 rr = d.g2_sigma * sqrt_n (-2.0 * log_n (c));
-                                 x_0 = d.g2_xctr; y_0 = d.g2_yctr;
-                              }
-                            else
-                              {
-                                 double c = uniform (st);
-                                 double rmax = d.l1_rmax / d.l1_hwhm;
-                                 rr = d.l1_hwhm * sqrt (expm1 (c * log1p (rmax * rmax)));
-                                 x_0 = d.l1_xctr; y_0 = d.l1_yctr;
-                              }
-                            double sn, cs;
-                            sincos_turn (uniform (st), sn, cs);
-                            dx += x_0 + rr * cs;
-                            dy += y_0 + rr * sn;
-                            if (d.extend == 0)
-                              {
-                                 if (dx < 0.0) dx = 0.0;
-                                 if (dy < 0.0) dy = 0.0;
-                              }
-                         }
-                       s.ccd[id] = (int8_t) g.id;
-                       if (is_hrc_s)
-                         {
-                            const int cid = g.id;
-                            double u = d.pix_u[cid], v = d.pix_v[cid];
-                            u += div_n (dx, d.u_pixel_size);
-                            v += div_n (dy, d.v_pixel_size);
-                            s.upix[id] = (float) u;
-                            s.vpix[id] = (float) v;
-                            s.ypix[id] = (float) (d.pix_x0[cid] + (u - d.pix_u0[cid]));
-                            s.zpix[id] = (float) (d.pix_y0[cid] + (v - d.pix_v0[cid]));
-                         }
-                       else
-                         {
-                            s.ypix[id] = (float) (d.pix_x0[0] + div_n (dx, d.u_pixel_size));
-                            s.zpix[id] = (float) (d.pix_y0[0] + div_n (dy, d.v_pixel_size));
-                         }
-                    }
-               }
-             p = rot_inv (d.matrix, p);
-             x = rot_inv (d.matrix, x);
-             x.x += d.offset[0];
-             x.y += d.offset[1];
-             x.z += d.offset[2];
-          }
-        s.x0[id] = x.x; s.x1[id] = x.y; s.x2[id] = x.z;
-        s.p0[id] = p.x; s.p1[id] = p.y; s.p2[id] = p.z;
-        s.flags[id] = flags;
-        keep = (flags & BAD_PHOTON_MASK) == 0;
-     }
-   return keep;
+   const uint32_t flags = RELAY ? at (relay->flags, slot) : at (s.flags, id);
+   if (flags & BAD_PHOTON_MASK) return false;
+   const vec3 x = RELAY ? v3 (at (relay->x0, slot), at (relay->x1, slot), at (relay->x2, slot)) : v3 (at (s.x0, id), at (s.x1, id), at (s.x2, id));
+   const vec3 p = RELAY ? v3 (at (relay->p0, slot), at (relay->p1, slot), at (relay->p2, slot)) : v3 (at (s.p0, id), at (s.p1, id), at (s.p2, id));
+   return detect_core<FEF, KIND> (d, fa, da, s, id, RELAY ? at (relay->tag, slot) : at (s.tag, id),
+                                  RELAY ? at (relay->energy, slot) : at (s.energy, id), x, p, flags, tstart, seed, source_id);
 }
 
 } // namespace mxg

@@ -90,6 +90,23 @@ __device__ __forceinline__ double uniform (Stream &s)
    return (double) u * (1.0 / ((double) 0xFFFFFFFFu));
 }
 
+// A Gaussian pair from two uniforms in the unit disk (polar method): false
+// when they fall outside.
+__device__ __forceinline__ bool polar_pair (double u1, double u2, double &g1, double &g2, double &g)
+{
+   g1 = fma (2.0, u1, -1.0);
+   g2 = fma (2.0, u2, -1.0);
+   g = fma (g1, g1, g2 * g2);
+   return (g < 1.0) && (g != 0.0);
+}
+
+// its scale sqrt (-2 log (g) / g), as l / sqrt (l g): 0 < g < 1, so l > 0
+__device__ __forceinline__ double polar_scale (double g)
+{
+   const double l = -2.0 * log_n (g);
+   return l * rsqrt_n (l * g);
+}
+
 __device__ __forceinline__ double gaussian (Stream &s)
 {
    if (s.have_gauss)
@@ -98,17 +115,92 @@ __device__ __forceinline__ double gaussian (Stream &s)
         return s.g2;
      }
    s.have_gauss = 1;
-   double g1, g2, g;
-   do
+   double g1, g2, g, u1;
+   do u1 = uniform (s);
+   while (!polar_pair (u1, uniform (s), g1, g2, g));
+   const double f = polar_scale (g);
+   s.g2 = g2 * f;
+   return g1 * f;
+}
+
+// The same stream with its words kept in LDS.  Lanes of a wave that reject
+// draws fall out of step, and a stream in registers then makes a block at
+// nearly every draw, for the lanes that are out; here a lane has up to eight
+// words in hand, so that a block is made for all lanes at once (top_up) and
+// only a lane that rejects several times makes one for itself.  ring: the
+// lane's column of the wave's kRing rows of 64 words; word w of the stream
+// is in row w mod kRing.
+constexpr uint32_t kRing = 8;
+struct RingStream
+{
+   uint32_t k0, k1, c0, c1, c3;
+   uint32_t next, end;           // the next word, the words made (a multiple of 4)
+   uint32_t *ring;
+   int have_gauss;
+   double g2;
+};
+
+__device__ __forceinline__ void ring_init (RingStream &s, uint32_t *ring, unsigned long long seed, uint32_t tag,
+                                           uint32_t stage, uint32_t source_id, uint32_t word)
+{
+   s.k0 = (uint32_t) seed;
+   s.k1 = (uint32_t) (seed >> 32);
+   s.c0 = tag; s.c1 = stage; s.c3 = source_id;
+   s.next = word;
+   s.end = word & ~3u;
+   s.ring = ring;
+   s.have_gauss = 0;
+   s.g2 = 0.0;
+}
+
+__device__ __forceinline__ void ring_fill (RingStream &s)
+{
+   uint32_t w0, w1, w2, w3;
+   philox (s.c0, s.c1, s.end >> 2, s.c3, s.k0, s.k1, w0, w1, w2, w3);
+   uint32_t *r = s.ring + (s.end & (kRing - 1u)) * 64u;
+   r[0] = w0;
+   r[64] = w1;
+   r[128] = w2;
+   r[192] = w3;
+   s.end += 4;
+}
+
+// another block where there is room for it
+__device__ __forceinline__ void top_up (RingStream &s)
+{
+   if ((int) (s.end - s.next) <= 4) ring_fill (s);
+}
+
+// at least n words in hand (n <= 5)
+__device__ __forceinline__ void need (RingStream &s, int n)
+{
+   while ((int) (s.end - s.next) < n) ring_fill (s);
+}
+
+// the next word, in hand already
+__device__ __forceinline__ double take (RingStream &s)
+{
+   const uint32_t u = s.ring[(s.next & (kRing - 1u)) * 64u];
+   s.next++;
+   return (double) u * (1.0 / ((double) 0xFFFFFFFFu));
+}
+
+__device__ __forceinline__ double gaussian (RingStream &s)
+{
+   if (s.have_gauss)
      {
-        g1 = 2.0 * uniform (s) - 1.0;
-        g2 = 2.0 * uniform (s) - 1.0;
-        g = g1 * g1 + g2 * g2;
+        s.have_gauss = 0;
+        return s.g2;
      }
-   while ((g >= 1.0) || (g == 0.0));
-   // sqrt (l / g) as l / sqrt (l g): 0 < g < 1, so l > 0
-   const double l = -2.0 * log_n (g);
-   const double f = l * rsqrt_n (l * g);
+   s.have_gauss = 1;
+   double g1, g2, g;
+   for (;;)
+     {
+        need (s, 2);
+        const double u1 = take (s), u2 = take (s);
+        if (polar_pair (u1, u2, g1, g2, g)) break;
+     }
+   const double f = polar_scale (g);
    s.g2 = g2 * f;
    return g1 * f;
 }
@@ -481,19 +573,26 @@ __device__ __forceinline__ double reflectivity (double cos_theta, double beta, d
 
 // ---- WFold scattering-angle tables -------------------------------------------------
 
-__device__ __forceinline__ double fold_theta (const double *__restrict__ fa, const float *__restrict__ farena, double p)
+// The angle of one scattering array at p: 0 below its table, a power law
+// above, linear between its entries.
+struct FoldRecord
 {
-   double p_min = fa[1];
-   if (p < p_min) return 0.0;
-   double p_max = fa[3];
-   if (p > p_max) return pow (fa[4] * (1.0 - p), fa[5]);
-   unsigned int num = (unsigned int) fa[6];
-   const float *t = farena + (unsigned int) fa[7];
-   double delta_i = div_n (p - p_min, fa[2]);
-   unsigned int i = (unsigned int) delta_i;
-   if (i + 1 >= num) return (double) t[num - 1];
+   double e_alpha, p_min, delta_p, p_max, norm, expon, num, off;
+};
+
+__device__ __forceinline__ double fold_theta (const FoldRecord &f, const float *__restrict__ farena, double p)
+{
+   if (p < f.p_min) return 0.0;
+   if (p > f.p_max) return pow (f.norm * (1.0 - p), f.expon);
+   const unsigned int num = (unsigned int) f.num;
+   const float *t = farena + (unsigned int) f.off;
+   double delta_i = div_n (p - f.p_min, f.delta_p);
+   const unsigned int i = (unsigned int) delta_i;
+   // past the last interval: the last entry twice
+   const unsigned int i0 = (i + 1 >= num) ? num - 1 : i, i1 = (i + 1 >= num) ? num - 1 : i + 1;
    delta_i -= (double) i;
-   return (1.0 - delta_i) * (double) t[i] + delta_i * (double) t[i + 1];
+   const double t0 = (double) t[i0], t1 = (double) t[i1];
+   return (i1 == i0) ? t0 : (1.0 - delta_i) * t0 + delta_i * t1;
 }
 
 // e_alphas: the table's e_alpha values (float32 file values, exact in
@@ -509,8 +608,8 @@ __device__ __forceinline__ double wfold_interp (const mxg_wfold &w, const float 
                                                 const float *__restrict__ cnt = nullptr)
 {
    if (w.n_arrays == 0) return 0.0;
-   const double *arrays = da + w.arrays_off;
-   if (w.n_arrays == 1) return fold_theta (arrays, fa, r);
+   const FoldRecord *arrays = (const FoldRecord *) (da + w.arrays_off);
+   if (w.n_arrays == 1) return fold_theta (arrays[0], fa, r);
    double e_alpha = energy * sin_alpha;
    unsigned int i;
    if constexpr (sizeof (T) == sizeof (float))
@@ -520,8 +619,10 @@ __device__ __forceinline__ double wfold_interp (const mxg_wfold &w, const float 
      i = search_w (e_alpha, e_alphas, w.n_arrays);
    if (i == w.n_arrays) i--;
    if (i == 0) i++;
-   double theta_0 = fold_theta (arrays + (i - 1) * MXG_FOLD_STRIDE, fa, r);
-   double theta_1 = fold_theta (arrays + i * MXG_FOLD_STRIDE, fa, r);
+   // both records at once, before what is asked of them branches
+   const FoldRecord f0 = arrays[i - 1], f1 = arrays[i];
+   const double theta_0 = fold_theta (f0, fa, r);
+   const double theta_1 = fold_theta (f1, fa, r);
    double e0 = (double) e_alphas[i - 1], e1 = (double) e_alphas[i];
    return theta_0 + div_n ((theta_1 - theta_0) * (e_alpha - e0), e1 - e0);
 }

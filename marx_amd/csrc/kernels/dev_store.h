@@ -6,6 +6,7 @@
 #include <stdint.h>
 #include "marx_gpu.h"
 #include "marx_gpu_cfg.h"
+#include "dev_math.h"
 
 namespace mxg {
 
@@ -26,6 +27,24 @@ struct Soa
    int8_t *sup[4];
    uint32_t *tag;
 };
+
+// The stages' search tables as the host lays them out for LDS (hrma_image,
+// grating_image), in HBM: 16-byte words at img, n16 of them.
+struct LdsImage
+{
+   const uint4 *img;
+   uint32_t n16;
+};
+
+// Copies n16 16-byte words of a host-made LDS image into LDS.  Every thread
+// has several loads in flight: the staging is one round of memory latency,
+// where copying table by table it was a dozen.
+__device__ __forceinline__ void stage_image (const uint4 *__restrict__ img, uint32_t n16, unsigned char *lds)
+{
+   uint4 *dst = (uint4 *) lds;
+#pragma unroll 4
+   for (uint32_t w = threadIdx.x; w < n16; w += blockDim.x) dst[w] = img[w];
+}
 
 // Per-stage launch arguments: the active index list in, the survivors out.
 //
@@ -74,17 +93,48 @@ struct PhotonOut
    int shell;
 };
 
+// Entry i of a column.  Columns are below 2^32 bytes (a launch takes at most
+// 2^28 photons), so the byte offset is formed in 32 bits and added to the
+// column's address, a scalar, by the memory instruction itself.
+template <class T>
+__device__ __forceinline__ T &at (T *col, uint32_t i)
+{
+   return *(T *) ((char *) col + (uint32_t) (i * (uint32_t) sizeof (T)));
+}
+
+// the path columns of photon id
+__device__ __forceinline__ void store_path (const Soa &s, uint32_t id, vec3 x, vec3 p, uint32_t flags)
+{
+   at (s.x0, id) = x.x; at (s.x1, id) = x.y; at (s.x2, id) = x.z;
+   at (s.p0, id) = p.x; at (s.p1, id) = p.y; at (s.p2, id) = p.z;
+   at (s.flags, id) = flags;
+}
+
 // a survivor's row of a relay
 __device__ __forceinline__ void relay_put (const Relay &r, uint32_t q, const PhotonOut &o)
 {
-   r.x0[q] = o.x0; r.x1[q] = o.x1; r.x2[q] = o.x2;
-   r.p0[q] = o.p0; r.p1[q] = o.p1; r.p2[q] = o.p2;
-   r.energy[q] = o.energy;
-   r.tag[q] = o.tag;
-   r.flags[q] = o.flags;
-   r.shell[q] = (uint8_t) o.shell;
+   at (r.x0, q) = o.x0; at (r.x1, q) = o.x1; at (r.x2, q) = o.x2;
+   at (r.p0, q) = o.p0; at (r.p1, q) = o.p1; at (r.p2, q) = o.p2;
+   at (r.energy, q) = o.energy;
+   at (r.tag, q) = o.tag;
+   at (r.flags, q) = o.flags;
+   at (r.shell, q) = (uint8_t) o.shell;
 }
 
+
+// A kernel's first argument, read again from its argument segment.  A loop
+// that uses some thirty columns loads their addresses where it needs them;
+// the compiler would otherwise load them all before the loop, more than the
+// scalar registers hold, and keep the rest in lanes of vector registers, an
+// instruction and a wait for each use.
+template <class T>
+__device__ __forceinline__ T kernel_args ()
+{
+   typedef const __attribute__ ((address_space (4))) T *Segment;
+   Segment p = (Segment) __builtin_amdgcn_kernarg_segment_ptr ();
+   asm volatile ("" : "+s" (p));
+   return *(const T *) p;
+}
 
 struct BlockRange { uint32_t lo, hi; };
 
@@ -225,9 +275,10 @@ struct HrmaScratch
 {
    uint32_t *idx_mid;      // photons that hit the paraboloid (capacity entries)
    uint32_t *n_mid;        // its length (written by k_compact)
-   uint32_t *rng_pos;      // per photon: random-stream position at the split
+   uint32_t *rng_pos;      // per photon: random-stream word at the split
    uint32_t reflect_grid;  // blocks of k_hrma_reflect
    int reflect_waves;      // 2, 3 or 4: the instance of k_hrma_reflect launched
+   LdsImage image;         // the mirror's tables
    uint32_t *n_mid_copy = nullptr;  // when non-null, also receives the middle list's length
 };
 
@@ -249,7 +300,7 @@ hipError_t launch_hrma (const mxg_config *cfg, const mxg_config *hcfg, const flo
 // stream positions in rng_pos) to io's survivor segments (io.grid blocks;
 // the caller compacts them); waves: the instance launched (2, 3 or 4)
 hipError_t launch_hrma_reflect (const mxg_config *cfg, const mxg_config *hcfg, const float *fa,
-                                const double *da, Soa s, ListIO io, const uint32_t *rng_pos, int waves,
+                                const double *da, Soa s, ListIO io, const uint32_t *rng_pos, LdsImage image, int waves,
                                 unsigned long long seed, uint32_t source_id, const Relay *relay_out,
                                 hipStream_t st);
 // The blocks of k_grating that one CU holds at once for configuration hcfg
@@ -257,15 +308,14 @@ hipError_t launch_hrma_reflect (const mxg_config *cfg, const mxg_config *hcfg, c
 // the runtime cannot say.  A grid of whole rounds of them measured fastest
 // (HETG + ACIS-S: 3 blocks per CU 0.36 ms, 4 0.47 ms, 8 0.40 ms).
 uint32_t grating_blocks_per_cu (const mxg_config *hcfg);
-// hcfg: the host copy of cfg (for the layout of the tables the kernel
-// stages in LDS); letg: the instance compiled for the LETG pass; relay_in,
+// hcfg: the host copy of cfg; image: the tables the kernel stages in LDS; letg: the instance compiled for the LETG pass; relay_in,
 // when non-null:
 // the input list is the mirror's with this relay, whose rows the kernel
 // reads instead of the store's; relay_out, when non-null: the survivors go
 // to it for launch_detect, which stores their x, p and flags (the kernel
 // stores those of the photons it drops only)
 hipError_t launch_grating (const mxg_config *cfg, const mxg_config *hcfg, const float *fa, const double *da, Soa s,
-                           ListIO io, uint32_t n_upper, unsigned long long seed,
+                           ListIO io, LdsImage image, uint32_t n_upper, unsigned long long seed,
                            uint32_t source_id, bool letg, const Relay *relay_in, const Relay *relay_out,
                            hipStream_t st);
 // fef: run the variant with the ACIS FEF step (the configuration read a FEF
@@ -298,6 +348,15 @@ hipError_t launch_source (const mxg_config *cfg, const float *fa, const double *
                           uint32_t *first_over, uint32_t *count, uint32_t *count_copy, uint32_t *idx, bool point,
                           bool entry_follows, hipStream_t st);
 
+// The arrival-time scan alone (launch_source's first pass, n > 0): ticks and
+// tile_tot filled, *first_over set to 0xFFFFFFFF, and the wall clock at its
+// start in *begin when non-null; *tile_off: the tiles' offsets for
+// source_photon (null for a single tile, whose offset is 0).
+hipError_t launch_source_scan (const mxg_config *cfg, const float *fa, const double *da, uint32_t n,
+                               uint32_t tag_start, unsigned long long seed, uint32_t source_id, uint64_t *ticks,
+                               uint64_t *tile_tot, uint32_t *first_over, uint64_t *begin, bool point,
+                               const uint64_t **tile_off, hipStream_t st);
+
 // Batched point sources (see source.hip): n photons over nsrc sources with
 // prefix offsets off[nsrc + 1] and unit directions dir[3 nsrc]; point: the
 // configured shape is a point (the instance without the extended shapes);
@@ -309,43 +368,8 @@ hipError_t launch_batch_source (const mxg_config *cfg, const double *da, Soa s, 
                                 uint32_t grid, bool point, bool entry_follows,
                                 hipStream_t st);
 
-// The batched pass as one persistent launch (persist.hip): blocks take
-// tiles of `tile` photons (a multiple of kBlock, at most kMaxPersistTile)
-// from *work and run every stage on them; the detected photons of the batch
-// end in idx_out / *n_out in id order, as after the staged pass.
-// stage_count (4 entries) receives the photons into the reflection and out
-// of the mirror, grating and detector; seg (n entries), tile_count and
-// tile_off (ceil(n / tile) entries each) are scratch.  ev, when non-null:
-// two events around the persistent kernel.
+// largest persistent tile of a schedule
 constexpr uint32_t kMaxPersistTile = 4096;
-// waves per SIMD of the persistent kernel: 3 (168 VGPRs, 250-660 B of
-// spills per lane) measured 7 percent faster than 4 (128 VGPRs) and than 2
-// (no spills) on the batched ACIS-I pass
-#ifndef MXG_PERSIST_WAVES
-#define MXG_PERSIST_WAVES 3
-#endif
-struct PersistLaunch
-{
-   const mxg_config *cfg;        // device copy
-   const mxg_config *hcfg;       // host copy (LDS layout)
-   const float *fa;
-   const double *da;
-   Soa s;
-   uint32_t n;
-   const uint32_t *off;
-   uint32_t nsrc;
-   const double *dir;
-   const uint32_t *tag_start;
-   double exposure, start_time;
-   unsigned long long seed;
-   uint32_t *rng_pos, *work, *stage_count;
-   uint32_t tile, blocks;
-   uint32_t *seg, *tile_count, *tile_off, *idx_out, *n_out;
-   int grating;                  // 0 none, 1 HETG, 2 LETG
-   int kind;                     // detector family, -1 none
-   hipEvent_t *ev;
-};
-hipError_t launch_batch_persistent (const PersistLaunch &p, hipStream_t st);
 
 // The differentiable mirror (diff.hip).
 struct DiffOut

@@ -8,7 +8,10 @@
 #include <stdarg.h>
 #include <stdint.h>
 
+#include "hrma_stage.h"
+#include "grating_stage.h"
 #include "dev_store.h"
+#include "passes.h"
 #include "mxg_columns.h"
 #include "mxg_device.h"
 
@@ -32,6 +35,8 @@ mxg_config g_hcfg;                 // host copy of the device configuration
 int g_num_cus = 0;
 float *d_fa = nullptr;
 double *d_da = nullptr;
+unsigned char *d_images = nullptr;  // the LDS images: the mirror's, then the grating's
+LdsImage g_mirror_image, g_grating_image;
 size_t d_fa_cap = 0, d_da_cap = 0;
 unsigned int g_cfg_gen = 0;
 
@@ -49,6 +54,10 @@ uint32_t *d_counts = nullptr;      // [0],[1] list lengths, [2] source cut, [4] 
                                    // [8..15] per-stage survivor counts, [32] the persistent
                                    // pass's tile counter, [36..39] its stage counts
 uint32_t *h_counts = nullptr;      // pinned host copy of d_counts[8..15], read once per call
+TraceReport *d_trace = nullptr;    // running sums of the trace as chunk kernels (passes.hip)
+TraceReport *h_trace = nullptr;    // ... and its report, in pinned memory
+uint32_t *d_trace_n = nullptr, *d_trace_counts = nullptr;  // its length and block counts
+double g_clock_khz = 1.0e5;        // rate of the device's wall clock
 uint32_t *d_tile_cnt = nullptr;    // the persistent pass's per-tile counts and offsets
 size_t g_tile_cap = 0;             // entries of each
 int g_cur = 0;                     // list holding the active photons
@@ -112,6 +121,38 @@ int fail (const char *fmt, ...)
    return fail ("%s failed: %s", #call, hipGetErrorString (e_)); } while (0)
 
 size_t align256 (size_t n) { return (n + 255) & ~(size_t) 255; }
+
+// Bytes kept for each LDS image: what a CU has.  A larger one is not made
+// (n16 stays past what a launch accepts).
+constexpr size_t kImageBytes = 160 * 1024;
+
+// The LDS images of configuration *cfg into d_images (held since the set-up),
+// on the library's stream.
+int sync_images (const mxg_config *cfg, const float *fa, const double *da)
+{
+   static unsigned char host[2][kImageBytes];
+   const bool letg = cfg->grating.type == MARX_GRATING_LETG;
+   const bool grating = letg || (cfg->grating.type == MARX_GRATING_HETG);
+   const HrmaLds lay = hrma_lds_layout (cfg->hrma, da);
+   const GratingLds glay = grating ? grating_lds_layout (cfg->grating, letg) : GratingLds {};
+   const size_t m = hrma_image_bytes (lay);
+   const size_t g = grating ? grating_image_bytes (glay) : 0;
+   HIPCHECK (hipStreamSynchronize (g_stream));
+   if (m <= kImageBytes)
+     {
+        hrma_image (cfg->hrma, fa, da, lay, host[0]);
+        HIPCHECK (hipMemcpyAsync (d_images, host[0], m, hipMemcpyHostToDevice, g_stream));
+     }
+   if (grating && (g <= kImageBytes))
+     {
+        grating_image (cfg->grating, fa, da, glay, letg, host[1]);
+        HIPCHECK (hipMemcpyAsync (d_images + kImageBytes, host[1], g, hipMemcpyHostToDevice, g_stream));
+     }
+   HIPCHECK (hipStreamSynchronize (g_stream));
+   g_mirror_image = LdsImage {(const uint4 *) d_images, (uint32_t) (m / 16)};
+   g_grating_image = LdsImage {(const uint4 *) (d_images + kImageBytes), (uint32_t) (g / 16)};
+   return 0;
+}
 
 __global__ void k_set_u32 (uint32_t *p, uint32_t v) { *p = v; }
 
@@ -462,6 +503,20 @@ int mxgd_init (void)
    HIPCHECK (hipMalloc (&d_seg_count, kMaxSegments * sizeof (uint32_t)));
    HIPCHECK (hipMemset (d_counts, 0, 64 * sizeof (uint32_t)));
    HIPCHECK (hipHostMalloc ((void **) &h_counts, kSlots * sizeof (uint32_t), hipHostMallocDefault));
+   {
+      TraceReport zero;
+      memset (&zero, 0, sizeof (zero));
+      HIPCHECK (hipMalloc (&d_images, 2 * kImageBytes));
+      HIPCHECK (hipMalloc (&d_trace_n, sizeof (uint32_t)));
+      HIPCHECK (hipMalloc (&d_trace_counts, 4 * kMaxSegments * sizeof (uint32_t)));
+      HIPCHECK (hipMalloc (&d_trace, sizeof (TraceReport)));
+      HIPCHECK (hipMemcpy (d_trace, &zero, sizeof (zero), hipMemcpyHostToDevice));
+      HIPCHECK (hipHostMalloc ((void **) &h_trace, sizeof (TraceReport), hipHostMallocCoherent));
+      memset (h_trace, 0, sizeof (TraceReport));
+      int khz = 0;
+      HIPCHECK (hipDeviceGetAttribute (&khz, hipDeviceAttributeWallClockRate, dev));
+      if (khz > 0) g_clock_khz = (double) khz;
+   }
    if (scratch_setup (dev)) return -1;
    g_inited = 1;
    return 0;
@@ -509,6 +564,7 @@ int mxgd_sync_config (const mxg_config *cfg, const float *fa, unsigned int nf,
    g_grating_bpc = grating_blocks_per_cu (&g_hcfg);
    if (nf) HIPCHECK (hipMemcpy (d_fa, fa, nf * sizeof (float), hipMemcpyHostToDevice));
    if (nd) HIPCHECK (hipMemcpy (d_da, da, nd * sizeof (double), hipMemcpyHostToDevice));
+   if (sync_images (cfg, fa, da)) return -1;
    g_cfg_gen = generation;
    return 0;
 }
@@ -623,7 +679,7 @@ int mxgd_run_mirror (double source_distance, unsigned long long seed, int slot, 
    if (begin_stage (slot)) return -1;
    bool timed = (slot >= 0) && (g_upper > 0);
    HrmaScratch hs = {d_idx_mid, d_counts + 4, d_rng_pos, stage_grid (g_upper, MXGD_K_REFLECT),
-                     (int) g_sched.reflect_waves};
+                     (int) g_sched.reflect_waves, g_mirror_image};
    // photons entering each kernel: the active list, the middle list (the
    // latter's length copied by k_compact)
    if (timed) hs.n_mid_copy = slot_count (MXGD_SLOT_HRMA_REFLECT);
@@ -663,7 +719,7 @@ int mxgd_run_grating (unsigned long long seed, int slot, float *ms, int relay_in
         if (skip_stage (io)) return -1;
      }
    else
-     HIPCHECK (launch_grating (d_cfg, &g_hcfg, d_fa, d_da, g_soa, io, g_upper, seed, 0,
+     HIPCHECK (launch_grating (d_cfg, &g_hcfg, d_fa, d_da, g_soa, io, g_grating_image, g_upper, seed, 0,
                                g_hcfg.grating.type == MARX_GRATING_LETG, rin, rout, g_stream));
    g_relay_have = out_k;
    return end_stage (slot, ms);
@@ -802,6 +858,136 @@ int mxgd_set_created (unsigned int m)
 {
    if (m > g_n) return fail ("%u photons created in a store of %u", m, g_n);
    g_n = m;
+   return 0;
+}
+
+/* ---- the trace as chunk kernels ------------------------------------------------- */
+
+namespace {
+
+TraceArgs trace_args (unsigned int n, double exposure, double start_time, unsigned long long seed)
+{
+   TraceArgs a;
+   memset (&a, 0, sizeof (a));
+   a.cfg = d_cfg;
+   a.fa = d_fa;
+   a.da = d_da;
+   a.s = g_soa;
+   a.n = n;
+   a.seed = seed;
+   a.exposure = exposure;
+   a.start_time = start_time;
+   a.tstart = start_time;
+   a.rng_pos = d_rng_pos;
+   a.mirror = g_mirror_image;
+   a.grating = g_grating_image;
+   a.sums = d_trace;
+   a.report = h_trace;
+   a.n_dev = d_trace_n;
+   return a;
+}
+
+// The lists of the trace as kernels over the chunk, sized for n photons.
+PassLists pass_lists (unsigned int n)
+{
+   PassLists l;
+   l.create.idx_in = nullptr;
+   l.create.idx_out = d_idx_mid;
+   l.create.n_out = d_counts + 4;
+   l.create.seg = d_seg;
+   l.create.seg_count = d_seg_count;
+   l.create.grid = stage_grid (n, MXGD_K_ENTER);
+   l.create.n_in = d_trace_n;
+   l.mirror = l.create;
+   l.mirror.idx_in = d_idx_mid;
+   l.mirror.n_in = d_counts + 4;
+   l.mirror.idx_out = d_idx[0];
+   l.mirror.n_out = d_counts;
+   l.mirror.grid = stage_grid (n, MXGD_K_REFLECT);
+   l.relay = g_relay[0];
+   l.counts = d_trace_counts;
+   l.diffract_grid = stage_grid (n, MXGD_K_DETECT);
+   return l;
+}
+
+// The counts of the last launch by timing slot (the stream is synchronised),
+// and with ms its times: the stages of a kernel share its time by the cycles
+// its sampled blocks spent in each, and the source's includes the arrival-time
+// scan.
+void read_trace (unsigned int n, bool scanned, float *ms, unsigned int *counts)
+{
+   const TraceReport &r = *h_trace;
+   const bool grating = (g_hcfg.grating.type == MARX_GRATING_HETG) || (g_hcfg.grating.type == MARX_GRATING_LETG);
+   const uint32_t mirror = grating ? r.in[2] : r.in[4];
+   memset (counts, 0, kSlots * sizeof (unsigned int));
+   counts[0] = (scanned && (r.first_over < n)) ? r.first_over + 1 : n;
+   counts[1] = mirror;
+   counts[2] = grating ? r.in[4] : 0;
+   counts[3] = (g_hcfg.det.type > 0) ? r.in[5] : 0;
+   counts[MXGD_SLOT_HRMA_ENTER] = r.in[0];
+   counts[MXGD_SLOT_HRMA_REFLECT] = r.in[1];
+   if (ms == nullptr) return;
+   memset (ms, 0, kSlots * sizeof (float));
+   double t[6], scan = scanned ? (double) (r.create - r.scan) / g_clock_khz : 0.0;
+   const double length[3] = {(double) (r.mirror - r.create), (double) ((grating ? r.diffract : r.end) - r.mirror),
+                             grating ? (double) (r.end - r.diffract) : 0.0};
+   for (int k = 0; k < 6; k++)
+     {
+        const double both = (double) (r.busy[k & ~1] + r.busy[k | 1]);
+        t[k] = (both > 0.0) ? length[k / 2] / g_clock_khz * (double) r.busy[k] / both : 0.0;
+     }
+   // the second part of the mirror's kernel is the detector without a grating
+   if (!grating)
+     {
+        t[5] = t[3];
+        t[3] = 0.0;
+     }
+   ms[0] = (float) (t[0] + scan);
+   ms[1] = (float) (t[1] + t[2]);
+   ms[2] = (float) (t[3] + t[4]);
+   ms[3] = (float) t[5];
+   ms[MXGD_SLOT_HRMA_ENTER] = (float) t[1];
+   ms[MXGD_SLOT_HRMA_REFLECT] = (float) t[2];
+}
+
+} // namespace
+
+int mxgd_passes_fit (void)
+{
+   return (d_cfg != nullptr) && !g_hcfg.det.fef_on && (g_mirror_image.n16 <= 64 * 1024 / 16)
+     && (g_grating_image.n16 <= 64 * 1024 / 16);
+}
+
+int mxgd_run_passes (unsigned int n, unsigned int tag_start, double start_time, double exposure_time,
+                     unsigned long long seed, float *ms, unsigned int *counts)
+{
+   g_relay_have = -1;
+   if (!d_cfg) return fail ("configuration not on the device");
+   if (n == 0) return fail ("no photons to trace");
+   if (n > (1u << 26)) return fail ("chunk of %u photons exceeds the 2^26 limit of one launch", n);
+   if (ensure_capacity (n)) return -1;
+   TraceArgs a = trace_args (n, exposure_time, start_time, seed);
+   a.tag_start = tag_start;
+   const bool scanned = (g_hcfg.src.time_mode == MXG_TIME_POISSON);
+   if (scanned)
+     {
+        a.ticks = d_ticks;
+        a.first_over = d_counts + 2;
+        HIPCHECK (launch_source_scan (d_cfg, d_fa, d_da, n, tag_start, seed, 0, d_ticks, d_tile_tot, a.first_over,
+                                      &d_trace->scan, g_hcfg.src.type == MXG_SOURCE_POINT, &a.tile_off, g_stream));
+     }
+   HIPCHECK (launch_passes (a, &g_hcfg, pass_lists (n), g_stream));
+   HIPCHECK (hipStreamSynchronize (g_stream));
+   read_trace (n, scanned, ms, counts);
+   g_n = n;
+   g_upper = 0;
+   return 0;
+}
+
+int mxgd_read_passes (unsigned int n, float *ms, unsigned int *counts)
+{
+   HIPCHECK (hipStreamSynchronize (g_stream));
+   read_trace (n, false, ms, counts);
    return 0;
 }
 
@@ -1052,64 +1238,20 @@ int mxgd_run_batch_source (unsigned int n, double exposure, double start_time,
    return 0;
 }
 
-int mxgd_run_batch_persistent (unsigned int n, double exposure, double start_time,
-                               unsigned long long seed, int slot)
+int mxgd_run_batch_passes (unsigned int n, double exposure, double start_time, unsigned long long seed)
 {
    g_relay_have = -1;
    if (!d_cfg) return fail ("configuration not on the device");
-   if ((n > g_capacity) || (g_batch_nsrc == 0)) return fail ("batch not prepared");
-   if (g_sched.persist_tile == 0) return fail ("the schedule has no persistent tile");
-   if (g_hcfg.det.fef_on) return fail ("the persistent pass has no FEF step");
-   if (g_hcfg.src.type != MXG_SOURCE_POINT) return fail ("the persistent pass traces point sources only");
-   const uint32_t tiles = (n + g_sched.persist_tile - 1) / g_sched.persist_tile;
-   if (tiles > g_tile_cap) return fail ("persistent pass of %u tiles exceeds %zu", tiles, g_tile_cap);
-   bool timed = (slot >= 0) && (slot < kSlots) && !g_capturing;
-   if (timed)
-     {
-        HIPCHECK (hipEventRecord (g_tev[slot][0], g_stream));
-        g_slot_used[slot] = 1;
-     }
-   PersistLaunch p;
-   p.cfg = d_cfg;
-   p.hcfg = &g_hcfg;
-   p.fa = d_fa;
-   p.da = d_da;
-   p.s = g_soa;
-   p.n = n;
-   p.off = d_batch_off;
-   p.nsrc = g_batch_nsrc;
-   p.dir = d_batch_dir;
-   p.tag_start = d_batch_tag;
-   p.exposure = exposure;
-   p.start_time = start_time;
-   p.seed = seed;
-   p.rng_pos = d_rng_pos;
-   p.work = d_counts + 32;
-   p.stage_count = d_counts + 36;
-   p.tile = g_sched.persist_tile;
-   p.blocks = (uint32_t) (g_num_cus > 0 ? g_num_cus : 256) * g_sched.persist_blocks_per_cu;
-   p.seg = d_seg;
-   p.tile_count = d_tile_cnt;
-   p.tile_off = d_tile_cnt + g_tile_cap;
-   p.idx_out = d_idx[1];
-   p.n_out = d_counts + 1;
-   p.grating = (g_hcfg.grating.type == MARX_GRATING_HETG) ? 1 : (g_hcfg.grating.type == MARX_GRATING_LETG) ? 2 : 0;
-   p.kind = (g_hcfg.det.type > 0) ? detector_kind (g_hcfg) : -1;
-   p.ev = nullptr;
-   HIPCHECK (launch_batch_persistent (p, g_stream));
-   if (timed)
-     HIPCHECK (hipEventRecord (g_tev[slot][1], g_stream));
-   // the per-stage counts where the staged pass leaves them: photons into
-   // the two mirror kernels, out of the mirror, grating and detector
-   hipLaunchKernelGGL (k_set_u32, dim3 (1), dim3 (1), 0, g_stream, d_counts + 8 + MXGD_SLOT_HRMA_ENTER, (uint32_t) n);
-   hipLaunchKernelGGL (k_copy_u32, dim3 (1), dim3 (1), 0, g_stream, d_counts + 8 + MXGD_SLOT_HRMA_REFLECT,
-                       d_counts + 36);
-   for (int k = 1; k <= 3; k++)
-     hipLaunchKernelGGL (k_copy_u32, dim3 (1), dim3 (1), 0, g_stream, d_counts + 8 + k, d_counts + 36 + k);
-   HIPCHECK (hipGetLastError ());
-   g_cur = 1;
+   if ((n == 0) || (n > g_capacity) || (g_batch_nsrc == 0)) return fail ("batch not prepared");
+   TraceArgs a = trace_args (n, exposure, start_time, seed);
+   a.off = d_batch_off;
+   a.nsrc = g_batch_nsrc;
+   a.dir = d_batch_dir;
+   a.batch_tag = d_batch_tag;
+   HIPCHECK (launch_passes (a, &g_hcfg, pass_lists (n), g_stream));
+   g_cur = 0;
    g_n = n;
-   g_upper = n;
+   g_upper = 0;
    return 0;
 }
 
@@ -1345,6 +1487,7 @@ int mxgd_trace_noalloc (const mxg_soa_view *v, unsigned int n, unsigned int tag_
         if (nd) HIPCHECK (hipMemcpyAsync (d_da, da, nd * sizeof (double), hipMemcpyHostToDevice, g_stream));
         HIPCHECK (hipStreamSynchronize (g_stream));
         memcpy (&g_hcfg, cfg, sizeof (mxg_config));
+        if (sync_images (cfg, fa, da)) return -1;
         g_grating_bpc = grating_blocks_per_cu (&g_hcfg);
         g_cfg_gen = generation;
      }
@@ -1414,14 +1557,14 @@ int mxgd_trace_noalloc (const mxg_soa_view *v, unsigned int n, unsigned int tag_
       return hipGetLastError ();
    };
    HIPCHECK (clear_out ());
-   HrmaScratch hs = {mid, counts + 4, rng, io (MXGD_K_REFLECT).grid, (int) g_sched.reflect_waves};
+   HrmaScratch hs = {mid, counts + 4, rng, io (MXGD_K_REFLECT).grid, (int) g_sched.reflect_waves, g_mirror_image};
    HIPCHECK (launch_hrma (c_cfg, cfg, c_fa, c_da, s, io (MXGD_K_ENTER), hs, n, cfg->src.distance, seed, 0,
                           nullptr, false, g_stream, nullptr));
    cur = 1 - cur;
    if ((cfg->grating.type == MARX_GRATING_HETG) || (cfg->grating.type == MARX_GRATING_LETG))
      {
         HIPCHECK (clear_out ());
-        HIPCHECK (launch_grating (c_cfg, cfg, c_fa, c_da, s, io (MXGD_K_GRATING), n, seed, 0,
+        HIPCHECK (launch_grating (c_cfg, cfg, c_fa, c_da, s, io (MXGD_K_GRATING), g_grating_image, n, seed, 0,
                                   cfg->grating.type == MARX_GRATING_LETG, nullptr, nullptr, g_stream));
         cur = 1 - cur;
      }

@@ -354,15 +354,16 @@ __device__ __forceinline__ double wfold_d1 (const mxg_wfold &w, const float *__r
 {
    dval = 0.0;
    if (w.n_arrays == 0) return 0.0;
-   const double *arrays = da + w.arrays_off;
-   if (w.n_arrays == 1) return fold_theta (arrays, fa, r);
+   const FoldRecord *arrays = (const FoldRecord *) (da + w.arrays_off);
+   if (w.n_arrays == 1) return fold_theta (arrays[0], fa, r);
    const double *e_alphas = da + w.e_alphas_off;
    double e_alpha = energy * sin_alpha;
    unsigned int i = search_w (e_alpha, e_alphas, w.n_arrays);
    if (i == w.n_arrays) i--;
    if (i == 0) i++;
-   double theta_0 = fold_theta (arrays + (i - 1) * MXG_FOLD_STRIDE, fa, r);
-   double theta_1 = fold_theta (arrays + i * MXG_FOLD_STRIDE, fa, r);
+   const FoldRecord f0 = arrays[i - 1], f1 = arrays[i];
+   const double theta_0 = fold_theta (f0, fa, r);
+   const double theta_1 = fold_theta (f1, fa, r);
    double e0 = e_alphas[i - 1], e1 = e_alphas[i];
    dval = (theta_1 - theta_0) / (e1 - e0) * energy;
    return theta_0 + (theta_1 - theta_0) * (e_alpha - e0) / (e1 - e0);

@@ -10,18 +10,18 @@ namespace mxg {
 // RIN: the input list is the mirror's with relay rin (list entry i at row
 // rin.pos[i]); ROUT: the survivors' columns also go to rout at their
 // segment slots.  The block first stages the search tables (energies,
-// bucket counts, orders, sectors) in LDS at the layout lay: they are the
+// bucket counts, orders, sectors; grating_image) in LDS: they are the
 // targets of each photon's chains of dependent loads.
 template <bool LETG, int W, bool RIN, bool ROUT>
 __global__ __launch_bounds__ (kBlock, W > 0 ? W : 1)
 void k_grating (const mxg_config *__restrict__ cfg, const float *__restrict__ fa,
                 const double *__restrict__ da, Soa s, ListIO io,
-                unsigned long long seed, uint32_t source_id, GratingLds lay, Relay rin, Relay rout)
+                unsigned long long seed, uint32_t source_id, LdsImage image, Relay rin, Relay rout)
 {
    const mxg_grating_cfg &gc = cfg->grating;
    extern __shared__ __align__ (16) unsigned char lds[];
    float *ltab = (float *) (lds + kGratingTabOff);
-   stage_grating_tables (gc, fa, da, lay, LETG, lds, ltab);
+   stage_image (image.img, image.n16, lds);
    __syncthreads ();
    const GratingLds *L = (const GratingLds *) lds;
    __shared__ uint32_t seg_wc[2 * (kBlock / 64)];
@@ -49,29 +49,29 @@ void k_grating (const mxg_config *__restrict__ cfg, const float *__restrict__ fa
 template <bool LETG, int W>
 static void launch_io (dim3 g, size_t lds_bytes, hipStream_t st, const mxg_config *cfg, const float *fa,
                        const double *da, Soa s, ListIO io, unsigned long long seed, uint32_t source_id,
-                       const GratingLds &lay, const Relay *rin, const Relay *rout)
+                       const LdsImage &image, const Relay *rin, const Relay *rout)
 {
    const Relay a = rin ? *rin : Relay {}, b = rout ? *rout : Relay {};
    const dim3 blk (kBlock);
    if (rin && rout)
      hipLaunchKernelGGL ((k_grating<LETG, W, true, true>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, lay, a, b);
+                         source_id, image, a, b);
    else if (rin)
      hipLaunchKernelGGL ((k_grating<LETG, W, true, false>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, lay, a, b);
+                         source_id, image, a, b);
    else if (rout)
      hipLaunchKernelGGL ((k_grating<LETG, W, false, true>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, lay, a, b);
+                         source_id, image, a, b);
    else
      hipLaunchKernelGGL ((k_grating<LETG, W, false, false>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, lay, a, b);
+                         source_id, image, a, b);
 }
 
 uint32_t grating_blocks_per_cu (const mxg_config *hcfg)
 {
    const bool letg = hcfg->grating.type == MARX_GRATING_LETG;
    const GratingLds lay = grating_lds_layout (hcfg->grating, letg);
-   const size_t lds_bytes = kGratingTabOff + (size_t) lay.floats * sizeof (float);
+   const size_t lds_bytes = grating_image_bytes (lay);
    int n = 0;
    const hipError_t e
      = letg ? hipOccupancyMaxActiveBlocksPerMultiprocessor (&n, k_grating<true, MXG_LETG_GRATING_WAVES, false, false>,
@@ -82,21 +82,20 @@ uint32_t grating_blocks_per_cu (const mxg_config *hcfg)
 }
 
 hipError_t launch_grating (const mxg_config *cfg, const mxg_config *hcfg, const float *fa, const double *da,
-                           Soa s, ListIO io, uint32_t n_upper, unsigned long long seed,
+                           Soa s, ListIO io, LdsImage image, uint32_t n_upper, unsigned long long seed,
                            uint32_t source_id, bool letg, const Relay *relay_in, const Relay *relay_out,
                            hipStream_t st)
 {
    if (n_upper == 0) return hipSuccess;
    const dim3 g (io.grid);
-   const GratingLds lay = grating_lds_layout (hcfg->grating, letg);
-   const size_t lds_bytes = kGratingTabOff + (size_t) lay.floats * sizeof (float);
+   const size_t lds_bytes = (size_t) image.n16 * 16;
    if (lds_bytes > 64 * 1024)
      return hipErrorInvalidConfiguration;
    if (letg)
-     launch_io<true, MXG_LETG_GRATING_WAVES> (g, lds_bytes, st, cfg, fa, da, s, io, seed, source_id, lay,
+     launch_io<true, MXG_LETG_GRATING_WAVES> (g, lds_bytes, st, cfg, fa, da, s, io, seed, source_id, image,
                                              relay_in, relay_out);
    else
-     launch_io<false, MXG_GRATING_WAVES> (g, lds_bytes, st, cfg, fa, da, s, io, seed, source_id, lay, relay_in,
+     launch_io<false, MXG_GRATING_WAVES> (g, lds_bytes, st, cfg, fa, da, s, io, seed, source_id, image, relay_in,
                                          relay_out);
    hipError_t e = hipGetLastError ();
    if (e == hipSuccess) e = launch_compact (io, st, relay_out ? relay_out->pos : nullptr);

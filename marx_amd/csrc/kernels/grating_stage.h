@@ -13,6 +13,7 @@
 //   one lane touches two contiguous rows.
 #pragma once
 
+#include <string.h>
 #include "dev_common.h"
 #include "dev_store.h"
 
@@ -269,33 +270,33 @@ inline GratingLds grating_lds_layout (const mxg_grating_cfg &gc, bool letg)
    return lay;
 }
 
-// Stages the tables of lay in LDS (the layout at lds, the tables at ltab =
-// lds + kGratingTabOff); letg as for the layout.  The caller synchronises.
-__device__ __forceinline__ void stage_grating_tables (const mxg_grating_cfg &gc, const float *__restrict__ fa,
-                                                      const double *__restrict__ da, const GratingLds &lay,
-                                                      bool letg, unsigned char *lds, float *ltab)
+// The LDS image of the tables of lay, made by the host from the arenas fa,
+// da: lay at 0, the tables at kGratingTabOff (letg as for the layout),
+// grating_image_bytes of it, a multiple of 16.
+inline size_t grating_image_bytes (const GratingLds &lay)
 {
-   if (threadIdx.x == 0) *(GratingLds *) lds = lay;
+   return (kGratingTabOff + (size_t) lay.floats * sizeof (float) + 15) & ~(size_t) 15;
+}
+
+inline void grating_image (const mxg_grating_cfg &gc, const float *fa, const double *da, const GratingLds &lay,
+                           bool letg, unsigned char *img)
+{
+   memset (img, 0, grating_image_bytes (lay));
+   memcpy (img, &lay, sizeof (lay));
+   float *tab = (float *) (img + kGratingTabOff);
+   auto put = [&] (uint32_t at, uint32_t off, uint32_t n) { if (n) memcpy (tab + at, fa + off, n * sizeof (float)); };
    for (int k = 0; k < 6; k++)
      {
         if ((k >= MXG_NUM_SHELLS) && !(letg && ((k == MXG_NUM_SHELLS) ? gc.has_fine : gc.has_coarse)))
           continue;
         const mxg_grating &g = grating_of (gc, k);
-        for (uint32_t w = threadIdx.x; w < g.num_energies; w += blockDim.x)
-          ltab[lay.e[k] + w] = fa[g.energies_off + w];
-        const uint32_t nb = bucket_floats (g.e_bucket);
-        for (uint32_t w = threadIdx.x; w < nb; w += blockDim.x)
-          ltab[lay.bk[k] + w] = fa[g.e_bucket.off + w];
-        for (uint32_t w = threadIdx.x; w < g.num_orders; w += blockDim.x)
-          ltab[lay.ord[k] + w] = fa[g.orders_off + w];
+        put (lay.e[k], g.energies_off, g.num_energies);
+        put (lay.bk[k], g.e_bucket.off, bucket_floats (g.e_bucket));
+        put (lay.ord[k], g.orders_off, g.num_orders);
      }
    for (int sh = 0; sh < MXG_NUM_SHELLS; sh++)
-     {
-        double *dst = (double *) (ltab + lay.sec[sh]);
-        const uint32_t n = 6 * gc.sectors[sh].n;
-        for (uint32_t w = threadIdx.x; w < n; w += blockDim.x)
-          dst[w] = da[gc.sectors[sh].off + w];
-     }
+     if (gc.sectors[sh].n)
+       memcpy (tab + lay.sec[sh], da + gc.sectors[sh].off, 6 * gc.sectors[sh].n * sizeof (double));
 }
 
 // The tables of grating k (0-3 by shell, 4 fine, 5 coarse) and, for k < 4,
@@ -327,16 +328,107 @@ __device__ __forceinline__ GratingTabs grating_tabs (const mxg_grating_cfg &gc, 
    return t;
 }
 
-// k_grating's work for photon id: vignetting, the Rowland torus, the order
-// draw and diffraction, and for LETG the support gratings.  True when the
-// photon leaves the grating stage alive, its columns then also in o.
+// The stream of a photon after its vignetting and order draws.
+__device__ __forceinline__ void resume_diffraction (Stream &st, unsigned long long seed, uint32_t tag,
+                                                    uint32_t source_id)
+{
+   uint32_t w0, w1;
+   stream_init (st, seed, tag, MXG_STAGE_GRATING, source_id);
+   philox (st.c0, st.c1, 0u, st.c3, st.k0, st.k1, w0, w1, st.b0, st.b1);
+   st.c2 = 1;
+   st.pos = 2;
+}
+
+// The grating stage of one photon in two parts, at the order draw: most
+// photons find no order (four in five for HETG), and what follows costs
+// more than what comes before.
+enum GratingStep
+{
+   GRATING_VIGNETTED,           // flags only: the photon keeps its path
+   GRATING_NO_ORDER,            // its path is final
+   GRATING_DIFFRACTS            // on the torus, in the grating's frame, with an order
+};
+
+// The vignetting draw, the frame rotation, the Rowland torus and the order
+// draw of a photon of shell `shell`.  STAGED: the search tables are read from
+// LDS (layout L, tables ltab, as k_grating stages them), else from the
+// arenas.
+template <bool STAGED>
+__device__ __forceinline__ GratingStep grating_enter_core (const mxg_grating_cfg &gc, const float *__restrict__ fa,
+                                                           const double *__restrict__ da, const GratingLds *L,
+                                                           const float *ltab, int shell, double energy, vec3 &x,
+                                                           vec3 &p, uint32_t &flags, int8_t &order, Stream &st)
+{
+   const mxg_grating &g = gc.g[shell];
+   if (uniform (st) > g.vig)
+     {
+        flags |= PHOTON_MIRROR_VBLOCKED;
+        return GRATING_VIGNETTED;
+     }
+   x = turn_x_f (x, g.disp_cos, -g.disp_sin);
+   p = turn_x_f (p, g.disp_cos, -g.disp_sin);
+   if (!torus_intersect (x, p, gc.rowland[shell]))
+     flags |= PHOTON_UNDIFFRACTED;
+   const GratingTabs t = grating_tabs<STAGED> (gc, shell, fa, da, L, ltab);
+   const int k = draw_order (g, fa, t.E, t.bcnt, (double) (float) energy, uniform (st));
+   if (k >= 0)
+     {
+        order = (int8_t) (int) t.orders[k];
+        return GRATING_DIFFRACTS;
+     }
+   flags |= PHOTON_UNDIFFRACTED;
+   x = turn_x_f (x, g.disp_cos, g.disp_sin);
+   p = turn_x_f (p, g.disp_cos, g.disp_sin);
+   return GRATING_NO_ORDER;
+}
+
+// A GRATING_DIFFRACTS photon from there on: the diffraction, for LETG the
+// support gratings (their orders to sup), and the rotation back.  True when
+// it leaves the grating alive.
+template <bool LETG, bool STAGED>
+__device__ __forceinline__ bool grating_leave_core (const mxg_grating_cfg &gc, const float *__restrict__ fa,
+                                                    const double *__restrict__ da, const GratingLds *L,
+                                                    const float *ltab, int shell, double energy, int8_t order,
+                                                    vec3 &x, vec3 &p, uint32_t &flags, int8_t *const *sup,
+                                                    uint32_t id, Stream &st)
+{
+   const mxg_grating &g = gc.g[shell];
+   const GratingTabs t = grating_tabs<STAGED> (gc, shell, fa, da, L, ltab);
+   if (-1 == diffract_photon (g, t.nsec, t.sec, 0.0, energy, x, p, (int) order, st))
+     flags |= PHOTON_UNDIFFRACTED;
+   if constexpr (LETG)
+     {
+        const double ef = (double) (float) energy;
+        for (int pass = 0; pass < 4; pass++)
+          {
+             const bool fine = (pass == 0);
+             if (fine ? !gc.has_fine : !gc.has_coarse) continue;
+             if (flags & BAD_PHOTON_MASK) continue;
+             const double theta = (pass == 0) ? MXG_PI / 2.0
+               : (pass == 1) ? MXG_PI / 3.0
+               : (pass == 2) ? 2.0 * MXG_PI / 3.0 : 0.0;
+             int8_t so = at (sup[pass], id);
+             if (-1 == diffract_from (fine ? gc.fine : gc.coarse,
+                                      grating_tabs<STAGED> (gc, fine ? MXG_NUM_SHELLS : MXG_NUM_SHELLS + 1, fa, da, L,
+                                                            ltab),
+                                      fa, theta, energy, ef, x, p, so, st))
+               flags |= PHOTON_UNDIFFRACTED;
+             at (sup[pass], id) = so;
+          }
+     }
+   x = turn_x_f (x, g.disp_cos, g.disp_sin);
+   p = turn_x_f (p, g.disp_cos, g.disp_sin);
+   return (flags & BAD_PHOTON_MASK) == 0;
+}
+
+// k_grating's work for photon id: both parts on the store's columns.  True
+// when the photon leaves the grating stage alive, its columns then also in o.
 // RELAY: its incoming x, p, energy, tag, flags and shell are read from row
 // `slot` of *relay instead of the store, where the mirror left x, p and
 // flags for this stage to write (a vignetted photon's as they came).
 // HANDOFF: the photons it keeps go on to the detector through o, and the
 // detector stores their x, p and flags; only the photons it drops have
-// theirs stored here.  STAGED: the search tables are read from LDS (layout
-// L, tables ltab, as k_grating stages them), else from the arenas.
+// theirs stored here.  STAGED: as grating_enter_core.
 template <bool LETG, bool RELAY = false, bool HANDOFF = false, bool STAGED = false>
 __device__ __forceinline__ bool grating_one (const mxg_grating_cfg &gc, const float *__restrict__ fa,
                                              const double *__restrict__ da, Soa s, uint32_t id,
@@ -345,78 +437,32 @@ __device__ __forceinline__ bool grating_one (const mxg_grating_cfg &gc, const fl
                                              const GratingLds *L = nullptr, const float *ltab = nullptr)
 {
    bool keep = false;
-   uint32_t flags = RELAY ? relay->flags[slot] : s.flags[id];
+   uint32_t flags = RELAY ? at (relay->flags, slot) : at (s.flags, id);
    if ((flags & BAD_PHOTON_MASK) == 0)
      {
         Stream st;
-        const uint32_t tag = RELAY ? relay->tag[slot] : s.tag[id];
+        const uint32_t tag = RELAY ? at (relay->tag, slot) : at (s.tag, id);
         stream_init (st, seed, tag, MXG_STAGE_GRATING, source_id);
-        const int shell = RELAY ? (int) relay->shell[slot] : (int) s.shell[id];
-        const mxg_grating &g = gc.g[shell];
-        if (uniform (st) > g.vig)
+        const int shell = RELAY ? (int) at (relay->shell, slot) : (int) at (s.shell, id);
+        vec3 x = RELAY ? v3 (at (relay->x0, slot), at (relay->x1, slot), at (relay->x2, slot)) : v3 (at (s.x0, id), at (s.x1, id), at (s.x2, id));
+        vec3 p = RELAY ? v3 (at (relay->p0, slot), at (relay->p1, slot), at (relay->p2, slot)) : v3 (at (s.p0, id), at (s.p1, id), at (s.p2, id));
+        const double energy = RELAY ? at (relay->energy, slot) : at (s.energy, id);
+        int8_t order = 0;
+        const GratingStep step = grating_enter_core<STAGED> (gc, fa, da, L, ltab, shell, energy, x, p, flags, order, st);
+        if (step == GRATING_DIFFRACTS)
           {
-             s.flags[id] = flags | PHOTON_MIRROR_VBLOCKED;
-             if (RELAY)
-               {
-                  s.x0[id] = relay->x0[slot]; s.x1[id] = relay->x1[slot]; s.x2[id] = relay->x2[slot];
-                  s.p0[id] = relay->p0[slot]; s.p1[id] = relay->p1[slot]; s.p2[id] = relay->p2[slot];
-               }
+             at (s.order, id) = order;
+             keep = grating_leave_core<LETG, STAGED> (gc, fa, da, L, ltab, shell, energy, order, x, p, flags, s.sup, id,
+                                                      st);
           }
-        else
-          {
-             vec3 x = RELAY ? v3 (relay->x0[slot], relay->x1[slot], relay->x2[slot])
-                            : v3 (s.x0[id], s.x1[id], s.x2[id]);
-             vec3 p = RELAY ? v3 (relay->p0[slot], relay->p1[slot], relay->p2[slot])
-                            : v3 (s.p0[id], s.p1[id], s.p2[id]);
-             const double energy = RELAY ? relay->energy[slot] : s.energy[id];
-             const double ef = (double) (float) energy;
-             int8_t order = s.order[id];
-
-             x = turn_x_f (x, g.disp_cos, -g.disp_sin);
-             p = turn_x_f (p, g.disp_cos, -g.disp_sin);
-             if (!torus_intersect (x, p, gc.rowland[shell]))
-               flags |= PHOTON_UNDIFFRACTED;
-             if (-1 == diffract_from (g, grating_tabs<STAGED> (gc, shell, fa, da, L, ltab), fa, 0.0, energy,
-                                      ef, x, p, order, st))
-               flags |= PHOTON_UNDIFFRACTED;
-             s.order[id] = order;
-
-             if constexpr (LETG)
-               {
-                  for (int pass = 0; pass < 4; pass++)
-                    {
-                       const bool fine = (pass == 0);
-                       if (fine ? !gc.has_fine : !gc.has_coarse) continue;
-                       if (flags & BAD_PHOTON_MASK) continue;
-                       const double theta = (pass == 0) ? MXG_PI / 2.0
-                         : (pass == 1) ? MXG_PI / 3.0
-                         : (pass == 2) ? 2.0 * MXG_PI / 3.0 : 0.0;
-                       int8_t so = s.sup[pass][id];
-                       if (-1 == diffract_from (fine ? gc.fine : gc.coarse,
-                                                grating_tabs<STAGED> (gc, fine ? MXG_NUM_SHELLS : MXG_NUM_SHELLS + 1,
-                                                                      fa, da, L, ltab),
-                                                fa, theta, energy, ef, x, p, so, st))
-                         flags |= PHOTON_UNDIFFRACTED;
-                       s.sup[pass][id] = so;
-                    }
-               }
-
-             x = turn_x_f (x, g.disp_cos, g.disp_sin);
-             p = turn_x_f (p, g.disp_cos, g.disp_sin);
-             keep = (flags & BAD_PHOTON_MASK) == 0;
-             if (!(HANDOFF && keep))
-               {
-                  s.x0[id] = x.x; s.x1[id] = x.y; s.x2[id] = x.z;
-                  s.p0[id] = p.x; s.p1[id] = p.y; s.p2[id] = p.z;
-                  s.flags[id] = flags;
-               }
-             o.x0 = x.x; o.x1 = x.y; o.x2 = x.z;
-             o.p0 = p.x; o.p1 = p.y; o.p2 = p.z;
-             o.energy = energy;
-             o.tag = tag;
-             o.flags = flags;
-             o.shell = shell;
-          }
+        if (!RELAY && (step == GRATING_VIGNETTED)) at (s.flags, id) = flags;
+        else if (!(HANDOFF && keep)) store_path (s, id, x, p, flags);
+        o.x0 = x.x; o.x1 = x.y; o.x2 = x.z;
+        o.p0 = p.x; o.p1 = p.y; o.p2 = p.z;
+        o.energy = energy;
+        o.tag = tag;
+        o.flags = flags;
+        o.shell = shell;
      }
    return keep;
 }

@@ -27,12 +27,12 @@ __global__ __launch_bounds__ (kBlock, MXG_ENTER_WAVES)
 #else
 __global__ __launch_bounds__ (kBlock)
 #endif
-void k_hrma_enter (const mxg_config *__restrict__ cfg, Soa s, ListIO io,
+void k_hrma_enter (const uint4 *__restrict__ image, Soa s, ListIO io,
                    uint32_t *__restrict__ rng_pos, uint32_t tilted, double source_distance,
                    unsigned long long seed, uint32_t source_id)
 {
-   __shared__ __align__ (16) unsigned char lds[sizeof (mxg_hrma_cfg)];
-   stage_hrma_cfg (cfg, lds);
+   __shared__ __align__ (16) unsigned char lds[kHrmaLayOff];
+   stage_image (image, kHrmaLayOff / 16, lds);
    __syncthreads ();
    const mxg_hrma_cfg &h = *(const mxg_hrma_cfg *) lds;
    __shared__ uint32_t seg_wc[2 * (kBlock / 64)];
@@ -62,15 +62,17 @@ void k_hrma_enter (const mxg_config *__restrict__ cfg, Soa s, ListIO io,
 // grating, which stores their x, p and flags.
 template <int WAVES, bool RELAY>
 __global__ __launch_bounds__ (kBlock, WAVES)
-void k_hrma_reflect (const mxg_config *__restrict__ cfg, const float *__restrict__ fa,
+void k_hrma_reflect (const float *__restrict__ fa,
                      const double *__restrict__ da, Soa s, ListIO io,
                      const uint32_t *__restrict__ rng_pos, unsigned long long seed,
-                     uint32_t source_id, HrmaLds lay, Relay relay)
+                     uint32_t source_id, LdsImage image, Relay relay)
 {
    extern __shared__ __align__ (16) unsigned char lds[];
+   __shared__ uint32_t rings[kBlock / 64][kRing][64];
    float *ltab = (float *) (lds + kHrmaTabOff);
-   stage_hrma_tables (cfg, fa, da, lay, lds, ltab);
+   stage_image (image.img, image.n16, lds);
    __syncthreads ();
+   uint32_t *ring = &rings[threadIdx.x >> 6][0][threadIdx.x & 63u];
 
    const mxg_hrma_cfg &h = *(const mxg_hrma_cfg *) lds;
    const HrmaLds &L = *(const HrmaLds *) (lds + kHrmaLayOff);
@@ -87,7 +89,7 @@ void k_hrma_reflect (const mxg_config *__restrict__ cfg, const float *__restrict
         if (i < range.hi)
           {
              id = io.idx_in[i];
-             keep = hrma_reflect_one<RELAY> (h, ltab, L, fa, da, s, id, rng_pos, seed, source_id, o);
+             keep = hrma_reflect_one<RELAY> (h, ltab, L, fa, da, ring, s, id, rng_pos, seed, source_id, o);
           }
         const uint32_t q = survivors.add (keep, id);
         if (RELAY && keep) relay_put (relay, q, o);
@@ -96,24 +98,23 @@ void k_hrma_reflect (const mxg_config *__restrict__ cfg, const float *__restrict
 }
 
 hipError_t launch_hrma_reflect (const mxg_config *cfg, const mxg_config *hcfg, const float *fa,
-                                const double *da, Soa s, ListIO io, const uint32_t *rng_pos, int waves,
+                                const double *da, Soa s, ListIO io, const uint32_t *rng_pos, LdsImage image, int waves,
                                 unsigned long long seed, uint32_t source_id, const Relay *relay_out,
                                 hipStream_t st)
 {
-   const HrmaLds lay = hrma_lds_layout (hcfg->hrma);
-   size_t lds_bytes = kHrmaTabOff + (size_t) lay.floats * sizeof (float);
+   const size_t lds_bytes = (size_t) image.n16 * 16;
    if (lds_bytes > 64 * 1024)
      return hipErrorInvalidConfiguration;
-   typedef void (*ReflectFn) (const mxg_config *, const float *, const double *, Soa, ListIO,
-                              const uint32_t *, unsigned long long, uint32_t, HrmaLds, Relay);
+   typedef void (*ReflectFn) (const float *, const double *, Soa, ListIO,
+                              const uint32_t *, unsigned long long, uint32_t, LdsImage, Relay);
    const bool r = relay_out != nullptr;
    const ReflectFn reflect
      = (waves <= 2) ? (r ? k_hrma_reflect<2, true> : k_hrma_reflect<2, false>)
        : (waves == 3) ? (r ? k_hrma_reflect<3, true> : k_hrma_reflect<3, false>)
        : (r ? k_hrma_reflect<MXG_REFLECT_WAVES_TOP, true> : k_hrma_reflect<MXG_REFLECT_WAVES_TOP, false>);
    const Relay rel = r ? *relay_out : Relay {};
-   hipLaunchKernelGGL (reflect, dim3 (io.grid), dim3 (kBlock), lds_bytes, st, cfg, fa, da, s, io, rng_pos,
-                       seed, source_id, lay, rel);
+   hipLaunchKernelGGL (reflect, dim3 (io.grid), dim3 (kBlock), lds_bytes, st, fa, da, s, io, rng_pos,
+                       seed, source_id, image, rel);
    return hipGetLastError ();
 }
 
@@ -123,8 +124,7 @@ hipError_t launch_hrma (const mxg_config *cfg, const mxg_config *hcfg, const flo
                         const Relay *relay_out, bool fresh, hipStream_t st, hipEvent_t *ev)
 {
    if (n_upper == 0) return hipSuccess;
-   const HrmaLds lay = hrma_lds_layout (hcfg->hrma);
-   if (kHrmaTabOff + (size_t) lay.floats * sizeof (float) > 64 * 1024)
+   if (hs.image.n16 > 64 * 1024 / 16)
      return hipErrorInvalidConfiguration;
 
    // io.idx_in -> k_hrma_enter -> middle list -> k_hrma_reflect -> io.idx_out
@@ -139,17 +139,17 @@ hipError_t launch_hrma (const mxg_config *cfg, const mxg_config *hcfg, const flo
    if (ev) e = hipEventRecord (ev[0], st);
    if (e != hipSuccess) return e;
    if (fresh)
-     hipLaunchKernelGGL (k_hrma_enter<true>, dim3 (a.grid), dim3 (kBlock), 0, st, cfg, s, a, hs.rng_pos,
-                         lay.tilted, source_distance, seed, source_id);
+     hipLaunchKernelGGL (k_hrma_enter<true>, dim3 (a.grid), dim3 (kBlock), 0, st, hs.image.img, s, a, hs.rng_pos,
+                         hrma_tilted (hcfg->hrma), source_distance, seed, source_id);
    else
-     hipLaunchKernelGGL (k_hrma_enter<false>, dim3 (a.grid), dim3 (kBlock), 0, st, cfg, s, a, hs.rng_pos,
-                         lay.tilted, source_distance, seed, source_id);
+     hipLaunchKernelGGL (k_hrma_enter<false>, dim3 (a.grid), dim3 (kBlock), 0, st, hs.image.img, s, a, hs.rng_pos,
+                         hrma_tilted (hcfg->hrma), source_distance, seed, source_id);
    e = hipGetLastError ();
    if ((e == hipSuccess) && ev) e = hipEventRecord (ev[1], st);
    if (e == hipSuccess) e = launch_compact (a, st);
    if ((e == hipSuccess) && ev) e = hipEventRecord (ev[2], st);
    if (e == hipSuccess)
-     e = launch_hrma_reflect (cfg, hcfg, fa, da, s, b, hs.rng_pos, hs.reflect_waves, seed, source_id, relay_out,
+     e = launch_hrma_reflect (cfg, hcfg, fa, da, s, b, hs.rng_pos, hs.image, hs.reflect_waves, seed, source_id, relay_out,
                               st);
    if ((e == hipSuccess) && ev) e = hipEventRecord (ev[3], st);
    if (e == hipSuccess) e = launch_compact (b, st, relay_out ? relay_out->pos : nullptr);

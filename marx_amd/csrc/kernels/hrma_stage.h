@@ -10,16 +10,15 @@
 //   (wfold.c:334-369) -> cap struts -> hyperboloid: the same -> post-collimator
 //   struts.  Geometry is FP64.
 //
-// The mirror's work is split in two at the paraboloid hit (hrma_enter_one,
-// hrma_reflect_one).  The stream position is the Philox block counter c2
-// and the index of the next unused word of the current block, packed as
-// (c2 << 3) | pos.  No Gaussian variate is pending at the split (none is
-// drawn before it), and the buffered block is recomputed from c2 - 1 on
-// resumption.  (A second split at the hyperboloid hit, each part on the
-// photons still alive, measured 37 percent slower: the second kernel
-// repeats the stream resumption, the table lookups and the LDS staging.)
+// The mirror's work is split in two at the paraboloid hit (hrma_enter_core,
+// hrma_reflect_core).  The stream position handed on is the number of words
+// drawn; no Gaussian variate is pending there.  (A second split at the
+// hyperboloid hit, each part on the photons still alive, measured 37 percent
+// slower: the second kernel repeats the stream resumption, the table lookups
+// and the LDS staging.)
 #pragma once
 
+#include <string.h>
 #include "dev_common.h"
 #include "dev_store.h"
 
@@ -84,12 +83,13 @@ __device__ __forceinline__ vec3 conic_normal (double a, double b, vec3 x)
 // about n by a uniform azimuth; the two are at right angles, and u and n are,
 // so the rotations have no component along their axes, and they keep the
 // length 1 to rounding.
-__device__ __forceinline__ void blur_normal (vec3 &n, double blur, Stream &st)
+__device__ __forceinline__ void blur_normal (vec3 &n, double blur, RingStream &st)
 {
    const double n2 = fma (n.y, n.y, n.z * n.z);
    const double il = rsqrt_n (n2);
    double s, c;
-   sincos_turn (uniform (st), s, c);
+   need (st, 1);
+   sincos_turn (take (st), s, c);
    const double cl = c * il, sl = s * il, sx = sl * n.x;
    const vec3 u = v3 (-(sl * n2), fma (sx, n.y, cl * n.z), fma (sx, n.z, -(cl * n.y)));
    double phi = blur * (1.0 / 3600.0 * MXG_PI / 180.0);
@@ -139,22 +139,29 @@ __device__ __forceinline__ int reflect_at (const mxg_hrma_cfg &h, const mxg_shel
                                            const float *__restrict__ fa,
                                            const double *__restrict__ da,
                                            const float *__restrict__ e_alphas,
-                                           const float *__restrict__ ea_cnt, Stream &st)
+                                           const float *__restrict__ ea_cnt, RingStream &st)
 {
    vec3 normal = conic_normal (S.conic_a[k], S.conic_b[k], x);
    if (h.use_blur)
      blur_normal (normal, S.blur[k], st);
    const double p_dot_n = dot_f (p, normal);
-   if ((h.ideal == 0) && fresnel_absorbs (uniform (st), fabs (p_dot_n), m))
-     return -1;
+   if (h.ideal == 0)
+     {
+        need (st, 1);
+        if (fresnel_absorbs (take (st), fabs (p_dot_n), m)) return -1;
+     }
    p = along_f (p, -2.0 * p_dot_n, normal);
    if (h.use_wfold == 0)
      return 0;
-   double r = uniform (st);
+   // a block for every lane with room: usually the scatter's two words here
+   // and four more for the other surface
+   top_up (st);
+   need (st, 2);
+   const double r = take (st);
    double dg = wfold_interp (S.wfold[k], fa, da, e_alphas, energy, -p_dot_n, r, &S.ea_bucket[k], ea_cnt);
    dg *= S.scat_factor[k];
    if (dg > MXG_PI / 4) return -1;
-   if (uniform (st) < 0.5) dg = -dg;
+   if (take (st) < 0.5) dg = -dg;
    // p turned by dg about p x n, which is at right angles to p and not of
    // length 1: cos p + sin (p x n) x p, with (p x n) x p = n - p (p . n)
    // and p . n = -p_dot_n after the reflection
@@ -162,15 +169,6 @@ __device__ __forceinline__ int reflect_at (const mxg_hrma_cfg &h, const mxg_shel
    sincos_small (dg, &sn, &cs);
    p = unit_f (lin2_f (fma (sn, p_dot_n, cs), p, sn, normal));
    return 0;
-}
-
-// Copies the mirror configuration (a multiple of 4 bytes) into LDS.
-__device__ __forceinline__ void stage_hrma_cfg (const mxg_config *__restrict__ cfg, unsigned char *lds)
-{
-   constexpr uint32_t cfg_words = sizeof (mxg_hrma_cfg) / 4;
-   const uint32_t *src = (const uint32_t *) &cfg->hrma;
-   uint32_t *dst = (uint32_t *) lds;
-   for (uint32_t w = threadIdx.x; w < cfg_words; w += blockDim.x) dst[w] = src[w];
 }
 
 // Offsets (in floats) of the tables staged in LDS by k_hrma_reflect.
@@ -209,8 +207,11 @@ inline uint32_t hrma_tilted (const mxg_hrma_cfg &h)
 constexpr size_t kHrmaLayOff = (sizeof (mxg_hrma_cfg) + 15) & ~(size_t) 15;
 constexpr size_t kHrmaTabOff = (kHrmaLayOff + sizeof (HrmaLds) + 15) & ~(size_t) 15;
 
-// The LDS layout of the reflection tables for configuration h (host side).
-inline HrmaLds hrma_lds_layout (const mxg_hrma_cfg &h)
+// The LDS layout of the reflection tables for configuration h, whose e_alpha
+// values are in da (host side).  WFold tables on the same e_alpha values (the
+// standard ones all are) share them, which lets a CU hold four blocks of the
+// reflection with their streams instead of three.
+inline HrmaLds hrma_lds_layout (const mxg_hrma_cfg &h, const double *da)
 {
    HrmaLds lay;
    uint32_t f = 0;
@@ -224,6 +225,20 @@ inline HrmaLds hrma_lds_layout (const mxg_hrma_cfg &h)
         lay.bk_corr[sh] = f; f += bucket_floats (S.corr_bucket);
         for (int k = 0; k < 2; k++)
           {
+             int same = -1;
+             for (int q = 0; (q < 2 * sh + k) && (same < 0); q++)
+               {
+                  const mxg_wfold &o = h.shell[q / 2].wfold[q % 2], &w = S.wfold[k];
+                  if ((o.n_arrays == w.n_arrays)
+                      && !memcmp (da + o.e_alphas_off, da + w.e_alphas_off, w.n_arrays * sizeof (double)))
+                    same = q;
+               }
+             if (same >= 0)
+               {
+                  lay.ea[sh][k] = lay.ea[same / 2][same % 2];
+                  lay.bk_ea[sh][k] = lay.bk_ea[same / 2][same % 2];
+                  continue;
+               }
              lay.ea[sh][k] = f;
              f += S.wfold[k].n_arrays;
              lay.bk_ea[sh][k] = f;
@@ -235,87 +250,94 @@ inline HrmaLds hrma_lds_layout (const mxg_hrma_cfg &h)
    return lay;
 }
 
-// bucket counts of table b from the float arena into LDS at dst
-__device__ __forceinline__ void stage_bucket (const mxg_bucket &b, const float *__restrict__ fa, float *dst)
+// The LDS image of the mirror configuration and the reflection tables (the
+// binary-search targets of every photon), made by the host from the arenas
+// fa, da: the configuration at 0, lay at kHrmaLayOff, the tables at
+// kHrmaTabOff + the offsets of lay: hrma_image_bytes of it, a multiple of 16.
+inline size_t hrma_image_bytes (const HrmaLds &lay)
 {
-   if (!b.ok) return;
-   for (uint32_t w = threadIdx.x; w <= b.nb; w += blockDim.x) dst[w] = fa[b.off + w];
+   return (kHrmaTabOff + (size_t) lay.floats * sizeof (float) + 15) & ~(size_t) 15;
 }
 
-// Stages the mirror configuration and the reflection tables (the
-// binary-search targets of every photon) in LDS: the configuration copy at
-// lds, lay at lds + kHrmaLayOff, the tables at ltab (lds + kHrmaTabOff) +
-// the offsets of lay.  The caller synchronises.
-__device__ __forceinline__ void stage_hrma_tables (const mxg_config *__restrict__ cfg, const float *__restrict__ fa,
-                                                   const double *__restrict__ da, const HrmaLds &lay,
-                                                   unsigned char *lds, float *ltab)
+inline void hrma_image (const mxg_hrma_cfg &h, const float *fa, const double *da, const HrmaLds &lay,
+                        unsigned char *img)
 {
-   stage_hrma_cfg (cfg, lds);
-   if (threadIdx.x == 0) *(HrmaLds *) (lds + kHrmaLayOff) = lay;
-   {
-      const mxg_hrma_cfg &gh = cfg->hrma;
-      for (uint32_t w = threadIdx.x; w < gh.opt_n; w += blockDim.x)
-        {
-           ltab[lay.opt + w] = fa[gh.opt_e_off + w];
-           ltab[lay.opt + gh.opt_n + w] = fa[gh.opt_beta_off + w];
-           ltab[lay.opt + 2 * gh.opt_n + w] = fa[gh.opt_delta_off + w];
-        }
-      stage_bucket (gh.opt_bucket, fa, ltab + lay.bk_opt);
-      for (int sh = 0; sh < MXG_NUM_SHELLS; sh++)
-        {
-           const mxg_shell_cfg &S = gh.shell[sh];
-           for (uint32_t w = threadIdx.x; w < S.corr_n; w += blockDim.x)
-             {
-                ltab[lay.corr_e[sh] + w] = fa[S.corr_e_off + w];
-                ltab[lay.corr_f[sh] + w] = fa[S.corr_f_off + w];
-             }
-           stage_bucket (S.corr_bucket, fa, ltab + lay.bk_corr[sh]);
-           for (int k = 0; k < 2; k++)
-             {
-                for (uint32_t w = threadIdx.x; w < S.wfold[k].n_arrays; w += blockDim.x)
-                  ltab[lay.ea[sh][k] + w] = (float) da[S.wfold[k].e_alphas_off + w];
-                stage_bucket (S.ea_bucket[k], fa, ltab + lay.bk_ea[sh][k]);
-             }
-        }
-   }
+   memset (img, 0, hrma_image_bytes (lay));
+   memcpy (img, &h, sizeof (h));
+   memcpy (img + kHrmaLayOff, &lay, sizeof (lay));
+   float *tab = (float *) (img + kHrmaTabOff);
+   auto put = [&] (uint32_t at, uint32_t off, uint32_t n) { if (n) memcpy (tab + at, fa + off, n * sizeof (float)); };
+   put (lay.opt, h.opt_e_off, h.opt_n);
+   put (lay.opt + h.opt_n, h.opt_beta_off, h.opt_n);
+   put (lay.opt + 2 * h.opt_n, h.opt_delta_off, h.opt_n);
+   put (lay.bk_opt, h.opt_bucket.off, bucket_floats (h.opt_bucket));
+   for (int sh = 0; sh < MXG_NUM_SHELLS; sh++)
+     {
+        const mxg_shell_cfg &S = h.shell[sh];
+        put (lay.corr_e[sh], S.corr_e_off, S.corr_n);
+        put (lay.corr_f[sh], S.corr_f_off, S.corr_n);
+        put (lay.bk_corr[sh], S.corr_bucket.off, bucket_floats (S.corr_bucket));
+        for (int k = 0; k < 2; k++)
+          {
+             for (uint32_t w = 0; w < S.wfold[k].n_arrays; w++)
+               tab[lay.ea[sh][k] + w] = (float) da[S.wfold[k].e_alphas_off + w];
+             put (lay.bk_ea[sh][k], S.ea_bucket[k].off, bucket_floats (S.ea_bucket[k]));
+          }
+     }
 }
 
 // The source-to-paraboloid part of the mirror for an unabsorbed photon with
 // tag `tag` and direction p (tilted: HrmaLds): vignetting, aperture, precollimator struts,
 // frame change and the paraboloid intersection.  False when vignetting
 // blocks the photon (nothing else is drawn); else true, with its position
-// x, direction p, shell si and the mirror's marks added to flags; *hit: it
-// hit the paraboloid, its random-stream position in *rng.
+// x, direction p, shell si and the mirror's marks added to flags; hit: it
+// hit the paraboloid; its random-stream position in rng (3 words, 4 with
+// vignetting, unless a draw was repeated).
 __device__ __forceinline__ bool hrma_enter_core (const mxg_hrma_cfg &h, uint32_t tilted, uint32_t tag,
                                                  double source_distance,
                                                  unsigned long long seed, uint32_t source_id, vec3 &x,
                                                  vec3 &p, int &si, uint32_t &flags, bool &hit, uint32_t &rng)
 {
-   Stream st;
-   stream_init (st, seed, tag, MXG_STAGE_MIRROR, source_id);
    hit = false;
-   if ((h.ideal == 0) && (uniform (st) > h.vignetting))
-     return false;
+   uint32_t w0, w1, w2, w3;
+   philox (tag, MXG_STAGE_MIRROR, 0u, source_id, (uint32_t) seed, (uint32_t) (seed >> 32), w0, w1, w2, w3);
+   const double unit = 1.0 / ((double) 0xFFFFFFFFu);
+   if (h.ideal == 0)
+     {
+        if ((double) w0 * unit > h.vignetting) return false;
+        w0 = w1;
+        w1 = w2;
+        w2 = w3;
+     }
 
    // aperture: shell by cumulative area, radius, open quadrant
-   for (;;)
+   const double r = (double) w0 * unit;
+   si = 0;
+   for (int k = 0; k < MXG_NUM_SHELLS - 1; k++) si += (r >= h.shell[k].area_fraction) ? 1 : 0;
+   bool ok = r < h.shell[MXG_NUM_SHELLS - 1].area_fraction;
+   double u_radius = (double) w1 * unit, theta = (double) w2 * unit;
+   ok = ok && (0 != (h.shell[si].shutter_bitmap & (1u << (unsigned int) (4.0 * theta))));
+   rng = h.ideal ? 3u : 4u;
+   if (!ok)
      {
-        double r = uniform (st);
-        si = -1;
-        for (int k = 0; k < MXG_NUM_SHELLS; k++)
-          if (r < h.shell[k].area_fraction) { si = k; break; }
-        if (si >= 0) break;
+        // a draw outside the open aperture is repeated: the draws again, as
+        // the stream takes them
+        Stream st;
+        stream_init (st, seed, tag, MXG_STAGE_MIRROR, source_id);
+        if (h.ideal == 0) (void) uniform (st);
+        for (si = -1; si < 0; )
+          {
+             const double q = uniform (st);
+             for (int k = 0; k < MXG_NUM_SHELLS; k++)
+               if (q < h.shell[k].area_fraction) { si = k; break; }
+          }
+        u_radius = uniform (st);
+        do theta = uniform (st);
+        while (0 == (h.shell[si].shutter_bitmap & (1u << (unsigned int) (4.0 * theta))));
+        rng = 4u * st.c2 - 4u + (uint32_t) st.pos;
      }
    const mxg_shell_cfg &S = h.shell[si];
-   double radius = S.min_radius + (S.max_radius - S.min_radius) * uniform (st);
-   double theta;
-   unsigned int quad;
-   do
-     {
-        theta = uniform (st);
-        quad = (unsigned int) (4.0 * theta);
-     }
-   while (0 == (S.shutter_bitmap & (1u << quad)));
+   const double radius = S.min_radius + (S.max_radius - S.min_radius) * u_radius;
    double sn, cs;
    sincos_turn (theta - 1.0 / 8.0, sn, cs);
    x.z = radius * cs;
@@ -343,10 +365,7 @@ __device__ __forceinline__ bool hrma_enter_core (const mxg_hrma_cfg &h, uint32_t
    if (!conic_hit (S.conic_a[0], S.conic_b[0], S.conic_c[0], x, p, ipx, S.conic_xmin[0], S.conic_xmax[0]))
      flags |= PHOTON_UNREFLECTED;
    else
-     {
-        hit = true;
-        rng = (st.c2 << 3) | (uint32_t) st.pos;
-     }
+     hit = true;
    return true;
 }
 
@@ -362,50 +381,31 @@ __device__ __forceinline__ bool hrma_enter_one (const mxg_hrma_cfg &h, uint32_t 
                                                 unsigned long long seed, uint32_t source_id)
 {
    bool keep = false;
-   uint32_t flags = FRESH ? 0u : s.flags[id];
+   uint32_t flags = FRESH ? 0u : at (s.flags, id);
    if ((flags & BAD_PHOTON_MASK) == 0)
      {
-        vec3 x, p = v3 (s.p0[id], s.p1[id], s.p2[id]);
+        vec3 x, p = v3 (at (s.p0, id), at (s.p1, id), at (s.p2, id));
         int si;
         uint32_t rng = 0;
-        if (!hrma_enter_core (h, tilted, s.tag[id], source_distance, seed, source_id, x, p, si, flags, keep, rng))
+        if (!hrma_enter_core (h, tilted, at (s.tag, id), source_distance, seed, source_id, x, p, si, flags, keep, rng))
           {
-             s.flags[id] = flags | PHOTON_MIRROR_VBLOCKED;
+             at (s.flags, id) = flags | PHOTON_MIRROR_VBLOCKED;
              if (FRESH)
                {
-                  s.x0[id] = 0.0; s.x1[id] = 0.0; s.x2[id] = 0.0;
-                  s.shell[id] = 0;
+                  at (s.x0, id) = 0.0; at (s.x1, id) = 0.0; at (s.x2, id) = 0.0;
+                  at (s.shell, id) = 0;
                }
           }
         else
           {
              if (keep) rng_pos[id] = rng;
-             s.x0[id] = x.x; s.x1[id] = x.y; s.x2[id] = x.z;
-             s.p0[id] = p.x; s.p1[id] = p.y; s.p2[id] = p.z;
-             s.shell[id] = (uint8_t) si;
-             s.flags[id] = flags;
+             at (s.x0, id) = x.x; at (s.x1, id) = x.y; at (s.x2, id) = x.z;
+             at (s.p0, id) = p.x; at (s.p1, id) = p.y; at (s.p2, id) = p.z;
+             at (s.shell, id) = (uint8_t) si;
+             at (s.flags, id) = flags;
           }
      }
    return keep;
-}
-
-// The stream of photon id at the mirror's split, saved by hrma_enter_one.
-__device__ __forceinline__ void resume_stream (Stream &st, const uint32_t *__restrict__ rng_pos, uint32_t id)
-{
-   const uint32_t w = rng_pos[id];
-   st.c2 = w >> 3;
-   st.pos = (int) (w & 7u);
-   if (st.pos < 4)
-     {
-        // the block again, less the words already used
-        philox (st.c0, st.c1, st.c2 - 1u, st.c3, st.k0, st.k1, st.b0, st.b1, st.b2, st.b3);
-        for (int k = 0; k < st.pos; k++)
-          {
-             st.b0 = st.b1;
-             st.b1 = st.b2;
-             st.b2 = st.b3;
-          }
-     }
 }
 
 // The photon's optical constants and the square root of its shell's area
@@ -435,28 +435,21 @@ __device__ __forceinline__ MirrorIndex mirror_index (const mxg_hrma_cfg &h, cons
    return m;
 }
 
-// k_hrma_reflect's work for photon id of the middle list: paraboloid
-// reflection, cap struts, hyperboloid, post-collimator struts.  ltab: the
-// tables staged in LDS at the offsets lay.  True when the photon leaves the
-// mirror, its columns then also in o.  HANDOFF: such photons go on to the
-// grating through o, and the grating stores their x, p and flags; only the
-// photons the mirror drops have theirs stored here.
-template <bool HANDOFF = false>
-__device__ __forceinline__ bool hrma_reflect_one (const mxg_hrma_cfg &h, const float *ltab, const HrmaLds &lay,
-                                                  const float *__restrict__ fa, const double *__restrict__ da,
-                                                  Soa s, uint32_t id, const uint32_t *__restrict__ rng_pos,
-                                                  unsigned long long seed, uint32_t source_id, PhotonOut &o)
+// From the paraboloid hit on: reflection, cap struts, hyperboloid,
+// post-collimator struts, for the photon with tag `tag`, shell si, position x
+// on the paraboloid and direction p, its stream at word rng (ring: RingStream).  ltab: the tables
+// staged in LDS at the offsets lay.  True when the photon leaves the mirror.
+__device__ __forceinline__ bool hrma_reflect_core (const mxg_hrma_cfg &h, const float *ltab, const HrmaLds &lay,
+                                                   const float *__restrict__ fa, const double *__restrict__ da,
+                                                   uint32_t *ring, uint32_t tag, int si, double energy, uint32_t rng,
+                                                   unsigned long long seed, uint32_t source_id, vec3 &x, vec3 &p,
+                                                   uint32_t &flags)
 {
-   uint32_t flags = s.flags[id];
-   const int si = s.shell[id];
    const mxg_shell_cfg &S = h.shell[si];
-   Stream st;
-   const uint32_t tag = s.tag[id];
-   stream_init (st, seed, tag, MXG_STAGE_MIRROR, source_id);
-   resume_stream (st, rng_pos, id);
-   vec3 x = v3 (s.x0[id], s.x1[id], s.x2[id]);
-   vec3 p = v3 (s.p0[id], s.p1[id], s.p2[id]);
-   const double energy = s.energy[id];
+   RingStream st;
+   ring_init (st, ring, seed, tag, MXG_STAGE_MIRROR, source_id, rng);
+   ring_fill (st);
+   top_up (st);
    const MirrorIndex m = mirror_index (h, S, si, ltab, lay, energy);
    const uint32_t tilted = __builtin_amdgcn_readfirstlane (lay.tilted);
 
@@ -499,13 +492,30 @@ __device__ __forceinline__ bool hrma_reflect_one (const mxg_hrma_cfg &h, const f
                }
           }
      }
-   const bool keep = (flags & BAD_PHOTON_MASK) == 0;
-   if (!(HANDOFF && keep))
-     {
-        s.x0[id] = x.x; s.x1[id] = x.y; s.x2[id] = x.z;
-        s.p0[id] = p.x; s.p1[id] = p.y; s.p2[id] = p.z;
-        s.flags[id] = flags;
-     }
+   return (flags & BAD_PHOTON_MASK) == 0;
+}
+
+// k_hrma_reflect's work for photon id of the middle list (hrma_reflect_core
+// on the store's columns).  True when the photon leaves the mirror, its
+// columns then also in o.  HANDOFF: such photons go on to the grating
+// through o, and the grating stores their x, p and flags; only the photons
+// the mirror drops have theirs stored here.
+template <bool HANDOFF = false>
+__device__ __forceinline__ bool hrma_reflect_one (const mxg_hrma_cfg &h, const float *ltab, const HrmaLds &lay,
+                                                  const float *__restrict__ fa, const double *__restrict__ da,
+                                                  uint32_t *ring, Soa s, uint32_t id,
+                                                  const uint32_t *__restrict__ rng_pos,
+                                                  unsigned long long seed, uint32_t source_id, PhotonOut &o)
+{
+   uint32_t flags = at (s.flags, id);
+   const int si = at (s.shell, id);
+   const uint32_t tag = at (s.tag, id);
+   vec3 x = v3 (at (s.x0, id), at (s.x1, id), at (s.x2, id));
+   vec3 p = v3 (at (s.p0, id), at (s.p1, id), at (s.p2, id));
+   const double energy = at (s.energy, id);
+   const bool keep = hrma_reflect_core (h, ltab, lay, fa, da, ring, tag, si, energy, rng_pos[id], seed, source_id, x,
+                                        p, flags);
+   if (!(HANDOFF && keep)) store_path (s, id, x, p, flags);
    o.x0 = x.x; o.x1 = x.y; o.x2 = x.z;
    o.p0 = p.x; o.p1 = p.y; o.p2 = p.z;
    o.energy = energy;

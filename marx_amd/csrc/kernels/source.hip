@@ -22,59 +22,24 @@
 
 namespace mxg {
 
-constexpr int kTile = 2048;          // photons per scan tile
-constexpr int kPer = kTile / kBlock; // photons per thread
-
-__device__ __forceinline__ uint64_t gap_ticks (double e)
-{
-   return (uint64_t) (e * 4294967296.0 + 0.5);
-}
-
-// The source stream of photon `tag` (source.c:268-384): its energy, its
-// direction and, for Poisson arrivals, the gap to the photon before in
-// 2^-32 units of the mean gap (else its uniform arrival time t).  Both
-// passes over the photons draw through this, so they see the same values.
-// POINT: compiled for a point source only (its direction is the source's,
-// with no draw); GAP: only the gap is wanted (the energy draw, one uniform
-// for either spectrum, is skipped over without its table search).
-template <bool POINT, bool GAP = false>
-__device__ __forceinline__ void source_draws (const mxg_source_cfg &src, const float *__restrict__ fa,
-                                              const double *__restrict__ da, uint32_t tag,
-                                              unsigned long long seed, uint32_t source_id, bool poisson,
-                                              double &energy, vec3 &p, uint64_t &gap, double &t)
-{
-   Stream st;
-   stream_init (st, seed, tag, MXG_STAGE_SOURCE, source_id);
-   if (GAP)
-     {
-        (void) uniform (st);
-        energy = 0.0;
-     }
-   else
-     energy = draw_energy (src, da, st);
-   if (POINT)
-     p = ld3 (src.p);
-   else
-     p = extended_direction (src, fa, ld3 (src.p), ld3 (src.p_normal), ld3 (src.line_normal), src.line_alpha, st);
-   gap = 0;
-   t = 0.0;
-   if (poisson)
-     gap = gap_ticks (expn (st));
-   else
-     t = src.uniform_tmax * uniform (st);
-}
-
 // Poisson arrivals, first pass: each photon's gap (the source stream's
 // draws up to it, no photon stored), the inclusive scan of the gaps within
-// its tile of kTile photons in ticks[i], the tile's total in tile_tot.
+// its tile of kTile photons in ticks[i], the tile's total in tile_tot.  Also
+// clears *first_over for the pass after, and leaves the clock in *begin.
 template <bool POINT>
 __global__ __launch_bounds__ (kBlock)
 void k_source_scan (const mxg_config *__restrict__ cfg, const float *__restrict__ fa,
                     const double *__restrict__ da, uint32_t n, uint32_t tag_start,
                     unsigned long long seed, uint32_t source_id, uint64_t *__restrict__ ticks,
-                    uint64_t *__restrict__ tile_tot)
+                    uint64_t *__restrict__ tile_tot, uint32_t *__restrict__ first_over,
+                    uint64_t *__restrict__ begin)
 {
    const mxg_source_cfg &src = cfg->src;
+   if ((blockIdx.x == 0) && (threadIdx.x == 0))
+     {
+        *first_over = 0xFFFFFFFFu;
+        if (begin) *begin = wall_clock64 ();
+     }
    __shared__ uint64_t sk[kTile];
    __shared__ uint64_t warp_tot[kBlock / 64];
    if (src.time_mode != MXG_TIME_POISSON)
@@ -162,54 +127,6 @@ void k_scan_tiles (uint64_t *__restrict__ tile_tot, uint32_t ntiles)
      }
 }
 
-// A photon as the source makes it: energy, time, direction (dithered when
-// configured, with the offsets d) and whether it is active.
-struct NewPhoton
-{
-   double energy, t;
-   vec3 p;
-   float d[3];
-   bool dithered, active;
-};
-
-// Photon i: its draws; with Poisson arrivals its time from the first pass's
-// scan and its tile's offset tile_off, whether it is active (the first
-// photon, or its predecessor arrives before the exposure) and, for the first
-// photon at or past the exposure, *first_over (unique: the times do not
-// decrease); the INTERNAL dither.  POINT: as in source_draws.
-template <bool POINT>
-__device__ __forceinline__ NewPhoton source_photon (const mxg_source_cfg &src, const float *__restrict__ fa,
-                                                    const double *__restrict__ da, uint32_t i, uint32_t tag,
-                                                    double exposure_time, double start_time,
-                                                    unsigned long long seed, uint32_t source_id,
-                                                    const uint64_t *__restrict__ ticks,
-                                                    const uint64_t *__restrict__ tile_off,
-                                                    uint32_t *__restrict__ first_over)
-{
-   NewPhoton ph;
-   const bool poisson = (src.time_mode == MXG_TIME_POISSON);
-   uint64_t k;
-   source_draws<POINT> (src, fa, da, tag, seed, source_id, poisson, ph.energy, ph.p, k, ph.t);
-   ph.active = true;
-   if (poisson)
-     {
-        const uint64_t toff = tile_off[i / kTile];
-        const double mt = src.mean_time;
-        ph.t = mt * ((double) (ticks[i] + toff) * (1.0 / 4294967296.0));
-        if ((exposure_time > 0.0) && (i > 0))
-          {
-             const uint64_t Sp = ((i % kTile) == 0) ? toff : ticks[i - 1] + toff;
-             const double tp = mt * ((double) Sp * (1.0 / 4294967296.0));
-             ph.active = !(exposure_time <= tp);
-          }
-        if (ph.active && (exposure_time > 0.0) && (exposure_time <= ph.t)) *first_over = i;
-     }
-   ph.dithered = (src.dither_mode == MXG_DITHER_INTERNAL);
-   if (ph.dithered)
-     ph.p = internal_dither (src, ph.p, tag, ph.t, start_time, seed, source_id, ph.d);
-   return ph;
-}
-
 // Photon i, one per thread (source_photon): every column written once, and
 // idx[i] = i for an active photon.  ENTRY: the mirror's entry follows with
 // the photons as fresh and writes their position, shell and flags, so
@@ -271,6 +188,26 @@ __global__ void k_source_count (uint32_t n, const uint32_t *__restrict__ first_o
 
 __global__ void k_reset (uint32_t *p, uint32_t v) { *p = v; }
 
+hipError_t launch_source_scan (const mxg_config *cfg, const float *fa, const double *da, uint32_t n,
+                               uint32_t tag_start, unsigned long long seed, uint32_t source_id, uint64_t *ticks,
+                               uint64_t *tile_tot, uint32_t *first_over, uint64_t *begin, bool point,
+                               const uint64_t **tile_off, hipStream_t st)
+{
+   const uint32_t ntiles = (n + kTile - 1) / kTile;
+   void (*scan) (const mxg_config *, const float *, const double *, uint32_t, uint32_t, unsigned long long, uint32_t,
+                 uint64_t *, uint64_t *, uint32_t *, uint64_t *)
+     = point ? k_source_scan<true> : k_source_scan<false>;
+   hipLaunchKernelGGL (scan, dim3 (ntiles), dim3 (kBlock), 0, st, cfg, fa, da, n, tag_start, seed, source_id, ticks,
+                       tile_tot, first_over, begin);
+   *tile_off = nullptr;
+   if (ntiles > 1)
+     {
+        hipLaunchKernelGGL (k_scan_tiles, dim3 (1), dim3 (kScanThreads), 0, st, tile_tot, ntiles);
+        *tile_off = tile_tot;
+     }
+   return hipGetLastError ();
+}
+
 hipError_t launch_source (const mxg_config *cfg, const float *fa, const double *da, Soa s, uint32_t n,
                           uint32_t tag_start, double exposure_time, double start_time,
                           unsigned long long seed, uint32_t source_id, uint64_t *ticks, uint64_t *tile_tot,
@@ -283,22 +220,17 @@ hipError_t launch_source (const mxg_config *cfg, const float *fa, const double *
         if (count_copy) hipLaunchKernelGGL (k_reset, dim3 (1), dim3 (1), 0, st, count_copy, 0u);
         return hipGetLastError ();
      }
-   const uint32_t ntiles = (n + kTile - 1) / kTile;
    const uint32_t blocks = (n + kBlock - 1) / kBlock;
-   hipLaunchKernelGGL (k_reset, dim3 (1), dim3 (1), 0, st, first_over, 0xFFFFFFFFu);
-   if (point)
-     hipLaunchKernelGGL (k_source_scan<true>, dim3 (ntiles), dim3 (kBlock), 0, st, cfg, fa, da, n, tag_start,
-                         seed, source_id, ticks, tile_tot);
-   else
-     hipLaunchKernelGGL (k_source_scan<false>, dim3 (ntiles), dim3 (kBlock), 0, st, cfg, fa, da, n, tag_start,
-                         seed, source_id, ticks, tile_tot);
-   hipLaunchKernelGGL (k_scan_tiles, dim3 (1), dim3 (kScanThreads), 0, st, tile_tot, ntiles);
+   const uint64_t *tile_off;
+   hipError_t e = launch_source_scan (cfg, fa, da, n, tag_start, seed, source_id, ticks, tile_tot, first_over, nullptr,
+                                      point, &tile_off, st);
+   if (e != hipSuccess) return e;
    void (*kern) (const mxg_config *, const float *, const double *, Soa, uint32_t, uint32_t, double, double,
                  unsigned long long, uint32_t, const uint64_t *, const uint64_t *, uint32_t *, uint32_t *)
      = point ? (entry_follows ? k_source<true, true> : k_source<true, false>)
              : (entry_follows ? k_source<false, true> : k_source<false, false>);
    hipLaunchKernelGGL (kern, dim3 (blocks), dim3 (kBlock), 0, st, cfg, fa, da, s, n, tag_start, exposure_time,
-                       start_time, seed, source_id, ticks, tile_tot, first_over, idx);
+                       start_time, seed, source_id, ticks, tile_off, first_over, idx);
    hipLaunchKernelGGL (k_source_count, dim3 (1), dim3 (1), 0, st, n, first_over, count, count_copy);
    return hipGetLastError ();
 }

@@ -7,6 +7,15 @@
 
 namespace mxg {
 
+// A store to a column that no later stage reads, or few photons of it:
+// it is left out of the cache, which then holds the columns that the next
+// stages read and write again.
+template <class T>
+__device__ __forceinline__ void put_once (T *p, T v)
+{
+   __builtin_nontemporal_store (v, p);
+}
+
 // every column of photon i set as a fresh photon of the given energy,
 // direction, time and tag, with no dither offsets; a column that a later
 // step writes is left out (with_t, with_p, with_dith false; with_entry
@@ -16,34 +25,38 @@ __device__ __forceinline__ void init_photon (Soa s, uint32_t i, double energy, v
                                              uint32_t tag, bool with_t = true, bool with_p = true,
                                              bool with_dith = true, bool with_entry = true)
 {
-   s.energy[i] = energy;
+   at (s.energy, i) = energy;
    if (with_p)
      {
-        s.p0[i] = p.x; s.p1[i] = p.y; s.p2[i] = p.z;
+        at (s.p0, i) = p.x; at (s.p1, i) = p.y; at (s.p2, i) = p.z;
      }
    if (with_entry)
      {
-        s.x0[i] = 0.0; s.x1[i] = 0.0; s.x2[i] = 0.0;
-        s.flags[i] = 0u;
-        s.shell[i] = 0;
+        at (s.x0, i) = 0.0; at (s.x1, i) = 0.0; at (s.x2, i) = 0.0;
+        at (s.flags, i) = 0u;
+        at (s.shell, i) = 0;
      }
-   if (with_t) s.t[i] = t;
-   s.ypix[i] = 0.0f; s.zpix[i] = 0.0f; s.upix[i] = 0.0f; s.vpix[i] = 0.0f;
+   if (with_t) put_once (&at (s.t, i), t);
+   put_once (&at (s.ypix, i), 0.0f); put_once (&at (s.zpix, i), 0.0f);
+   put_once (&at (s.upix, i), 0.0f); put_once (&at (s.vpix, i), 0.0f);
    if (with_dith)
-     for (int q = 0; q < 6; q++) s.dith[q][i] = 0.0f;
-   s.pi[i] = 0.0f;
-   s.pha[i] = 0;
-   s.ccd[i] = 0; s.region[i] = 0; s.order[i] = 0;
-   for (int q = 0; q < 4; q++) s.sup[q][i] = 0;
-   s.tag[i] = tag;
+     for (int q = 0; q < 6; q++) put_once (&at (s.dith[q], i), 0.0f);
+   put_once (&at (s.pi, i), 0.0f);
+   put_once (&at (s.pha, i), (int16_t) 0);
+   put_once (&at (s.ccd, i), (int8_t) 0); put_once (&at (s.region, i), (int8_t) 0); put_once (&at (s.order, i), (int8_t) 0);
+   for (int q = 0; q < 4; q++) put_once (&at (s.sup[q], i), (int8_t) 0);
+   put_once (&at (s.tag, i), tag);
 }
 
 // the dither state of photon i: the three pointing offsets d (ra, dec,
 // roll), the other three columns zero
 __device__ __forceinline__ void store_dith (Soa s, uint32_t i, const float d[3])
 {
-   s.dith[0][i] = d[0]; s.dith[1][i] = d[1]; s.dith[2][i] = d[2];
-   s.dith[3][i] = 0.0f; s.dith[4][i] = 0.0f; s.dith[5][i] = 0.0f;
+   for (int q = 0; q < 3; q++)
+     {
+        put_once (&at (s.dith[q], i), d[q]);
+        put_once (&at (s.dith[q + 3], i), 0.0f);
+     }
 }
 
 // The direction of a photon of the configured source shape about the source
@@ -131,14 +144,22 @@ __device__ __forceinline__ double rotation_axis (vec3 a, vec3 b, vec3 &c)
    return theta;
 }
 
+// sine and cosine of the turn by the nominal roll, internal_dither's when the
+// roll does not vary (roll_amp = 0)
+__device__ __forceinline__ void roll_turn (const mxg_source_cfg &src, double *roll)
+{
+   sincos_small (-(double) (float) src.nominal_roll, &roll[0], &roll[1]);
+}
+
 // INTERNAL dither (dither.c:167-182, 551-581, 609-658) of the photon with
 // tag `tag`, direction p and arrival time t: the Lissajous pointing offset
 // at that time, returned in d as float (as the reference stores the dither
 // state), Gaussian aspect blur, and the rotation of the direction, which is
-// returned.
+// returned.  roll, non-null only where the roll does not vary: sine and
+// cosine of roll_turn.
 __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3 p, uint32_t tag, double t,
                                                  double start_time, unsigned long long seed,
-                                                 uint32_t source_id, float d[3])
+                                                 uint32_t source_id, float d[3], const double *roll = nullptr)
 {
    Stream st;
    stream_init (st, seed, tag, MXG_STAGE_DITHER, source_id);
@@ -152,10 +173,16 @@ __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3
    d[0] = fra; d[1] = fdec; d[2] = froll;
    double delta_ra = src.aspect_blur * gaussian (st);
    double delta_dec = src.aspect_blur * gaussian (st);
-   double ra = (double) fra + delta_ra, dec = (double) fdec + delta_dec, roll = froll;
+   const double ra = (double) fra + delta_ra, dec = (double) fdec + delta_dec;
 
    double sr, cr;
-   sincos_small (-roll, &sr, &cr);
+   if (roll)
+     {
+        sr = roll[0];
+        cr = roll[1];
+     }
+   else
+     sincos_small (-(double) froll, &sr, &cr);
    p = reunit_f (turn_x_f (p, cr, sr));
    double sin_ra, cos_ra, sin_dec, cos_dec;
    sincos_small (ra, &sin_ra, &cos_ra);
@@ -178,9 +205,103 @@ __device__ __forceinline__ void apply_internal_dither (const mxg_source_cfg &src
                                                        unsigned long long seed, uint32_t source_id)
 {
    float d[3];
-   vec3 p = internal_dither (src, v3 (s.p0[i], s.p1[i], s.p2[i]), s.tag[i], t, start_time, seed, source_id, d);
+   vec3 p = internal_dither (src, v3 (at (s.p0, i), at (s.p1, i), at (s.p2, i)), at (s.tag, i), t, start_time, seed, source_id, d);
    store_dith (s, i, d);
-   s.p0[i] = p.x; s.p1[i] = p.y; s.p2[i] = p.z;
+   at (s.p0, i) = p.x; at (s.p1, i) = p.y; at (s.p2, i) = p.z;
+}
+
+// ---- one source ------------------------------------------------------------------
+
+constexpr int kTile = 2048;          // photons per scan tile
+constexpr int kPer = kTile / kBlock; // photons per thread
+
+__device__ __forceinline__ uint64_t gap_ticks (double e)
+{
+   return (uint64_t) (e * 4294967296.0 + 0.5);
+}
+
+// The source stream of photon `tag` (source.c:268-384): its energy, its
+// direction and, for Poisson arrivals, the gap to the photon before in
+// 2^-32 units of the mean gap (else its uniform arrival time t).  Both
+// passes over the photons draw through this, so they see the same values.
+// POINT: compiled for a point source only (its direction is the source's,
+// with no draw); GAP: only the gap is wanted (the energy draw, one uniform
+// for either spectrum, is skipped over without its table search).
+template <bool POINT, bool GAP = false>
+__device__ __forceinline__ void source_draws (const mxg_source_cfg &src, const float *__restrict__ fa,
+                                              const double *__restrict__ da, uint32_t tag,
+                                              unsigned long long seed, uint32_t source_id, bool poisson,
+                                              double &energy, vec3 &p, uint64_t &gap, double &t)
+{
+   Stream st;
+   stream_init (st, seed, tag, MXG_STAGE_SOURCE, source_id);
+   if (GAP)
+     {
+        (void) uniform (st);
+        energy = 0.0;
+     }
+   else
+     energy = draw_energy (src, da, st);
+   if (POINT)
+     p = ld3 (src.p);
+   else
+     p = extended_direction (src, fa, ld3 (src.p), ld3 (src.p_normal), ld3 (src.line_normal), src.line_alpha, st);
+   gap = 0;
+   t = 0.0;
+   if (poisson)
+     gap = gap_ticks (expn (st));
+   else
+     t = src.uniform_tmax * uniform (st);
+}
+
+// A photon as the source makes it: energy, time, direction (dithered when
+// configured, with the offsets d) and whether it is active.
+struct NewPhoton
+{
+   double energy, t;
+   vec3 p;
+   float d[3];
+   bool dithered, active;
+};
+
+// Photon i: its draws; with Poisson arrivals its time from the first pass's
+// scan and its tile's offset tile_off (null: a single tile), whether it is active (the first
+// photon, or its predecessor arrives before the exposure) and, for the first
+// photon at or past the exposure, *first_over (unique: the times do not
+// decrease); the INTERNAL dither.  POINT: as in source_draws.
+template <bool POINT>
+__device__ __forceinline__ NewPhoton source_photon (const mxg_source_cfg &src, const float *__restrict__ fa,
+                                                    const double *__restrict__ da, uint32_t i, uint32_t tag,
+                                                    double exposure_time, double start_time,
+                                                    unsigned long long seed, uint32_t source_id,
+                                                    const uint64_t *__restrict__ ticks,
+                                                    const uint64_t *__restrict__ tile_off,
+                                                    uint32_t *__restrict__ first_over,
+                                                    const double *roll = nullptr)
+{
+   NewPhoton ph;
+   const bool poisson = (src.time_mode == MXG_TIME_POISSON);
+   uint64_t k;
+   source_draws<POINT> (src, fa, da, tag, seed, source_id, poisson, ph.energy, ph.p, k, ph.t);
+   ph.active = true;
+   if (poisson)
+     {
+        const uint64_t toff = tile_off ? tile_off[i / kTile] : 0ull;
+        const double mt = src.mean_time;
+        ph.t = mt * ((double) (ticks[i] + toff) * (1.0 / 4294967296.0));
+        if ((exposure_time > 0.0) && (i > 0))
+          {
+             const uint64_t Sp = ((i % kTile) == 0) ? toff : ticks[i - 1] + toff;
+             const double tp = mt * ((double) Sp * (1.0 / 4294967296.0));
+             ph.active = !(exposure_time <= tp);
+          }
+        if (ph.active && (exposure_time > 0.0) && (exposure_time <= ph.t))
+          __hip_atomic_store (first_over, i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+     }
+   ph.dithered = (src.dither_mode == MXG_DITHER_INTERNAL);
+   if (ph.dithered)
+     ph.p = internal_dither (src, ph.p, tag, ph.t, start_time, seed, source_id, ph.d, roll);
+   return ph;
 }
 
 // ---- batched point sources ------------------------------------------------------
@@ -206,44 +327,82 @@ __device__ __forceinline__ uint32_t source_of (const uint32_t *__restrict__ off,
    return lo;
 }
 
-// Photon i of the batch (tag t0 + i): k_batch_source's work for one photon.
-// POINT: compiled for point sources only (the extended shapes' code, and
-// its registers, left out); ENTRY: the mirror's entry follows with the
-// photon as fresh (see init_photon), so its position, shell and flags are
-// left to it.
+// source_of for the photons first, first + 1, ... of a wave's lanes, by all
+// of its lanes: the wave looks for the first photon's source with a probe a
+// lane, a step for each factor of 64 sources, and each lane goes on from
+// there.
+__device__ __forceinline__ uint32_t source_of_wave (const uint32_t *__restrict__ off, uint32_t nsrc, uint32_t first,
+                                                    uint32_t i)
+{
+   const uint32_t lane = __lane_id ();
+   uint32_t lo = 0, hi = nsrc;         // off[lo] <= first < off[hi]
+   while (hi - lo > 1)
+     {
+        const uint32_t step = (hi - lo + 63u) / 64u, at = lo + lane * step;
+        const uint32_t c = (uint32_t) __popcll (__ballot ((at < hi) && (off[at] <= first)));
+        lo += (c - 1u) * step;
+        hi = (hi - lo < step) ? hi : lo + step;
+     }
+   // the sources are mostly longer than a wave
+   for (int k = 0; k < 4; k++)
+     {
+        if (i < off[lo + 1]) return lo;
+        if (lo + 2 >= nsrc) return nsrc - 1;
+        lo++;
+     }
+   hi = nsrc;
+   while (hi > lo + 1)
+     {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (off[mid] <= i) lo = mid;
+        else hi = mid;
+     }
+   return lo;
+}
+
+// Photon i of the batch, of source k, with tag `tag`.  POINT: compiled for point sources
+// only (the extended shapes' code, and its registers, left out).
+template <bool POINT>
+__device__ __forceinline__ NewPhoton batch_photon (const mxg_source_cfg &src, const double *__restrict__ da, uint32_t k,
+                                                   uint32_t tag, const double *__restrict__ dir, double exposure,
+                                                   double start_time, unsigned long long seed,
+                                                   const double *roll = nullptr)
+{
+   NewPhoton ph;
+   Stream st;
+   stream_init (st, seed, tag, MXG_STAGE_SOURCE, 0u);
+   ph.energy = draw_energy (src, da, st);
+   ph.p = v3 (dir[3 * k], dir[3 * k + 1], dir[3 * k + 2]);
+   if (!POINT && (src.type != MXG_SOURCE_POINT))
+     {
+        // the shape about this source's direction: its normal as the
+        // source set-up makes it, and the rotation of -x onto it
+        vec3 nrm = v3 (-ph.p.y / ph.p.x, 1.0, 0.0);
+        normalize (nrm);
+        vec3 ln = v3 (0.0, 0.0, 0.0);
+        double la = 0.0;
+        if (src.type == MXG_SOURCE_LINE) la = rotation_axis (v3 (-1.0, 0.0, 0.0), ph.p, ln);
+        ph.p = extended_direction (src, nullptr, ph.p, nrm, ln, la, st);
+     }
+   ph.t = exposure * uniform (st);
+   ph.active = true;
+   ph.dithered = (src.dither_mode == MXG_DITHER_INTERNAL);
+   if (ph.dithered) ph.p = internal_dither (src, ph.p, tag, ph.t, start_time, seed, 0u, ph.d, roll);
+   return ph;
+}
+
+// Photon i of the batch (tag t0 + i) written to the store: k_batch_source's
+// work for one photon.  ENTRY: the mirror's entry follows with the photon as
+// fresh (see init_photon), so its position, shell and flags are left to it.
 template <bool POINT, bool ENTRY = false>
 __device__ __forceinline__ void batch_source_one (const mxg_source_cfg &src, const double *__restrict__ da, Soa s,
                                                   uint32_t i, const uint32_t *__restrict__ off, uint32_t nsrc,
                                                   const double *__restrict__ dir, uint32_t t0, double exposure,
                                                   double start_time, unsigned long long seed)
 {
-   const uint32_t k = source_of (off, nsrc, i);
-   const uint32_t tag = t0 + i;
-   Stream st;
-   stream_init (st, seed, tag, MXG_STAGE_SOURCE, 0u);
-   double energy = draw_energy (src, da, st);
-   vec3 p = v3 (dir[3 * k], dir[3 * k + 1], dir[3 * k + 2]);
-   if (!POINT && (src.type != MXG_SOURCE_POINT))
-     {
-        // the shape about this source's direction: its normal as the
-        // source set-up makes it, and the rotation of -x onto it
-        vec3 nrm = v3 (-p.y / p.x, 1.0, 0.0);
-        normalize (nrm);
-        vec3 ln = v3 (0.0, 0.0, 0.0);
-        double la = 0.0;
-        if (src.type == MXG_SOURCE_LINE) la = rotation_axis (v3 (-1.0, 0.0, 0.0), p, ln);
-        p = extended_direction (src, nullptr, p, nrm, ln, la, st);
-     }
-   double t = exposure * uniform (st);
-   if (src.dither_mode == MXG_DITHER_INTERNAL)
-     {
-        float d[3];
-        p = internal_dither (src, p, tag, t, start_time, seed, 0u, d);
-        init_photon (s, i, energy, p, t, tag, true, true, false, !ENTRY);
-        store_dith (s, i, d);
-     }
-   else
-     init_photon (s, i, energy, p, t, tag, true, true, true, !ENTRY);
+   const NewPhoton ph = batch_photon<POINT> (src, da, source_of (off, nsrc, i), t0 + i, dir, exposure, start_time, seed);
+   init_photon (s, i, ph.energy, ph.p, ph.t, t0 + i, true, true, !ph.dithered, !ENTRY);
+   if (ph.dithered) store_dith (s, i, ph.d);
 }
 
 } // namespace mxg
