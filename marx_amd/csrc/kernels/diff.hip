@@ -73,7 +73,7 @@ template <int N> __device__ __forceinline__ Dual<N> operator* (Dual<N> a, Dual<N
 {
    Dual<N> r; r.v = a.v * b.v;
 #pragma unroll
-   for (int j = 0; j < N; j++) r.d[j] = a.d[j] * b.v + a.v * b.d[j];
+   for (int j = 0; j < N; j++) r.d[j] = fma (a.d[j], b.v, a.v * b.d[j]);
    return r;
 }
 template <int N> __device__ __forceinline__ Dual<N> operator* (double a, Dual<N> b)
@@ -86,17 +86,25 @@ template <int N> __device__ __forceinline__ Dual<N> operator* (double a, Dual<N>
 template <int N> __device__ __forceinline__ Dual<N> operator* (Dual<N> b, double a) { return a * b; }
 template <int N> __device__ __forceinline__ Dual<N> operator/ (Dual<N> a, Dual<N> b)
 {
-   Dual<N> r; r.v = a.v / b.v;
-   double ib = 1.0 / b.v;
+   const double ib = rcp_n (b.v);
+   Dual<N> r; r.v = div_r (a.v, b.v, ib);
 #pragma unroll
-   for (int j = 0; j < N; j++) r.d[j] = (a.d[j] - r.v * b.d[j]) * ib;
+   for (int j = 0; j < N; j++) r.d[j] = fma (-r.v, b.d[j], a.d[j]) * ib;
    return r;
 }
-template <int N> __device__ __forceinline__ Dual<N> operator/ (Dual<N> a, double b)
+// a b + c
+template <int N> __device__ __forceinline__ Dual<N> dfma (Dual<N> a, Dual<N> b, Dual<N> c)
 {
-   Dual<N> r; r.v = a.v / b;
+   Dual<N> r; r.v = fma (a.v, b.v, c.v);
 #pragma unroll
-   for (int j = 0; j < N; j++) r.d[j] = a.d[j] / b;
+   for (int j = 0; j < N; j++) r.d[j] = fma (a.d[j], b.v, fma (a.v, b.d[j], c.d[j]));
+   return r;
+}
+template <int N> __device__ __forceinline__ Dual<N> dfma (double a, Dual<N> b, Dual<N> c)
+{
+   Dual<N> r; r.v = fma (a, b.v, c.v);
+#pragma unroll
+   for (int j = 0; j < N; j++) r.d[j] = fma (a, b.d[j], c.d[j]);
    return r;
 }
 template <int N> __device__ __forceinline__ Dual<N> operator+ (Dual<N> a, double b) { a.v += b; return a; }
@@ -106,17 +114,25 @@ template <int N> __device__ __forceinline__ Dual<N> operator- (double a, Dual<N>
 
 template <int N> __device__ __forceinline__ Dual<N> dsqrt (Dual<N> a)
 {
-   Dual<N> r; r.v = sqrt (a.v);
-   double f = (r.v > 0.0) ? 0.5 / r.v : 0.0;
+   Dual<N> r; r.v = sqrt_n (a.v);
+   const double f = (N > 0 && r.v > 0.0) ? 0.5 * rcp_n (r.v) : 0.0;
 #pragma unroll
    for (int j = 0; j < N; j++) r.d[j] = a.d[j] * f;
    return r;
 }
-template <int N> __device__ __forceinline__ Dual<N> dfabs (Dual<N> a) { return (a.v < 0.0) ? -a : a; }
+// 1 / sqrt (a), a > 0
+template <int N> __device__ __forceinline__ Dual<N> drsqrt (Dual<N> a)
+{
+   Dual<N> r; r.v = rsqrt_n (a.v);
+   const double f = -0.5 * r.v * (r.v * r.v);
+#pragma unroll
+   for (int j = 0; j < N; j++) r.d[j] = a.d[j] * f;
+   return r;
+}
 template <int N> __device__ __forceinline__ void dsincos (Dual<N> a, Dual<N> &s, Dual<N> &c)
 {
    double sv, cv;
-   sincos (a.v, &sv, &cv);
+   sincos_small (a.v, &sv, &cv);
    s.v = sv; c.v = cv;
 #pragma unroll
    for (int j = 0; j < N; j++) { s.d[j] = cv * a.d[j]; c.d[j] = -sv * a.d[j]; }
@@ -139,74 +155,43 @@ template <int N> __device__ __forceinline__ DVec<N> dsub (const DVec<N> &a, cons
 }
 template <int N> __device__ __forceinline__ Dual<N> ddot (const DVec<N> &a, const DVec<N> &b)
 {
-   return a.x * b.x + a.y * b.y + a.z * b.z;
+   return dfma (a.z, b.z, dfma (a.y, b.y, a.x * b.x));
 }
 template <int N> __device__ __forceinline__ DVec<N> dcross (const DVec<N> &a, const DVec<N> &b)
 {
    DVec<N> c;
-   c.z = a.x * b.y - a.y * b.x;
-   c.x = a.y * b.z - a.z * b.y;
-   c.y = a.z * b.x - a.x * b.z;
+   c.x = dfma (a.y, b.z, -(a.z * b.y));
+   c.y = dfma (a.z, b.x, -(a.x * b.z));
+   c.z = dfma (a.x, b.y, -(a.y * b.x));
    return c;
 }
-template <int N>
-__device__ __forceinline__ DVec<N> dax1_bx2 (Dual<N> a, const DVec<N> &x1, Dual<N> b, const DVec<N> &x2)
+template <int N> __device__ __forceinline__ DVec<N> dscale (Dual<N> a, const DVec<N> &x)
 {
    DVec<N> r;
-   r.x = a * x1.x + b * x2.x;
-   r.y = a * x1.y + b * x2.y;
-   r.z = a * x1.z + b * x2.z;
+   r.x = a * x.x; r.y = a * x.y; r.z = a * x.z;
    return r;
 }
+// a x + b y
 template <int N>
-__device__ __forceinline__ DVec<N> dax1_bx2_cx3 (Dual<N> a, const DVec<N> &x1, Dual<N> b, const DVec<N> &x2,
-                                                 Dual<N> c, const DVec<N> &x3)
+__device__ __forceinline__ DVec<N> dlin2 (Dual<N> a, const DVec<N> &x, Dual<N> b, const DVec<N> &y)
 {
    DVec<N> r;
-   r.x = a * x1.x + b * x2.x + c * x3.x;
-   r.y = a * x1.y + b * x2.y + c * x3.y;
-   r.z = a * x1.z + b * x2.z + c * x3.z;
+   r.x = dfma (a, x.x, b * y.x);
+   r.y = dfma (a, x.y, b * y.y);
+   r.z = dfma (a, x.z, b * y.z);
    return r;
 }
 
-// the vector length of dev_common.h's length(), on values for the ordering
-template <int N> __device__ __forceinline__ Dual<N> dlength (const DVec<N> &a)
+// a / |a|
+template <int N> __device__ __forceinline__ DVec<N> dunit (const DVec<N> &a)
 {
-   Dual<N> x = dfabs (a.x), y = dfabs (a.y), z = dfabs (a.z), t;
-   if (z.v < x.v) { t = z; z = x; x = t; }
-   if (z.v < y.v) { t = z; z = y; y = t; }
-   if (z.v == 0.0) return dc<N> (0.0);
-   x = x / z;
-   y = y / z;
-   return z * dsqrt (1.0 + x * x + y * y);
+   return dscale (drsqrt (ddot (a, a)), a);
 }
 
-template <int N> __device__ __forceinline__ void dnormalize (DVec<N> &a)
+// ... of a vector that a rotation keeps of length 1 to rounding (reunit_f)
+template <int N> __device__ __forceinline__ DVec<N> dreunit (const DVec<N> &a)
 {
-   Dual<N> len = dlength (a);
-   if (len.v != 0.0)
-     {
-        a.x = a.x / len;
-        a.y = a.y / len;
-        a.z = a.z / len;
-     }
-}
-
-template <int N>
-__device__ __forceinline__ DVec<N> drotate_unit_vector1 (const DVec<N> &p, const DVec<N> &n, Dual<N> c, Dual<N> s)
-{
-   Dual<N> pn = ddot (p, n);
-   DVec<N> u = dax1_bx2_cx3 (c, p, pn * (1.0 - c), n, s, dcross (n, p));
-   dnormalize (u);
-   return u;
-}
-
-template <int N>
-__device__ __forceinline__ DVec<N> drotate_unit_vector (const DVec<N> &p, const DVec<N> &n, Dual<N> theta)
-{
-   Dual<N> s, c;
-   dsincos (theta, s, c);
-   return drotate_unit_vector1 (p, n, c, s);
+   return dscale (dfma (-0.5, ddot (a, a), dc<N> (1.5)), a);
 }
 
 // M x for a tilt matrix M(az, el): value m, derivatives dm[0] (az, tangent
@@ -215,12 +200,13 @@ template <int N>
 __device__ __forceinline__ Dual<N> dm3_row (const double *m, const double (*dm)[9], int row, const DVec<N> &x)
 {
    const double *a = m + 3 * row;
-   Dual<N> o = a[0] * x.x + a[1] * x.y + a[2] * x.z;
+   Dual<N> o = dfma (a[2], x.z, dfma (a[1], x.y, a[0] * x.x));
    if constexpr (N >= 2)
-     {
-        o.d[0] += dm[0][3 * row] * x.x.v + dm[0][3 * row + 1] * x.y.v + dm[0][3 * row + 2] * x.z.v;
-        o.d[1] += dm[1][3 * row] * x.x.v + dm[1][3 * row + 1] * x.y.v + dm[1][3 * row + 2] * x.z.v;
-     }
+     for (int j = 0; j < 2; j++)
+       {
+          const double *b = dm[j] + 3 * row;
+          o.d[j] = fma (b[2], x.z.v, fma (b[1], x.y.v, fma (b[0], x.x.v, o.d[j])));
+       }
    return o;
 }
 
@@ -249,101 +235,57 @@ template <int N> __device__ __forceinline__ DVec<N> dto_osac (const mxg_diff_she
 }
 
 // ---- the reflectivity and its derivative by cos(theta) ---------------------------
+//
+// With m = n^2 - 1 and w = sqrt (m + c^2), the amplitudes are E = (c - w) /
+// (c + w) across and (n^2 c - w) / (n^2 c + w) along the plane of incidence,
+// w' = c / w, and from w^2 - c^2 = m
+//   d|E|^2 / dc = -4 |m|^2 Re (w) / (|c + w|^4 |w|^2)
+//   d|E|^2 / dc = 4 |m|^2 Re (n^2 conj ((c^2 (2 + m) - 1) w)) / (|n^2 c + w|^4 |w|^2).
+// The reflectivity (reflect.c:39-77) is the mean of the two |E|^2.
 
-struct D1 { double v, d; };
-__device__ __forceinline__ D1 d1 (double v, double d = 0.0) { D1 r; r.v = v; r.d = d; return r; }
-__device__ __forceinline__ D1 operator+ (D1 a, D1 b) { return d1 (a.v + b.v, a.d + b.d); }
-__device__ __forceinline__ D1 operator- (D1 a, D1 b) { return d1 (a.v - b.v, a.d - b.d); }
-__device__ __forceinline__ D1 operator- (D1 a) { return d1 (-a.v, -a.d); }
-__device__ __forceinline__ D1 operator* (D1 a, D1 b) { return d1 (a.v * b.v, a.d * b.v + a.v * b.d); }
-__device__ __forceinline__ D1 operator/ (D1 a, D1 b)
+struct MirrorOptics
 {
-   double q = a.v / b.v;
-   return d1 (q, (a.d - q * b.d) / b.v);
-}
-__device__ __forceinline__ D1 d1sqrt (D1 a)
-{
-   double s = sqrt (a.v);
-   return d1 (s, (s > 0.0) ? a.d * 0.5 / s : 0.0);
-}
-__device__ __forceinline__ D1 d1fabs (D1 a) { return (a.v < 0.0) ? -a : a; }
+   double mr, mi;                // m = n^2 - 1, n = 1 - delta + i beta
+};
 
-struct C1 { D1 r, i; };
-
-__device__ __forceinline__ C1 c1mul (C1 a, C1 b)
+__device__ __forceinline__ MirrorOptics mirror_optics (double beta, double delta)
 {
-   C1 z; z.r = a.r * b.r - a.i * b.i; z.i = a.r * b.i + a.i * b.r; return z;
-}
-__device__ __forceinline__ C1 c1div (C1 z1, C1 z2)
-{
-   C1 z;
-   D1 ratio, denom;
-   if (fabs (z2.r.v) > fabs (z2.i.v))
-     {
-        ratio = z2.i / z2.r;
-        denom = z2.r + z2.i * ratio;
-        z.r = (z1.r + ratio * z1.i) / denom;
-        z.i = (z1.i - z1.r * ratio) / denom;
-     }
-   else
-     {
-        ratio = z2.r / z2.i;
-        denom = z2.r * ratio + z2.i;
-        z.r = (z1.r * ratio + z1.i) / denom;
-        z.i = (z1.i * ratio - z1.r) / denom;
-     }
-   return z;
-}
-__device__ __forceinline__ C1 c1_a_bz (D1 a, double b, C1 z1)
-{
-   C1 z; z.r = a + d1 (b) * z1.r; z.i = d1 (b) * z1.i; return z;
-}
-__device__ __forceinline__ C1 c1_az1_bz2 (D1 a, C1 z1, double b, C1 z2)
-{
-   C1 z; z.r = a * z1.r + d1 (b) * z2.r; z.i = a * z1.i + d1 (b) * z2.i; return z;
-}
-__device__ __forceinline__ D1 c1abs (C1 z)
-{
-   D1 fr = d1fabs (z.r), fi = d1fabs (z.i), ratio;
-   if (fr.v > fi.v)
-     {
-        ratio = z.i / z.r;
-        return fr * d1sqrt (d1 (1.0) + ratio * ratio);
-     }
-   if (fi.v == 0.0) return d1 (0.0);
-   ratio = z.r / z.i;
-   return fi * d1sqrt (d1 (1.0) + ratio * ratio);
-}
-__device__ __forceinline__ C1 c1sqrt (C1 a)
-{
-   D1 r = c1abs (a);
-   if (r.v == 0.0) return a;
-   if (a.r.v >= 0.0)
-     {
-        a.r = d1sqrt (d1 (0.5) * (r + a.r));
-        a.i = d1 (0.5) * a.i / a.r;
-     }
-   else
-     {
-        r = d1sqrt (d1 (0.5) * (r - a.r));
-        a.r = d1 (0.5) * a.i / r;
-        a.i = r;
-        if (a.r.v < 0.0) { a.r = -a.r; a.i = -a.i; }
-     }
-   return a;
+   MirrorOptics o;
+   o.mr = fma (delta, delta - 2.0, -(beta * beta));
+   o.mi = 2.0 * (1.0 - delta) * beta;
+   return o;
 }
 
-// reflectivity (value and d/d cos_theta) of dev_common.h's reflectivity()
-__device__ __forceinline__ D1 reflectivity_d1 (double cos_theta, double beta, double delta)
+// the reflectivity at cos (theta) = c; SLOPE: its derivative in dr
+template <bool SLOPE>
+__device__ __forceinline__ double reflectivity_at (double c, const MirrorOptics &o, double &dr)
 {
-   D1 c = d1 (cos_theta, 1.0);
-   C1 n; n.r = d1 (1.0 - delta); n.i = d1 (beta);
-   D1 sin_theta = d1sqrt (d1 (1.0) - c * c);
-   C1 nsqr = c1mul (n, n);
-   C1 root = c1sqrt (c1_a_bz (-(sin_theta * sin_theta), 1.0, nsqr));
-   C1 e_perp = c1div (c1_a_bz (c, -1.0, root), c1_a_bz (c, 1.0, root));
-   C1 e_par = c1div (c1_az1_bz2 (c, nsqr, -1.0, root), c1_az1_bz2 (c, nsqr, 1.0, root));
-   return d1 (0.5) * (e_par.r * e_par.r + e_par.i * e_par.i + e_perp.r * e_perp.r + e_perp.i * e_perp.i);
+   const double c2 = c * c, wr2 = fma (c, c, o.mr), wi2 = o.mi;
+   // the principal square root of wr2 + i wi2 by the half-angle formulas
+   double inv;
+   const double mod = sqrt_n (fma (wr2, wr2, wi2 * wi2));
+   const double big = sqrt_rsqrt_n (fmax (0.5 * (mod + fabs (wr2)), 1e-300), inv);
+   const double small = 0.5 * wi2 * inv;
+   const double wr = (wr2 >= 0.0) ? big : fabs (small);
+   const double wi = (wr2 >= 0.0) ? small : copysign (big, small);
+   const double i2 = wi * wi, nr = 1.0 + o.mr;
+   const double d1 = c - wr, s1 = c + wr;
+   const double A = fma (d1, d1, i2), B = fma (s1, s1, i2);
+   const double xr = nr * c, xi = o.mi * c;
+   const double e1 = xr - wr, e2 = xi - wi, f1 = xr + wr, f2 = xi + wi;
+   const double C = fma (e1, e1, e2 * e2), D = fma (f1, f1, f2 * f2);
+   const double ibd = rcp_n (B * D);
+   const double ib = ibd * D, id = ibd * B;       // 1 / B, 1 / D
+   if (SLOPE)
+     {
+        const double m2 = fma (o.mr, o.mr, o.mi * o.mi);
+        // u = (c^2 (2 + m) - 1) w, then Re (n^2 conj (u))
+        const double tr = fma (c2, 2.0 + o.mr, -1.0), ti = c2 * o.mi;
+        const double ur = fma (tr, wr, -(ti * wi)), ui = fma (tr, wi, ti * wr);
+        const double par = fma (nr, ur, o.mi * ui);
+        dr = 2.0 * m2 * rcp_n (fmax (mod, 1e-300)) * fma (par * id, id, -(wr * ib) * ib);
+     }
+   return 0.5 * fma (A, ib, C * id);
 }
 
 // WFold angle at (energy, sin_alpha, r) and its derivative by sin_alpha
@@ -365,23 +307,26 @@ __device__ __forceinline__ double wfold_d1 (const mxg_wfold &w, const float *__r
    const double theta_0 = fold_theta (f0, fa, r);
    const double theta_1 = fold_theta (f1, fa, r);
    double e0 = e_alphas[i - 1], e1 = e_alphas[i];
-   dval = (theta_1 - theta_0) / (e1 - e0) * energy;
-   return theta_0 + (theta_1 - theta_0) * (e_alpha - e0) / (e1 - e0);
+   const double slope = div_n (theta_1 - theta_0, e1 - e0);
+   dval = slope * energy;
+   return fma (slope, e_alpha - e0, theta_0);
 }
 
 // ---- one photon -----------------------------------------------------------------------
 
+// conic_hit (hrma_stage.h) on duals
 template <int N>
-__device__ __forceinline__ bool dconic_intersection (double a, double b, double c, DVec<N> &x0, const DVec<N> &p,
-                                                     double xmin, double xmax)
+__device__ __forceinline__ bool dconic_hit (double a, double b, double c, DVec<N> &x0, const DVec<N> &p,
+                                            double xmin, double xmax)
 {
-   Dual<N> t_plus = -x0.x / p.x;
-   Dual<N> x_y = x0.y + t_plus * p.y;
-   Dual<N> x_z = x0.z + t_plus * p.z;
-   Dual<N> alpha = a * (p.x * p.x) - 1.0;
-   Dual<N> beta = b * p.x - 2.0 * (p.y * x_y + p.z * x_z);
-   Dual<N> gamma = c - x_z * x_z - x_y * x_y;
-   Dual<N> t_minus;
+   const Dual<N> t0 = -x0.x / p.x;
+   const Dual<N> x_y = dfma (t0, p.y, x0.y);
+   const Dual<N> x_z = dfma (t0, p.z, x0.z);
+   const Dual<N> alpha = dfma (a * p.x, p.x, dc<N> (-1.0));
+   const Dual<N> beta = dfma (b, p.x, -2.0 * dfma (p.y, x_y, p.z * x_z));
+   const Dual<N> gamma = dfma (-x_y, x_y, dfma (-x_z, x_z, dc<N> (c)));
+   Dual<N> t_plus, t_minus;
+   bool minus_ok = false;
    if (alpha.v == 0.0)
      {
         if (beta.v == 0.0) return false;
@@ -389,75 +334,73 @@ __device__ __forceinline__ bool dconic_intersection (double a, double b, double 
      }
    else
      {
-        // the roots of dev_common.h's quadratic_root(), on duals
-        Dual<N> bsqr = beta * beta;
-        Dual<N> ac4 = alpha * gamma * 4.0;
-        Dual<N> neg_b_over_2a = -beta / (2.0 * alpha);
-        if (bsqr.v > ac4.v)
+        const Dual<N> disc = dfma (beta, beta, -4.0 * (alpha * gamma));
+        if (!(disc.v >= 0.0)) return false;
+        const Dual<N> root = dsqrt (disc);
+        const Dual<N> q = (beta.v < 0.0) ? beta - root : beta + root;
+        t_plus = -2.0 * (gamma / q);
+        t_minus = t_plus;
+        if (fabs (p.x.v * q.v) <= 2.0001 * fmax (fabs (xmin), fabs (xmax)) * fabs (alpha.v))
           {
-             Dual<N> factor = 1.0 + dsqrt (1.0 - ac4 / bsqr);
-             t_plus = -2.0 * gamma / (beta * factor);
-             t_minus = neg_b_over_2a * factor;
+             t_minus = -0.5 * (q / alpha);
+             const double x_minus = p.x.v * t_minus.v;
+             minus_ok = (x_minus >= xmin) && (x_minus < xmax);
           }
-        else if (bsqr.v == ac4.v)
-          t_plus = t_minus = neg_b_over_2a;
-        else
-          return false;
      }
-   Dual<N> x_plus = p.x * t_plus;
-   Dual<N> x_minus = p.x * t_minus;
-   bool plus_ok = (x_plus.v >= xmin) && (x_plus.v < xmax);
-   bool minus_ok = (x_minus.v >= xmin) && (x_minus.v < xmax);
-   Dual<N> t;
-   if (plus_ok)
-     t = (minus_ok && (x_minus.v > x_plus.v)) ? t_minus : t_plus;
-   else if (minus_ok)
-     t = t_minus;
-   else
-     return false;
+   const double x_plus = p.x.v * t_plus.v;
+   const bool plus_ok = (x_plus >= xmin) && (x_plus < xmax);
+   if (!(plus_ok || minus_ok)) return false;
+   const bool minus = minus_ok && !(plus_ok && (x_plus >= p.x.v * t_minus.v));
+   const Dual<N> t = minus ? t_minus : t_plus;
    x0.x = p.x * t;
-   x0.y = x_y + p.y * t;
-   x0.z = x_z + p.z * t;
+   x0.y = dfma (p.y, t, x_y);
+   x0.z = dfma (p.z, t, x_z);
    return true;
 }
 
 // reflection at x on conic k: normal blur, survival weight, specular
-// reflection, WFold scatter.  false: scattered past pi/4.
+// reflection, WFold scatter (the rotations as in hrma_stage.h: about axes
+// at right angles).  false: scattered past pi/4.
 template <int N>
 __device__ __forceinline__ bool dreflect_at (const mxg_hrma_cfg &h, const mxg_shell_cfg &S, int k,
                                              const DVec<N> &x, DVec<N> &p, Dual<N> &w, double energy,
-                                             double beta, double delta, double corr,
+                                             const MirrorOptics &optics, double corr,
                                              const float *__restrict__ fa,
                                              const double *__restrict__ da, Stream &st)
 {
    DVec<N> n;
-   n.x = (S.conic_a[k] - 1) * x.x + 0.5 * S.conic_b[k];
+   n.x = dfma (S.conic_a[k] - 1.0, x.x, dc<N> (0.5 * S.conic_b[k]));
    n.y = -x.y;
    n.z = -x.z;
-   dnormalize (n);
+   n = dunit (n);
    if (h.use_blur)
      {
-        Dual<N> len = dsqrt (n.y * n.y + n.z * n.z);
-        DVec<N> perp;
-        perp.x = dc<N> (0.0);
-        perp.y = n.z / len;
-        perp.z = -n.y / len;
-        double phi = (2.0 * MXG_PI) * uniform (st);
-        perp = drotate_unit_vector (perp, n, dc<N> (phi));
-        phi = S.blur[k] * (1.0 / 3600.0 * MXG_PI / 180.0);
+        double sn, cs;
+        const Dual<N> n2 = dfma (n.y, n.y, n.z * n.z);
+        const Dual<N> il = drsqrt (n2);
+        sincos_turn (uniform (st), sn, cs);
+        const Dual<N> cl = cs * il, sl = sn * il, sx = sl * n.x;
+        DVec<N> u;
+        u.x = -(sl * n2);
+        u.y = dfma (sx, n.y, cl * n.z);
+        u.z = dfma (sx, n.z, -(cl * n.y));
+        double phi = S.blur[k] * (1.0 / 3600.0 * MXG_PI / 180.0);
         phi = phi * gaussian (st);
-        n = drotate_unit_vector (n, perp, dc<N> (phi));
+        sincos_small (phi, &sn, &cs);
+        n = dreunit (dlin2 (dc<N> (cs), n, dc<N> (sn), dcross (u, n)));
      }
-   Dual<N> p_dot_n = ddot (p, n);
+   const Dual<N> p_dot_n = ddot (p, n);
    if (h.ideal == 0)
      {
-        D1 r = reflectivity_d1 (fabs (p_dot_n.v), beta, delta);
-        Dual<N> c = dfabs (p_dot_n);
-        Dual<N> R = r.d * c;             // the derivative part; its value is replaced next
-        R.v = r.v;
+        double dr = 0.0;
+        Dual<N> R;
+        R.v = reflectivity_at<(N > 0)> (fabs (p_dot_n.v), optics, dr);
+        const double f = (p_dot_n.v < 0.0) ? -dr : dr;
+#pragma unroll
+        for (int j = 0; j < N; j++) R.d[j] = f * p_dot_n.d[j];
         w = w * (R * corr);
      }
-   p = dax1_bx2 (dc<N> (1.0), p, -2.0 * p_dot_n, n);
+   p = dlin2 (dc<N> (1.0), p, -2.0 * p_dot_n, n);
    if (h.use_wfold == 0)
      return true;
    double r = uniform (st);
@@ -468,7 +411,9 @@ __device__ __forceinline__ bool dreflect_at (const mxg_hrma_cfg &h, const mxg_sh
    dg = dg * S.scat_factor[k];
    if (dg.v > MXG_PI / 4) return false;
    if (uniform (st) < 0.5) dg = -dg;
-   p = drotate_unit_vector (p, dcross (p, n), dg);
+   Dual<N> sn, cs;
+   dsincos (dg, sn, cs);
+   p = dunit (dlin2 (dfma (sn, p_dot_n, cs), p, sn, n));
    return true;
 }
 
@@ -541,9 +486,8 @@ __device__ __forceinline__ bool diff_enter (const mxg_hrma_cfg &h, const mxg_sou
         quad = (unsigned int) (4.0 * theta);
      }
    while (0 == (S.shutter_bitmap & (1u << quad)));
-   theta = (2.0 * MXG_PI) * (theta - 1.0 / 8.0);
    double sn, cs;
-   sincos (theta, &sn, &cs);
+   sincos_turn (theta - 1.0 / 8.0, sn, cs);
 
    ph.t0 = dto_osac<N> (D, 0);
    ph.t1 = dto_osac<N> (D, 1);
@@ -555,16 +499,14 @@ __device__ __forceinline__ bool diff_enter (const mxg_hrma_cfg &h, const mxg_sou
    p = dv<N> (ld3 (src.p));
    if (src.distance > 0.0)
      {
-        p = dax1_bx2 (dc<N> (1.0), x, dc<N> (src.distance), p);
-        dnormalize (p);
+        p = dunit (dlin2 (dc<N> (1.0), x, dc<N> (src.distance), p));
      }
    if (h.use_struts && in_strut_shadow (h, val (x), val (p), rcp_n (p.x.v), h.pre_struts))
      return false;
    x = dadd (x, ph.t0);
    x = dm3_vmul (D.fwd[0], D.dfwd[0], x);
    p = dm3_vmul (D.fwd[0], D.dfwd[0], p);
-   return dconic_intersection (S.conic_a[0], S.conic_b[0], S.conic_c[0], x, p, S.conic_xmin[0],
-                               S.conic_xmax[0]);
+   return dconic_hit (S.conic_a[0], S.conic_b[0], S.conic_c[0], x, p, S.conic_xmin[0], S.conic_xmax[0]);
 }
 
 // Every photon to its paraboloid intersection, values only.  A lost photon
@@ -651,6 +593,7 @@ void k_diff_forward (const mxg_config *__restrict__ cfg, const float *__restrict
              if (h.use_scale)
                corr = sqrt ((double) interp_f (ef, fa + S.corr_e_off, fa + S.corr_f_off, S.corr_n));
           }
+        const MirrorOptics optics = mirror_optics (beta, delta);
         for (int k = 0; (k < 2) && alive; k++)
           {
              if (k == 1)
@@ -658,14 +601,13 @@ void k_diff_forward (const mxg_config *__restrict__ cfg, const float *__restrict
                   x = dadd (x, ph.t1);
                   x = dm3_vmul (D.fwd[1], D.dfwd[1], x);
                   p = dm3_vmul (D.fwd[1], D.dfwd[1], p);
-                  if (!dconic_intersection (S.conic_a[1], S.conic_b[1], S.conic_c[1], x, p,
-                                            S.conic_xmin[1], S.conic_xmax[1]))
+                  if (!dconic_hit (S.conic_a[1], S.conic_b[1], S.conic_c[1], x, p, S.conic_xmin[1], S.conic_xmax[1]))
                     {
                        alive = false;
                        break;
                     }
                }
-             if (!dreflect_at (h, S, k, x, p, w, ph.energy, beta, delta, corr, fa, da, ph.st))
+             if (!dreflect_at (h, S, k, x, p, w, ph.energy, optics, corr, fa, da, ph.st))
                {
                   alive = false;
                   break;
