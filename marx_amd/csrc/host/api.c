@@ -165,9 +165,40 @@ static int copy_back (Marx_Photon_Type *pt)
    return 0;
 }
 
-static int finish_stage (Marx_Photon_Type *pt, int force_copy)
+/* A stage (MXGD_STAGE_*) on the caller's list, its records and sorted_index
+ * back there unless the copies are lazy (last: the stage ends a lazily
+ * synchronised chunk). */
+static int run_stage (Marx_Photon_Type *pt, int stage, double arg, int last)
 {
-   if (Lazy_Sync && !force_copy)
+   int status = 1;
+   if (-1 == sync_config ())
+     return -1;
+   if ((Lazy_Sync == 0) && (pt->num_sorted <= pt->n_photons))
+     {
+        unsigned int n = 0;
+        Device_Trace = 0;
+        Resident = NULL;
+        status = mxgd_stage_on_list (stage, arg, Seed, pt->attributes, pt->n_photons, pt->sorted_index,
+                                     pt->sorted_energies, pt->num_sorted, &n);
+        if (status == 0)
+          {
+             pt->num_sorted = n;
+             Resident = pt;
+             Resident_Tag_Start = pt->tag_start;
+             return 0;
+          }
+     }
+   if ((status == 1) && (-1 == make_resident (pt)))
+     return -1;
+   if ((status == -1)
+       || (-1 == ((stage == MXGD_STAGE_MIRROR) ? mxgd_run_mirror (arg, Seed, -1, NULL, 0, 0)
+                  : (stage == MXGD_STAGE_GRATING) ? mxgd_run_grating (Seed, -1, NULL, 0, 0)
+                  : mxgd_run_detect (arg, Seed, -1, NULL, 0))))
+     {
+        mxg_error ("%s", mxgd_last_error ());
+        return -1;
+     }
+   if (Lazy_Sync && !last)
      return 0;
    return copy_back (pt);
 }
@@ -214,14 +245,7 @@ int marx_mirror_reflect (Marx_Photon_Type *pt, int verbose)
    if (pt->history & MARX_MIRROR_SHELL_OK)
      return 0;
    pt->history |= MARX_MIRROR_SHELL_OK;
-   if ((-1 == sync_config ()) || (-1 == make_resident (pt)))
-     return -1;
-   if (-1 == mxgd_run_mirror (pt->source_distance, Seed, -1, NULL, 0, 0))
-     {
-        mxg_error ("%s", mxgd_last_error ());
-        return -1;
-     }
-   return finish_stage (pt, 0);
+   return run_stage (pt, MXGD_STAGE_MIRROR, pt->source_distance, 0);
 }
 
 /* ---- grating (grating.c:44-114) ------------------------------------------------ */
@@ -281,14 +305,7 @@ int marx_grating_diffract (Marx_Photon_Type *pt, int verbose)
    if (pt->history & MARX_ORDER_OK)
      return 0;
    pt->history |= grating_history ();
-   if ((-1 == sync_config ()) || (-1 == make_resident (pt)))
-     return -1;
-   if (-1 == mxgd_run_grating (Seed, -1, NULL, 0, 0))
-     {
-        mxg_error ("%s", mxgd_last_error ());
-        return -1;
-     }
-   return finish_stage (pt, 0);
+   return run_stage (pt, MXGD_STAGE_GRATING, 0.0, 0);
 }
 
 /* ---- detector (detector.c:298-379) ------------------------------------------- */
@@ -330,14 +347,7 @@ int marx_detect (Marx_Photon_Type *pt, int verbose)
    if (pt->history & MARX_DET_NUM_OK)
      return 0;
    pt->history |= detector_history ();
-   if ((-1 == sync_config ()) || (-1 == make_resident (pt)))
-     return -1;
-   if (-1 == mxgd_run_detect (pt->start_time, Seed, -1, NULL, 0))
-     {
-        mxg_error ("%s", mxgd_last_error ());
-        return -1;
-     }
-   return finish_stage (pt, 1);
+   return run_stage (pt, MXGD_STAGE_DETECT, pt->start_time, 1);
 }
 
 /* ---- source (source.c:268-384) ------------------------------------------------- */
@@ -576,8 +586,7 @@ int marx_create_photons (Marx_Source_Type *st, Marx_Photon_Type *pt, unsigned in
         return -1;
      }
    /* the records, and their energy order sorted on the device */
-   if ((n > 0) && ((-1 == mxgd_download_aos (pt->attributes, n))
-                   || (-1 == mxgd_sort_store_by_energy (n, pt->sorted_index, pt->sorted_energies))))
+   if (-1 == mxgd_download_sorted (pt->attributes, n, pt->sorted_index, pt->sorted_energies))
      {
         mxg_error ("%s", mxgd_last_error ());
         return -1;

@@ -51,19 +51,23 @@ uint32_t *d_seg = nullptr;         // per-block survivor segments of the running
 uint32_t *d_seg_count = nullptr;   // kMaxSegments entries
 uint32_t *d_rng_pos = nullptr;     // the mirror's per-photon stream position
 uint32_t *d_counts = nullptr;      // [0],[1] list lengths, [2] source cut, [4] middle list,
-                                   // [8..15] per-stage survivor counts, [32] the persistent
-                                   // pass's tile counter, [36..39] its stage counts
+                                   // [8..15] per-stage survivor counts, [24] a host list's length
 uint32_t *h_counts = nullptr;      // pinned host copy of d_counts[8..15], read once per call
 TraceReport *d_trace = nullptr;    // running sums of the trace as chunk kernels (passes.hip)
 TraceReport *h_trace = nullptr;    // ... and its report, in pinned memory
 uint32_t *d_trace_n = nullptr, *d_trace_counts = nullptr;  // its length and block counts
 double g_clock_khz = 1.0e5;        // rate of the device's wall clock
-uint32_t *d_tile_cnt = nullptr;    // the persistent pass's per-tile counts and offsets
-size_t g_tile_cap = 0;             // entries of each
 int g_cur = 0;                     // list holding the active photons
 unsigned int g_upper = 0;          // host-side upper bound of the active count
 Marx_Photon_Attr_Type *d_aos = nullptr;
 size_t g_aos_cap = 0;
+// stages on a host list, chunk by chunk (mxgd_stage_on_list)
+constexpr unsigned int kChunks = 8;
+hipStream_t g_copy_stream = nullptr;    // the link's copies beside the stage's kernels
+hipEvent_t g_copy_ev[kChunks + 1];      // chunk k's records are on the device; [kChunks]: order between the streams
+uint32_t *d_active = nullptr;           // the list as the caller gave it
+uint8_t *d_marks = nullptr;             // 1: the photon is on it
+size_t g_marks_cap = 0;                 // entries of both
 uint64_t *d_ticks = nullptr;       // arrival-time scan (fixed-point gaps)
 void *d_relay_mem = nullptr;       // two stage-to-stage relays (capacity rows each)
 Relay g_relay[2] = {};
@@ -163,10 +167,10 @@ __global__ void k_iota (uint32_t *idx, uint32_t n)
 }
 
 __global__ __launch_bounds__ (kBlock)
-void k_aos_to_soa (const Marx_Photon_Attr_Type *__restrict__ a, Soa s, uint32_t n)
+void k_aos_to_soa (const Marx_Photon_Attr_Type *__restrict__ a, Soa s, uint32_t lo, uint32_t hi)
 {
-   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-   if (i >= n) return;
+   const uint32_t i = lo + blockIdx.x * blockDim.x + threadIdx.x;
+   if (i >= hi) return;
    const Marx_Photon_Attr_Type &at = a[i];
    s.energy[i] = at.energy;
    s.x0[i] = at.x.x; s.x1[i] = at.x.y; s.x2[i] = at.x.z;
@@ -186,13 +190,12 @@ void k_aos_to_soa (const Marx_Photon_Attr_Type *__restrict__ a, Soa s, uint32_t 
    s.tag[i] = at.tag;
 }
 
-__global__ __launch_bounds__ (kBlock)
-void k_soa_to_aos (Marx_Photon_Attr_Type *__restrict__ a, Soa s, uint32_t n)
+constexpr int kWords = sizeof (Marx_Photon_Attr_Type) / 8;
+static_assert (sizeof (Marx_Photon_Attr_Type) % 8 == 0, "record is whole 8-byte words");
+
+// photon i's record at dst
+__device__ __forceinline__ void put_record (const Soa &s, uint32_t i, uint64_t *dst)
 {
-   static_assert (sizeof (Marx_Photon_Attr_Type) % 8 == 0, "record is whole 8-byte words");
-   constexpr int kWords = sizeof (Marx_Photon_Attr_Type) / 8;
-   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-   if (i >= n) return;
    // built in zeroed words and stored word by word, so that the record's
    // padding bytes are zero (a struct copy may leave them indeterminate)
    union { Marx_Photon_Attr_Type at; uint64_t w[kWords]; } u;
@@ -214,8 +217,118 @@ void k_soa_to_aos (Marx_Photon_Attr_Type *__restrict__ a, Soa s, uint32_t n)
    at.ccd_num = s.ccd[i]; at.detector_region = s.region[i]; at.order = s.order[i];
    for (int k = 0; k < 4; k++) at.support_orders[k] = s.sup[k][i];
    at.tag = s.tag[i];
-   uint64_t *dst = (uint64_t *) (a + i);
    for (int k = 0; k < kWords; k++) dst[k] = u.w[k];
+}
+
+__global__ __launch_bounds__ (kBlock)
+void k_soa_to_aos (Marx_Photon_Attr_Type *__restrict__ a, Soa s, uint32_t n)
+{
+   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+   if (i < n) put_record (s, i, (uint64_t *) (a + i));
+}
+
+// ---- a stage on a host list (mxgd_stage_on_list) ----
+
+__global__ void k_zero_bytes (uint8_t *__restrict__ a, uint32_t n)
+{
+   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+   if (i < n) a[i] = 0;
+}
+
+__global__ void k_mark_listed (const uint32_t *__restrict__ list, uint32_t m, uint32_t n, uint8_t *__restrict__ marks)
+{
+   const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+   if ((q < m) && (list[q] < n)) marks[list[q]] = 1;
+}
+
+// The marked photons of [lo, hi) into list, their number added to *count, in
+// no order (their results do not depend on it: the draws follow the tags).
+__global__ __launch_bounds__ (kBlock)
+void k_list_marked (const uint8_t *__restrict__ marks, uint32_t lo, uint32_t hi, uint32_t *__restrict__ list,
+                    uint32_t *__restrict__ count)
+{
+   __shared__ uint32_t wc[kBlock / 64], at0;
+   const uint32_t i = lo + blockIdx.x * kBlock + threadIdx.x;
+   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+   const bool on = (i < hi) && marks[i];
+   const unsigned long long mask = __ballot (on);
+   if (lane == 0) wc[wave] = (uint32_t) __popcll (mask);
+   __syncthreads ();
+   if (threadIdx.x == 0)
+     {
+        uint32_t t = 0;
+        for (int w = 0; w < kBlock / 64; w++) t += wc[w];
+        at0 = t ? atomicAdd (count, t) : 0u;
+     }
+   __syncthreads ();
+   uint32_t q = at0 + (uint32_t) __popcll (mask & ((1ull << lane) - 1ull));
+   for (int w = 0; w < wave; w++) q += wc[w];
+   if (on) list[q] = i;
+}
+
+// The records of the listed photons straight into the caller's list in
+// pinned host memory.  A block builds kBlock of them in LDS and its lanes
+// write them word by word side by side, so that the link carries whole runs:
+// MI355X, 1e6 records of 136 bytes: every one 2.49 ms (55 GB/s), one in three
+// 0.95 ms, one in sixteen 0.20 ms; a DMA copy of all of them takes 2.38 ms.
+__global__ __launch_bounds__ (kBlock)
+void k_records_out (uint64_t *__restrict__ host, Soa s, const uint32_t *__restrict__ list,
+                    const uint32_t *__restrict__ count)
+{
+   __shared__ uint64_t rec[kBlock * kWords];
+   __shared__ uint32_t ids[kBlock];
+   const uint32_t m = *count;
+   for (uint32_t base = blockIdx.x * kBlock; base < m; base += gridDim.x * kBlock)
+     {
+        const uint32_t rows = (m - base < (uint32_t) kBlock) ? m - base : (uint32_t) kBlock;
+        if (threadIdx.x < rows)
+          {
+             const uint32_t id = list[base + threadIdx.x];
+             ids[threadIdx.x] = id;
+             put_record (s, id, rec + threadIdx.x * kWords);
+          }
+        __syncthreads ();
+        for (uint32_t t = threadIdx.x; t < rows * kWords; t += kBlock)
+          host[(size_t) ids[t / kWords] * kWords + t % kWords] = rec[t];
+        __syncthreads ();
+     }
+}
+
+// list[0 .. *n_list) without the photons now flagged bad, in order, into io
+__global__ __launch_bounds__ (kBlock)
+void k_still_listed (const uint32_t *__restrict__ list, const uint32_t *__restrict__ flags, uint32_t n, ListIO io)
+{
+   __shared__ uint32_t wc[2 * (kBlock / 64)];
+   const BlockRange range = block_range (*io.n_in, blockIdx.x, gridDim.x);
+   SegWriter sw (io, range, wc);
+   for (uint32_t base = range.lo; base < range.hi; base += kBlock)
+     {
+        const uint32_t q = base + threadIdx.x;
+        uint32_t id = 0;
+        bool keep = false;
+        if (q < range.hi)
+          {
+             id = list[q];
+             keep = (id < n) && ((flags[id] & BAD_PHOTON_MASK) == 0u);
+          }
+        sw.add (keep, id);
+     }
+   sw.finish (io);
+}
+
+// the active list and its energies into pinned host arrays, its length too
+__global__ __launch_bounds__ (kBlock)
+void k_list_out (const uint32_t *__restrict__ list, const uint32_t *__restrict__ n, const double *__restrict__ energy,
+                 uint32_t *__restrict__ index, double *__restrict__ energies, uint32_t *__restrict__ length)
+{
+   const uint32_t m = *n;
+   for (uint32_t q = blockIdx.x * kBlock + threadIdx.x; q < m; q += gridDim.x * kBlock)
+     {
+        const uint32_t id = list[q];
+        index[q] = id;
+        energies[q] = energy[id];
+     }
+   if ((blockIdx.x == 0) && (threadIdx.x == 0)) *length = m;
 }
 
 int ensure_capacity (size_t n)
@@ -235,10 +348,8 @@ int ensure_capacity (size_t n)
    if (d_idx_mid) { (void) hipFree (d_idx_mid); d_idx_mid = nullptr; }
    if (d_seg) { (void) hipFree (d_seg); d_seg = nullptr; }
    if (d_rng_pos) { (void) hipFree (d_rng_pos); d_rng_pos = nullptr; }
-   if (d_tile_cnt) { (void) hipFree (d_tile_cnt); d_tile_cnt = nullptr; }
    if (d_relay_mem) { (void) hipFree (d_relay_mem); d_relay_mem = nullptr; }
    g_capacity = 0;
-   g_tile_cap = 0;
    HIPCHECK (hipMalloc (&mem, total));
    HIPCHECK (hipMalloc (&d_ticks, cap * sizeof (uint64_t)));
    HIPCHECK (hipMalloc (&d_tile_tot, (cap / 2048 + 2) * sizeof (uint64_t)));
@@ -247,9 +358,6 @@ int ensure_capacity (size_t n)
    HIPCHECK (hipMalloc (&d_idx_mid, cap * sizeof (uint32_t)));
    HIPCHECK (hipMalloc (&d_seg, cap * sizeof (uint32_t)));
    HIPCHECK (hipMalloc (&d_rng_pos, cap * sizeof (uint32_t)));
-   // tiles of at least kBlock photons
-   HIPCHECK (hipMalloc (&d_tile_cnt, 2 * (cap / kBlock + 1) * sizeof (uint32_t)));
-   g_tile_cap = cap / kBlock + 1;
    {
       // each relay: seven double, three 32-bit and one byte column
       const size_t dcol = align256 (cap * sizeof (double)), ucol = align256 (cap * sizeof (uint32_t));
@@ -491,6 +599,9 @@ int mxgd_init (void)
      return fail ("device %d is %s; this library is built for gfx950", dev, prop.gcnArchName);
    g_num_cus = prop.multiProcessorCount;
    HIPCHECK (hipStreamCreateWithFlags (&g_stream, hipStreamNonBlocking));
+   HIPCHECK (hipStreamCreateWithFlags (&g_copy_stream, hipStreamNonBlocking));
+   for (unsigned int k = 0; k <= kChunks; k++)
+     HIPCHECK (hipEventCreateWithFlags (&g_copy_ev[k], hipEventDisableTiming));
    HIPCHECK (hipEventCreate (&g_ev0));
    HIPCHECK (hipEventCreate (&g_ev1));
    for (int k = 0; k < kSlots; k++)
@@ -581,7 +692,7 @@ int mxgd_upload_aos (const Marx_Photon_Attr_Type *at, unsigned int n,
         HIPCHECK (hipMemcpyAsync (d_aos, at, (size_t) n * sizeof (Marx_Photon_Attr_Type),
                                   hipMemcpyHostToDevice, g_stream));
         hipLaunchKernelGGL (k_aos_to_soa, dim3 ((n + kBlock - 1) / kBlock), dim3 (kBlock), 0,
-                            g_stream, d_aos, g_soa, (uint32_t) n);
+                            g_stream, d_aos, g_soa, 0u, (uint32_t) n);
         HIPCHECK (hipGetLastError ());
      }
    g_cur = 0;
@@ -1353,7 +1464,8 @@ size_t g_sort_cap = 0, g_sort_tmp = 0;
 double *d_gather = nullptr;          // energies of the active list
 size_t g_gather_cap = 0;
 // pinned host allocations made for photon lists
-void **g_pinned = nullptr;
+struct Pinned { void *p; size_t bytes; };
+Pinned *g_pinned = nullptr;
 size_t g_pinned_n = 0, g_pinned_cap = 0;
 
 int sort_buffers (size_t n)
@@ -1388,19 +1500,20 @@ void *mxgd_host_alloc (size_t bytes)
    if (g_pinned_n == g_pinned_cap)
      {
         size_t cap = g_pinned_cap ? 2 * g_pinned_cap : 64;
-        void **q = (void **) realloc (g_pinned, cap * sizeof (void *));
+        Pinned *q = (Pinned *) realloc (g_pinned, cap * sizeof (Pinned));
         if (q == nullptr) { (void) hipHostFree (p); return nullptr; }
         g_pinned = q;
         g_pinned_cap = cap;
      }
-   g_pinned[g_pinned_n++] = p;
+   g_pinned[g_pinned_n].p = p;
+   g_pinned[g_pinned_n++].bytes = bytes;
    return p;
 }
 
 int mxgd_host_free (void *p)
 {
    for (size_t k = 0; k < g_pinned_n; k++)
-     if (g_pinned[k] == p)
+     if (g_pinned[k].p == p)
        {
           g_pinned[k] = g_pinned[--g_pinned_n];
           (void) hipStreamSynchronize (g_stream);
@@ -1410,11 +1523,19 @@ int mxgd_host_free (void *p)
    return 0;
 }
 
-int mxgd_sort_store_by_energy (unsigned int n, unsigned int *index, double *energies)
+// the records [0, n) of list memory p, by the library's allocation: true
+// when all of them lie in it (kernels may write there)
+static bool is_pinned (const void *p, size_t bytes)
 {
-   if (mxgd_init ()) return -1;
-   if (n > g_n) return fail ("sort of %u photons in a store of %u", n, g_n);
-   if (n == 0) return 0;
+   for (size_t k = 0; k < g_pinned_n; k++)
+     if (g_pinned[k].p == p) return bytes <= g_pinned[k].bytes;
+   return false;
+}
+
+// the sort of the store's first n energies and its result on their way to
+// the host, on g_stream
+static int queue_energy_sort (unsigned int n, unsigned int *index, double *energies)
+{
    if (sort_buffers (n)) return -1;
    char *b = (char *) d_sort;
    double *k_in = (double *) b; b += align256 (g_sort_cap * sizeof (double));
@@ -1425,8 +1546,125 @@ int mxgd_sort_store_by_energy (unsigned int n, unsigned int *index, double *ener
    HIPCHECK (sort_energies (g_soa.energy, n, k_in, v_in, k_out, v_out, b, &tmp, g_stream));
    HIPCHECK (hipMemcpyAsync (index, v_out, (size_t) n * sizeof (uint32_t), hipMemcpyDeviceToHost, g_stream));
    HIPCHECK (hipMemcpyAsync (energies, k_out, (size_t) n * sizeof (double), hipMemcpyDeviceToHost, g_stream));
+   return 0;
+}
+
+int mxgd_sort_store_by_energy (unsigned int n, unsigned int *index, double *energies)
+{
+   if (mxgd_init ()) return -1;
+   if (n > g_n) return fail ("sort of %u photons in a store of %u", n, g_n);
+   if (n == 0) return 0;
+   if (queue_energy_sort (n, index, energies)) return -1;
    HIPCHECK (hipStreamSynchronize (g_stream));
    return 0;
+}
+
+int mxgd_download_sorted (Marx_Photon_Attr_Type *at, unsigned int n, unsigned int *index, double *energies)
+{
+   if (mxgd_init ()) return -1;
+   if (n > g_n) return fail ("download of %u photons from a store of %u", n, g_n);
+   if (n == 0) return 0;
+   if (ensure_aos (n) || sort_buffers (n)) return -1;
+   hipLaunchKernelGGL (k_soa_to_aos, dim3 ((n + kBlock - 1) / kBlock), dim3 (kBlock), 0,
+                       g_stream, d_aos, g_soa, (uint32_t) n);
+   HIPCHECK (hipGetLastError ());
+   HIPCHECK (hipEventRecord (g_copy_ev[kChunks], g_stream));
+   HIPCHECK (hipStreamWaitEvent (g_copy_stream, g_copy_ev[kChunks], 0));
+   hipError_t e = hipMemcpyAsync (at, d_aos, (size_t) n * sizeof (Marx_Photon_Attr_Type), hipMemcpyDeviceToHost,
+                                  g_copy_stream);
+   int status = (e == hipSuccess) ? queue_energy_sort (n, index, energies) : fail ("hipMemcpy: %s", hipGetErrorString (e));
+   // nothing writes to the caller's memory after the return, failed or not
+   if ((hipStreamSynchronize (g_copy_stream) != hipSuccess) || (hipStreamSynchronize (g_stream) != hipSuccess))
+     status = fail ("download of %u photons failed", n);
+   return status;
+}
+
+static int stage_on_chunks (int stage, double arg, unsigned long long seed, Marx_Photon_Attr_Type *at, unsigned int n,
+                            unsigned int *index, double *energies, unsigned int nactive)
+{
+   // the records on their way, in order; the device's copy of them is free
+   // once what g_stream holds is done
+   const unsigned int chunk = ((n + kChunks - 1) / kChunks > 65536u) ? (n + kChunks - 1) / kChunks : 65536u;
+   HIPCHECK (hipEventRecord (g_copy_ev[kChunks], g_stream));
+   HIPCHECK (hipStreamWaitEvent (g_copy_stream, g_copy_ev[kChunks], 0));
+   if (nactive)
+     HIPCHECK (hipMemcpyAsync (d_active, index, (size_t) nactive * sizeof (uint32_t), hipMemcpyHostToDevice, g_stream));
+   for (unsigned int lo = 0, c = 0; lo < n; lo += chunk, c++)
+     {
+        const unsigned int m = (n - lo < chunk) ? n - lo : chunk;
+        HIPCHECK (hipMemcpyAsync (d_aos + lo, at + lo, (size_t) m * sizeof (Marx_Photon_Attr_Type),
+                                  hipMemcpyHostToDevice, g_copy_stream));
+        HIPCHECK (hipEventRecord (g_copy_ev[c], g_copy_stream));
+     }
+   const dim3 block (kBlock);
+   hipLaunchKernelGGL (k_zero_bytes, dim3 ((n + kBlock - 1) / kBlock), block, 0, g_stream, d_marks, n);
+   if (nactive)
+     hipLaunchKernelGGL (k_mark_listed, dim3 ((nactive + kBlock - 1) / kBlock), block, 0, g_stream, d_active, nactive,
+                         n, d_marks);
+   hipLaunchKernelGGL (k_set_u32, dim3 (1), dim3 (1), 0, g_stream, d_counts + 24, (uint32_t) nactive);
+   HIPCHECK (hipGetLastError ());
+   g_cur = 0;
+   g_n = n;
+   for (unsigned int lo = 0, c = 0; lo < n; lo += chunk, c++)
+     {
+        const unsigned int m = (n - lo < chunk) ? n - lo : chunk;
+        const uint32_t blocks = (m + kBlock - 1) / kBlock;
+        const uint32_t *listed = d_idx[g_cur], *n_listed = d_counts + g_cur;
+        HIPCHECK (hipStreamWaitEvent (g_stream, g_copy_ev[c], 0));
+        hipLaunchKernelGGL (k_aos_to_soa, dim3 (blocks), block, 0, g_stream, d_aos, g_soa, lo, lo + m);
+        hipLaunchKernelGGL (k_set_u32, dim3 (1), dim3 (1), 0, g_stream, d_counts + g_cur, 0u);
+        hipLaunchKernelGGL (k_list_marked, dim3 (blocks), block, 0, g_stream, d_marks, lo, lo + m, d_idx[g_cur],
+                            d_counts + g_cur);
+        HIPCHECK (hipGetLastError ());
+        g_upper = (m < nactive) ? m : nactive;
+        if ((stage == MXGD_STAGE_MIRROR) ? mxgd_run_mirror (arg, seed, -1, nullptr, 0, 0)
+            : (stage == MXGD_STAGE_GRATING) ? mxgd_run_grating (seed, -1, nullptr, 0, 0)
+            : mxgd_run_detect (arg, seed, -1, nullptr, 0))
+          return -1;
+        hipLaunchKernelGGL (k_records_out, dim3 (blocks), block, 0, g_stream, (uint64_t *) at, g_soa, listed, n_listed);
+        HIPCHECK (hipGetLastError ());
+     }
+   // the list less the photons absorbed, in its order
+   g_upper = nactive;
+   ListIO io = list_io (MXGD_K_ENTER);
+   io.n_in = d_counts + 24;
+   hipLaunchKernelGGL (k_still_listed, dim3 (io.grid), block, 0, g_stream, d_active, g_soa.flags, n, io);
+   HIPCHECK (launch_compact (io, g_stream));
+   g_cur = 1 - g_cur;
+   const uint32_t blocks = (nactive + kBlock - 1) / kBlock;
+   hipLaunchKernelGGL (k_list_out, dim3 (blocks ? blocks : 1u), block, 0, g_stream, d_idx[g_cur], d_counts + g_cur,
+                       g_soa.energy, index, energies, h_counts);
+   HIPCHECK (hipGetLastError ());
+   return 0;
+}
+
+int mxgd_stage_on_list (int stage, double arg, unsigned long long seed, Marx_Photon_Attr_Type *at, unsigned int n,
+                        unsigned int *index, double *energies, unsigned int nactive, unsigned int *n_out)
+{
+   if (mxgd_init ()) return -1;
+   if ((n == 0) || (nactive > n) || !is_pinned (at, (size_t) n * sizeof (Marx_Photon_Attr_Type))
+       || !is_pinned (index, (size_t) nactive * sizeof (uint32_t))
+       || !is_pinned (energies, (size_t) nactive * sizeof (double)))
+     return 1;
+   g_relay_have = -1;
+   if (ensure_capacity (n) || ensure_aos (n)) return -1;
+   if (n > g_marks_cap)
+     {
+        if (d_marks) (void) hipFree (d_marks);
+        if (d_active) (void) hipFree (d_active);
+        d_marks = nullptr;
+        d_active = nullptr;
+        g_marks_cap = 0;
+        HIPCHECK (hipMalloc (&d_marks, n));
+        HIPCHECK (hipMalloc (&d_active, (size_t) n * sizeof (uint32_t)));
+        g_marks_cap = n;
+     }
+   int status = stage_on_chunks (stage, arg, seed, at, n, index, energies, nactive);
+   // nothing reads or writes the caller's memory after the return, failed or not
+   if ((hipStreamSynchronize (g_copy_stream) != hipSuccess) || (hipStreamSynchronize (g_stream) != hipSuccess))
+     status = fail ("stage on a host list of %u photons failed", n);
+   if (status == 0) *n_out = h_counts[0];
+   return status;
 }
 
 int mxgd_download_active (unsigned int *index, double *energies, unsigned int cap, unsigned int *n_out)

@@ -1,0 +1,74 @@
+"""The drop-in stages on host lists (marx_mirror_reflect,
+marx_grating_diffract, marx_detect): lists in the library's pinned memory,
+whose records travel in overlapping parts, against the same lists in plain
+memory, which are copied whole.  Byte for byte: the records, sorted_index and
+sorted_energies.
+
+- lengths around the block and around one part (65536 records), one past
+  eight whole parts, where the parts grow;
+- sorted_index out of order and without a third of the photons, whose
+  records stay as they are; no photon listed; a listed photon that is
+  flagged bad already."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from marx_amd import Photons, Tracer
+from marx_amd._lib import check
+from tests.test_gpu_source import ON_AXIS
+
+
+class Plain:
+    """A copy of a list in numpy's memory."""
+
+    def __init__(self, p):
+        self.pt = type(p.pt)()
+        ctypes.pointer(self.pt)[0] = p.pt
+        self.records = p.attrs.copy()
+        self.index = np.ctypeslib.as_array(p.pt.sorted_index, shape=(p.capacity,)).copy()
+        self.energies = np.ctypeslib.as_array(p.pt.sorted_energies, shape=(p.capacity,)).copy()
+        self.pt.attributes = self.records.ctypes.data
+        self.pt.sorted_index = self.index.ctypes.data_as(type(p.pt.sorted_index))
+        self.pt.sorted_energies = self.energies.ctypes.data_as(type(p.pt.sorted_energies))
+
+
+def _views(p):
+    a = p.records if isinstance(p, Plain) else p.attrs
+    m = p.pt.num_sorted
+    return (a.view(np.uint8), np.ctypeslib.as_array(p.pt.sorted_index, shape=(max(m, 1),))[:m],
+            np.ctypeslib.as_array(p.pt.sorted_energies, shape=(max(m, 1),))[:m])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grating,det", [("HETG", "ACIS-S"), ("LETG", "HRC-S")])
+@pytest.mark.parametrize("n,listed", [(1, "all"), (257, "some"), (65536, "all"), (65537, "some"), (8 * 65536 + 1, "some"),
+                                      (1000, "none")])
+def test_pinned_lists_match_plain_ones(gpu, grating, det, n, listed):
+    t = Tracer(seed=17, GratingType=grating, DetectorType=det, SourceType="POINT", SpectrumType="FLAT", MinEnergy=0.5,
+               MaxEnergy=7.0, DitherModel="INTERNAL", **ON_AXIS)
+    t.init_source(SourceFlux=n / (1.0e4 * t.geometric_area))
+    p = Photons(n)
+    assert t.create_photons(p, n) == n
+    rng = np.random.default_rng(n)
+    if listed != "all":
+        keep = np.sort(rng.permutation(n)[: (2 * n) // 3 if listed == "some" else 0])
+        idx = rng.permutation(keep).astype(np.uint32)
+        np.ctypeslib.as_array(p.pt.sorted_index, shape=(n,))[: len(idx)] = idx
+        np.ctypeslib.as_array(p.pt.sorted_energies, shape=(n,))[: len(idx)] = p.attrs["energy"][idx]
+        p.pt.num_sorted = len(idx)
+        if len(idx):
+            p.attrs["flags"][idx[0]] = 0x08
+    rows = p.attrs.view(np.uint8).reshape(n, -1)
+    before = rows.copy()
+    unlisted = np.ones(n, bool)
+    unlisted[p.sorted_index()] = False
+    q = Plain(p)
+    for stage in (t.lib.marx_mirror_reflect, t.lib.marx_grating_diffract, t.lib.marx_detect):
+        check(stage(p.ptr, 0), "stage")
+        check(stage(ctypes.pointer(q.pt), 0), "stage")
+        assert p.pt.num_sorted == q.pt.num_sorted and p.pt.history == q.pt.history
+        for a, b in zip(_views(p), _views(q)):
+            assert np.array_equal(a, b)
+    assert np.array_equal(rows[unlisted], before[unlisted])
+    assert p.pt.num_sorted < max(n // 4, 2)
