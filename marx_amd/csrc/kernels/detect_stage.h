@@ -351,7 +351,7 @@ static __device__ __noinline__ double contam_transmission (const mxg_contam &c, 
 template <bool FEF, int KIND>
 __device__ __forceinline__ bool detect_core (const mxg_detector_cfg &d, const float *__restrict__ fa,
                                              const double *__restrict__ da, const Soa &s, uint32_t id, uint32_t tag,
-                                             double energy, vec3 x, vec3 p, uint32_t flags, double tstart,
+                                             double energy, vec3 &x, vec3 &p, uint32_t &flags, double tstart,
                                              unsigned long long seed, uint32_t source_id)
 {
    constexpr bool is_acis = (KIND == MXG_DET_ACIS);
@@ -563,7 +563,6 @@ __device__ __forceinline__ bool detect_core (const mxg_detector_cfg &d, const fl
         x.y += d.offset[1];
         x.z += d.offset[2];
      }
-store_path (s, id, x, p, flags);
    return (flags & BAD_PHOTON_MASK) == 0;
 }
 
@@ -575,12 +574,15 @@ __device__ __forceinline__ bool detect_one (const mxg_detector_cfg &d, const flo
                                             unsigned long long seed, uint32_t source_id,
                                             const Relay *relay = nullptr, uint32_t slot = 0)
 {
-   const uint32_t flags = RELAY ? at (relay->flags, slot) : at (s.flags, id);
+   uint32_t flags = RELAY ? at (relay->flags, slot) : at (s.flags, id);
    if (flags & BAD_PHOTON_MASK) return false;
-   const vec3 x = RELAY ? v3 (at (relay->x0, slot), at (relay->x1, slot), at (relay->x2, slot)) : v3 (at (s.x0, id), at (s.x1, id), at (s.x2, id));
-   const vec3 p = RELAY ? v3 (at (relay->p0, slot), at (relay->p1, slot), at (relay->p2, slot)) : v3 (at (s.p0, id), at (s.p1, id), at (s.p2, id));
-   return detect_core<FEF, KIND> (d, fa, da, s, id, RELAY ? at (relay->tag, slot) : at (s.tag, id),
-                                  RELAY ? at (relay->energy, slot) : at (s.energy, id), x, p, flags, tstart, seed, source_id);
+   vec3 x = RELAY ? v3 (at (relay->x0, slot), at (relay->x1, slot), at (relay->x2, slot)) : v3 (at (s.x0, id), at (s.x1, id), at (s.x2, id));
+   vec3 p = RELAY ? v3 (at (relay->p0, slot), at (relay->p1, slot), at (relay->p2, slot)) : v3 (at (s.p0, id), at (s.p1, id), at (s.p2, id));
+   const bool keep = detect_core<FEF, KIND> (d, fa, da, s, id, RELAY ? at (relay->tag, slot) : at (s.tag, id),
+                                             RELAY ? at (relay->energy, slot) : at (s.energy, id), x, p, flags, tstart,
+                                             seed, source_id);
+   store_path (s, id, x, p, flags);
+   return keep;
 }
 
 } // namespace mxg

@@ -20,10 +20,15 @@
 // (38 percent) through the short part that follows; that costs less than
 // writing, listing and reading the survivors.
 //
+// k_mirror's wave stores what it dropped and what it finished in one go: as
+// two stores, each of which wrote part of the lines, it took 0.58 ms (batch
+// of 6e7: 3.90, now 3.41).  Waves with ranges of their own, without the
+// block's barrier, took longer (0.55): a block's waves share lines.
+//
 // What bounds them now (MI355X, HETG + ACIS-S, 1e7 photons): k_create 0.50 ms,
 // 1.28 GB written (126 bytes a photon: once each) and the vector ALUs busy 58
-// percent of the time; k_mirror 0.58 ms, 1.35 GB, the ALUs busy 55 percent at
-// four waves a SIMD; k_diffract 0.16 ms.  As kernels a stage: source 0.41,
+// percent of the time; k_mirror 0.54 ms, 1.35 GB, the ALUs busy 60 percent at
+// four waves a SIMD; k_diffract 0.15 ms.  As kernels a stage: source 0.41,
 // entry 0.25, reflection 0.68, grating 0.36, detector 0.17 ms.  One launch of
 // independent waves that queue photons for each stage in LDS measured 1.62 ms
 // in all against 1.37: its three waves a SIMD wait for memory at every stage.
@@ -187,12 +192,15 @@ void k_mirror (TraceArgs a, ListIO io, Relay out, uint32_t *__restrict__ counts)
    const uint32_t t0 = a.batch_tag ? *a.batch_tag : a.tag_start;
    const BlockRange range = block_range (*io.n_in, blockIdx.x, gridDim.x);
    SegWriter ordered (io, range, seg_wc);
+   // a lane's list entry is read a photon ahead
+   uint32_t next = (range.lo + threadIdx.x < range.hi) ? io.idx_in[range.lo + threadIdx.x] : 0u;
    uint32_t mirrored = 0, detected = 0;
    PartClock clock;
 
    for (uint32_t base = range.lo; base < range.hi; base += kBlock)
      {
-        const uint32_t i = base + threadIdx.x;
+        const uint32_t i = base + threadIdx.x, entry = next;
+        if (i + kBlock < range.hi) next = io.idx_in[i + kBlock];
         bool keep = false;
         uint32_t id = 0, flags = PHOTON_UNREFLECTED;
         int si = 0;
@@ -200,7 +208,6 @@ void k_mirror (TraceArgs a, ListIO io, Relay out, uint32_t *__restrict__ counts)
         vec3 x, p;
         if (i < range.hi)
           {
-             const uint32_t entry = io.idx_in[i];
              id = entry & kIdMask;
              si = (int) ((entry >> kIdBits) & 3u);
              flags = (entry & kBlocked) ? PHOTON_MIRROR_VBLOCKED : 0u;
@@ -209,7 +216,6 @@ void k_mirror (TraceArgs a, ListIO io, Relay out, uint32_t *__restrict__ counts)
              energy = at (a.s.energy, id);
              const uint32_t rng = (entry & kOddStream) ? a.rng_pos[id] : usual;
              keep = hrma_reflect_core (h, ltab, L, a.fa, a.da, ring, t0 + id, si, energy, rng, a.seed, 0u, x, p, flags);
-             if (!keep || (!G && (KIND < 0))) store_path (a.s, id, x, p, flags);
           }
         clock.spent (0);
         mirrored += (uint32_t) __popcll (__ballot (keep));
@@ -222,8 +228,9 @@ void k_mirror (TraceArgs a, ListIO io, Relay out, uint32_t *__restrict__ counts)
                   stream_init (st, a.seed, t0 + id, MXG_STAGE_GRATING, 0u);
                   keep = GRATING_DIFFRACTS == grating_enter_core<false> (a.cfg->grating, a.fa, a.da, nullptr, nullptr, si,
                                                                          energy, x, p, flags, order, st);
-                  if (!keep) store_path (a.s, id, x, p, flags);
                }
+             // dropped by either stage: one store for both
+             if ((i < range.hi) && !keep) store_path (a.s, id, x, p, flags);
              const uint32_t q = ordered.add (keep, id);
              if (keep)
                {
@@ -245,6 +252,8 @@ void k_mirror (TraceArgs a, ListIO io, Relay out, uint32_t *__restrict__ counts)
                                                 a.seed, 0u);
              detected += (uint32_t) __popcll (__ballot (keep));
           }
+        // the mirror's and the detector's photons in one store
+        if (!G && (i < range.hi)) store_path (a.s, id, x, p, flags);
         clock.spent (1);
      }
    if (G) ordered.finish (io);
@@ -291,7 +300,6 @@ void k_diffract (TraceArgs a, const uint32_t *__restrict__ idx, const uint32_t *
              resume_diffraction (st, a.seed, t0 + id, 0u);
              keep = grating_leave_core<LETG, true> (a.cfg->grating, a.fa, a.da, (const GratingLds *) lds, gtab,
                                                     (int) at (in.shell, q), energy, order, x, p, flags, a.s.sup, id, st);
-             if (!keep || (KIND < 0)) store_path (a.s, id, x, p, flags);
           }
         diffracted += (uint32_t) __popcll (__ballot (keep));
         clock.spent (0);
@@ -301,8 +309,9 @@ void k_diffract (TraceArgs a, const uint32_t *__restrict__ idx, const uint32_t *
                keep = detect_core<false, KIND> (a.cfg->det, a.fa, a.da, a.s, id, t0 + id, energy, x, p, flags, a.tstart,
                                                 a.seed, 0u);
              detected += (uint32_t) __popcll (__ballot (keep));
-             clock.spent (1);
           }
+        if (i < range.hi) store_path (a.s, id, x, p, flags);
+        clock.spent (1);
      }
    block_counts (diffracted, detected, wave_counts, counts + 2 * blockIdx.x);
    clock.finish (a.sums, 4);
