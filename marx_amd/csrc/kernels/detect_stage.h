@@ -1,5 +1,5 @@
 // detect_stage.h -- the per-photon work of focal-plane detection, shared by
-// the stage kernel (detect.hip) and the one-launch batch pass (persist.hip).
+// the stage kernel (detect.hip) and the chunk kernels (passes.hip).
 //
 // ACIS-S / ACIS-I (marx/libsrc/acis-s.c:138-248, acis-i.c:56-167): detector
 //   transform, first chip whose plane hit lies inside it (detector.c:56-168),

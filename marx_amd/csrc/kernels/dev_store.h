@@ -102,12 +102,43 @@ __device__ __forceinline__ T &at (T *col, uint32_t i)
    return *(T *) ((char *) col + (uint32_t) (i * (uint32_t) sizeof (T)));
 }
 
+// a column entry that the kernel writes and no kernel reads soon
+template <class T>
+__device__ __forceinline__ void put_once (T *p, T v)
+{
+   __builtin_nontemporal_store (v, p);
+}
+
 // the path columns of photon id
 __device__ __forceinline__ void store_path (const Soa &s, uint32_t id, vec3 x, vec3 p, uint32_t flags)
 {
    at (s.x0, id) = x.x; at (s.x1, id) = x.y; at (s.x2, id) = x.z;
    at (s.p0, id) = p.x; at (s.p1, id) = p.y; at (s.p2, id) = p.z;
    at (s.flags, id) = flags;
+}
+
+// Chunks of more photons than this store their paths past the caches in the
+// kernels whose waves fill nearly every line: the columns of so many (126
+// bytes a photon) do not stay in the 256 MB cache until they are read, and
+// keeping them costs its bandwidth.  MI355X, trace of n photons with the
+// paths kept and past it: ACIS-S n = 1e6 149 and 151 us, 3e6 318 and 337,
+// 4e6 464 and 419, 6e6 714 and 590; HETG + ACIS-S 2e6 253 and 264, 3e6 379
+// and 366, 6e6 780 and 651.
+constexpr uint32_t kCachedPhotons = 3u << 20;
+
+// store_path in a chunk of n photons
+__device__ __forceinline__ void chunk_path (const Soa &s, uint32_t n, uint32_t id, vec3 x, vec3 p, uint32_t flags)
+{
+   if (n <= kCachedPhotons) store_path (s, id, x, p, flags);
+   else
+     {
+        // (the compiler would make one of the two alternatives, the first)
+        asm volatile ("; past the caches");
+        put_once (&at (s.x0, id), x.x); put_once (&at (s.x1, id), x.y); put_once (&at (s.x2, id), x.z);
+        put_once (&at (s.p0, id), p.x); put_once (&at (s.p1, id), p.y); put_once (&at (s.p2, id), p.z);
+        put_once (&at (s.flags, id), flags);
+        asm volatile ("; to here");
+     }
 }
 
 // a survivor's row of a relay

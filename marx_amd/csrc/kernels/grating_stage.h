@@ -1,5 +1,5 @@
 // grating_stage.h -- the per-photon work of the HETG / LETG stage, shared by
-// the stage kernel (grating.hip) and the one-launch batch pass (persist.hip).
+// the stage kernel (grating.hip) and the chunk kernels (passes.hip).
 //
 // Per photon (the operations of marx/libsrc/diffract.c:974-1130):
 //   grating vignetting draw -> rotate about X into the grating frame ->

@@ -1,6 +1,6 @@
 // hrma_stage.h -- the per-photon work of the HRMA stage (marx/libsrc/hrma.c),
-// shared by the stage kernels (hrma.hip) and the one-launch batch pass
-// (persist.hip).
+// shared by the stage kernels (hrma.hip) and the chunk kernels
+// (passes.hip).
 //
 // Per photon (the operations of marx/libsrc/hrma.c:1161-1341):
 //   vignetting draw -> aperture sampling by cumulative shell area, radius and

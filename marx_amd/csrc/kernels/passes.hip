@@ -25,9 +25,13 @@
 // of 6e7: 3.90, now 3.41).  Waves with ranges of their own, without the
 // block's barrier, took longer (0.55): a block's waves share lines.
 //
-// What bounds them now (MI355X, HETG + ACIS-S, 1e7 photons): k_create 0.50 ms,
-// 1.28 GB written (126 bytes a photon: once each) and the vector ALUs busy 58
-// percent of the time; k_mirror 0.54 ms, 1.35 GB, the ALUs busy 60 percent at
+// Paths of large chunks go past the caches from k_create and k_mirror
+// (chunk_path): the lines are nearly whole and nobody reads them before the
+// kernel ends.  With plain stores k_create took 0.525 ms; k_diffract's few
+// photons a line are merged in the cache (0.150 ms, 0.168 past it).
+//
+// What bounds them now (MI355X, HETG + ACIS-S, 1e7 photons): k_create 0.37 ms,
+// 1.28 GB written (126 bytes a photon: once each); k_mirror 0.54 ms, 1.35 GB, the ALUs busy 60 percent at
 // four waves a SIMD; k_diffract 0.15 ms.  As kernels a stage: source 0.41,
 // entry 0.25, reflection 0.68, grating 0.36, detector 0.17 ms.  One launch of
 // independent waves that queue photons for each stage in LDS measured 1.62 ms
@@ -141,7 +145,7 @@ void k_create (TraceArgs first, ListIO io, uint32_t tilted)
                   si = 0;
                   flags = PHOTON_MIRROR_VBLOCKED;
                }
-             store_path (a.s, i, x, p, flags);
+             chunk_path (a.s, a.n, i, x, p, flags);
              at (a.s.shell, i) = (uint8_t) si;
              entry = i | ((uint32_t) si << kIdBits) | (flags ? kBlocked : 0u) | ((rng != usual) ? kOddStream : 0u);
           }
@@ -230,7 +234,7 @@ void k_mirror (TraceArgs a, ListIO io, Relay out, uint32_t *__restrict__ counts)
                                                                          energy, x, p, flags, order, st);
                }
              // dropped by either stage: one store for both
-             if ((i < range.hi) && !keep) store_path (a.s, id, x, p, flags);
+             if ((i < range.hi) && !keep) chunk_path (a.s, a.n, id, x, p, flags);
              const uint32_t q = ordered.add (keep, id);
              if (keep)
                {
@@ -253,7 +257,7 @@ void k_mirror (TraceArgs a, ListIO io, Relay out, uint32_t *__restrict__ counts)
              detected += (uint32_t) __popcll (__ballot (keep));
           }
         // the mirror's and the detector's photons in one store
-        if (!G && (i < range.hi)) store_path (a.s, id, x, p, flags);
+        if (!G && (i < range.hi)) chunk_path (a.s, a.n, id, x, p, flags);
         clock.spent (1);
      }
    if (G) ordered.finish (io);

@@ -1,5 +1,5 @@
 // source_stage.h -- the per-photon work of photon creation shared by the
-// source kernels (source.hip) and the one-launch batch pass (persist.hip).
+// source kernels (source.hip) and the chunk kernels (passes.hip).
 #pragma once
 
 #include "dev_common.h"
@@ -10,12 +10,6 @@ namespace mxg {
 // A store to a column that no later stage reads, or few photons of it:
 // it is left out of the cache, which then holds the columns that the next
 // stages read and write again.
-template <class T>
-__device__ __forceinline__ void put_once (T *p, T v)
-{
-   __builtin_nontemporal_store (v, p);
-}
-
 // every column of photon i set as a fresh photon of the given energy,
 // direction, time and tag, with no dither offsets; a column that a later
 // step writes is left out (with_t, with_p, with_dith false; with_entry
