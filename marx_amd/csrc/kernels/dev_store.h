@@ -405,9 +405,11 @@ constexpr uint32_t kMaxPersistTile = 4096;
 // The differentiable mirror (diff.hip).
 struct DiffOut
 {
-   double *w, *y, *z;           // n values each
+   // a row for each photon that reached the paraboloid, in the list's order
+   double *w, *y, *z;           // n values each, of which the rows
    double *dw, *dy, *dz;        // MXG_DIFF_NPAR x n derivatives each
-   uint8_t *shell;
+   uint8_t *row_shell;
+   uint8_t *shell;              // by photon
    double *block_w;             // per-block summed weight
 };
 hipError_t launch_diff_forward (const mxg_config *cfg, const float *fa, const double *da,
@@ -416,7 +418,7 @@ hipError_t launch_diff_forward (const mxg_config *cfg, const float *fa, const do
                                 float *win_partial, float *slice_sum, DiffOut out, const ListIO &enter,
                                 uint32_t grid, double *wsum_dev, int tangents, hipStream_t st,
                                 hipEvent_t *ev);
-hipError_t launch_diff_adjoint (uint32_t n, DiffOut in, const mxg_image_spec *spec, const float *g,
+hipError_t launch_diff_adjoint (uint32_t n, const uint32_t *n_rows, DiffOut in, int tangents, const mxg_image_spec *spec, const float *g,
                                 double *partial, uint32_t grid, double *grad_dev, hipStream_t st,
                                 hipEvent_t *ev);
 

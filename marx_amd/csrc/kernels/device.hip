@@ -84,7 +84,7 @@ DiffOut g_diff_out;
 unsigned int g_diff_n = 0;
 mxg_image_spec g_diff_spec;
 uint32_t g_diff_grid = 0;
-bool g_diff_tangents = false;      // the last forward pass kept derivatives
+int g_diff_tangents = 0;           // derivatives the last forward pass carried: none, 2 or MXG_DIFF_NPAR
 unsigned long long g_diff_pass = 0; // forward passes made (over every caller)
 hipEvent_t g_diff_ev[6];           // around k_diff_enter + k_compact, k_diff_forward, k_diff_adjoint
 float g_diff_ms[3] = {0.0f, 0.0f, 0.0f};
@@ -1117,10 +1117,10 @@ int diff_buffers (size_t n, uint32_t grid)
         while (cap < n) cap *= 2;
         if (d_diff) { HIPCHECK (hipStreamSynchronize (g_stream)); (void) hipFree (d_diff); d_diff = nullptr; }
         g_diff_cap = 0;
-        // 3 + 3 * MXG_DIFF_NPAR doubles, one byte and two list words per photon
+        // 3 + 3 * MXG_DIFF_NPAR doubles, two bytes and two list words per photon
         size_t dbl = align256 (cap * sizeof (double));
         size_t u32 = align256 (cap * sizeof (uint32_t));
-        size_t total = (3 + 3 * MXG_DIFF_NPAR) * dbl + align256 (cap) + 2 * u32;
+        size_t total = (3 + 3 * MXG_DIFF_NPAR) * dbl + 2 * align256 (cap) + 2 * u32;
         HIPCHECK (hipMalloc (&d_diff, total));
         char *q = (char *) d_diff;
         g_diff_out.w = (double *) q; q += dbl;
@@ -1130,6 +1130,7 @@ int diff_buffers (size_t n, uint32_t grid)
         g_diff_out.dy = (double *) q; q += MXG_DIFF_NPAR * dbl;
         g_diff_out.dz = (double *) q; q += MXG_DIFF_NPAR * dbl;
         g_diff_out.shell = (uint8_t *) q; q += align256 (cap);
+        g_diff_out.row_shell = (uint8_t *) q; q += align256 (cap);
         d_diff_list = (uint32_t *) q;      // segments, then the list
         g_diff_cap = cap;
      }
@@ -1190,7 +1191,7 @@ int mxgd_diff_forward (const mxg_diff_cfg *d, unsigned int n, unsigned int tag_s
    g_diff_n = n;
    g_diff_spec = *spec;
    g_diff_grid = grid;
-   g_diff_tangents = (tangents != 0);
+   g_diff_tangents = nt;
    g_diff_pass++;
    return 0;
 }
@@ -1207,7 +1208,7 @@ int mxgd_diff_adjoint (unsigned long long pass, unsigned int npix, const float *
      return fail ("gradient image of %u pixels a side for a forward pass of %u", npix, g_diff_spec.npix);
    if (!g_diff_tangents)
      return fail ("the last forward pass (mxg_diff_image) kept no derivatives; call mxg_diff_forward");
-   HIPCHECK (launch_diff_adjoint (g_diff_n, g_diff_out, &g_diff_spec, g, d_diff_partial, g_diff_grid,
+   HIPCHECK (launch_diff_adjoint (g_diff_n, d_diff_u32 + 1, g_diff_out, g_diff_tangents, &g_diff_spec, g, d_diff_partial, g_diff_grid,
                                   d_diff_small + 8, g_stream, g_diff_ev + 4));
    HIPCHECK (hipMemcpyAsync (grad, d_diff_small + 8, kDiffGrad * sizeof (double),
                              hipMemcpyDeviceToHost, g_stream));
@@ -1231,36 +1232,43 @@ int mxgd_diff_state (unsigned int n, double *w, double *y, double *z, double *dw
      return fail ("no forward pass of %u photons", n);
    if (!g_diff_tangents && (dw || dy || dz))
      return fail ("the last forward pass (mxg_diff_image) kept no derivatives");
-   const size_t b = (size_t) n * sizeof (double);
    HIPCHECK (hipStreamSynchronize (g_stream));
-   if (w) HIPCHECK (hipMemcpy (w, g_diff_out.w, b, hipMemcpyDeviceToHost));
-   if (y) HIPCHECK (hipMemcpy (y, g_diff_out.y, b, hipMemcpyDeviceToHost));
-   if (z) HIPCHECK (hipMemcpy (z, g_diff_out.z, b, hipMemcpyDeviceToHost));
-   if (dw) HIPCHECK (hipMemcpy (dw, g_diff_out.dw, MXG_DIFF_NPAR * b, hipMemcpyDeviceToHost));
-   if (dy) HIPCHECK (hipMemcpy (dy, g_diff_out.dy, MXG_DIFF_NPAR * b, hipMemcpyDeviceToHost));
-   if (dz) HIPCHECK (hipMemcpy (dz, g_diff_out.dz, MXG_DIFF_NPAR * b, hipMemcpyDeviceToHost));
-   if (dw || dy || dz)
+   // the device holds rows of the photons that reached the paraboloid, and
+   // what k_diff_forward<2> does not leave out of them; the others' are zero
+   const size_t m = g_diff_listed;
+   const uint32_t *d_list = d_diff_list + align256 (g_diff_cap * sizeof (uint32_t)) / sizeof (uint32_t);
+   uint32_t *ids = (uint32_t *) malloc ((m ? m : 1) * sizeof (uint32_t));
+   if (ids == nullptr) return fail ("out of memory");
+   double *row = (double *) malloc ((m ? m : 1) * sizeof (double)), *wv = (double *) malloc ((m ? m : 1) * sizeof (double));
+   hipError_t e = ((row == nullptr) || (wv == nullptr)) ? hipErrorOutOfMemory : hipSuccess;
+   if ((e == hipSuccess) && m) e = hipMemcpy (ids, d_list, m * sizeof (uint32_t), hipMemcpyDeviceToHost);
+   if ((e == hipSuccess) && m) e = hipMemcpy (wv, g_diff_out.w, m * sizeof (double), hipMemcpyDeviceToHost);
+   // dst (n entries): column col of the rows, or the constant c without one;
+   // zero for photons of weight 0 when derivative is set
+   auto fill = [&] (double *dst, const double *col, double c, bool derivative)
      {
-        // photons lost before the paraboloid have no derivative columns on
-        // the device (see k_diff_enter): their derivatives are 0
-        double *wv = w;
-        if (wv == nullptr)
-          {
-             wv = (double *) malloc (b);
-             if (wv == nullptr) return fail ("out of memory");
-             hipError_t e = hipMemcpy (wv, g_diff_out.w, b, hipMemcpyDeviceToHost);
-             if (e != hipSuccess) { free (wv); return fail ("hipMemcpy: %s", hipGetErrorString (e)); }
-          }
-        for (unsigned int i = 0; i < n; i++)
-          if (wv[i] == 0.0)
-            for (int j = 0; j < MXG_DIFF_NPAR; j++)
-              {
-                 if (dw) dw[(size_t) j * n + i] = 0.0;
-                 if (dy) dy[(size_t) j * n + i] = 0.0;
-                 if (dz) dz[(size_t) j * n + i] = 0.0;
-              }
-        if (wv != w) free (wv);
+        memset (dst, 0, (size_t) n * sizeof (double));
+        if ((e == hipSuccess) && m && (col != nullptr))
+          e = hipMemcpy (row, col, m * sizeof (double), hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return;
+        for (size_t q = 0; q < m; q++)
+          if (!derivative || (wv[q] != 0.0)) dst[ids[q]] = (col != nullptr) ? row[q] : c;
+     };
+   if (w) fill (w, g_diff_out.w, 0.0, false);
+   if (y) fill (y, g_diff_out.y, 0.0, false);
+   if (z) fill (z, g_diff_out.z, 0.0, false);
+   for (int j = 0; j < MXG_DIFF_NPAR; j++)
+     {
+        const size_t o = (size_t) j * n;
+        const bool tilts = (g_diff_tangents == 2);
+        if (dw) fill (dw + o, (tilts && (j > 1)) ? nullptr : g_diff_out.dw + o, 0.0, true);
+        if (dy) fill (dy + o, (tilts && ((j == 2) || (j == 3))) ? nullptr : g_diff_out.dy + o, (j == 2) ? 1.0 : 0.0, true);
+        if (dz) fill (dz + o, (tilts && ((j == 2) || (j == 3))) ? nullptr : g_diff_out.dz + o, (j == 3) ? 1.0 : 0.0, true);
      }
+   free (ids);
+   free (row);
+   free (wv);
+   if (e != hipSuccess) return fail ("mxg_diff_state: %s", hipGetErrorString (e));
    if (shell) HIPCHECK (hipMemcpy (shell, g_diff_out.shell, n, hipMemcpyDeviceToHost));
    return 0;
 }

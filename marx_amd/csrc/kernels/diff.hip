@@ -509,11 +509,12 @@ __device__ __forceinline__ bool diff_enter (const mxg_hrma_cfg &h, const mxg_sou
    return dconic_hit (S.conic_a[0], S.conic_b[0], S.conic_c[0], x, p, S.conic_xmin[0], S.conic_xmax[0]);
 }
 
-// Every photon to its paraboloid intersection, values only.  A lost photon
-// gets its final weight, position and shell here (weight 0, position 0; its
-// derivative columns are not written: a photon of weight 0 adds nothing to
-// the gradient and the adjoint does not read them); the others are listed,
-// in order, for k_diff_forward.
+// Every photon to its paraboloid intersection, values only: its shell, and
+// those that are not lost listed, in order, for k_diff_forward, whose rows
+// are dense: row q of its columns is entry q of the list.  (About half of
+// the photons are lost.  With the columns by photon this kernel also wrote
+// the lost ones' zeros, and the adjoint read lines half of which it did not
+// need: 0.150 and 0.220 ms for 1e7 photons, now 0.137 and 0.116.)
 __global__ __launch_bounds__ (kBlock)
 void k_diff_enter (const mxg_config *__restrict__ cfg, const double *__restrict__ da,
                    const mxg_diff_cfg *__restrict__ dcfg, uint32_t n, uint32_t tag_start,
@@ -532,11 +533,7 @@ void k_diff_enter (const mxg_config *__restrict__ cfg, const double *__restrict_
           {
              DiffPhoton<0> ph;
              keep = diff_enter<0> (h, src, da, dcfg, tag_start + i, seed, ph);
-             if (!keep)
-               {
-                  out.w[i] = 0.0; out.y[i] = 0.0; out.z[i] = 0.0;
-                  out.shell[i] = (uint8_t) ph.si;
-               }
+             out.shell[i] = (uint8_t) ph.si;
           }
         sw.add (keep, i);
      }
@@ -632,15 +629,17 @@ void k_diff_forward (const mxg_config *__restrict__ cfg, const float *__restrict
         else
           w = dc<N> (0.0);
 
-        out.w[i] = w.v; out.y[i] = yf.v; out.z[i] = zf.v;
+        put_once (&out.w[q], w.v);
+        put_once (&out.y[q], yf.v);
+        put_once (&out.z[q], zf.v);
         if constexpr (N == kNP)
           {
 #pragma unroll
              for (int j = 0; j < kNP; j++)
                {
-                  out.dw[(size_t) j * n + i] = w.d[j];
-                  out.dy[(size_t) j * n + i] = yf.d[j];
-                  out.dz[(size_t) j * n + i] = zf.d[j];
+                  out.dw[(size_t) j * n + q] = w.d[j];
+                  out.dy[(size_t) j * n + q] = yf.d[j];
+                  out.dz[(size_t) j * n + q] = zf.d[j];
                }
           }
         else if constexpr (N == 2)
@@ -648,21 +647,20 @@ void k_diff_forward (const mxg_config *__restrict__ cfg, const float *__restrict
              // tilts as traced; the translations (decenter y, decenter z,
              // despace x) move the exit point by themselves and leave the
              // direction and weight alone: d(y, z) = (1, 0), (0, 1),
-             // -(p_y, p_z) / p_x, dw = 0
-             const double one = alive ? 1.0 : 0.0;
-             const double dyx = -ib * p.y.v, dzx = -ib * p.z.v;
-             const double dws[kNP] = {w.d[0], w.d[1], 0.0, 0.0, 0.0};
-             const double dys[kNP] = {yf.d[0], yf.d[1], one, 0.0, alive ? dyx : 0.0};
-             const double dzs[kNP] = {zf.d[0], zf.d[1], 0.0, one, alive ? dzx : 0.0};
+             // -(p_y, p_z) / p_x, dw = 0.  Only what is not a constant is
+             // stored (k_diff_adjoint<true>, mxgd_diff_state): 11 doubles a
+             // photon, not 18.
 #pragma unroll
-             for (int j = 0; j < kNP; j++)
+             for (int j = 0; j < 2; j++)
                {
-                  out.dw[(size_t) j * n + i] = dws[j];
-                  out.dy[(size_t) j * n + i] = dys[j];
-                  out.dz[(size_t) j * n + i] = dzs[j];
+                  put_once (&out.dw[(size_t) j * n + q], w.d[j]);
+                  put_once (&out.dy[(size_t) j * n + q], yf.d[j]);
+                  put_once (&out.dz[(size_t) j * n + q], zf.d[j]);
                }
+             put_once (&out.dy[(size_t) 4 * n + q], -ib * p.y.v);
+             put_once (&out.dz[(size_t) 4 * n + q], -ib * p.z.v);
           }
-        out.shell[i] = (uint8_t) si;
+        put_once (&out.row_shell[q], (uint8_t) si);
 
         if (w.v != 0.0)
           {
@@ -737,9 +735,14 @@ __global__ void k_zero_f (float *__restrict__ a, size_t n)
    for (; i < n; i += stride) a[i] = 0.0f;
 }
 
-// per-block partial gradients: 4 shell pairs x kNP parameters
+// per-block partial gradients: 4 shell pairs x kNP parameters.  TILTS: the
+// forward pass carried the tilts only, and the translations' constant
+// derivatives are not in memory: bound by the columns it reads, 89 bytes a
+// photon instead of 145 (1e7 photons, 4.77e6 rows: 0.297 -> 0.220 ms, and 0.116
+// on dense rows).
+template <bool TILTS>
 __global__ __launch_bounds__ (kBlock)
-void k_diff_adjoint (uint32_t n, DiffOut in, ImageSpec sp, const float *__restrict__ g,
+void k_diff_adjoint (uint32_t n, const uint32_t *__restrict__ n_rows, DiffOut in, ImageSpec sp, const float *__restrict__ g,
                      double *__restrict__ partial)
 {
    constexpr int kG = MXG_NUM_SHELLS * kNP;
@@ -747,7 +750,7 @@ void k_diff_adjoint (uint32_t n, DiffOut in, ImageSpec sp, const float *__restri
    double acc[kG];
 #pragma unroll
    for (int q = 0; q < kG; q++) acc[q] = 0.0;
-   const BlockRange range = block_range (n, blockIdx.x, gridDim.x);
+   const BlockRange range = block_range (*n_rows, blockIdx.x, gridDim.x);
    const double inv_pix = 1.0 / sp.pix;
 
    for (uint32_t i = range.lo + threadIdx.x; i < range.hi; i += blockDim.x)
@@ -759,6 +762,13 @@ void k_diff_adjoint (uint32_t n, DiffOut in, ImageSpec sp, const float *__restri
 #pragma unroll
         for (int j = 0; j < kNP; j++)
           {
+             if (TILTS && (j > 1))
+               {
+                  dw[j] = 0.0;
+                  dy[j] = (j == 2) ? 1.0 : (j == 3) ? 0.0 : in.dy[(size_t) j * n + i];
+                  dz[j] = (j == 2) ? 0.0 : (j == 3) ? 1.0 : in.dz[(size_t) j * n + i];
+                  continue;
+               }
              dw[j] = in.dw[(size_t) j * n + i];
              dy[j] = in.dy[(size_t) j * n + i];
              dz[j] = in.dz[(size_t) j * n + i];
@@ -781,7 +791,7 @@ void k_diff_adjoint (uint32_t n, DiffOut in, ImageSpec sp, const float *__restri
              gu += gc * bu[c];
              gv += gc * bv[c];
           }
-        const int s = in.shell[i];
+        const int s = in.row_shell[i];
 #pragma unroll
         for (int j = 0; j < kNP; j++)
           {
@@ -865,13 +875,15 @@ hipError_t launch_diff_forward (const mxg_config *cfg, const float *fa, const do
    return hipGetLastError ();
 }
 
-hipError_t launch_diff_adjoint (uint32_t n, DiffOut in, const mxg_image_spec *spec, const float *g,
+hipError_t launch_diff_adjoint (uint32_t n, const uint32_t *n_rows, DiffOut in, int tangents, const mxg_image_spec *spec, const float *g,
                                 double *partial, uint32_t grid, double *grad_dev, hipStream_t st,
                                 hipEvent_t *ev)
 {
    ImageSpec sp = {spec->npix, spec->pixel_size, spec->center_y, spec->center_z};
    if (ev) (void) hipEventRecord (ev[0], st);
-   hipLaunchKernelGGL (k_diff_adjoint, dim3 (grid), dim3 (kBlock), 0, st, n, in, sp, g, partial);
+   void (*adjoint) (uint32_t, const uint32_t *, DiffOut, ImageSpec, const float *, double *)
+     = (tangents == 2) ? k_diff_adjoint<true> : k_diff_adjoint<false>;
+   hipLaunchKernelGGL (adjoint, dim3 (grid), dim3 (kBlock), 0, st, n, n_rows, in, sp, g, partial);
    if (ev) (void) hipEventRecord (ev[1], st);
    hipLaunchKernelGGL (k_diff_sum, dim3 (MXG_NUM_SHELLS * kNP), dim3 (kBlock), 0, st, partial, grid,
                        grad_dev, (uint32_t) (MXG_NUM_SHELLS * kNP));
