@@ -70,27 +70,23 @@ BYTES_PER_PHOTON = {
     "k_hrma_reflect": (4 + 4 + 1 + 4 + 4 + 24 + 24 + 8) + (24 + 24 + 4 + 4),
     "grating": (4 + 4 + 4 + 1 + 8 + 24 + 24 + 1) + (24 + 24 + 4 + 1 + 4),
     "detector": (4 + 4 + 4 + 8 + 8 + 24 + 24) + (24 + 24 + 4 + 1 + 4 + 4 + 4),
-    # per photon entering: in: list index; out: w, y, z, their 3 x 5
-    # derivatives, shell (the image stays in L2 / LDS)
-    "k_diff_forward": 4 + 8 * (3 + 15) + 1,
-    # per photon of weight != 0 (the others: their weight, 8 B): in: y, z,
-    # the 15 derivatives, shell
-    "k_diff_adjoint": 8 * (2 + 15) + 1,
+    # per listed photon: in: list index; out: w, y, z, the 8 derivatives that
+    # are not constants, shell (the image stays in L2 / LDS)
+    "k_diff_forward": 4 + 8 * (3 + 8) + 1,
+    # per listed photon, in: w, y, z, the 8 derivatives, shell
+    "k_diff_adjoint": 8 * (3 + 8) + 1,
 }
 # HBM bytes per photon entering a kernel, measured with rocprofv3 counters
 # (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 per dispatch, the factors that make a
 # 1 GiB device copy read back 1 GiB each way); commands and figures in
-# profiles/pmc_hetg_acis_s_1e7.md and profiles/pmc_letg_diff.md.  Absent
+# profiles/pmc_hetg_acis_s_1e7.md.  Absent
 # when not measured for the current kernels.
 # The figure is not measured inside this run (counters need their own
 # profiler runs): each entry names the profile it comes from, and the bench
 # line carries that name beside `traffic`.
 TRAFFIC_BYTES_PER_PHOTON = {
-    ("hetg-acis-s", "k_hrma_reflect"): (312.9, "profiles/pmc_hetg_acis_s_1e7.md"),
-    ("letg-hrc-s", "k_hrma_reflect"): (321.2, "profiles/pmc_letg_diff.md"),
-    ("letg-hrc-s", "grating"): (333.9, "profiles/pmc_letg_diff.md"),
-    # per listed photon
-    ("diff", "k_diff_forward"): (357.1, "profiles/pmc_letg_diff.md"),
+    # k_mirror's, per photon that hit a paraboloid
+    ("hetg-acis-s", "k_hrma_reflect"): (232.1, "profiles/pmc_hetg_acis_s_1e7.md"),
 }
 
 
@@ -187,8 +183,11 @@ def kernel_roofline(cfg, kernels):
     units = kernels[dom]["photons_in"]
     traffic, traffic_src = traffic_of(cfg, dom, units)
     return {"bound": "valu", "pipe": VALU_PIPE,
-            "kernel": "k_grating (stage)" if dom == "grating" else
-                      "k_detect (stage)" if dom == "detector" else dom,
+            # the chunk kernels do two stages each; their time is shared
+            # between those by the cycles that sampled blocks spend in each
+            "kernel": {"grating": "k_mirror and k_diffract (grating part)", "detector": "detector part",
+                       "k_hrma_enter": "k_create (entry part)",
+                       "k_hrma_reflect": "k_mirror (reflection part)"}.get(dom, dom),
             "achieved": kernels[dom]["tflops"], "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
             "frac": kernels[dom]["tflops"] / PEAK_FP64_TFLOPS,
             "traffic": traffic, "traffic_source": traffic_src,
@@ -230,9 +229,6 @@ def measure_batched(args, tmp, torch):
     progress(f"{K} graph-launched steps: {elapsed / K * 1e3:.2f} ms per step")
 
     # per-kernel device times from one uncaptured pass of the same batch
-    # under the staged schedule (the persistent pass is one kernel), which
-    # the per-source loop below also uses
-    tracer.set_schedule(persistent_tile=0)
     tracer.trace_batch(dirs, counts, exposure=T, use_graph=False)
     sms = tracer.stage_ms()
     kms, kin = tracer.kernel_stats()
@@ -254,8 +250,6 @@ def measure_batched(args, tmp, torch):
     torch.cuda.synchronize()
     loop_s = time.perf_counter() - t0
     progress(f"per-source loop: {loop_s:.2f} s")
-    tracer.set_schedule(persistent_tile=sched["persistent_tile"],
-                        persistent_blocks_per_cu=sched["persistent_blocks_per_cu"])
 
     out = {
         "metric": "photons/s traced (HRMA+grating+detector) 1 GPU vs host CPU; gradient evals/s",
@@ -265,7 +259,7 @@ def measure_batched(args, tmp, torch):
         "config": {"workload": DESCRIPTION[cfg], "name": cfg, "sources": len(counts),
                    "photons_per_step": N, "exposure_s": T, "detected_per_step": detected / K},
         "schedule": sched, "autotuned_pass_ms": tuned_ms,
-        "pass": "persistent" if sched["persistent_tile"] else "staged",
+        "pass": "chunk kernels",
         "per_source_loop": {"value": N / loop_s, "unit": "photons/s", "seconds": loop_s,
                             "sources": len(counts)},
         "batched_over_loop": value / (N / loop_s),
@@ -349,7 +343,7 @@ def measure_diff(args, torch):
     kernels = {}
     byt = {"k_diff_enter": None,
            "k_diff_forward": BYTES_PER_PHOTON["k_diff_forward"] * listed,
-           "k_diff_adjoint": 8 * N + BYTES_PER_PHOTON["k_diff_adjoint"] * weighted}
+           "k_diff_adjoint": BYTES_PER_PHOTON["k_diff_adjoint"] * listed}
     for name, ms_k, n_in in (("k_diff_enter", ent_ms / K, N), ("k_diff_forward", fwd_ms / K, listed),
                              ("k_diff_adjoint", adj_ms / K, N)):
         t = ms_k * 1e-3

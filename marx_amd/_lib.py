@@ -81,7 +81,7 @@ class SoaView(ctypes.Structure):
 class Schedule(ctypes.Structure):
     """mxg_schedule: blocks per CU of the source, paraboloid, reflection,
     grating and detector kernels, the reflection kernel's waves per SIMD, and
-    the persistent pass's tile (0: the staged pass) and blocks per CU."""
+    two values that are kept but choose nothing any more (mxg_schedule)."""
     _fields_ = [("blocks_per_cu", ctypes.c_uint * 5), ("reflect_waves", ctypes.c_uint),
                 ("persistent_tile", ctypes.c_uint), ("persistent_blocks_per_cu", ctypes.c_uint)]
 

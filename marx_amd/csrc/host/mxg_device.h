@@ -110,9 +110,10 @@ int mxgd_read_passes (unsigned int n, float *ms, unsigned int *counts);
 
 /* Launch schedule: blocks per CU of the stage kernels (the grating's 0: one
  * round of the blocks a CU holds at once) and the minimum waves
- * per SIMD of the reflection kernel (2, 3 or 4); persist_tile != 0: the
- * batched pass as one persistent launch of persist_blocks_per_cu blocks per
- * CU over tiles of persist_tile photons (a multiple of 256, at most 4096). */
+ * per SIMD of the reflection kernel (2, 3 or 4).  The chunk kernels take the
+ * grids of the entry (k_create), the reflection (k_mirror) and the detector
+ * (k_diffract).  persist_tile (0 or a multiple of 256, at most 4096) and
+ * persist_blocks_per_cu (1..8) are checked and kept, and choose nothing. */
 enum { MXGD_K_SOURCE, MXGD_K_ENTER, MXGD_K_REFLECT, MXGD_K_GRATING, MXGD_K_DETECT, MXGD_NUM_K };
 typedef struct
 {

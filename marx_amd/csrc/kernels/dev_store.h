@@ -399,7 +399,7 @@ hipError_t launch_batch_source (const mxg_config *cfg, const double *da, Soa s, 
                                 uint32_t grid, bool point, bool entry_follows,
                                 hipStream_t st);
 
-// largest persistent tile of a schedule
+// largest persistent tile that a schedule may name
 constexpr uint32_t kMaxPersistTile = 4096;
 
 // The differentiable mirror (diff.hip).

@@ -99,9 +99,11 @@ double *d_diff_small = nullptr;    // summed weight, gradient
 mxg_diff_cfg *d_diff_cfg = nullptr;
 // launch schedule and graph capture
 // Default grids: whole rounds of the blocks a CU holds at once, where that
-// measured fastest (HETG + ACIS-S): the entry (five blocks a CU) at three
-// rounds, 0.240 ms against 0.264 at 8 blocks per CU; the reflection (two to
-// four) at 12 blocks, 0.668 against 0.676; the grating one round (0).
+// measured fastest (HETG + ACIS-S, as kernels a stage): the entry (five
+// blocks a CU) at three rounds, 0.240 ms against 0.264 at 8 blocks per CU;
+// the reflection (two to four) at 12 blocks, 0.668 against 0.676; the grating
+// one round (0).  The chunk kernels take the entry's, the reflection's and
+// the detector's: k_mirror holds four blocks a CU, 12 are three rounds.
 mxgd_schedule g_sched = {{8, 15, 12, 0, 8}, MXG_REFLECT_WAVES_DEFAULT, 0, 2};
 uint32_t g_grating_bpc = 8;        // one round of k_grating blocks per CU (grating_blocks_per_cu)
 int g_capturing = 0;
@@ -599,9 +601,6 @@ int mxgd_init (void)
      return fail ("device %d is %s; this library is built for gfx950", dev, prop.gcnArchName);
    g_num_cus = prop.multiProcessorCount;
    HIPCHECK (hipStreamCreateWithFlags (&g_stream, hipStreamNonBlocking));
-   HIPCHECK (hipStreamCreateWithFlags (&g_copy_stream, hipStreamNonBlocking));
-   for (unsigned int k = 0; k <= kChunks; k++)
-     HIPCHECK (hipEventCreateWithFlags (&g_copy_ev[k], hipEventDisableTiming));
    HIPCHECK (hipEventCreate (&g_ev0));
    HIPCHECK (hipEventCreate (&g_ev1));
    for (int k = 0; k < kSlots; k++)
@@ -1531,6 +1530,17 @@ int mxgd_host_free (void *p)
    return 0;
 }
 
+// The copy stream and its events, made when a host list first needs them: a
+// process that only traces on the device keeps one hardware queue.
+static int copy_stream (void)
+{
+   if (g_copy_stream != nullptr) return 0;
+   for (unsigned int k = 0; k <= kChunks; k++)
+     if (g_copy_ev[k] == nullptr) HIPCHECK (hipEventCreateWithFlags (&g_copy_ev[k], hipEventDisableTiming));
+   HIPCHECK (hipStreamCreateWithFlags (&g_copy_stream, hipStreamNonBlocking));
+   return 0;
+}
+
 // the records [0, n) of list memory p, by the library's allocation: true
 // when all of them lie in it (kernels may write there)
 static bool is_pinned (const void *p, size_t bytes)
@@ -1572,7 +1582,7 @@ int mxgd_download_sorted (Marx_Photon_Attr_Type *at, unsigned int n, unsigned in
    if (mxgd_init ()) return -1;
    if (n > g_n) return fail ("download of %u photons from a store of %u", n, g_n);
    if (n == 0) return 0;
-   if (ensure_aos (n) || sort_buffers (n)) return -1;
+   if (ensure_aos (n) || sort_buffers (n) || copy_stream ()) return -1;
    hipLaunchKernelGGL (k_soa_to_aos, dim3 ((n + kBlock - 1) / kBlock), dim3 (kBlock), 0,
                        g_stream, d_aos, g_soa, (uint32_t) n);
    HIPCHECK (hipGetLastError ());
@@ -1655,7 +1665,7 @@ int mxgd_stage_on_list (int stage, double arg, unsigned long long seed, Marx_Pho
        || !is_pinned (energies, (size_t) nactive * sizeof (double)))
      return 1;
    g_relay_have = -1;
-   if (ensure_capacity (n) || ensure_aos (n)) return -1;
+   if (ensure_capacity (n) || ensure_aos (n) || copy_stream ()) return -1;
    if (n > g_marks_cap)
      {
         if (d_marks) (void) hipFree (d_marks);

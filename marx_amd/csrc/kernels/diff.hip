@@ -107,10 +107,6 @@ template <int N> __device__ __forceinline__ Dual<N> dfma (double a, Dual<N> b, D
    for (int j = 0; j < N; j++) r.d[j] = fma (a, b.d[j], c.d[j]);
    return r;
 }
-template <int N> __device__ __forceinline__ Dual<N> operator+ (Dual<N> a, double b) { a.v += b; return a; }
-template <int N> __device__ __forceinline__ Dual<N> operator+ (double b, Dual<N> a) { a.v = b + a.v; return a; }
-template <int N> __device__ __forceinline__ Dual<N> operator- (Dual<N> a, double b) { a.v -= b; return a; }
-template <int N> __device__ __forceinline__ Dual<N> operator- (double a, Dual<N> b) { return dc<N> (a) - b; }
 
 template <int N> __device__ __forceinline__ Dual<N> dsqrt (Dual<N> a)
 {

@@ -250,8 +250,8 @@ class Tracer:
         """Sets the launch schedule: blocks_per_cu for every kernel, or per
         kernel (source=, enter=, reflect=, grating=, detect=; grating=0,
         the default, is one round of the blocks a CU holds at once), the
-        reflection kernel's waves per SIMD, and the persistent pass's tile
-        (0: the staged pass) and blocks per CU."""
+        reflection kernel's waves per SIMD, and the two persistent_ values,
+        which are checked and kept but choose nothing any more."""
         s = Schedule()
         check(self.lib.mxg_get_schedule(ctypes.byref(s)), "mxg_get_schedule")
         for i, k in enumerate(Schedule.KERNELS):
