@@ -455,6 +455,16 @@ __device__ __forceinline__ void normalize (vec3 &a)
 
 __device__ __forceinline__ vec3 unit (vec3 a) { normalize (a); return a; }
 
+// a / |a| of a vector that the caller gave, of any length (rays of a plug-in
+// or a ray file, a batch's directions): unit_f where the squared length
+// allows it, else normalize, which leaves a zero vector alone
+__device__ __forceinline__ vec3 unit_given (vec3 a)
+{
+   const double l2 = dot_f (a, a);
+   if ((l2 > 1e-290) && (l2 < 1e290)) return scale_f (rsqrt_n (l2), a);
+   return unit (a);
+}
+
 __device__ __forceinline__ double dot (vec3 a, vec3 b)
 {
    return a.x * b.x + a.y * b.y + a.z * b.z;

@@ -61,7 +61,8 @@ __device__ __forceinline__ void store_dith (Soa s, uint32_t i, const float d[3])
 // (s-line.c:89-98); a pixel of an image drawn from its cumulative
 // distribution (fa + image_off), uniform within the pixel, the image centre
 // at -x rotated onto the source direction (s-image.c:284-324).  The draws
-// follow the energy in the source stream.
+// follow the energy in the source stream.  p need not be of length 1 (a
+// batch's directions are the caller's): the result is.
 __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, const float *__restrict__ fa,
                                                     vec3 p, vec3 p_normal, vec3 line_normal, double line_alpha,
                                                     Stream &st)
@@ -70,18 +71,18 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
    if (src.type == MXG_SOURCE_DISK)
      {
         sincos_turn (uniform (st), sn, cs);
-        const vec3 normal = reunit_f (turn_f (p_normal, p, cs, sn));
+        const vec3 normal = unit_given (turn_f (p_normal, p, cs, sn));
         double x0 = src.disk_theta_min / src.disk_theta;
         x0 = x0 * x0;
         double x1 = 1.0 - x0;
         double rnd = src.disk_theta * sqrt_n (x0 + x1 * uniform (st));
         sincos_small (rnd, &sn, &cs);
-        return reunit_f (turn_f (p, normal, cs, sn));
+        return unit_given (turn_f (p, normal, cs, sn));
      }
    if ((src.type == MXG_SOURCE_GAUSS) || (src.type == MXG_SOURCE_BETA))
      {
         sincos_turn (uniform (st), sn, cs);
-        const vec3 normal = reunit_f (turn_f (p_normal, p, cs, sn));
+        const vec3 normal = unit_given (turn_f (p_normal, p, cs, sn));
         double rnd;
         do rnd = uniform (st);
         while (rnd == 0.0);
@@ -90,7 +91,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         else
           rnd = src.beta_core * sqrt (pow (rnd, src.beta_xpon) - 1.0);
         sincos_small (rnd, &sn, &cs);
-        return reunit_f (turn_f (p, normal, cs, sn));
+        return unit_given (turn_f (p, normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_IMAGE)
      {
@@ -105,7 +106,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         sincos_small (x, &sx, &cx);
         sincos_small (y, &sy, &cy);
         sincos_r (line_alpha, sn, cs);
-        return reunit_f (turn_f (v3 (-cy * cx, cy * sx, -sy), line_normal, cs, sn));
+        return unit_given (turn_f (v3 (-cy * cx, cy * sx, -sy), line_normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_LINE)
      {
@@ -114,7 +115,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         const double sin_theta = -sn;
         vec3 q = v3 (-cs, sin_theta * src.line_cos_phi, sin_theta * src.line_sin_phi);
         sincos_r (line_alpha, sn, cs);
-        return reunit_f (turn_f (q, line_normal, cs, sn));
+        return unit_given (turn_f (q, line_normal, cs, sn));
      }
    return p;
 }
@@ -149,7 +150,7 @@ __device__ __forceinline__ void roll_turn (const mxg_source_cfg &src, double *ro
 // tag `tag`, direction p and arrival time t: the Lissajous pointing offset
 // at that time, returned in d as float (as the reference stores the dither
 // state), Gaussian aspect blur, and the rotation of the direction, which is
-// returned.  roll, non-null only where the roll does not vary: sine and
+// returned with length 1 whatever the length of p.  roll, non-null only where the roll does not vary: sine and
 // cosine of roll_turn.
 __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3 p, uint32_t tag, double t,
                                                  double start_time, unsigned long long seed,
@@ -177,7 +178,8 @@ __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3
      }
    else
      sincos_small (-(double) froll, &sr, &cr);
-   p = reunit_f (turn_x_f (p, cr, sr));
+   // the first rotation takes directions that the library did not make
+   p = unit_given (turn_x_f (p, cr, sr));
    double sin_ra, cos_ra, sin_dec, cos_dec;
    sincos_small (ra, &sin_ra, &cos_ra);
    sincos_small (dec, &sin_dec, &cos_dec);
