@@ -163,11 +163,12 @@ __device__ __forceinline__ int reflect_at (const mxg_hrma_cfg &h, const mxg_shel
    if (dg > MXG_PI / 4) return -1;
    if (take (st) < 0.5) dg = -dg;
    // p turned by dg about p x n, which is at right angles to p and not of
-   // length 1: cos p + sin (p x n) x p, with (p x n) x p = n - p (p . n)
-   // and p . n = -p_dot_n after the reflection
+   // length 1: cos p + sin (p x n) x p, with (p x n) x p = n |p|^2 - p (p . n)
+   // and p . n = -p_dot_n after the reflection (|p| is 1 unless a caller's
+   // list holds other directions)
    double sn, cs;
    sincos_small (dg, &sn, &cs);
-   p = unit_f (lin2_f (fma (sn, p_dot_n, cs), p, sn, normal));
+   p = unit_f (lin2_f (fma (sn, p_dot_n, cs), p, sn * dot_f (p, p), normal));
    return 0;
 }
 

@@ -1,11 +1,12 @@
 """Directions that the library did not make and that are not of length 1: the
 rays of a USER plug-in (a ray file's go through the same kernel), a batch's
-directions.  The dither and the extended shapes make them unit vectors; against
-the CPU oracle at the bars of tests/parity.py."""
+directions, a photon list.  The dither and the extended shapes make them unit
+vectors, the mirror takes them as they are; against the CPU oracle at the bars
+of tests/parity.py."""
 import numpy as np
 import pytest
 
-from marx_amd import Photons, Tracer
+from marx_amd import Photons, Tracer, offaxis_directions, on_axis_photons
 from oracle.oracle import Oracle
 from tests.parity import compare
 from tests.test_gpu_batch import ON_AXIS, _batch, _download, _oracle
@@ -30,7 +31,7 @@ def test_user_rays(gpu, tmp_path, length):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,dither,par", [
-    ("POINT", "INTERNAL", {}), ("DISK", "NONE", {"S-DiskTheta0": 5.0, "S-DiskTheta1": 40.0}),
+    ("POINT", "INTERNAL", {}), ("POINT", "NONE", {}), ("DISK", "NONE", {"S-DiskTheta0": 5.0, "S-DiskTheta1": 40.0}),
     ("GAUSS", "INTERNAL", {"S-GaussSigma": 20.0}), ("LINE", "NONE", {"S-LineTheta": 300.0, "S-LinePhi": 60.0})])
 @pytest.mark.parametrize("length", (0.5, 2.0))
 def test_batch_directions(gpu, tmp_path, shape, dither, par, length):
@@ -39,3 +40,19 @@ def test_batch_directions(gpu, tmp_path, shape, dither, par, length):
     t.trace_batch(dirs, counts, tag_start=9, start_time=0.0, exposure=2.0e4, use_graph=False)
     compare(_download(t, int(counts.sum())), _oracle(t, dirs, counts, 9, 0.0, 2.0e4, "NONE"), max_flips=2,
             label=f"{shape} of length {length}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length", LENGTHS)
+def test_lists_at_the_mirror(gpu, length):
+    n = 60_000
+    t = Tracer(seed=6, GratingType="NONE", DetectorType="NONE")
+    rec = on_axis_photons(n, 1.49)
+    rec["p"] = length * offaxis_directions(np.full(n, 2.0e-3), np.linspace(0.0, 2.0 * np.pi, n))
+    pg, po = Photons(n), Photons(n)
+    pg.load(rec)
+    po.load(rec)
+    t.reflect(pg)
+    Oracle(t).reflect(po)
+    compare(pg.active, po.active, max_flips=2, label=f"list of length {length}")
+    assert ((pg.active["flags"] & 0xFF) == 0).any()
