@@ -503,7 +503,8 @@ __device__ __forceinline__ vec3 rotate_vector1 (vec3 p, vec3 n, double c, double
 // sin and cos of t; below 2^-6 rad (the arcsecond-to-arcminute angles of
 // the mirror blur, WFold scatter and dither offsets) from their Taylor
 // polynomials through t^7 and t^8 (truncation below 1e-20 relative: the
-// result differs from sincos's by rounding only), else sincos_r.
+// result differs from sincos's by rounding only), else sincos_r, whose range
+// it has.
 __device__ __forceinline__ void sincos_small (double t, double *sn, double *cs)
 {
    if (fabs (t) < 0.015625)
@@ -516,6 +517,13 @@ __device__ __forceinline__ void sincos_small (double t, double *sn, double *cs)
      }
    else
      sincos_r (t, *sn, *cs);
+}
+
+// sin and cos of any t
+__device__ __forceinline__ void sincos_any (double t, double *sn, double *cs)
+{
+   if (fabs (t) < 1048576.0) sincos_small (t, sn, cs);
+   else sincos (t, sn, cs);
 }
 
 __device__ __forceinline__ vec3 ld3 (const double *a) { return v3 (a[0], a[1], a[2]); }

@@ -117,6 +117,12 @@ __device__ __forceinline__ void quarter_turns (int k, double s, double c, double
    co = ((k + 1) & 2) ? -b : b;
 }
 
+// k mod 2^32 of a whole number |k| < 2^51 (a conversion to int ends at 2^31)
+__device__ __forceinline__ int low_bits (double k)
+{
+   return __double2loint (k + 6755399441055744.0);      // 1.5 x 2^52
+}
+
 // sin and cos of 2 pi u, |u| < 2^20: the quarter turns are taken off
 // exactly, before the product with 2 pi
 __device__ __forceinline__ void sincos_turn (double u, double &s, double &c)
@@ -127,9 +133,10 @@ __device__ __forceinline__ void sincos_turn (double u, double &s, double &c)
    quarter_turns ((int) k, sx, cx, s, c);
 }
 
-// sin and cos of x, |x| < 2^20: k quarter turns are taken off in two parts
-// of pi / 2 (53 bits each, their products exact in the fma), and what the
-// second subtraction rounds off goes on as the tail
+// sin and cos of x, |x| < 2^20 (to 2^50 with an absolute error below 2e-16):
+// k quarter turns are taken off in two parts of pi / 2 (53 bits each: the
+// first product and difference are exact in the fma), and what the second
+// subtraction rounds off goes on as the tail
 __device__ __forceinline__ void sincos_r (double x, double &s, double &c)
 {
    const double k = rint (x * 0.63661977236758134308);
@@ -137,7 +144,7 @@ __device__ __forceinline__ void sincos_r (double x, double &s, double &c)
    const double r = fma (-k, 6.1232339957367660e-17, r1);
    double sx, cx;
    sincos_poly (r, fma (-k, 6.1232339957367660e-17, r1 - r), sx, cx);
-   quarter_turns ((int) k, sx, cx, s, c);
+   quarter_turns (low_bits (k), sx, cx, s, c);
 }
 
 // sin of x, |x| < 2^20: k half turns are taken off, |r| <= pi / 2 goes into
@@ -161,7 +168,13 @@ __device__ __forceinline__ double sin_r (double x)
    p = fma_k (p, z, 1.0 / 120.0);
    p = fma_k (p, z, -1.0 / 6.0);
    const double s = fma (p * z, r, r);
-   return ((int) k & 1) ? -s : s;
+   return (low_bits (k) & 1) ? -s : s;
+}
+
+// sin of any x
+__device__ __forceinline__ double sin_any (double x)
+{
+   return (fabs (x) < 1048576.0) ? sin_r (x) : sin (x);
 }
 
 // log (x), x > 0 and normal: x = 2^e (1 + f), sqrt (1/2) <= 1 + f <

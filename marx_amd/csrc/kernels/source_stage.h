@@ -60,7 +60,9 @@ __device__ __forceinline__ void store_dith (Soa s, uint32_t i, const float d[3])
 // (s-gauss.c:121-137, s-beta.c:108-124); uniform along a line
 // (s-line.c:89-98); a pixel of an image drawn from its cumulative
 // distribution (fa + image_off), uniform within the pixel, the image centre
-// at -x rotated onto the source direction (s-image.c:284-324).  The draws
+// at -x rotated onto the source direction (s-image.c:284-324).  The angles may
+// be of any size: a beta profile of beta near 1/2 has tails of 1e6 radians and
+// far more.  The draws
 // follow the energy in the source stream.  p need not be of length 1 (a
 // batch's directions are the caller's): the result is.
 __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, const float *__restrict__ fa,
@@ -76,7 +78,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         x0 = x0 * x0;
         double x1 = 1.0 - x0;
         double rnd = src.disk_theta * sqrt_n (x0 + x1 * uniform (st));
-        sincos_small (rnd, &sn, &cs);
+        sincos_any (rnd, &sn, &cs);
         return unit_given (turn_f (p, normal, cs, sn));
      }
    if ((src.type == MXG_SOURCE_GAUSS) || (src.type == MXG_SOURCE_BETA))
@@ -90,7 +92,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
           rnd = src.gauss_sigma * sqrt_n (-log_n (rnd));
         else
           rnd = src.beta_core * sqrt (pow (rnd, src.beta_xpon) - 1.0);
-        sincos_small (rnd, &sn, &cs);
+        sincos_any (rnd, &sn, &cs);
         return unit_given (turn_f (p, normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_IMAGE)
@@ -103,15 +105,15 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         y = y * src.image_yscale;
         x = x * src.image_xscale;
         double sx, cx, sy, cy;
-        sincos_small (x, &sx, &cx);
-        sincos_small (y, &sy, &cy);
+        sincos_any (x, &sx, &cx);
+        sincos_any (y, &sy, &cy);
         sincos_r (line_alpha, sn, cs);
         return unit_given (turn_f (v3 (-cy * cx, cy * sx, -sy), line_normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_LINE)
      {
         double theta = src.line_theta * (-1.0 + 2.0 * uniform (st));
-        sincos_small (theta, &sn, &cs);
+        sincos_any (theta, &sn, &cs);
         const double sin_theta = -sn;
         vec3 q = v3 (-cs, sin_theta * src.line_cos_phi, sin_theta * src.line_sin_phi);
         sincos_r (line_alpha, sn, cs);
@@ -143,7 +145,7 @@ __device__ __forceinline__ double rotation_axis (vec3 a, vec3 b, vec3 &c)
 // roll does not vary (roll_amp = 0)
 __device__ __forceinline__ void roll_turn (const mxg_source_cfg &src, double *roll)
 {
-   sincos_small (-(double) (float) src.nominal_roll, &roll[0], &roll[1]);
+   sincos_any (-(double) (float) src.nominal_roll, &roll[0], &roll[1]);
 }
 
 // INTERNAL dither (dither.c:167-182, 551-581, 609-658) of the photon with
@@ -158,13 +160,14 @@ __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3
 {
    Stream st;
    stream_init (st, seed, tag, MXG_STAGE_DITHER, source_id);
-   // the angles as the reference rounds them: the state is kept as float
+   // the angles as the reference rounds them: the state is kept as float; the
+   // phases grow with the time since the start over the period, without limit
    const double tt = (2.0 * MXG_PI) * (start_time + t);
-   float fra = (float) (src.ra_amp * sin_r (div_n (tt, src.ra_period) + src.ra_phase));
-   float fdec = (float) (src.dec_amp * sin_r (div_n (tt, src.dec_period) + src.dec_phase));
+   float fra = (float) (src.ra_amp * sin_any (tt / src.ra_period + src.ra_phase));
+   float fdec = (float) (src.dec_amp * sin_any (tt / src.dec_period + src.dec_phase));
    float froll = (float) src.nominal_roll;
    if (src.roll_amp != 0.0)
-     froll = (float) (src.nominal_roll + src.roll_amp * sin_r (div_n (tt, src.roll_period) + src.roll_phase));
+     froll = (float) (src.nominal_roll + src.roll_amp * sin_any (tt / src.roll_period + src.roll_phase));
    d[0] = fra; d[1] = fdec; d[2] = froll;
    double delta_ra = src.aspect_blur * gaussian (st);
    double delta_dec = src.aspect_blur * gaussian (st);
