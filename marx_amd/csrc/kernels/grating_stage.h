@@ -134,8 +134,8 @@ __device__ __forceinline__ int draw_order (const mxg_grating &g, const float *__
           v = ya;
         else
           {
-             double a = ya, b = yb;
-             v = (float) (a + div_n ((b - a) * (e - x_0), dx_10));
+             const double a = ya, b = yb, num = (b - a) * (e - x_0);
+             v = (float) (a + (inside ? div_n (num, dx_10) : num / dx_10));   // outside, e may be infinite
           }
         if (r <= (double) v)
           return (int) k;
@@ -149,7 +149,9 @@ __device__ __forceinline__ int diffract_photon (const mxg_grating &g, unsigned i
                                                 double theta, double energy, vec3 x, vec3 &p, int order,
                                                 Stream &st)
 {
-   const double n_lambda_over_d = div_n ((double) order * (2.0 * MXG_PI * MXG_HBAR_C), g.period * energy);
+   // the general division: a list's energy may be 0, whose photons no order
+   // but the zeroth lets pass, or infinite
+   const double n_lambda_over_d = (double) order * (2.0 * MXG_PI * MXG_HBAR_C) / (g.period * energy);
    // the facet's normal -x / |x|, and the directions along (l, in the x-z
    // plane) and across (d) its grooves: n . l = 0, so d has length 1
    vec3 n = unit_f (x);
