@@ -482,7 +482,7 @@ __device__ __forceinline__ bool detect_core (const mxg_detector_cfg &d, const fl
                   const mxg_qe_table *fq;
                   if (is_hrc_s)
                     {
-                       double t = div_n (d.shield_x - x.x, p.x);
+                       const double t = (d.shield_x - x.x) / p.x;   // infinite along the plane
                        region = filter_region (d, x.y + t * p.y, x.z + t * p.z);
                        if (region < 0) ok = false;
                        fq = d.filter_qe + (region < 0 ? 0 : region);

@@ -1,5 +1,6 @@
 """Records of a photon list that no source makes, at the edges of the stages'
-divisions: energies of 0 and infinity and next to them; against the CPU oracle."""
+divisions: energies of 0 and infinity and next to them, rays along the shield's
+plane at HRC-S; against the CPU oracle."""
 import numpy as np
 import pytest
 
@@ -66,3 +67,19 @@ def test_energies_at_the_detector(gpu, det, energy):
     t.detect(pg)
     Oracle(t).detect(po)
     _agree(pg.active, po.active, f"{det} {energy}")
+
+
+@pytest.mark.gpu
+def test_rays_along_the_shield(gpu):
+    t = Tracer(seed=82, GratingType="NONE", DetectorType="HRC-S")
+    n = 20_000
+    rec = on_axis_photons(n, 1.0)
+    rng = np.random.default_rng(2)
+    rec["x"] = rng.uniform((-0.5, -1.0, -8.0), (3.0, 1.0, 8.0), (n, 3))
+    rec["p"] = 0.0
+    rec["p"][:, 1] = np.where(rng.random(n) < 0.5, 1.0, -1.0)
+    pg, po = _pair(rec)
+    t.detect(pg)
+    Oracle(t).detect(po)
+    _agree(pg.active, po.active, "HRC-S")
+    assert (po.active["flags"] != po.active["flags"][0]).any()
