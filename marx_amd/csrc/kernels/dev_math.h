@@ -12,7 +12,7 @@
 // Largest error over 2^20 arguments against 80-bit arithmetic, in units of
 // the last place, beside the general form's: division and square root 0.50
 // (0.50), 1 / sqrt 0.99 (1.48 as 1 / sqrt (x)), log 1.07 (0.63), sine and
-// cosine of an angle 0.84 (0.77); of a turn, 1.4e-16 in all (6.9e-16 as
+// cosine of an angle 0.75 (0.77); of a turn, 1.4e-16 in all (6.9e-16 as
 // sincos (2 pi u), whose argument is rounded).
 #pragma once
 
@@ -83,7 +83,8 @@ __device__ __forceinline__ double sqrt_n (double x)
 
 // sin and cos of x + tail, |x| <= pi / 4 (a little more does no harm), tail
 // below an ulp of x: the Taylor series through x^17 and x^16 (truncation
-// below 2e-18)
+// below 2e-18).  TAIL: what the squares round off is carried too.
+template <bool TAIL>
 __device__ __forceinline__ void sincos_poly (double x, double tail, double &s, double &c)
 {
    const double z = x * x;
@@ -95,7 +96,6 @@ __device__ __forceinline__ void sincos_poly (double x, double tail, double &s, d
    p = fma_k (p, z, -1.0 / 5040.0);
    p = fma_k (p, z, 1.0 / 120.0);
    p = fma_k (p, z, -1.0 / 6.0);
-   s = x + fma (p * z, x, tail);
    double q = 1.0 / 20922789888000.0;
    q = fma_k (q, z, -1.0 / 87178291200.0);
    q = fma_k (q, z, 1.0 / 479001600.0);
@@ -105,7 +105,15 @@ __device__ __forceinline__ void sincos_poly (double x, double tail, double &s, d
    q = fma_k (q, z, 1.0 / 24.0);
    // 1 - z / 2 is rounded once, and what it lost goes back with the rest
    const double w = 0.5 * z, a = 1.0 - w;
-   c = a + fma (z * z, q, fma (-x, tail, (1.0 - a) - w));
+   double lost = (1.0 - a) - w;
+   if (TAIL)
+     {
+        s = x + fma (p, z * x, fma (-w, tail, tail));
+        lost = fma (-x, tail, fma (-0.5, fma (x, x, -z), lost));
+     }
+   else
+     s = x + p * z * x;
+   c = a + fma (z * z, q, lost);
 }
 
 // (s, c) turned by k quarter turns
@@ -129,7 +137,7 @@ __device__ __forceinline__ void sincos_turn (double u, double &s, double &c)
 {
    const double k = rint (4.0 * u);
    double sx, cx;
-   sincos_poly (6.283185307179586477 * fma (-0.25, k, u), 0.0, sx, cx);
+   sincos_poly<false> (6.283185307179586477 * fma (-0.25, k, u), 0.0, sx, cx);
    quarter_turns ((int) k, sx, cx, s, c);
 }
 
@@ -143,32 +151,16 @@ __device__ __forceinline__ void sincos_r (double x, double &s, double &c)
    const double r1 = fma (-k, 1.5707963267948965580, x);
    const double r = fma (-k, 6.1232339957367660e-17, r1);
    double sx, cx;
-   sincos_poly (r, fma (-k, 6.1232339957367660e-17, r1 - r), sx, cx);
+   sincos_poly<true> (r, fma (-k, 6.1232339957367660e-17, r1 - r), sx, cx);
    quarter_turns (low_bits (k), sx, cx, s, c);
 }
 
-// sin of x, |x| < 2^20: k half turns are taken off, |r| <= pi / 2 goes into
-// the Taylor series through r^23 (truncation below 2e-18); one series instead
-// of the two of sincos_r
+// sin of x, |x| < 2^20
 __device__ __forceinline__ double sin_r (double x)
 {
-   const double k = rint (x * 0.31830988618379067154);
-   double r = fma (-k, 3.1415926535897931160, x);
-   r = fma (-k, 1.2246467991473532e-16, r);
-   const double z = r * r;
-   double p = -1.0 / 25852016738884976640000.0;
-   p = fma_k (p, z, 1.0 / 51090942171709440000.0);
-   p = fma_k (p, z, -1.0 / 121645100408832000.0);
-   p = fma_k (p, z, 1.0 / 355687428096000.0);
-   p = fma_k (p, z, -1.0 / 1307674368000.0);
-   p = fma_k (p, z, 1.0 / 6227020800.0);
-   p = fma_k (p, z, -1.0 / 39916800.0);
-   p = fma_k (p, z, 1.0 / 362880.0);
-   p = fma_k (p, z, -1.0 / 5040.0);
-   p = fma_k (p, z, 1.0 / 120.0);
-   p = fma_k (p, z, -1.0 / 6.0);
-   const double s = fma (p * z, r, r);
-   return (low_bits (k) & 1) ? -s : s;
+   double s, c;
+   sincos_r (x, s, c);
+   return s;
 }
 
 // sin of any x
