@@ -100,11 +100,10 @@ __device__ __forceinline__ bool polar_pair (double u1, double u2, double &g1, do
    return (g < 1.0) && (g != 0.0);
 }
 
-// its scale sqrt (-2 log (g) / g), as l / sqrt (l g): 0 < g < 1, so l > 0
+// its scale sqrt (-2 log (g) / g), 0 < g < 1
 __device__ __forceinline__ double polar_scale (double g)
 {
-   const double l = -2.0 * log_n (g);
-   return l * rsqrt_n (l * g);
+   return sqrt_n (div_n (-2.0 * log_n (g), g));
 }
 
 __device__ __forceinline__ double gaussian (Stream &s)

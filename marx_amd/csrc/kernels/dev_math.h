@@ -11,9 +11,10 @@
 // rounding makes a residual exact; the polynomials are the Taylor series.
 // Largest error over 2^20 arguments against 80-bit arithmetic, in units of
 // the last place, beside the general form's: division and square root 0.50
-// (0.50), 1 / sqrt 0.99 (1.48 as 1 / sqrt (x)), log 1.07 (0.63), sine and
-// cosine of an angle 0.75 (0.77); of a turn, 1.4e-16 in all (6.9e-16 as
-// sincos (2 pi u), whose argument is rounded).
+// (0.50), 1 / sqrt 0.99 (1.48 as 1 / sqrt (x)), log 0.54 (0.63), sine and
+// cosine of an angle 0.75 (0.77), the polar method's sqrt (-2 log (g) / g)
+// 1.17 (1.18); of a turn, 1.4e-16 in all (6.9e-16 as sincos (2 pi u), whose
+// argument is rounded).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -171,7 +172,8 @@ __device__ __forceinline__ double sin_any (double x)
 
 // log (x), x > 0 and normal: x = 2^e (1 + f), sqrt (1/2) <= 1 + f <
 // sqrt (2), log (1 + f) = 2 atanh (f / (2 + f)) by its series (through
-// the 21st power: truncation below 2e-17 of it)
+// the 21st power: truncation below 1e-18 of it).  The quotient and the sum
+// with e log (2) keep what they round off.
 __device__ __forceinline__ double log_n (double x)
 {
    double m = __builtin_amdgcn_frexp_mant (x);
@@ -181,8 +183,8 @@ __device__ __forceinline__ double log_n (double x)
         m = m + m;
         e--;
      }
-   const double f = m - 1.0;
-   const double s = div_n (f, 2.0 + f);
+   const double f = m - 1.0, t = 2.0 + f, r = rcp_n (t);
+   const double s = div_r (f, t, r);
    const double z = s * s;
    double p = 2.0 / 21.0;
    p = fma_k (p, z, 2.0 / 19.0);
@@ -194,10 +196,12 @@ __device__ __forceinline__ double log_n (double x)
    p = fma_k (p, z, 2.0 / 7.0);
    p = fma_k (p, z, 2.0 / 5.0);
    p = fma_k (p, z, 2.0 / 3.0);
-   p = p * z;
-   // 2 s = f - s f: the large part f is exact
-   const double k = (double) e;
-   return fma (k, 0.69314718055994528623, f) - fma (s, f - p, k * -2.3190468138462995584e-17);
+   // f - s (2 + f), with the rounding f - (t - 2) of t
+   const double rest = fma (-s, f - (t - 2.0), fma (-s, t, f)) * r;
+   const double k = (double) e, s2 = s + s;
+   const double h = fma (k, 0.69314718055994528623, s2);
+   const double l = fma (k, 0.69314718055994528623, -h) + s2;
+   return h + (l + fma (k, 2.3190468138462995584e-17, fma (p, z * s, rest + rest)));
 }
 
 // a ^ b ^ c, one instruction on gfx950
