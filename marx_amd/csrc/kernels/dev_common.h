@@ -100,10 +100,14 @@ __device__ __forceinline__ bool polar_pair (double u1, double u2, double &g1, do
    return (g < 1.0) && (g != 0.0);
 }
 
-// its scale sqrt (-2 log (g) / g), 0 < g < 1
+// its scale f = sqrt (l / g), l = -2 log (g): l / sqrt (l g), and a step of
+// Newton's method on f^2 g = l (0 < g < 1, so l > 0)
 __device__ __forceinline__ double polar_scale (double g)
 {
-   return sqrt_n (div_n (-2.0 * log_n (g), g));
+   const double l = -2.0 * log_n (g);
+   const double y = rsqrt_n (l * g), f = l * y, fg = f * g;
+   const double rest = fma (-f, fma (f, g, -fg), fma (-f, fg, l));
+   return fma (rest, 0.5 * y, f);
 }
 
 __device__ __forceinline__ double gaussian (Stream &s)

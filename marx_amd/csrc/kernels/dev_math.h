@@ -13,7 +13,7 @@
 // the last place, beside the general form's: division and square root 0.50
 // (0.50), 1 / sqrt 0.99 (1.48 as 1 / sqrt (x)), log 0.54 (0.63), sine and
 // cosine of an angle 0.75 (0.77), the polar method's sqrt (-2 log (g) / g)
-// 1.17 (1.18); of a turn, 1.4e-16 in all (6.9e-16 as sincos (2 pi u), whose
+// 0.90 (1.18); of a turn, 1.4e-16 in all (6.9e-16 as sincos (2 pi u), whose
 // argument is rounded).
 #pragma once
 
@@ -51,6 +51,12 @@ __device__ __forceinline__ double div_r (double a, double b, double r)
 __device__ __forceinline__ double div_n (double a, double b)
 {
    return div_r (a, b, rcp_n (b));
+}
+
+// a / b as div_n, and as the general form where a or b is 0, infinite or NaN
+__device__ __forceinline__ double div_x (double a, double b)
+{
+   return __builtin_amdgcn_div_fixup (div_n (a, b), b, a);
 }
 
 // 1 / sqrt (x); x > 0 and normal

@@ -53,6 +53,14 @@ __device__ __forceinline__ void store_dith (Soa s, uint32_t i, const float d[3])
      }
 }
 
+// a / |a|, of a vector that a rotation made from a unit vector or, GIVEN, from
+// one of any length
+template <bool GIVEN>
+__device__ __forceinline__ vec3 unit_of (vec3 a)
+{
+   return GIVEN ? unit_given (a) : reunit_f (a);
+}
+
 // The direction of a photon of the configured source shape about the source
 // direction p (p_normal: a unit vector normal to p; line_normal and
 // line_alpha: the rotation of -x onto p): a point source's p; uniform over
@@ -63,8 +71,9 @@ __device__ __forceinline__ void store_dith (Soa s, uint32_t i, const float d[3])
 // at -x rotated onto the source direction (s-image.c:284-324).  The angles may
 // be of any size: a beta profile of beta near 1/2 has tails of 1e6 radians and
 // far more.  The draws
-// follow the energy in the source stream.  p need not be of length 1 (a
-// batch's directions are the caller's): the result is.
+// follow the energy in the source stream.  GIVEN: p is the caller's and need
+// not be of length 1 (a batch's directions); the result is.
+template <bool GIVEN>
 __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, const float *__restrict__ fa,
                                                     vec3 p, vec3 p_normal, vec3 line_normal, double line_alpha,
                                                     Stream &st)
@@ -73,18 +82,18 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
    if (src.type == MXG_SOURCE_DISK)
      {
         sincos_turn (uniform (st), sn, cs);
-        const vec3 normal = unit_given (turn_f (p_normal, p, cs, sn));
+        const vec3 normal = unit_of<GIVEN> (turn_f (p_normal, p, cs, sn));
         double x0 = src.disk_theta_min / src.disk_theta;
         x0 = x0 * x0;
         double x1 = 1.0 - x0;
         double rnd = src.disk_theta * sqrt_n (x0 + x1 * uniform (st));
         sincos_any (rnd, &sn, &cs);
-        return unit_given (turn_f (p, normal, cs, sn));
+        return unit_of<GIVEN> (turn_f (p, normal, cs, sn));
      }
    if ((src.type == MXG_SOURCE_GAUSS) || (src.type == MXG_SOURCE_BETA))
      {
         sincos_turn (uniform (st), sn, cs);
-        const vec3 normal = unit_given (turn_f (p_normal, p, cs, sn));
+        const vec3 normal = unit_of<GIVEN> (turn_f (p_normal, p, cs, sn));
         double rnd;
         do rnd = uniform (st);
         while (rnd == 0.0);
@@ -93,7 +102,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         else
           rnd = src.beta_core * sqrt (pow (rnd, src.beta_xpon) - 1.0);
         sincos_any (rnd, &sn, &cs);
-        return unit_given (turn_f (p, normal, cs, sn));
+        return unit_of<GIVEN> (turn_f (p, normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_IMAGE)
      {
@@ -108,7 +117,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         sincos_any (x, &sx, &cx);
         sincos_any (y, &sy, &cy);
         sincos_r (line_alpha, sn, cs);
-        return unit_given (turn_f (v3 (-cy * cx, cy * sx, -sy), line_normal, cs, sn));
+        return unit_of<GIVEN> (turn_f (v3 (-cy * cx, cy * sx, -sy), line_normal, cs, sn));
      }
    if (src.type == MXG_SOURCE_LINE)
      {
@@ -117,7 +126,7 @@ __device__ __forceinline__ vec3 extended_direction (const mxg_source_cfg &src, c
         const double sin_theta = -sn;
         vec3 q = v3 (-cs, sin_theta * src.line_cos_phi, sin_theta * src.line_sin_phi);
         sincos_r (line_alpha, sn, cs);
-        return unit_given (turn_f (q, line_normal, cs, sn));
+        return unit_of<GIVEN> (turn_f (q, line_normal, cs, sn));
      }
    return p;
 }
@@ -152,8 +161,10 @@ __device__ __forceinline__ void roll_turn (const mxg_source_cfg &src, double *ro
 // tag `tag`, direction p and arrival time t: the Lissajous pointing offset
 // at that time, returned in d as float (as the reference stores the dither
 // state), Gaussian aspect blur, and the rotation of the direction, which is
-// returned with length 1 whatever the length of p.  roll, non-null only where the roll does not vary: sine and
+// returned; GIVEN: p is a direction that the library did not make, of any
+// length (the result's is 1).  roll, non-null only where the roll does not vary: sine and
 // cosine of roll_turn.
+template <bool GIVEN>
 __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3 p, uint32_t tag, double t,
                                                  double start_time, unsigned long long seed,
                                                  uint32_t source_id, float d[3], const double *roll = nullptr)
@@ -163,11 +174,11 @@ __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3
    // the angles as the reference rounds them: the state is kept as float; the
    // phases grow with the time since the start over the period, without limit
    const double tt = (2.0 * MXG_PI) * (start_time + t);
-   float fra = (float) (src.ra_amp * sin_any (tt / src.ra_period + src.ra_phase));
-   float fdec = (float) (src.dec_amp * sin_any (tt / src.dec_period + src.dec_phase));
+   float fra = (float) (src.ra_amp * sin_any (div_x (tt, src.ra_period) + src.ra_phase));
+   float fdec = (float) (src.dec_amp * sin_any (div_x (tt, src.dec_period) + src.dec_phase));
    float froll = (float) src.nominal_roll;
    if (src.roll_amp != 0.0)
-     froll = (float) (src.nominal_roll + src.roll_amp * sin_any (tt / src.roll_period + src.roll_phase));
+     froll = (float) (src.nominal_roll + src.roll_amp * sin_any (div_x (tt, src.roll_period) + src.roll_phase));
    d[0] = fra; d[1] = fdec; d[2] = froll;
    double delta_ra = src.aspect_blur * gaussian (st);
    double delta_dec = src.aspect_blur * gaussian (st);
@@ -181,8 +192,7 @@ __device__ __forceinline__ vec3 internal_dither (const mxg_source_cfg &src, vec3
      }
    else
      sincos_small (-(double) froll, &sr, &cr);
-   // the first rotation takes directions that the library did not make
-   p = unit_given (turn_x_f (p, cr, sr));
+   p = unit_of<GIVEN> (turn_x_f (p, cr, sr));
    double sin_ra, cos_ra, sin_dec, cos_dec;
    sincos_small (ra, &sin_ra, &cos_ra);
    sincos_small (dec, &sin_dec, &cos_dec);
@@ -204,7 +214,7 @@ __device__ __forceinline__ void apply_internal_dither (const mxg_source_cfg &src
                                                        unsigned long long seed, uint32_t source_id)
 {
    float d[3];
-   vec3 p = internal_dither (src, v3 (at (s.p0, i), at (s.p1, i), at (s.p2, i)), at (s.tag, i), t, start_time, seed, source_id, d);
+   vec3 p = internal_dither<true> (src, v3 (at (s.p0, i), at (s.p1, i), at (s.p2, i)), at (s.tag, i), t, start_time, seed, source_id, d);
    store_dith (s, i, d);
    at (s.p0, i) = p.x; at (s.p1, i) = p.y; at (s.p2, i) = p.z;
 }
@@ -244,7 +254,7 @@ __device__ __forceinline__ void source_draws (const mxg_source_cfg &src, const f
    if (POINT)
      p = ld3 (src.p);
    else
-     p = extended_direction (src, fa, ld3 (src.p), ld3 (src.p_normal), ld3 (src.line_normal), src.line_alpha, st);
+     p = extended_direction<false> (src, fa, ld3 (src.p), ld3 (src.p_normal), ld3 (src.line_normal), src.line_alpha, st);
    gap = 0;
    t = 0.0;
    if (poisson)
@@ -299,7 +309,7 @@ __device__ __forceinline__ NewPhoton source_photon (const mxg_source_cfg &src, c
      }
    ph.dithered = (src.dither_mode == MXG_DITHER_INTERNAL);
    if (ph.dithered)
-     ph.p = internal_dither (src, ph.p, tag, ph.t, start_time, seed, source_id, ph.d, roll);
+     ph.p = internal_dither<false> (src, ph.p, tag, ph.t, start_time, seed, source_id, ph.d, roll);
    return ph;
 }
 
@@ -381,12 +391,12 @@ __device__ __forceinline__ NewPhoton batch_photon (const mxg_source_cfg &src, co
         vec3 ln = v3 (0.0, 0.0, 0.0);
         double la = 0.0;
         if (src.type == MXG_SOURCE_LINE) la = rotation_axis (v3 (-1.0, 0.0, 0.0), ph.p, ln);
-        ph.p = extended_direction (src, nullptr, ph.p, nrm, ln, la, st);
+        ph.p = extended_direction<true> (src, nullptr, ph.p, nrm, ln, la, st);
      }
    ph.t = exposure * uniform (st);
    ph.active = true;
    ph.dithered = (src.dither_mode == MXG_DITHER_INTERNAL);
-   if (ph.dithered) ph.p = internal_dither (src, ph.p, tag, ph.t, start_time, seed, 0u, ph.d, roll);
+   if (ph.dithered) ph.p = internal_dither<true> (src, ph.p, tag, ph.t, start_time, seed, 0u, ph.d, roll);
    return ph;
 }
 

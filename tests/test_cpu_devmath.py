@@ -34,6 +34,7 @@ static int __double2loint (double x) { uint64_t u; memcpy (&u, &x, 8); return (i
 #define __builtin_amdgcn_rsq(x) coarse (1.0 / std::sqrt (x))
 #define __builtin_amdgcn_frexp_mant(x) mantissa (x)
 #define __builtin_amdgcn_frexp_exp(x) exponent (x)
+#define __builtin_amdgcn_div_fixup(q, b, a) ((std::isfinite (q) && (q) != 0.0) ? (q) : (a) / (b))
 #define __builtin_amdgcn_bitop3_b32(a, b, c, d) ((a) ^ (b) ^ (c))
 """
 
@@ -127,7 +128,7 @@ def worst(tmp_path_factory):
     return dict(zip(out[::2], map(float, out[1::2])))
 
 
-@pytest.mark.parametrize("name,bar", [("div", 0.502), ("sqrt", 0.502), ("rsqrt", 1.0), ("log", 0.63), ("polar", 1.18)]
+@pytest.mark.parametrize("name,bar", [("div", 0.502), ("sqrt", 0.502), ("rsqrt", 1.0), ("log", 0.63), ("polar", 0.95)]
                          + [(f"{f}{k}", 0.77) for f in ("sin", "cos") for k in range(4)])
 def test_largest_error_in_units_of_the_last_place(worst, name, bar):
     assert worst[name] <= bar
