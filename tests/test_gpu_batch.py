@@ -1,8 +1,10 @@
 """Batched point sources (mxg_trace_batch): one device pass over many sources
 with uneven photon counts, against the CPU oracle; the same photons as a
-per-source loop; independent of the launch schedule, staged or persistent;
-HIP-graph replays equal to eager passes; the autotuner installs a valid
-schedule."""
+per-source loop; independent of the launch schedule's grids, and of its
+persistent fields, which are kept and choose nothing; HIP-graph replays equal
+to eager passes; the autotuner installs a valid schedule.  (The kernels that
+the schedule's other fields choose between run with a FEF file and on host
+lists: tests/test_gpu_fef_trace.py.)"""
 import numpy as np
 import pytest
 
@@ -199,14 +201,10 @@ def test_graph_is_recaptured_after_the_store_grows(gpu, tmp_path):
                                                 ("HETG", "NONE", "NONE"), ("LETG", "ACIS-S", "NONE"),
                                                 ("HETG", "HRC-I", "INTERNAL")])
 def test_persistent_pass_equals_the_staged_pass(gpu, tmp_path, grating, det, dither):
-    """The batched pass as one persistent launch (blocks taking tiles of
-    photons from a work counter, every stage on a tile back to back) gives
-    the staged pass's records, detected list and stage counts, for tiles of
-    256 to 4096 photons at 1 to 8 blocks per CU, eager and graph-launched.
-    The staged pass hands survivors on through the dense relays (grating to
-    detector; mirror to an LETG grating) while the persistent pass reads
-    the store, so the combinations also check every detector family's and
-    both gratings' relay instances against the store path."""
+    """The schedule's persistent fields are accepted and change nothing: the
+    same records, detected list and stage counts with tiles of 256 to 4096
+    photons at 1 to 8 blocks per CU, eager and graph-launched, for every
+    detector family and both gratings."""
     t, dirs, counts = _batch(tmp_path, 48, grating=grating, det=det, dither=dither)
     n = int(counts.sum())
     t.set_schedule(blocks_per_cu=8, reflect_waves=4, persistent_tile=0)
