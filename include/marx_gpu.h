@@ -439,11 +439,12 @@ int mxg_set_schedule (const mxg_schedule *s);
 int mxg_get_schedule (mxg_schedule *s);
 
 /* Autotuner: times the batch of mxg_trace_batch (same arguments) under
- * candidate schedules -- blocks per CU in {2, 4, 8, 16} for every stage and
- * one round (0) for the grating, then 2, 3 and 4 waves for the reflection --
- * keeping for each the fastest (best of `repeats` runs), installs the
- * schedule found, and returns it in *best and the time of its graph-launched
- * pass in *best_ms. */
+ * candidate schedules -- blocks per CU in {2, 4, 8, 16} for each grid that the
+ * pass reads (mxg_schedule; with a FEF file, where every stage is a kernel of
+ * its own, every grid, one round (0) for the grating, then 2, 3 and 4 waves
+ * for the reflection) -- keeping for each the fastest (best of `repeats` runs)
+ * and what the pass does not read as it was, installs the schedule found, and
+ * returns it in *best and the time of its graph-launched pass in *best_ms. */
 int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsigned int *counts,
                         unsigned int tag_start, double start_time, double exposure,
                         unsigned int repeats, mxg_schedule *best, float *best_ms);

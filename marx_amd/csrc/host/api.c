@@ -934,8 +934,10 @@ int mxg_get_schedule (mxg_schedule *s)
    return 0;
 }
 
-/* per-kernel times of one timed (uncaptured) batch pass, best of repeats:
- * source, paraboloid, reflection, grating stage, detector stage */
+/* times of one timed (uncaptured) batch pass, best of repeats, by the schedule's
+ * grid that they depend on: those of source, paraboloid, reflection, grating
+ * and detector; of the chunk kernels k_create (the paraboloid's grid), k_mirror
+ * (the reflection's) and k_diffract (the detector's) */
 static int time_kernels (unsigned int num_sources, const double *dirs, const unsigned int *counts,
                          unsigned int tag_start, double start_time, double exposure,
                          unsigned int repeats, float best[5])
@@ -953,6 +955,15 @@ static int time_kernels (unsigned int num_sources, const double *dirs, const uns
         t[2] = Kernel_Ms[1];
         t[3] = Last_Slot_Ms[2];
         t[4] = Last_Slot_Ms[3];
+        if (mxgd_passes_fit ())
+          {
+             float ms[3];
+             mxgd_passes_kernel_ms (ms);
+             t[0] = t[3] = 0.0f;
+             t[1] = ms[0];
+             t[2] = ms[1];
+             t[4] = ms[2];
+          }
         for (int k = 0; k < 5; k++)
           if (t[k] < best[k]) best[k] = t[k];
      }
@@ -983,25 +994,35 @@ int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsi
    static const unsigned int bpc[4] = {2, 4, 8, 16};
    mxg_schedule cur, sel;
    float best_t[5], t[5], pass_ms;
-   int k, c;
+   int chunk, k, c;
+   /* the grids that the pass reads */
+   int reads[5] = {1, 1, 1, 1, 1};
 
    if (repeats == 0) repeats = 1;
-   if (-1 == mxg_get_schedule (&cur))
+   if ((-1 == sync_config ()) || (-1 == mxg_get_schedule (&cur)))
      return -1;
+   chunk = mxgd_passes_fit ();
+   if (chunk)
+     {
+        reads[0] = reads[3] = 0;
+        reads[4] = (Grating_Type == MARX_GRATING_HETG) || (Grating_Type == MARX_GRATING_LETG);
+     }
    sel = cur;
    sel.persistent_tile = 0;
    for (k = 0; k < 5; k++) best_t[k] = 1e30f;
-   /* blocks per CU, every stage at once (their times are independent) */
+   /* blocks per CU, every kernel's at once (a kernel's time depends on its own
+    * grid) */
    for (c = 0; c < 4; c++)
      {
         mxg_schedule s = sel;
-        for (k = 0; k < 5; k++) s.blocks_per_cu[k] = bpc[c];
+        for (k = 0; k < 5; k++)
+          if (reads[k]) s.blocks_per_cu[k] = bpc[c];
         if ((-1 == mxg_set_schedule (&s))
             || (-1 == time_kernels (num_sources, dirs, counts, tag_start, start_time, exposure,
                                     repeats, t)))
           goto fail;
         for (k = 0; k < 5; k++)
-          if (t[k] < best_t[k])
+          if (reads[k] && (t[k] < best_t[k]))
             {
                best_t[k] = t[k];
                sel.blocks_per_cu[k] = bpc[c];
@@ -1009,22 +1030,23 @@ int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsi
      }
    /* the grating at one round of the blocks a CU holds at once (0), which
     * none of the counts above need be (three for HETG) */
-   {
-      mxg_schedule s = sel;
-      s.blocks_per_cu[3] = 0;
-      if ((-1 == mxg_set_schedule (&s))
-          || (-1 == time_kernels (num_sources, dirs, counts, tag_start, start_time, exposure,
-                                  repeats, t)))
-        goto fail;
-      if (t[3] < best_t[3])
-        {
-           best_t[3] = t[3];
-           sel.blocks_per_cu[3] = 0;
-        }
-   }
+   if (!chunk)
+     {
+        mxg_schedule s = sel;
+        s.blocks_per_cu[3] = 0;
+        if ((-1 == mxg_set_schedule (&s))
+            || (-1 == time_kernels (num_sources, dirs, counts, tag_start, start_time, exposure,
+                                    repeats, t)))
+          goto fail;
+        if (t[3] < best_t[3])
+          {
+             best_t[3] = t[3];
+             sel.blocks_per_cu[3] = 0;
+          }
+     }
    /* the reflection kernel's register budget */
    best_t[2] = 1e30f;
-   for (c = 2; c <= 4; c++)
+   for (c = 2; (c <= 4) && !chunk; c++)
      {
         mxg_schedule s = sel;
         s.reflect_waves = (unsigned int) c;

@@ -107,6 +107,9 @@ int mxgd_run_passes (unsigned int n, unsigned int tag_start, double start_time, 
                      unsigned long long seed, float *ms, unsigned int *counts);
 /* Waits for the stream; ms and counts of the batch pass that ran last. */
 int mxgd_read_passes (unsigned int n, float *ms, unsigned int *counts);
+/* ms[3]: the times of k_create, k_mirror and (0 without a grating) k_diffract
+ * in the pass that was read last, each with the compaction after it. */
+void mxgd_passes_kernel_ms (float *ms);
 
 /* Launch schedule: blocks per CU of the stage kernels (the grating's 0: one
  * round of the blocks a CU holds at once) and the minimum waves

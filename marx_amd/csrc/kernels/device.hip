@@ -1020,6 +1020,8 @@ PassLists pass_lists (unsigned int n)
    return l;
 }
 
+float g_pass_ms[3];                // k_create, k_mirror, k_diffract of the pass read last
+
 // The counts of the last launch by timing slot (the stream is synchronised),
 // and with ms its times: the stages of a kernel share its time by the cycles
 // its sampled blocks spent in each, and the source's includes the arrival-time
@@ -1041,6 +1043,7 @@ void read_trace (unsigned int n, bool scanned, float *ms, unsigned int *counts)
    double t[6], scan = scanned ? (double) (r.create - r.scan) / g_clock_khz : 0.0;
    const double length[3] = {(double) (r.mirror - r.create), (double) ((grating ? r.diffract : r.end) - r.mirror),
                              grating ? (double) (r.end - r.diffract) : 0.0};
+   for (int k = 0; k < 3; k++) g_pass_ms[k] = (float) (length[k] / g_clock_khz);
    for (int k = 0; k < 6; k++)
      {
         const double both = (double) (r.busy[k & ~1] + r.busy[k | 1]);
@@ -1099,6 +1102,11 @@ int mxgd_read_passes (unsigned int n, float *ms, unsigned int *counts)
    HIPCHECK (hipStreamSynchronize (g_stream));
    read_trace (n, false, ms, counts);
    return 0;
+}
+
+void mxgd_passes_kernel_ms (float *ms)
+{
+   for (int k = 0; k < 3; k++) ms[k] = g_pass_ms[k];
 }
 
 /* ---- differentiable mirror ------------------------------------------------------ */

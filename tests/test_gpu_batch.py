@@ -163,6 +163,19 @@ def test_autotuner_installs_a_valid_schedule(gpu, tmp_path, grating, det):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("grating,det", [("NONE", "ACIS-I"), ("LETG", "HRC-S")])
+def test_autotuner_leaves_what_the_pass_does_not_read(gpu, tmp_path, grating, det):
+    """Without a FEF file the batch reads the grids of the paraboloid, the
+    reflection and, with a grating, the detector; the rest is the host lists'."""
+    t, dirs, counts = _batch(tmp_path, 32, grating=grating, det=det)
+    t.set_schedule(source=5, enter=6, reflect=7, grating=9, detect=11, reflect_waves=3)
+    sched, _ = t.autotune_batch(dirs, counts, repeats=2)
+    assert (sched["source"], sched["grating"], sched["reflect_waves"]) == (5, 9, 3)
+    assert {sched["enter"], sched["reflect"]} <= {2, 4, 8, 16}
+    assert sched["detect"] in ((11,) if grating == "NONE" else (2, 4, 8, 16))
+
+
+@pytest.mark.gpu
 def test_graph_is_recaptured_after_the_store_grows(gpu, tmp_path):
     """A captured batch graph holds the addresses of the photon store and of
     the batch's source arrays.  A device trace larger than the store (while
