@@ -36,6 +36,7 @@ int g_num_cus = 0;
 float *d_fa = nullptr;
 double *d_da = nullptr;
 unsigned char *d_images = nullptr;  // the LDS images: the mirror's, then the grating's
+unsigned char *h_images = nullptr;  // ... where the host makes them, in pinned memory
 LdsImage g_mirror_image, g_grating_image;
 size_t d_fa_cap = 0, d_da_cap = 0;
 unsigned int g_cfg_gen = 0;
@@ -133,30 +134,50 @@ size_t align256 (size_t n) { return (n + 255) & ~(size_t) 255; }
 constexpr size_t kImageBytes = 160 * 1024;
 
 // The LDS images of configuration *cfg into d_images (held since the set-up),
-// on the library's stream.
+// queued on the library's stream, which is idle: h_images is free.  An image
+// follows from its part of the configuration, as the arenas' entries never
+// change once a configuration holds their offsets, and is made when that part
+// is another one.
 int sync_images (const mxg_config *cfg, const float *fa, const double *da)
 {
-   static unsigned char host[2][kImageBytes];
+   static bool have_mirror, have_grating;
+   static mxg_hrma_cfg mirror;
+   static mxg_grating_cfg grating;
    const bool letg = cfg->grating.type == MARX_GRATING_LETG;
-   const bool grating = letg || (cfg->grating.type == MARX_GRATING_HETG);
-   const HrmaLds lay = hrma_lds_layout (cfg->hrma, da);
-   const GratingLds glay = grating ? grating_lds_layout (cfg->grating, letg) : GratingLds {};
-   const size_t m = hrma_image_bytes (lay);
-   const size_t g = grating ? grating_image_bytes (glay) : 0;
-   HIPCHECK (hipStreamSynchronize (g_stream));
-   if (m <= kImageBytes)
+   const bool with_grating = letg || (cfg->grating.type == MARX_GRATING_HETG);
+   if (!have_mirror || memcmp (&mirror, &cfg->hrma, sizeof (mirror)))
      {
-        hrma_image (cfg->hrma, fa, da, lay, host[0]);
-        HIPCHECK (hipMemcpyAsync (d_images, host[0], m, hipMemcpyHostToDevice, g_stream));
+        have_mirror = false;
+        const HrmaLds lay = hrma_lds_layout (cfg->hrma, da);
+        const size_t m = hrma_image_bytes (lay);
+        if (m <= kImageBytes)
+          {
+             hrma_image (cfg->hrma, fa, da, lay, h_images);
+             HIPCHECK (hipMemcpyAsync (d_images, h_images, m, hipMemcpyHostToDevice, g_stream));
+          }
+        g_mirror_image = LdsImage {(const uint4 *) d_images, (uint32_t) (m / 16)};
+        memcpy (&mirror, &cfg->hrma, sizeof (mirror));
+        have_mirror = true;
      }
-   if (grating && (g <= kImageBytes))
+   if (!with_grating)
      {
-        grating_image (cfg->grating, fa, da, glay, letg, host[1]);
-        HIPCHECK (hipMemcpyAsync (d_images + kImageBytes, host[1], g, hipMemcpyHostToDevice, g_stream));
+        g_grating_image = LdsImage {(const uint4 *) (d_images + kImageBytes), 0};
+        have_grating = false;
      }
-   HIPCHECK (hipStreamSynchronize (g_stream));
-   g_mirror_image = LdsImage {(const uint4 *) d_images, (uint32_t) (m / 16)};
-   g_grating_image = LdsImage {(const uint4 *) (d_images + kImageBytes), (uint32_t) (g / 16)};
+   else if (!have_grating || memcmp (&grating, &cfg->grating, sizeof (grating)))
+     {
+        have_grating = false;
+        const GratingLds lay = grating_lds_layout (cfg->grating, letg);
+        const size_t g = grating_image_bytes (lay);
+        if (g <= kImageBytes)
+          {
+             grating_image (cfg->grating, fa, da, lay, letg, h_images + kImageBytes);
+             HIPCHECK (hipMemcpyAsync (d_images + kImageBytes, h_images + kImageBytes, g, hipMemcpyHostToDevice, g_stream));
+          }
+        g_grating_image = LdsImage {(const uint4 *) (d_images + kImageBytes), (uint32_t) (g / 16)};
+        memcpy (&grating, &cfg->grating, sizeof (grating));
+        have_grating = true;
+     }
    return 0;
 }
 
@@ -617,6 +638,7 @@ int mxgd_init (void)
       TraceReport zero;
       memset (&zero, 0, sizeof (zero));
       HIPCHECK (hipMalloc (&d_images, 2 * kImageBytes));
+      HIPCHECK (hipHostMalloc ((void **) &h_images, 2 * kImageBytes, hipHostMallocDefault));
       HIPCHECK (hipMalloc (&d_trace_n, sizeof (uint32_t)));
       HIPCHECK (hipMalloc (&d_trace_counts, 4 * kMaxSegments * sizeof (uint32_t)));
       HIPCHECK (hipMalloc (&d_trace, sizeof (TraceReport)));
