@@ -101,7 +101,7 @@ int mxgd_run_batch_passes (unsigned int n, double exposure, double start_time, u
  * arrivals): source, mirror, grating and detector of n > 0 photons, then a
  * wait.  counts and ms (8 each) by timing slot as mxgd_read_timings gives
  * them.  mxgd_passes_fit: whether the device's configuration can take it
- * (no FEF step, tables that fit LDS). */
+ * (no FEF step). */
 int mxgd_passes_fit (void);
 int mxgd_run_passes (unsigned int n, unsigned int tag_start, double start_time, double exposure_time,
                      unsigned long long seed, float *ms, unsigned int *counts);

@@ -296,10 +296,6 @@ static __device__ __noinline__ bool apply_fef (const mxg_detector_cfg &d, const 
    return true;
 }
 
-// FEF: compiled with the ACIS FEF step (launched only when a FEF file was
-// read, so that the common case keeps the registers of the kernel without
-// it); W: waves per SIMD to leave room for (0 unbounded: ACIS and HRC both
-// measured slower bounded)
 // ACIS contamination: the transmission exp(-sum_i mu_i(E) (tau0_i + tau1_i
 // f(x, y))) at the chip pixel (cx, cy) (aciscontam.c:93-136), f the chip's
 // table or one of the two analytic models (aciscontam.c:141-185).  Out of

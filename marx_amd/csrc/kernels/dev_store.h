@@ -69,11 +69,13 @@ struct ListIO
 constexpr int kBlock = 256;
 constexpr uint32_t kMaxSegments = 8192;
 
-// A stage's survivors handed densely to the next stage: the columns the
+// A kernel's survivors handed densely to the next one: the columns the
 // grating and the detector read of a photon (x, p, energy, tag, flags,
-// shell), written by the producing kernel (the reflection, the grating) at
-// the survivor's segment slot (its position in seg), and pos, written by
-// k_compact: the slot of each entry of the compacted list.  After the
+// shell), written by the producing kernel at the survivor's segment slot (its
+// position in seg), and pos, written by k_compact: the slot of each entry of
+// the compacted list.  k_mirror hands the photons with an order to k_diffract
+// this way, and in traces and batches with a FEF file the reflection its
+// survivors to an LETG and either grating its own to the detector.  After the
 // mirror about one photon id in three is alive, after the grating one in
 // sixteen, so reading the double columns at the ids costs a cache line per
 // column for a few photons; the relay's rows are contiguous.
@@ -93,9 +95,12 @@ struct PhotonOut
    int shell;
 };
 
-// Entry i of a column.  Columns are below 2^32 bytes (a launch takes at most
-// 2^28 photons), so the byte offset is formed in 32 bits and added to the
-// column's address, a scalar, by the memory instruction itself.
+// Entry i of a column.  Columns are at most 2^32 bytes, so the byte offset is
+// formed in 32 bits and added to the column's address, a scalar, by the memory
+// instruction itself.  (Created chunks and batches hold at most 2^28 photons; a
+// host list as many as the store takes, whose capacity is a power of two and
+// at 292 bytes a photon, with its lists and relays, ends at 2^29 on a card of
+// 288 GB.)
 template <class T>
 __device__ __forceinline__ T &at (T *col, uint32_t i)
 {
@@ -262,25 +267,21 @@ hipError_t launch_pack_columns (const Soa &s, const uint32_t *idx, const uint32_
 
 // Minimum waves per SIMD of the mirror's reflection kernel unless the
 // launch schedule says otherwise (256 lanes per block = one wave per SIMD
-// per block).  Unbounded, the compiler gives it ~200 VGPRs, i.e. two waves
-// per SIMD, too few to hide its LDS and table-load latency; four waves
-// (128 VGPRs, a few spills) measured fastest on the HETG workload.
+// per block).  At 109 to 113 VGPRs, without spills, it holds four waves
+// whichever instance is launched; the instances differ in scheduling only.
 #define MXG_REFLECT_WAVES_DEFAULT 4
 // waves per SIMD that the compiler must leave room for (0: unbounded).
-// k_source needs fewer VGPRs than 4 waves allow (56 for a point source),
-// k_batch_source at 4 (from 175) measured 29 percent faster, the LETG
-// grating pass at 4 (from 218) 25 percent, the HETG grating pass at 3 (from
-// 208) 8 percent; the ACIS detector kernel needs 112 VGPRs (4 waves)
-// unbounded
+// The source kernels (50 to 70 VGPRs), the grating passes (68 to 91) and the
+// ACIS detector (91 to 94) need fewer than the 128 of four waves without
+// being told.
 #ifndef MXG_SOURCE_WAVES
 #define MXG_SOURCE_WAVES 4
 #endif
 #ifndef MXG_BATCH_SOURCE_WAVES
 #define MXG_BATCH_SOURCE_WAVES 4
 #endif
-// waves of the reflection kernel of the schedule's largest setting (4; 5
-// measured 21 percent slower), and of the aperture kernel (unbounded, 95
-// VGPRs; 6 and 8 measured slower)
+// waves of the reflection kernel of the schedule's largest setting, and of
+// the aperture kernel (unbounded, 52 VGPRs)
 #ifndef MXG_REFLECT_WAVES_TOP
 #define MXG_REFLECT_WAVES_TOP 4
 #endif
@@ -317,9 +318,9 @@ struct HrmaScratch
 // cfg: device copy; hcfg: host copy of the same configuration (launch
 // geometry and LDS layout are computed from it).  ev, when non-null, holds
 // four events recorded around k_hrma_enter (0, 1) and k_hrma_reflect (2, 3).
-// relay_out, when non-null: the mirror's survivors go to it for the grating
-// or the detector, which store their x, p and flags (the reflection kernel
-// stores those of the photons it drops only)
+// relay_out, when non-null: the mirror's survivors go to it for the grating,
+// which stores their x, p and flags (the reflection kernel stores those of
+// the photons it drops only)
 // fresh: the input photons come straight from launch_source with
 // entry_follows (unread flags, all zero; the entry writes every photon's
 // position, shell and flags)
@@ -339,12 +340,13 @@ hipError_t launch_hrma_reflect (const mxg_config *cfg, const mxg_config *hcfg, c
 // the runtime cannot say.  A grid of whole rounds of them measured fastest
 // (HETG + ACIS-S: 3 blocks per CU 0.36 ms, 4 0.47 ms, 8 0.40 ms).
 uint32_t grating_blocks_per_cu (const mxg_config *hcfg);
-// hcfg: the host copy of cfg; image: the tables the kernel stages in LDS; letg: the instance compiled for the LETG pass; relay_in,
-// when non-null:
-// the input list is the mirror's with this relay, whose rows the kernel
-// reads instead of the store's; relay_out, when non-null: the survivors go
-// to it for launch_detect, which stores their x, p and flags (the kernel
-// stores those of the photons it drops only)
+// hcfg: the host copy of cfg; image: the tables the kernel stages in LDS;
+// letg: the instance compiled for the LETG pass; relay_in, when non-null (with
+// letg and relay_out only): the input list is the mirror's with this relay,
+// whose rows the kernel reads instead of the store's; relay_out, when
+// non-null (without letg or with relay_in): the survivors go to it for
+// launch_detect, which stores their x, p and flags (the kernel stores those
+// of the photons it drops only)
 hipError_t launch_grating (const mxg_config *cfg, const mxg_config *hcfg, const float *fa, const double *da, Soa s,
                            ListIO io, LdsImage image, uint32_t n_upper, unsigned long long seed,
                            uint32_t source_id, bool letg, const Relay *relay_in, const Relay *relay_out,
@@ -357,8 +359,9 @@ inline int detector_kind (const mxg_config &c)
    return (c.det.type == MARX_DETECTOR_HRC_S) ? MXG_DET_HRC_S
      : (c.det.type == MARX_DETECTOR_HRC_I) ? MXG_DET_HRC_I : MXG_DET_ACIS;
 }
-// relay, when non-null: the input list is the one the previous stage left
-// with this relay, whose rows the kernel reads instead of the store's
+// relay, when non-null (ACIS with the FEF step only): the input list is the
+// one the grating left with this relay, whose rows the kernel reads instead
+// of the store's
 hipError_t launch_detect (const mxg_config *cfg, const float *fa, const double *da, Soa s,
                           ListIO io, uint32_t n_upper, double tstart,
                           unsigned long long seed, uint32_t source_id, bool fef, int kind,

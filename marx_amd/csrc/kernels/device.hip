@@ -1089,8 +1089,16 @@ void read_trace (unsigned int n, bool scanned, float *ms, unsigned int *counts)
 
 int mxgd_passes_fit (void)
 {
-   return (d_cfg != nullptr) && !g_hcfg.det.fef_on && (g_mirror_image.n16 <= 64 * 1024 / 16)
-     && (g_grating_image.n16 <= 64 * 1024 / 16);
+   return (d_cfg != nullptr) && !g_hcfg.det.fef_on;
+}
+
+// whether the tables that the chunk kernels stage fit their LDS
+static int images_fit (void)
+{
+   constexpr uint32_t limit = 64 * 1024 / 16;
+   if (g_mirror_image.n16 > limit) return fail ("the mirror's tables take %u bytes of LDS, of 64 KB", g_mirror_image.n16 * 16);
+   if (g_grating_image.n16 > limit) return fail ("the grating's tables take %u bytes of LDS, of 64 KB", g_grating_image.n16 * 16);
+   return 0;
 }
 
 int mxgd_run_passes (unsigned int n, unsigned int tag_start, double start_time, double exposure_time,
@@ -1100,7 +1108,7 @@ int mxgd_run_passes (unsigned int n, unsigned int tag_start, double start_time, 
    if (!d_cfg) return fail ("configuration not on the device");
    if (n == 0) return fail ("no photons to trace");
    if (n > (1u << 26)) return fail ("chunk of %u photons exceeds the 2^26 limit of one launch", n);
-   if (ensure_capacity (n)) return -1;
+   if (images_fit () || ensure_capacity (n)) return -1;
    TraceArgs a = trace_args (n, exposure_time, start_time, seed);
    a.tag_start = tag_start;
    const bool scanned = (g_hcfg.src.time_mode == MXG_TIME_POISSON);
@@ -1138,7 +1146,7 @@ namespace {
 constexpr int kDiffWin = 64 * 64;       // floats of one block's image window
 constexpr int kDiffGrad = MXG_NUM_SHELLS * MXG_DIFF_NPAR;
 
-int diff_buffers (size_t n, uint32_t grid)
+int diff_buffers (size_t n)
 {
    if ((n > g_diff_cap) || (d_diff_win == nullptr))
      {
@@ -1175,7 +1183,6 @@ int diff_buffers (size_t n, uint32_t grid)
         HIPCHECK (hipMalloc (&d_diff_u32, 4 * sizeof (uint32_t)));
         for (int k = 0; k < 6; k++) HIPCHECK (hipEventCreate (&g_diff_ev[k]));
      }
-   (void) grid;
    return 0;
 }
 
@@ -1189,7 +1196,7 @@ int mxgd_diff_forward (const mxg_diff_cfg *d, unsigned int n, unsigned int tag_s
    if (n > (1u << 28)) return fail ("%u photons exceed 2^28", n);
    if (spec->npix > 16384) return fail ("image of %u pixels a side exceeds 16384", spec->npix);
    uint32_t grid = stage_grid (n, MXGD_K_REFLECT);
-   if (diff_buffers (n ? n : 1, grid)) return -1;
+   if (diff_buffers (n ? n : 1)) return -1;
    g_diff_grid = 0;
    HIPCHECK (hipMemcpyAsync (d_diff_cfg, d, sizeof (mxg_diff_cfg), hipMemcpyHostToDevice, g_stream));
    // tangents by the tilts only for a source at infinity (the translations
@@ -1391,6 +1398,7 @@ int mxgd_run_batch_passes (unsigned int n, double exposure, double start_time, u
    g_relay_have = -1;
    if (!d_cfg) return fail ("configuration not on the device");
    if ((n == 0) || (n > g_capacity) || (g_batch_nsrc == 0)) return fail ("batch not prepared");
+   if (images_fit ()) return -1;
    TraceArgs a = trace_args (n, exposure, start_time, seed);
    a.off = d_batch_off;
    a.nsrc = g_batch_nsrc;

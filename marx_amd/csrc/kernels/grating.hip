@@ -46,27 +46,6 @@ void k_grating (const mxg_config *__restrict__ cfg, const float *__restrict__ fa
    survivors.finish (io);
 }
 
-template <bool LETG, int W>
-static void launch_io (dim3 g, size_t lds_bytes, hipStream_t st, const mxg_config *cfg, const float *fa,
-                       const double *da, Soa s, ListIO io, unsigned long long seed, uint32_t source_id,
-                       const LdsImage &image, const Relay *rin, const Relay *rout)
-{
-   const Relay a = rin ? *rin : Relay {}, b = rout ? *rout : Relay {};
-   const dim3 blk (kBlock);
-   if (rin && rout)
-     hipLaunchKernelGGL ((k_grating<LETG, W, true, true>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, image, a, b);
-   else if (rin)
-     hipLaunchKernelGGL ((k_grating<LETG, W, true, false>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, image, a, b);
-   else if (rout)
-     hipLaunchKernelGGL ((k_grating<LETG, W, false, true>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, image, a, b);
-   else
-     hipLaunchKernelGGL ((k_grating<LETG, W, false, false>), g, blk, lds_bytes, st, cfg, fa, da, s, io, seed,
-                         source_id, image, a, b);
-}
-
 uint32_t grating_blocks_per_cu (const mxg_config *hcfg)
 {
    const bool letg = hcfg->grating.type == MARX_GRATING_LETG;
@@ -91,12 +70,21 @@ hipError_t launch_grating (const mxg_config *cfg, const mxg_config *hcfg, const 
    const size_t lds_bytes = (size_t) image.n16 * 16;
    if (lds_bytes > 64 * 1024)
      return hipErrorInvalidConfiguration;
-   if (letg)
-     launch_io<true, MXG_LETG_GRATING_WAVES> (g, lds_bytes, st, cfg, fa, da, s, io, seed, source_id, image,
-                                             relay_in, relay_out);
+   const Relay none = {};
+   if (!relay_in && !relay_out)
+     hipLaunchKernelGGL ((letg ? k_grating<true, MXG_LETG_GRATING_WAVES, false, false>
+                               : k_grating<false, MXG_GRATING_WAVES, false, false>),
+                         g, dim3 (kBlock), lds_bytes, st, cfg, fa, da, s, io, seed, source_id, image, none, none);
+   // traces and batches with a FEF file: the mirror hands its survivors on to
+   // an LETG, and both gratings theirs to the detector
+   else if (letg && relay_in && relay_out)
+     hipLaunchKernelGGL ((k_grating<true, MXG_LETG_GRATING_WAVES, true, true>), g, dim3 (kBlock), lds_bytes, st, cfg, fa,
+                         da, s, io, seed, source_id, image, *relay_in, *relay_out);
+   else if (!letg && !relay_in)
+     hipLaunchKernelGGL ((k_grating<false, MXG_GRATING_WAVES, false, true>), g, dim3 (kBlock), lds_bytes, st, cfg, fa, da,
+                         s, io, seed, source_id, image, none, *relay_out);
    else
-     launch_io<false, MXG_GRATING_WAVES> (g, lds_bytes, st, cfg, fa, da, s, io, seed, source_id, image, relay_in,
-                                         relay_out);
+     return hipErrorInvalidValue;
    hipError_t e = hipGetLastError ();
    if (e == hipSuccess) e = launch_compact (io, st, relay_out ? relay_out->pos : nullptr);
    return e;

@@ -175,8 +175,8 @@ __device__ __forceinline__ void block_counts (uint32_t c0, uint32_t c1, uint32_t
      }
 }
 
-// G: 0 no grating, else HETG or LETG (the same code: the support gratings
-// come later); KIND: without a grating the detector family, -1 none.
+// G: with a grating, HETG or LETG (the same code: the support gratings come
+// later); KIND: without one the detector family, -1 none.
 // counts[2 b], [2 b + 1]: photons of block b out of the mirror, and detected.
 template <bool G, int KIND>
 __global__ __launch_bounds__ (kBlock, 4)

@@ -7,14 +7,13 @@
 
 namespace mxg {
 
-// A store to a column that no later stage reads, or few photons of it:
-// it is left out of the cache, which then holds the columns that the next
-// stages read and write again.
 // every column of photon i set as a fresh photon of the given energy,
 // direction, time and tag, with no dither offsets; a column that a later
 // step writes is left out (with_t, with_p, with_dith false; with_entry
 // false: the position, shell and flags, which the mirror's entry writes
-// for every photon it is given as fresh)
+// for every photon it is given as fresh).  The columns that no later stage
+// reads, or few photons of, are left out of the cache, which then holds those
+// that the next stages read and write again.
 __device__ __forceinline__ void init_photon (Soa s, uint32_t i, double energy, vec3 p, double t,
                                              uint32_t tag, bool with_t = true, bool with_p = true,
                                              bool with_dith = true, bool with_entry = true)
