@@ -31,8 +31,10 @@ if ROOT not in sys.path:
 # divs and sqrts of the restated reference algorithm, counted by the
 # op-counting oracle build on each workload:
 # `python -m oracle.opcount.opcount --photons 100000 --workload <name>`).
-# "grating" and "detector" are k_grating and k_detect.  Transcendental calls
-# per photon are listed beside.
+# The stages "source", "k_hrma_enter" (up to the paraboloid), "k_hrma_reflect"
+# (from there on), "grating" and "detector" are the reference's; the kernels do
+# several of them each (chunk_kernels).  Transcendental calls per photon are
+# listed beside.
 FLOPS_PER_PHOTON = {
     "hetg-acis-s": {"source": 146.0, "k_hrma_enter": 130.3, "k_hrma_reflect": 598.6,
                     "grating": 249.3, "detector": 200.1},
@@ -56,46 +58,42 @@ TRANSCENDENTALS_PER_PHOTON = {
                        "grating": 0.0, "detector": 0.17},
     "diff": {"k_diff_enter": 4.00, "k_diff_forward": 11.91 - 4.00, "k_diff_adjoint": 0.0},
 }
-# Algorithmic HBM bytes per photon entering each kernel: the structure-of-
-# arrays columns it must read and write, plus the active-list index in and
-# the survivor index out.
+# A created photon's record: every column once.
+RECORD_BYTES = 126
+# Algorithmic HBM bytes per photon entering each kernel of the differentiable
+# pass.
 BYTES_PER_PHOTON = {
-    # energy, p, t, tag, dither, scan word (the position, shell and flags
-    # are the mirror entry's to write)
-    "source": 8 + 24 + 8 + 4 + 24 + 8,
-    # in: index, tag, p (fresh photons: no flags read); out: x, p, shell,
-    # flags, stream position, index
-    "k_hrma_enter": (4 + 4 + 24) + (24 + 24 + 1 + 4 + 4 + 4),
-    # in: index, flags, shell, tag, stream position, x, p, energy; out: x, p, flags, index
-    "k_hrma_reflect": (4 + 4 + 1 + 4 + 4 + 24 + 24 + 8) + (24 + 24 + 4 + 4),
-    "grating": (4 + 4 + 4 + 1 + 8 + 24 + 24 + 1) + (24 + 24 + 4 + 1 + 4),
-    "detector": (4 + 4 + 4 + 8 + 8 + 24 + 24) + (24 + 24 + 4 + 1 + 4 + 4 + 4),
     # per listed photon: in: list index; out: w, y, z, the 8 derivatives that
     # are not constants, shell (the image stays in L2 / LDS)
     "k_diff_forward": 4 + 8 * (3 + 8) + 1,
     # per listed photon, in: w, y, z, the 8 derivatives, shell
     "k_diff_adjoint": 8 * (3 + 8) + 1,
 }
-# HBM bytes per photon entering a kernel, measured with rocprofv3 counters
-# (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 per dispatch, the factors that make a
-# 1 GiB device copy read back 1 GiB each way); commands and figures in
-# profiles/pmc_hetg_acis_s_1e7.md.  Absent
-# when not measured for the current kernels.
-# The figure is not measured inside this run (counters need their own
-# profiler runs): each entry names the profile it comes from, and the bench
-# line carries that name beside `traffic`.
+# HBM bytes per launch of a kernel and photon created, measured with rocprofv3
+# counters (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 per dispatch, the factors that
+# make a 1 GiB device copy read back 1 GiB each way); commands and figures in
+# the profile that an entry names.  Not measured inside this run (counters need
+# their own profiler runs): the bench line carries the profile's name beside
+# `traffic`.  Absent when not measured for the current kernels.
 TRAFFIC_BYTES_PER_PHOTON = {
-    # k_mirror's, per photon that hit a paraboloid
-    ("hetg-acis-s", "k_hrma_reflect"): (232.1, "profiles/pmc_hetg_acis_s_1e7.md"),
+    ("hetg-acis-s", "k_create"): (138.5, "profiles/pmc_hetg_acis_s_1e7.md"),
+    ("hetg-acis-s", "k_mirror + k_diffract"): (142.6, "profiles/pmc_hetg_acis_s_1e7.md"),
+    ("letg-hrc-s", "k_create"): (138.3, "profiles/pmc_letg_diff.md"),
+    ("letg-hrc-s", "k_mirror + k_diffract"): (153.6, "profiles/pmc_letg_diff.md"),
+    # per photon that reached a paraboloid
+    ("diff", "k_diff_forward"): (105.6, "profiles/pmc_letg_diff.md"),
 }
 
 
 def traffic_of(cfg, kernel, units):
-    """(HBM bytes per launch, source profile) of a kernel, or (None, None)."""
+    """(HBM bytes per launch of `units` created photons, source profile) of a
+    kernel, or (None, None)."""
     tb = TRAFFIC_BYTES_PER_PHOTON.get((cfg, kernel))
     if tb is None:
         return None, None
     return tb[0] * units, tb[1]
+
+
 DESCRIPTION = {
     "hetg-acis-s": "HETG + ACIS-S: on-axis point source, power law index 2 over 0.4-8 keV (FILE table), "
                    "HEG/MEG orders from the CALDB efficiency tables, INTERNAL dither 16 arcsec "
@@ -177,26 +175,55 @@ def cpu_baseline(tracer, target_seconds=20.0):
                       f"{threads} OpenMP threads), {dt:.1f} s"}
 
 
-def kernel_roofline(cfg, kernels):
-    """The roofline object for the slowest of the timed kernels."""
+def chunk_kernels(cfg, ms, created, hits, mirrored, detecting):
+    """Figures of the chunk kernels from their device times ms (k_create,
+    k_mirror, k_diffract, each with the list compaction after it) and the
+    photons created, on the paraboloid, out of the mirror and into the
+    detector.  k_mirror ends within the grating stage (at the order draw), so
+    with a grating it and k_diffract share one entry; without one k_mirror
+    does the detector too.
+
+    flops: the stages' algorithmic work.  bytes: what the kernels cannot do
+    without: k_create writes every photon's record and each hit's list entry;
+    of a hit, k_mirror reads entry, path and energy (60 bytes) and its path is
+    written once more (52); a photon with an order goes to k_diffract as a row
+    (77 bytes with its list entry, there and back; the photons into the
+    detector stand for them), and the detector's columns are 9 bytes."""
+    f, tr = FLOPS_PER_PHOTON[cfg], TRANSCENDENTALS_PER_PHOTON[cfg]
+    with_grating = f["grating"] > 0.0
+    work = {"k_create": (ms[0], created, {"source": created, "k_hrma_enter": created},
+                         created * RECORD_BYTES + 4.0 * hits)}
+    if with_grating:
+        work["k_mirror + k_diffract"] = (
+            ms[1] + ms[2], hits, {"k_hrma_reflect": hits, "grating": mirrored, "detector": detecting},
+            hits * 112.0 + detecting * (2 * 77.0 + 9.0))
+    else:
+        work["k_mirror"] = (ms[1], hits, {"k_hrma_reflect": hits, "detector": mirrored}, hits * 112.0 + mirrored * 9.0)
+    kernels = {}
+    for name, (t_ms, n_in, stages, byt) in work.items():
+        flops = sum(f[k] * n for k, n in stages.items())
+        traffic, traffic_src = traffic_of(cfg, name, created)
+        t = t_ms * 1e-3
+        kernels[name] = {"ms": t_ms, "photons_in": n_in, "flops": flops,
+                         "transcendentals": sum(tr[k] * n for k, n in stages.items()), "bytes": byt,
+                         "tflops": flops / t / 1e12 if t > 0 else None, "gbs": byt / t / 1e9 if t > 0 else None,
+                         "traffic": traffic, "traffic_source": traffic_src}
+    if with_grating:
+        kernels["k_mirror + k_diffract"].update(k_mirror_ms=ms[1], k_diffract_ms=ms[2])
+    return kernels
+
+
+def kernel_roofline(kernels):
+    """The roofline object for the slowest of chunk_kernels' entries."""
     dom = max(kernels, key=lambda k: kernels[k]["ms"])
-    units = kernels[dom]["photons_in"]
-    traffic, traffic_src = traffic_of(cfg, dom, units)
-    return {"bound": "valu", "pipe": VALU_PIPE,
-            # the chunk kernels do two stages each; their time is shared
-            # between those by the cycles that sampled blocks spend in each
-            "kernel": {"grating": "k_mirror and k_diffract (grating part)", "detector": "detector part",
-                       "k_hrma_enter": "k_create (entry part)",
-                       "k_hrma_reflect": "k_mirror (reflection part)"}.get(dom, dom),
-            "achieved": kernels[dom]["tflops"], "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-            "frac": kernels[dom]["tflops"] / PEAK_FP64_TFLOPS,
-            "traffic": traffic, "traffic_source": traffic_src,
-            "flops_per_photon": FLOPS_PER_PHOTON[cfg][dom],
-            "transcendentals_per_photon": TRANSCENDENTALS_PER_PHOTON[cfg][dom],
-            "photons_per_launch": units, "launch_ms": kernels[dom]["ms"],
-            "hbm": {"achieved": kernels[dom]["gbs"], "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                    "frac": kernels[dom]["gbs"] / PEAK_HBM_GBS,
-                    "bytes_per_photon": BYTES_PER_PHOTON[dom]}}
+    k = kernels[dom]
+    return {"bound": "valu", "pipe": VALU_PIPE, "kernel": dom,
+            "achieved": k["tflops"], "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
+            "frac": k["tflops"] / PEAK_FP64_TFLOPS, "traffic": k["traffic"], "traffic_source": k["traffic_source"],
+            "flops_per_launch": k["flops"], "transcendentals_per_launch": k["transcendentals"],
+            "photons_per_launch": k["photons_in"], "launch_ms": k["ms"],
+            "hbm": {"achieved": k["gbs"], "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": k["gbs"] / PEAK_HBM_GBS,
+                    "bytes_per_launch": k["bytes"]}}
 
 
 def measure_batched(args, tmp, torch):
@@ -231,15 +258,8 @@ def measure_batched(args, tmp, torch):
     # per-kernel device times from one uncaptured pass of the same batch
     tracer.trace_batch(dirs, counts, exposure=T, use_graph=False)
     sms = tracer.stage_ms()
-    kms, kin = tracer.kernel_stats()
-    c = tracer.stage_counts()
-    kernels = {}
-    for name, ms_k, n_k in (("k_hrma_enter", kms[0], kin[0]), ("k_hrma_reflect", kms[1], kin[1]),
-                            ("detector", sms[3], c[1])):
-        t = ms_k * 1e-3
-        kernels[name] = {"ms": ms_k, "photons_in": n_k,
-                         "tflops": FLOPS_PER_PHOTON[cfg][name] * n_k / t / 1e12 if t > 0 else None,
-                         "gbs": BYTES_PER_PHOTON[name] * n_k / t / 1e9 if t > 0 else None}
+    _, kin = tracer.kernel_stats()
+    kernels = chunk_kernels(cfg, tracer.pass_ms(), N, kin[1], tracer.stage_counts()[1], tracer.stage_counts()[2])
 
     # the plain per-source GPU loop over the same photons
     offs = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
@@ -263,7 +283,7 @@ def measure_batched(args, tmp, torch):
         "per_source_loop": {"value": N / loop_s, "unit": "photons/s", "seconds": loop_s,
                             "sources": len(counts)},
         "batched_over_loop": value / (N / loop_s),
-        "roofline": kernel_roofline(cfg, kernels),
+        "roofline": kernel_roofline(kernels),
         "stages_ms": {"source": sms[0], "mirror": sms[1], "detector": sms[3]},
         "kernels": kernels,
     }
@@ -693,15 +713,15 @@ def cpu_baseline_batch(tracer, dirs, counts, exposure, target_seconds=20.0):
                       f"task per source, {threads} threads), {dt:.1f} s"}
 
 
-GRID_CANDIDATES = {"enter": (4, 5, 8, 10, 15, 20), "reflect": (4, 8, 12, 16),
-                   "grating": (0, 2, 3, 4, 6, 8, 12), "detect": (1, 2, 4, 8)}
+GRID_CANDIDATES = {"enter": (2, 4, 5, 6, 8, 10, 12, 15, 20), "reflect": (2, 4, 8, 12, 16, 20),
+                   "detect": (1, 2, 3, 4, 5, 8, 10, 16)}
+GRID_KERNELS = {"enter": "k_create", "reflect": "k_mirror", "detect": "k_diffract"}
 
 
 def sweep_grids(args, tracer, step):
-    """Each stage kernel's time over candidate blocks per CU, one kernel at a
-    time with the others at the library's defaults (grating 0: one round of
-    the blocks a CU holds at once).  The mirror's kernels are timed alone
-    with HIP events, the grating and detector as their stages."""
+    """Each chunk kernel's device time (with the list compaction after it) over
+    candidate blocks per CU of the schedule's grid that it takes, one at a time
+    with the others at the library's defaults."""
     default = tracer.get_schedule()
     k = 0
     rows = []
@@ -714,16 +734,15 @@ def sweep_grids(args, tracer, step):
                     k += 1
                 ms = 0.0
                 for _ in range(args.steps):
-                    _, _, stage = step(k, timing=True)
+                    step(k)
                     k += 1
-                    kms, _ = tracer.kernel_stats()
-                    ms += {"enter": kms[0], "reflect": kms[1], "grating": stage[3], "detect": stage[4]}[kern]
-                rows.append({"kernel": kern, "blocks_per_cu": v, "ms": round(ms / args.steps, 4)})
+                    ms += tracer.pass_ms()[("enter", "reflect", "detect").index(kern)]
+                rows.append({"kernel": GRID_KERNELS[kern], "grid": kern, "blocks_per_cu": v, "ms": round(ms / args.steps, 4)})
                 print(json.dumps(rows[-1]), file=sys.stderr, flush=True)
                 tracer.set_schedule(**{kern: default[kern]})
     finally:
-        tracer.set_schedule(**{kk: default[kk] for kk in ("source", "enter", "reflect", "grating", "detect")})
-    return {"sweep": "blocks per CU of each stage kernel", "config": args.config, "steps": args.steps,
+        tracer.set_schedule(**{kk: default[kk] for kk in GRID_CANDIDATES})
+    return {"sweep": "blocks per CU of each chunk kernel", "config": args.config, "steps": args.steps,
             "warmup": args.warmup, "default": default, "rows": rows}
 
 
@@ -755,7 +774,7 @@ def measure():
     ap.add_argument("--exposure", type=float, default=50_000.0)
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU-baseline leg")
     ap.add_argument("--sweep-grids", action="store_true",
-                    help="instead of the bench line: each stage kernel's HIP-event time over candidate "
+                    help="instead of the bench line: each chunk kernel's device time over candidate "
                          "blocks per CU (the others at their defaults), one JSON line per candidate")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
                     help="after the steps, copy a MIB-MiB device buffer three times (the known-size "
@@ -804,17 +823,15 @@ def measure():
     torch.cuda.synchronize()
     stage_ms = {s: 0.0 for s in STAGES}
     stage_in = {s: 0 for s in STAGES}
-    kern_ms = {"k_hrma_enter": 0.0, "k_hrma_reflect": 0.0}
-    kern_in = {"k_hrma_enter": 0, "k_hrma_reflect": 0}
+    kern_ms = [0.0, 0.0, 0.0]
+    hits = 0
     detected = 0
     t0 = time.perf_counter()
     for k in range(args.steps):
         ncol, ndet, ms = step(args.warmup + k, timing=True)
         c = tracer.stage_counts()
-        kms, kin = tracer.kernel_stats()
-        for j, name in enumerate(("k_hrma_enter", "k_hrma_reflect")):
-            kern_ms[name] += kms[j]
-            kern_in[name] += kin[j]
+        kern_ms = [a + b for a, b in zip(kern_ms, tracer.pass_ms())]
+        hits += tracer.kernel_stats()[1][1]
         stage_ms["source"] += ms[0]
         stage_ms["mirror"] += ms[2]
         stage_ms["grating"] += ms[3]
@@ -829,25 +846,10 @@ def measure():
     K = args.steps
     value = K * N / elapsed
 
-    # per-kernel figures; the mirror's kernels are timed alone with HIP events
-    # on the library's stream, grating and detector are their stage (one
-    # kernel plus the list compaction)
-    kernels = {}
-    for name, ms_k, n_k in (("k_hrma_enter", kern_ms["k_hrma_enter"], kern_in["k_hrma_enter"]),
-                            ("k_hrma_reflect", kern_ms["k_hrma_reflect"], kern_in["k_hrma_reflect"]),
-                            ("grating", stage_ms["grating"], stage_in["grating"]),
-                            ("detector", stage_ms["detector"], stage_in["detector"])):
-        t = ms_k / K * 1e-3
-        kernels[name] = {"ms": ms_k / K, "photons_in": n_k / K,
-                         "tflops": FLOPS_PER_PHOTON[cfg][name] * n_k / K / t / 1e12 if t > 0 else None,
-                         "gbs": BYTES_PER_PHOTON[name] * n_k / K / t / 1e9 if t > 0 else None}
-
-    dom = max(kernels, key=lambda k: kernels[k]["ms"])
-    t_launch = kernels[dom]["ms"] * 1e-3
-    units = kernels[dom]["photons_in"]
-    achieved = kernels[dom]["tflops"]
-    achieved_bw = kernels[dom]["gbs"]
-    traffic, traffic_src = traffic_of(cfg, dom, units)
+    # per-kernel figures by the device's clock; the stages share a kernel's time
+    # by the cycles that a sample of its blocks spent in each (stages_ms)
+    kernels = chunk_kernels(cfg, [m / K for m in kern_ms], N, hits / K, stage_in["grating"] / K,
+                            stage_in["detector"] / K)
 
     out = {
         "metric": "photons/s traced (HRMA+grating+detector) 1 GPU vs host CPU; gradient evals/s",
@@ -865,18 +867,7 @@ def measure():
         "config": {"workload": DESCRIPTION[cfg], "name": cfg,
                    "photons_per_step": N, "exposure_s": T,
                    "detected_per_step": detected / K},
-        "roofline": {"bound": "valu", "pipe": VALU_PIPE,
-                     "kernel": "k_grating (stage)" if dom == "grating" else
-                               "k_detect (stage)" if dom == "detector" else dom,
-                     "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP64_TFLOPS, "traffic": traffic,
-                     "traffic_source": traffic_src,
-                     "flops_per_photon": FLOPS_PER_PHOTON[cfg][dom],
-                     "transcendentals_per_photon": TRANSCENDENTALS_PER_PHOTON[cfg][dom],
-                     "photons_per_launch": units, "launch_ms": t_launch * 1e3,
-                     "hbm": {"achieved": achieved_bw, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                             "frac": achieved_bw / PEAK_HBM_GBS,
-                             "bytes_per_photon": BYTES_PER_PHOTON[dom]}},
+        "roofline": kernel_roofline(kernels),
         "stages_ms": {s: stage_ms[s] / K for s in STAGES},
         "stage_photons_in": {s: stage_in[s] / K for s in STAGES},
         "kernels": kernels,

@@ -455,6 +455,13 @@ int mxg_autotune_batch (unsigned int num_sources, const double *dirs, const unsi
  * photons_in the photons each one processed (the photons entering the mirror,
  * and those that hit the paraboloid).  Either pointer may be NULL. */
 int mxg_last_kernel_stats (float ms[2], unsigned int photons_in[2]);
+/* Device times in milliseconds, by the device's clock, of the chunk kernels
+ * of the last mxg_trace_device or mxg_trace_batch call, each with the list
+ * compaction after it: k_create (source and paraboloid), k_mirror
+ * (reflections, then the torus and order draw or, without a grating, the
+ * detector) and k_diffract (diffraction and detector; 0 without a grating).
+ * All 0 when the stages ran as kernels of their own (a FEF file). */
+int mxg_last_pass_ms (float ms[3]);
 
 /* Copies the device-resident photons of the last mxg_trace_device call into
  * pt (AoS), setting n_photons, history and the pruned sorted_index. */

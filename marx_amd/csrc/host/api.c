@@ -617,6 +617,20 @@ static unsigned int Kernel_In[2];
 /* stage times (ms) of the last pass by timing slot; zero for a
  * graph-launched pass */
 static float Last_Slot_Ms[8];
+/* times of the chunk kernels of the last pass (mxg_last_pass_ms) */
+static float Pass_Ms[3];
+
+static void read_pass_ms (unsigned int n)
+{
+   memset (Pass_Ms, 0, sizeof (Pass_Ms));
+   if ((n > 0) && mxgd_passes_fit ()) mxgd_passes_kernel_ms (Pass_Ms);
+}
+
+int mxg_last_pass_ms (float ms[3])
+{
+   memcpy (ms, Pass_Ms, sizeof (Pass_Ms));
+   return 0;
+}
 
 int mxg_trace_device (unsigned int num, unsigned int tag_start, double start_time,
                       double exposure_time, unsigned int *num_collected,
@@ -682,6 +696,7 @@ int mxg_trace_device (unsigned int num, unsigned int tag_start, double start_tim
    Kernel_In[0] = counts[MXGD_SLOT_HRMA_ENTER];
    Kernel_In[1] = counts[MXGD_SLOT_HRMA_REFLECT];
    memcpy (Last_Slot_Ms, ms, sizeof (Last_Slot_Ms));
+   read_pass_ms (num);
    Resident = NULL;
    Last_Collected = n;
    Last_Tag_Start = tag_start;
@@ -800,6 +815,7 @@ static int batch_finish (unsigned int n, unsigned int tag_start, int with_gratin
    Last_History = hist;
    Device_Trace = 1;
    memcpy (Last_Slot_Ms, ms, sizeof (ms));
+   read_pass_ms (n);
    if (num_detected) *num_detected = Stage_Counts[3];
    return 0;
 }
@@ -957,12 +973,10 @@ static int time_kernels (unsigned int num_sources, const double *dirs, const uns
         t[4] = Last_Slot_Ms[3];
         if (mxgd_passes_fit ())
           {
-             float ms[3];
-             mxgd_passes_kernel_ms (ms);
              t[0] = t[3] = 0.0f;
-             t[1] = ms[0];
-             t[2] = ms[1];
-             t[4] = ms[2];
+             t[1] = Pass_Ms[0];
+             t[2] = Pass_Ms[1];
+             t[4] = Pass_Ms[2];
           }
         for (int k = 0; k < 5; k++)
           if (t[k] < best[k]) best[k] = t[k];

@@ -271,8 +271,8 @@ hipError_t launch_pack_columns (const Soa &s, const uint32_t *idx, const uint32_
 // whichever instance is launched; the instances differ in scheduling only.
 #define MXG_REFLECT_WAVES_DEFAULT 4
 // waves per SIMD that the compiler must leave room for (0: unbounded).
-// The source kernels (50 to 70 VGPRs), the grating passes (68 to 91) and the
-// ACIS detector (91 to 94) need fewer than the 128 of four waves without
+// The source kernels (50 to 70 VGPRs), the grating passes (75 to 89) and the
+// ACIS detector (94) need fewer than the 128 of four waves without
 // being told.
 #ifndef MXG_SOURCE_WAVES
 #define MXG_SOURCE_WAVES 4

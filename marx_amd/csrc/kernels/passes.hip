@@ -30,9 +30,10 @@
 // kernel ends.  With plain stores k_create took 0.525 ms; k_diffract's few
 // photons a line are merged in the cache (0.150 ms, 0.168 past it).
 //
-// What bounds them now (MI355X, HETG + ACIS-S, 1e7 photons): k_create 0.37 ms,
-// 1.28 GB written (126 bytes a photon: once each); k_mirror 0.54 ms, 1.35 GB, the ALUs busy 60 percent at
-// four waves a SIMD; k_diffract 0.15 ms.  As kernels a stage: source 0.41,
+// What bounds them now (MI355X, HETG + ACIS-S, 1e7 photons): k_create 0.39 ms,
+// 1.30 GB written (126 bytes a photon: once each), the ALUs busy 73 percent;
+// k_mirror 0.54 ms, 1.16 GB, the ALUs busy 60 percent at four waves a SIMD;
+// k_diffract 0.15 ms, 0.26 GB.  As kernels a stage: source 0.41,
 // entry 0.25, reflection 0.68, grating 0.36, detector 0.17 ms.  One launch of
 // independent waves that queue photons for each stage in LDS measured 1.62 ms
 // in all against 1.37: its three waves a SIMD wait for memory at every stage.

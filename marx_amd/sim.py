@@ -185,9 +185,16 @@ class Tracer:
         self.lib.mxg_last_stage_ms(m)
         return list(m)
 
+    def pass_ms(self):
+        """Device ms of k_create, k_mirror and k_diffract in the last
+        trace_device or trace_batch call (mxg_last_pass_ms)."""
+        m = (ctypes.c_float * 3)()
+        self.lib.mxg_last_pass_ms(m)
+        return list(m)
+
     def kernel_stats(self):
-        """(ms, photons_in) of the mirror's two kernels [aperture + paraboloid,
-        reflections] in the last timed trace_device call."""
+        """(ms, photons_in) of the mirror's two parts [aperture + paraboloid,
+        reflections] in the last trace_device call (mxg_last_kernel_stats)."""
         m = (ctypes.c_float * 2)()
         c = (ctypes.c_uint * 2)()
         self.lib.mxg_last_kernel_stats(m, c)

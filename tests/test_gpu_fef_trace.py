@@ -36,6 +36,7 @@ def _tracer(tmp_path, grating, det, shape, dither):
 def test_trace(gpu, tmp_path, grating, det, shape, dither, n, exposure):
     t = _tracer(tmp_path, grating, det, shape, dither)
     ncol, ndet, rec = _same(t, n, exposure=exposure, tag_start=3)
+    assert t.pass_ms() == [0.0, 0.0, 0.0]          # the stages are kernels of their own
     p = Photons(n)
     p.pt.tag_start, p.pt.start_time = 3, 20.0
     assert t.create_photons(p, n, exposure if exposure > 0.0 else None) == ncol

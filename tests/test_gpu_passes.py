@@ -99,3 +99,16 @@ def test_batches_with_small_and_empty_sources(gpu, counts, graph):
         got = p.active.copy()
         compare(got, _oracle(t, dirs, counts, tag, 7.0, 2.0e4, "NONE"), max_flips=1, label=f"{k} sources, tag {tag}")
         assert ndet == ((got["flags"] & 0xFF) == 0).sum()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grating", ["NONE", "HETG"])
+def test_kernel_times_are_the_stages(gpu, grating):
+    """The stages share the kernels' times; the source's has the scan besides."""
+    t = _tracer(grating, "ACIS-S", n=200_000)
+    _, _, ms = t.trace_device(200_000, timing=True)
+    create, mirror, diffract = t.pass_ms()
+    assert create > 0 and mirror > 0 and (diffract > 0) == (grating != "NONE")
+    enter, reflect = t.kernel_stats()[0]
+    assert mirror + diffract == pytest.approx(reflect + ms[3] + ms[4], rel=1e-5)
+    assert create < ms[0] + enter < create + 1.0
