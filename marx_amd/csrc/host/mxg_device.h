@@ -204,8 +204,8 @@ int mxgd_host_free (void *p);
 /* The store's first n photons in energy order with the index as tie-break:
  * their indices and energies into host arrays.  Synchronises. */
 int mxgd_sort_store_by_energy (unsigned int n, unsigned int *index, double *energies);
-/* mxgd_download_aos and mxgd_sort_store_by_energy, the records copied while
- * the sort runs. */
+/* mxgd_download_aos and mxgd_sort_store_by_energy, the records of a list as
+ * above copied while the sort runs. */
 int mxgd_download_sorted (Marx_Photon_Attr_Type *at, unsigned int n, unsigned int *index, double *energies);
 /* Stage `stage` (arg: the mirror's source distance, the detector's start
  * time) on a host list of n records whose active photons are
@@ -214,7 +214,8 @@ int mxgd_download_sorted (Marx_Photon_Attr_Type *at, unsigned int n, unsigned in
  * caller's arrays on return, *n_out their number; the store then holds every
  * record and the active list, as after mxgd_upload_aos and the stage.  The
  * copies up, the kernels and the copies down of successive parts of the list
- * overlap.  1: not done, the arrays are not such as mxgd_host_alloc gave. */
+ * overlap.  1: not done, the list is short or its arrays are not such as
+ * mxgd_host_alloc gave. */
 #define MXGD_STAGE_MIRROR 0
 #define MXGD_STAGE_GRATING 1
 #define MXGD_STAGE_DETECT 2

@@ -1588,6 +1588,23 @@ static bool is_pinned (const void *p, size_t bytes)
    return false;
 }
 
+// Lists of fewer photons are copied whole on the library's stream: the second
+// stream's events and the launches of the parts cost there what the overlap
+// saves or more, by a time that varies from process to process.  The drop-in
+// calls (HETG + ACIS-S) on n photons, copied whole and overlapped: n = 100 358
+// us and 365 to 427, 1000 425 and 366 to 470, 2000 459 and 391 to 491, 4000 503
+// and 414 to 513, 8000 617 and 473 to 549, 20000 841 and 625 to 661.
+constexpr unsigned int kOverlapFrom = 4096;
+
+// whether the copies of a list overlap its kernels: a long one, its n records
+// and m list entries in the library's pinned memory
+static bool overlaps (const Marx_Photon_Attr_Type *at, unsigned int n, const unsigned int *index, const double *energies,
+                      unsigned int m)
+{
+   return (n >= kOverlapFrom) && is_pinned (at, (size_t) n * sizeof (Marx_Photon_Attr_Type))
+     && is_pinned (index, (size_t) m * sizeof (uint32_t)) && is_pinned (energies, (size_t) m * sizeof (double));
+}
+
 // the sort of the store's first n energies and its result on their way to
 // the host, on g_stream
 static int queue_energy_sort (unsigned int n, unsigned int *index, double *energies)
@@ -1620,6 +1637,8 @@ int mxgd_download_sorted (Marx_Photon_Attr_Type *at, unsigned int n, unsigned in
    if (mxgd_init ()) return -1;
    if (n > g_n) return fail ("download of %u photons from a store of %u", n, g_n);
    if (n == 0) return 0;
+   if (!overlaps (at, n, index, energies, n))
+     return (mxgd_download_aos (at, n) || mxgd_sort_store_by_energy (n, index, energies)) ? -1 : 0;
    if (ensure_aos (n) || sort_buffers (n) || copy_stream ()) return -1;
    hipLaunchKernelGGL (k_soa_to_aos, dim3 ((n + kBlock - 1) / kBlock), dim3 (kBlock), 0,
                        g_stream, d_aos, g_soa, (uint32_t) n);
@@ -1698,10 +1717,7 @@ int mxgd_stage_on_list (int stage, double arg, unsigned long long seed, Marx_Pho
                         unsigned int *index, double *energies, unsigned int nactive, unsigned int *n_out)
 {
    if (mxgd_init ()) return -1;
-   if ((n == 0) || (nactive > n) || !is_pinned (at, (size_t) n * sizeof (Marx_Photon_Attr_Type))
-       || !is_pinned (index, (size_t) nactive * sizeof (uint32_t))
-       || !is_pinned (energies, (size_t) nactive * sizeof (double)))
-     return 1;
+   if ((nactive > n) || !overlaps (at, n, index, energies, nactive)) return 1;
    g_relay_have = -1;
    if (ensure_capacity (n) || ensure_aos (n) || copy_stream ()) return -1;
    if (n > g_marks_cap)

@@ -72,3 +72,25 @@ def test_pinned_lists_match_plain_ones(gpu, grating, det, n, listed):
             assert np.array_equal(a, b)
     assert np.array_equal(rows[unlisted], before[unlisted])
     assert p.pt.num_sorted < max(n // 4, 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,listed", [(4095, "some"), (4096, "some"), (4097, "all"), (5000, "none")])
+def test_lists_around_the_shortest_that_overlaps(gpu, n, listed):
+    test_pinned_lists_match_plain_ones(gpu, "HETG", "ACIS-S", n, listed)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 4095, 4096, 70_001])
+def test_created_lists_match_plain_ones(gpu, n):
+    t = Tracer(seed=18, GratingType="NONE", DetectorType="NONE", SourceType="POINT", SpectrumType="FLAT", MinEnergy=0.5,
+               MaxEnergy=7.0, DitherModel="INTERNAL", **ON_AXIS)
+    t.init_source(SourceFlux=n / (1.0e4 * t.geometric_area))
+    p = Photons(n)
+    q = Plain(p)
+    made = ctypes.c_uint()
+    assert t.create_photons(p, n) == n
+    check(t.lib.marx_create_photons(t.source, ctypes.pointer(q.pt), n, ctypes.byref(made), None), "create")
+    assert made.value == n and p.pt.num_sorted == q.pt.num_sorted == n
+    for a, b in zip(_views(p), _views(q)):
+        assert np.array_equal(a, b)
